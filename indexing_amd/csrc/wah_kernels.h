@@ -109,8 +109,6 @@ constexpr uint64_t kLongTailMin = 1ull << WAH_LONG_TAIL_MIN_LOG2;
 __host__ __device__ constexpr int tail_waves_per_eu(int items) {
   return items >= 16 ? 4 : kTailWavesPerEU;
 }
-constexpr int kScanItems = 8;
-constexpr int kScanTile = 256 * kScanItems;
 constexpr uint32_t kHistMaxBlocks = 2048;
 // Tile counters: radix launches 0-3 of pair-mode columns, then their tail;
 // radix launches 0-3 of run-mode columns, then their tail.
@@ -289,6 +287,27 @@ struct ScanArgs {
   uint32_t max_resident;
 };
 
+// State of the single-pass scans (wah_scan.hip), one per context: zero before
+// every launch, and zeroed again by the launch's last block.  The status words
+// (kScanStatusWords of them) follow it.
+struct ScanState {
+  uint32_t tiles[kLaneWords];  // per lane: word 0 the tile counter, word 1 its ended blocks
+  uint32_t done;               // lanes whose blocks have all ended
+  uint32_t fault;
+  uint64_t result[2];
+  uint32_t pad[58];
+};
+static_assert(sizeof(ScanState) % 256 == 0, "status words follow at a line boundary");
+// Tiles of the longest scan with room to spare: 2^30 elements in tiles of
+// 8192 at most.
+constexpr uint64_t kScanStatusWords = 1ull << 18;
+struct ScanRun {
+  ScanState* state;
+  uint64_t* status;
+  uint64_t* host;  // page-locked: fault, result[0], result[1] when the launch ends
+  uint32_t cus;    // compute units of the device
+};
+
 uint64_t scan_status_words(uint64_t n);
 
 // Optional hook called between kernel groups of the fused build (timing).
@@ -307,15 +326,17 @@ void launch_chunks(const uint32_t* rids, uint64_t n, uint32_t* chids, uint32_t* 
                    hipStream_t s);
 void launch_fills(const uint32_t* vals, const uint32_t* chids, uint64_t k, uint32_t* fills,
                   hipStream_t s);
-void launch_merge(const ScanArgs& a, const uint32_t* vals, const uint32_t* chids,
+void launch_merge(const ScanRun& a, const uint32_t* vals, const uint32_t* chids,
                   const uint32_t* lits, uint64_t n, uint32_t* ov, uint32_t* oc, uint32_t* ol,
-                  uint64_t* result, hipStream_t s);
-void launch_compact(const ScanArgs& a, const uint32_t* data, const uint32_t* valid, uint64_t n,
-                    int mode, uint32_t* out, uint64_t* result, hipStream_t s);
-void launch_colen(const ScanArgs& a, const uint32_t* vals, const uint32_t* fills, uint64_t k,
+                  hipStream_t s);
+// mode 0: keep data[i] where valid[i] != 0; 1: the nonzero words of the
+// interleaved (data[i], valid[i])
+void launch_compact(const ScanRun& a, const uint32_t* data, const uint32_t* valid, uint64_t n,
+                    int mode, uint32_t* out, hipStream_t s);
+void launch_colen(const ScanRun& a, const uint32_t* vals, const uint32_t* fills, uint64_t k,
                   uint32_t* keys, uint32_t* offsets, uint32_t* lengths,
                   wahgpu_counts_dev* counts, hipStream_t s);
-void launch_scan(const ScanArgs& a, const uint32_t* in, const uint32_t* heads, uint64_t n,
+void launch_scan(const ScanRun& a, const uint32_t* in, const uint32_t* heads, uint64_t n,
                  uint32_t* out, bool segmented, hipStream_t s);
 
 // Query side (wah_query.hip): WAH streams -> row bitmaps -> WAH streams.

@@ -16,8 +16,8 @@
 //   k_tail        sorted items -> chunk ids, OR-merged literals, fills,
 //                 zero-fill removal, word positions, keys and offsets
 //   k_finish      per column: k, lengths[i] = offsets[i+1] - offsets[i], fault
-// Staged kernels (what `phases` runs, one per reference stage) and the scan /
-// compaction primitives reuse the same look-back scheme.
+// The staged kernels (what `phases` runs, one per reference stage) that are
+// scans, and the scan / compaction primitives, are in wah_scan.hip.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -1805,21 +1805,9 @@ __global__ __launch_bounds__(kBlock) void k_finish(const DescHead* __restrict__ 
 }
 
 // ---------------------------------------------------------------------------
-// Staged kernels (one per reference stage) and primitives.
+// Staged kernels that are no scan (one per reference stage); wah_scan.hip holds
+// the others.
 // ---------------------------------------------------------------------------
-// lengths[i] = offsets[i+1] - offsets[i]; the last key runs to L.
-__global__ __launch_bounds__(kBlock) void k_lengths(const uint32_t* __restrict__ offsets,
-                                                    uint32_t* __restrict__ lengths,
-                                                    const wahgpu_counts_dev* __restrict__ counts,
-                                                    uint64_t cap) {
-  const uint64_t K = counts->keycnt < cap ? counts->keycnt : cap, L = counts->length;
-  for (uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x; i < K;
-       i += (uint64_t)gridDim.x * kBlock) {
-    const uint32_t end = (i + 1 < K) ? offsets[i + 1] : (uint32_t)L;
-    lengths[i] = end - offsets[i];
-  }
-}
-
 // Copy the sorted result of column 0 out of the pass buffers (stage API).
 __global__ __launch_bounds__(kBlock) void k_sort_finalize(
     const DescHead* __restrict__ desc, const ColState* __restrict__ cs, const uint32_t* values,
@@ -1855,234 +1843,6 @@ __global__ __launch_bounds__(kBlock) void k_fills(const uint32_t* __restrict__ v
        i += (uint64_t)gridDim.x * kBlock) {
     uint32_t c = chids[i];
     fills[i] = (i > 0 && vals[i] == vals[i - 1]) ? c - chids[i - 1] - 1u : c;
-  }
-}
-
-// Reduce-by-key OR over runs of equal (value, chid), any run length.  The
-// last element of each run writes (value, chid, OR) at index heads-1.
-template <int ITEMS>
-__global__ __launch_bounds__(kBlock) void k_merge(
-    const uint32_t* __restrict__ vals, const uint32_t* __restrict__ chids,
-    const uint32_t* __restrict__ lits, uint64_t n, uint32_t* __restrict__ out_v,
-    uint32_t* __restrict__ out_c, uint32_t* __restrict__ out_l, uint64_t* status,
-    uint32_t num_tiles, uint32_t* tile_counter, uint32_t lanes, uint64_t* result,
-    uint32_t* fault) {
-  constexpr int TILE = kBlock * ITEMS;
-  __shared__ uint64_t s_scan[kWaves];
-  __shared__ uint64_t s_prefix;
-  __shared__ uint32_t s_tile;
-  const int t = threadIdx.x;
-  uint32_t iter = 0;
-  for (;;) {
-    const uint32_t tile = next_tile(tile_counter, lanes, &s_tile, iter);
-    if (tile >= num_tiles) break;
-    const uint64_t g0 = (uint64_t)tile * TILE + (uint64_t)t * ITEMS;
-    uint32_t headmask = 0;
-    uint64_t agg = OpSegOr::identity();
-#pragma unroll
-    for (int i = 0; i < ITEMS; ++i) {
-      uint64_t g = g0 + i;
-      if (g < n) {
-        bool head = g == 0 || vals[g] != vals[g - 1] || chids[g] != chids[g - 1];
-        if (head) headmask |= 1u << i;
-        agg = OpSegOr::combine(agg, ((uint64_t)head << 32) | lits[g]);
-      }
-    }
-    uint64_t tile_agg;
-    uint64_t ex = block_exclusive<OpSegOr>(agg, s_scan, &tile_agg);
-    if (t == 0) s_prefix = lookback64<OpSegOr>(status, tile, tile_agg, fault);
-    __syncthreads();
-    uint64_t run = OpSegOr::combine(s_prefix, ex);
-#pragma unroll
-    for (int i = 0; i < ITEMS; ++i) {
-      uint64_t g = g0 + i;
-      if (g < n) {
-        bool head = (headmask >> i) & 1u;
-        run = OpSegOr::combine(run, ((uint64_t)head << 32) | lits[g]);
-        bool last = g + 1 == n || vals[g + 1] != vals[g] || chids[g + 1] != chids[g];
-        if (last) {
-          uint64_t idx = (run >> 32) - 1;
-          if (idx < n) {
-            out_v[idx] = vals[g];
-            out_c[idx] = chids[g];
-            out_l[idx] = (uint32_t)run;
-          } else {
-            atomicOr(fault, 2u);
-          }
-        }
-      }
-    }
-    if (tile == num_tiles - 1 && t == 0)
-      *result = (OpSegOr::combine(s_prefix, tile_agg) >> 32);
-    __syncthreads();
-  }
-}
-
-// Order-preserving compaction.  Mode 0: keep data[i] where valid[i] != 0
-// (include/stream_compaction.cl:124-160).  Mode 1: the interleaved words
-// (a[i], b[i]) with zero words dropped (fuse_fill_literals).
-template <int ITEMS, int MODE>
-__global__ __launch_bounds__(kBlock) void k_compact(
-    const uint32_t* __restrict__ a, const uint32_t* __restrict__ b, uint64_t n,
-    uint32_t* __restrict__ out, uint64_t* status, uint32_t num_tiles,
-    uint32_t* tile_counter, uint32_t lanes, uint64_t* result, uint32_t* fault) {
-  constexpr int TILE = kBlock * ITEMS;
-  const uint64_t cap = MODE == 0 ? n : 2 * n;
-  __shared__ uint64_t s_scan[kWaves];
-  __shared__ uint64_t s_prefix;
-  __shared__ uint32_t s_tile;
-  const int t = threadIdx.x;
-  uint32_t iter = 0;
-  for (;;) {
-    const uint32_t tile = next_tile(tile_counter, lanes, &s_tile, iter);
-    if (tile >= num_tiles) break;
-    const uint64_t g0 = (uint64_t)tile * TILE + (uint64_t)t * ITEMS;
-    uint64_t cnt = 0;
-#pragma unroll
-    for (int i = 0; i < ITEMS; ++i) {
-      uint64_t g = g0 + i;
-      if (g < n) {
-        if (MODE == 0) cnt += b[g] != 0u;
-        else cnt += (a[g] != 0u) + (b[g] != 0u);
-      }
-    }
-    uint64_t tile_agg;
-    uint64_t ex = block_exclusive<OpAdd>(cnt, s_scan, &tile_agg);
-    if (t == 0) s_prefix = lookback64<OpAdd>(status, tile, tile_agg, fault);
-    __syncthreads();
-    uint64_t pos = s_prefix + ex;
-    if (pos + cnt > cap) {  // never for a consistent scan
-      atomicOr(fault, 2u);
-      cnt = 0;
-      pos = 0;
-    }
-#pragma unroll
-    for (int i = 0; i < ITEMS; ++i) {
-      uint64_t g = g0 + i;
-      if (g < n) {
-        if (cnt == 0) break;
-        if (MODE == 0) {
-          if (b[g] != 0u) out[pos++] = a[g];
-        } else {
-          uint32_t x = a[g], y = b[g];
-          if (x) out[pos++] = x;
-          if (y) out[pos++] = y;
-        }
-      }
-    }
-    if (tile == num_tiles - 1 && t == 0) *result = s_prefix + tile_agg;
-    __syncthreads();
-  }
-}
-
-// compute_column_length over merged entries (values, fills): keys at value
-// changes, offsets = exclusive scan of (1 + (fill != 0)).
-template <int ITEMS>
-__global__ __launch_bounds__(kBlock) void k_colen(
-    const uint32_t* __restrict__ vals, const uint32_t* __restrict__ fills, uint64_t k,
-    uint32_t* __restrict__ out_keys, uint32_t* __restrict__ out_offsets, uint64_t* status,
-    uint32_t num_tiles, uint32_t* tile_counter, uint32_t lanes,
-    wahgpu_counts_dev* __restrict__ counts, uint32_t* fault) {
-  constexpr int TILE = kBlock * ITEMS;
-  __shared__ uint64_t s_scan[kWaves];
-  __shared__ uint64_t s_prefix;
-  __shared__ uint32_t s_tile;
-  const int t = threadIdx.x;
-  uint32_t iter = 0;
-  for (;;) {
-    const uint32_t tile = next_tile(tile_counter, lanes, &s_tile, iter);
-    if (tile >= num_tiles) break;
-    const uint64_t g0 = (uint64_t)tile * TILE + (uint64_t)t * ITEMS;
-    uint32_t W = 0, KH = 0;
-#pragma unroll
-    for (int i = 0; i < ITEMS; ++i) {
-      uint64_t g = g0 + i;
-      if (g < k) {
-        W += 1u + (fills[g] != 0u);
-        KH += (g == 0 || vals[g] != vals[g - 1]);
-      }
-    }
-    uint64_t tile_agg;
-    uint64_t ex = block_exclusive<OpAdd>(((uint64_t)KH << 31) | W, s_scan, &tile_agg);
-    if (t == 0) s_prefix = lookback64<OpAdd>(status, tile, tile_agg, fault);
-    __syncthreads();
-    const uint64_t pre = s_prefix + ex;
-    uint32_t pos = (uint32_t)(pre & 0x7FFFFFFFu);
-    uint32_t kidx = (uint32_t)(pre >> 31);
-#pragma unroll
-    for (int i = 0; i < ITEMS; ++i) {
-      uint64_t g = g0 + i;
-      if (g < k) {
-        if (g == 0 || vals[g] != vals[g - 1]) {
-          if (kidx < k) {
-            out_keys[kidx] = vals[g];
-            out_offsets[kidx] = pos;
-          } else {
-            atomicOr(fault, 2u);
-          }
-          ++kidx;
-        }
-        pos += 1u + (fills[g] != 0u);
-      }
-    }
-    if (tile == num_tiles - 1 && t == 0) {
-      uint64_t tot = s_prefix + tile_agg;
-      counts->length = tot & 0x7FFFFFFFu;
-      counts->keycnt = tot >> 31;
-    }
-    __syncthreads();
-  }
-}
-
-// Exclusive uint32 sum scan (include/scan.cl) and segmented inclusive sum
-// scan (include/segmented_scan.cl), single pass with look-back.
-template <int ITEMS, bool SEGMENTED>
-__global__ __launch_bounds__(kBlock) void k_scan(
-    const uint32_t* __restrict__ in, const uint32_t* __restrict__ heads, uint64_t n,
-    uint32_t* __restrict__ out, uint64_t* status, uint32_t num_tiles,
-    uint32_t* tile_counter, uint32_t lanes, uint32_t* fault) {
-  constexpr int TILE = kBlock * ITEMS;
-  __shared__ uint64_t s_scan[kWaves];
-  __shared__ uint64_t s_prefix;
-  __shared__ uint32_t s_tile;
-  using Op = typename std::conditional<SEGMENTED, OpSegAdd, OpAdd32>::type;
-  const int t = threadIdx.x;
-  uint32_t iter = 0;
-  for (;;) {
-    const uint32_t tile = next_tile(tile_counter, lanes, &s_tile, iter);
-    if (tile >= num_tiles) break;
-    const uint64_t g0 = (uint64_t)tile * TILE + (uint64_t)t * ITEMS;
-    uint64_t agg = Op::identity();
-#pragma unroll
-    for (int i = 0; i < ITEMS; ++i) {
-      uint64_t g = g0 + i;
-      if (g < n) {
-        uint64_t e = in[g];
-        if (SEGMENTED) e |= (uint64_t)(g == 0 || heads[g] != 0u) << 32;
-        agg = Op::combine(agg, e);
-      }
-    }
-    uint64_t tile_agg;
-    uint64_t ex = block_exclusive<Op>(agg, s_scan, &tile_agg);
-    if (t == 0) s_prefix = lookback64<Op>(status, tile, tile_agg, fault);
-    __syncthreads();
-    uint64_t run = Op::combine(s_prefix, ex);
-#pragma unroll
-    for (int i = 0; i < ITEMS; ++i) {
-      uint64_t g = g0 + i;
-      if (g < n) {
-        uint64_t e = in[g];
-        if (SEGMENTED) {
-          e |= (uint64_t)(g == 0 || heads[g] != 0u) << 32;
-          run = Op::combine(run, e);
-          out[g] = (uint32_t)run;
-        } else {
-          out[g] = (uint32_t)run;
-          run = Op::combine(run, e);
-        }
-      }
-    }
-    __syncthreads();
   }
 }
 
@@ -2251,8 +2011,6 @@ void launch_rank_selftest(uint32_t* ok, hipStream_t s) {
   hipLaunchKernelGGL(k_rank_selftest, dim3(64), dim3(256), 0, s, ok);
 }
 
-uint64_t scan_status_words(uint64_t n) { return (n + kScanTile - 1) / kScanTile; }
-
 static uint32_t grid_for(uint64_t n) {
   uint64_t g = (n + kBlock - 1) / kBlock;
   if (g > 8192) g = 8192;
@@ -2274,61 +2032,6 @@ void launch_fills(const uint32_t* vals, const uint32_t* chids, uint64_t k, uint3
                   hipStream_t s) {
   if (!k) return;
   hipLaunchKernelGGL(k_fills, dim3(grid_for(k)), dim3(kBlock), 0, s, vals, chids, k, fills);
-}
-
-static uint32_t scan_grid(uint64_t n, uint32_t max_resident, uint32_t* tiles_out) {
-  uint32_t tiles = (uint32_t)((n + kScanTile - 1) / kScanTile);
-  *tiles_out = tiles;
-  return tiles < max_resident ? tiles : max_resident;
-}
-
-void launch_merge(const ScanArgs& a, const uint32_t* vals, const uint32_t* chids,
-                  const uint32_t* lits, uint64_t n, uint32_t* ov, uint32_t* oc, uint32_t* ol,
-                  uint64_t* result, hipStream_t s) {
-  uint32_t tiles, grid = scan_grid(n, a.max_resident, &tiles);
-  if (!grid) return;
-  hipLaunchKernelGGL(k_merge<kScanItems>, dim3(grid), dim3(kBlock), 0, s, vals, chids, lits, n,
-                     ov, oc, ol, a.status, tiles, a.tile_counter, tile_lanes(grid), result,
-                     a.fault);
-}
-
-void launch_compact(const ScanArgs& a, const uint32_t* data, const uint32_t* valid, uint64_t n,
-                    int mode, uint32_t* out, uint64_t* result, hipStream_t s) {
-  uint32_t tiles, grid = scan_grid(n, a.max_resident, &tiles);
-  if (!grid) return;
-  if (mode == 0)
-    hipLaunchKernelGGL((k_compact<kScanItems, 0>), dim3(grid), dim3(kBlock), 0, s, data, valid,
-                       n, out, a.status, tiles, a.tile_counter, tile_lanes(grid), result,
-                       a.fault);
-  else
-    hipLaunchKernelGGL((k_compact<kScanItems, 1>), dim3(grid), dim3(kBlock), 0, s, data, valid,
-                       n, out, a.status, tiles, a.tile_counter, tile_lanes(grid), result,
-                       a.fault);
-}
-
-void launch_colen(const ScanArgs& a, const uint32_t* vals, const uint32_t* fills, uint64_t k,
-                  uint32_t* keys, uint32_t* offsets, uint32_t* lengths,
-                  wahgpu_counts_dev* counts, hipStream_t s) {
-  uint32_t tiles, grid = scan_grid(k, a.max_resident, &tiles);
-  if (grid)
-    hipLaunchKernelGGL(k_colen<kScanItems>, dim3(grid), dim3(kBlock), 0, s, vals, fills, k, keys,
-                       offsets, a.status, tiles, a.tile_counter, tile_lanes(grid), counts,
-                       a.fault);
-  uint32_t lg = grid_for(k);
-  if (lg > 1024) lg = 1024;
-  hipLaunchKernelGGL(k_lengths, dim3(lg), dim3(kBlock), 0, s, offsets, lengths, counts, k);
-}
-
-void launch_scan(const ScanArgs& a, const uint32_t* in, const uint32_t* heads, uint64_t n,
-                 uint32_t* out, bool segmented, hipStream_t s) {
-  uint32_t tiles, grid = scan_grid(n, a.max_resident, &tiles);
-  if (!grid) return;
-  if (segmented)
-    hipLaunchKernelGGL((k_scan<kScanItems, true>), dim3(grid), dim3(kBlock), 0, s, in, heads, n,
-                       out, a.status, tiles, a.tile_counter, tile_lanes(grid), a.fault);
-  else
-    hipLaunchKernelGGL((k_scan<kScanItems, false>), dim3(grid), dim3(kBlock), 0, s, in, heads, n,
-                       out, a.status, tiles, a.tile_counter, tile_lanes(grid), a.fault);
 }
 
 }  // namespace wah

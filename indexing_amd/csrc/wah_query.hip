@@ -367,7 +367,7 @@ __global__ __launch_bounds__(kBlock) void k_q_enc_write(const uint32_t* __restri
 
 // ---- launchers ---------------------------------------------------------------
 
-uint64_t decode_status_words(uint64_t len) { return (len + kDecTile - 1) / kDecTile + 1; }
+uint64_t scan_status_words(uint64_t n) { return (n + kDecTile - 1) / kDecTile; }
 uint64_t encode_tiles(uint64_t nrows) {
   const uint64_t chunks = (nrows + 30) / 31;
   return (chunks + kEncTile - 1) / kEncTile;

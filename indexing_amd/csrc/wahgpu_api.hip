@@ -20,6 +20,7 @@
 
 using wah::BuildArgs;
 using wah::ScanArgs;
+using wah::ScanRun;
 
 struct wahgpu_ctx {
   int device = 0;
@@ -33,6 +34,10 @@ struct wahgpu_ctx {
   uint32_t max_resident = 1024;
   std::string err;
   wahgpu_counts* pinned_counts = nullptr;  // host-pinned landing slot
+  // state of the single-pass scans: zero between launches (see ScanState)
+  wah::ScanState* scan_state = nullptr;
+  uint64_t* scan_host = nullptr;  // host-pinned: fault and results of a scan
+  uint32_t cus = 256;
   // per-kernel timing (wahgpu_timing_begin/end)
   std::vector<hipEvent_t> tev;  // max_calls x (WAHGPU_TIMING_GROUPS + 1)
   uint32_t tmax = 0, tcalls = 0;
@@ -353,6 +358,25 @@ int read_scan_result(wahgpu_ctx* c, const uint32_t* header, uint64_t* out) {
   return WAHGPU_OK;
 }
 
+// The context's scan state, for launches on its stream (one after another).
+// Results land in scan_host; a launch of no elements writes nothing, so they
+// start at zero.
+ScanRun scan_run(wahgpu_ctx* c) {
+  memset(c->scan_host, 0, 3 * sizeof(uint64_t));
+  return ScanRun{c->scan_state, reinterpret_cast<uint64_t*>(c->scan_state + 1), c->scan_host,
+                 c->cus};
+}
+// Waits for the stream and reads the result of its last scan.
+int scan_result(wahgpu_ctx* c, uint64_t* out) {
+  HIPCHK(c, hipStreamSynchronize(c->stream));
+  const volatile uint64_t* h = c->scan_host;
+  if (h[0])
+    return fail(c, WAHGPU_EHIP, "kernel reported fault " + std::to_string(h[0]) +
+                                    " (look-back wait gave up or index out of range)");
+  *out = h[1];
+  return WAHGPU_OK;
+}
+
 // Events bracketing phases; elapsed microseconds between consecutive marks.
 struct Marks {
   hipEvent_t ev[12];
@@ -472,6 +496,14 @@ int wahgpu_create(wahgpu_ctx** out, int device_ordinal, uint64_t arena_bytes) {
     return WAHGPU_EHIP;
   }
   c->stream = c->own_stream;
+  const uint64_t scan_bytes = sizeof(wah::ScanState) + wah::kScanStatusWords * 8;
+  if (hipHostMalloc(reinterpret_cast<void**>(&c->scan_host), 64, hipHostMallocDefault) != hipSuccess ||
+      hipMalloc(&c->scan_state, scan_bytes) != hipSuccess) {
+    (void)hipGetLastError();
+    wahgpu_destroy(c);
+    return WAHGPU_EHIP;
+  }
+  wah::launch_fill32(reinterpret_cast<uint32_t*>(c->scan_state), scan_bytes / 4, 0, c->stream);
   if (noalloc_lookup(c, device_ordinal) != WAHGPU_OK) {
     (void)hipGetLastError();
     wahgpu_destroy(c);
@@ -479,7 +511,7 @@ int wahgpu_create(wahgpu_ctx** out, int device_ordinal, uint64_t arena_bytes) {
   }
   hipDeviceProp_t prop;
   if (hipGetDeviceProperties(&prop, device_ordinal) == hipSuccess)
-    c->max_resident = (uint32_t)prop.multiProcessorCount * 4u;
+    c->cus = (uint32_t)prop.multiProcessorCount, c->max_resident = c->cus * 4u;
   // Radix ranking: LDS fetch-add when the device ranks same-address lanes in
   // lane order (checked here), else the ballot match.  WAHGPU_RANK=match or
   // =atomic overrides (the latter still requires the check to pass).
@@ -526,6 +558,8 @@ void wahgpu_destroy(wahgpu_ctx* c) {
   if (c->switch_ev) (void)hipEventDestroy(c->switch_ev);
   if (c->desc_stage) (void)hipHostFree(c->desc_stage);
   if (c->arena) (void)hipFree(c->arena);
+  if (c->scan_state) (void)hipFree(c->scan_state);
+  if (c->scan_host) (void)hipHostFree(c->scan_host);
   if (c->pinned_counts) (void)hipHostFree(c->pinned_counts);
   if (c->own_stream) (void)hipStreamDestroy(c->own_stream);
   delete c;
@@ -1283,7 +1317,7 @@ int wahgpu_build_staged(wahgpu_ctx* c, const uint32_t* values, uint64_t n, uint3
   HIPCHK(c, hipSetDevice(c->device));
   uint64_t nn = n ? n : 1;
   uint64_t bytes = build_scratch_bytes(caps_one(n, shape_for(c, n))) + align_up(nn * 4) * 12 + align_up(2 * nn * 4) +
-                   align_up(sizeof(wahgpu_counts)) + 4 * scan_scratch_bytes(2 * nn);
+                   align_up(sizeof(wahgpu_counts)) + 4 * scan_scratch_bytes(2 * nn);  // fixed arenas keep their limit
   rc = arena_reserve(c, bytes);
   if (rc) return rc;
   auto t0 = std::chrono::steady_clock::now();
@@ -1304,7 +1338,6 @@ int wahgpu_build_staged(wahgpu_ctx* c, const uint32_t* values, uint64_t n, uint3
   uint32_t* o_lengths = take<uint32_t>(c, nn);
   uint32_t* index = take<uint32_t>(c, 2 * nn);
   wahgpu_counts* d_counts = take<wahgpu_counts>(c, 1);
-  ScanScratch sm = carve_scan(c, nn), sf = carve_scan(c, 2 * nn), sc = carve_scan(c, nn);
   Marks m;
   m.init(times != nullptr);
   m.mark(c->stream);  // 0
@@ -1327,12 +1360,11 @@ int wahgpu_build_staged(wahgpu_ctx* c, const uint32_t* values, uint64_t n, uint3
     wah::launch_chunks(s_rids, n, chids, lits, c->stream);
     LAUNCHCHK(c);
     m.mark(c->stream);  // 3 chunks + literals
-    wah::launch_fill32(sm.base, sm.words, 0, c->stream);
-    wah::launch_merge(sm.args, s_keys, chids, lits, n, mv, mc, ml, sm.result, c->stream);
+    wah::launch_merge(scan_run(c), s_keys, chids, lits, n, mv, mc, ml, c->stream);
     LAUNCHCHK(c);
   }
   uint64_t k = 0;
-  rc = read_scan_result(c, sm.header, &k);  // k sizes the next launches (src/phases.cpp:890-903)
+  rc = scan_result(c, &k);  // k sizes the next launches (src/phases.cpp:890-903)
   if (rc) return rc;
   m.mark(c->stream);  // 4 merge
   {
@@ -1340,23 +1372,21 @@ int wahgpu_build_staged(wahgpu_ctx* c, const uint32_t* values, uint64_t n, uint3
     wah::launch_fills(mv, mc, k, fills, c->stream);
     LAUNCHCHK(c);
     m.mark(c->stream);  // 5 fills
-    wah::launch_fill32(sf.base, sf.words, 0, c->stream);
-    wah::launch_compact(sf.args, fills, ml, k, 1, index, sf.result, c->stream);
+    wah::launch_compact(scan_run(c), fills, ml, k, 1, index, c->stream);
     LAUNCHCHK(c);
   }
   uint64_t L = 0;
-  rc = read_scan_result(c, sf.header, &L);
+  rc = scan_result(c, &L);
   if (rc) return rc;
   m.mark(c->stream);  // 6 fuse
   {
     ORDERED(c);
-    wah::launch_fill32(sc.base, sc.words, 0, c->stream);
-    wah::launch_colen(sc.args, mv, fills, k, o_keys, o_offsets, o_lengths, d_counts, c->stream);
+    wah::launch_colen(scan_run(c), mv, fills, k, o_keys, o_offsets, o_lengths, d_counts, c->stream);
     LAUNCHCHK(c);
   }
   wahgpu_counts cc;
   uint64_t unused;
-  rc = read_scan_result(c, sc.header, &unused);  // fault word of the column kernel
+  rc = scan_result(c, &unused);  // fault word of the column kernel
   if (rc) return rc;
   rc = read_counts(c, d_counts, &cc);
   if (rc) return rc;
@@ -1440,16 +1470,14 @@ int wahgpu_merge_lit_by_val_chids(wahgpu_ctx* c, const uint32_t* d_values,
   int rc = check_n(c, n, 0);
   if (rc) return rc;
   HIPCHK(c, hipSetDevice(c->device));
-  rc = arena_reserve(c, scan_scratch_bytes(n));
+  rc = arena_reserve(c, scan_scratch_bytes(n));  // fixed arenas keep their limit
   if (rc) return rc;
-  ScanScratch s = carve_scan(c, n);
   ORDERED(c);
-  wah::launch_fill32(s.base, s.words, 0, c->stream);
-  wah::launch_merge(s.args, d_values, d_chids, d_lits, n, d_values_out, d_chids_out, d_lits_out,
-                    s.result, c->stream);
+  wah::launch_merge(scan_run(c), d_values, d_chids, d_lits, n, d_values_out, d_chids_out,
+                    d_lits_out, c->stream);
   LAUNCHCHK(c);
   order_guard_.end();  // no host wait holds the device order
-  return read_scan_result(c, s.header, k);
+  return scan_result(c, k);
 }
 
 int wahgpu_produce_fills(wahgpu_ctx* c, const uint32_t* d_values, const uint32_t* d_chids,
@@ -1469,15 +1497,13 @@ int wahgpu_fuse_fill_literals(wahgpu_ctx* c, const uint32_t* d_fills, const uint
   int rc = check_n(c, k, 0);
   if (rc) return rc;
   HIPCHK(c, hipSetDevice(c->device));
-  rc = arena_reserve(c, scan_scratch_bytes(k));
+  rc = arena_reserve(c, scan_scratch_bytes(k));  // fixed arenas keep their limit
   if (rc) return rc;
-  ScanScratch s = carve_scan(c, k);
   ORDERED(c);
-  wah::launch_fill32(s.base, s.words, 0, c->stream);
-  wah::launch_compact(s.args, d_fills, d_lits, k, 1, d_index, s.result, c->stream);
+  wah::launch_compact(scan_run(c), d_fills, d_lits, k, 1, d_index, c->stream);
   LAUNCHCHK(c);
   order_guard_.end();  // no host wait holds the device order
-  return read_scan_result(c, s.header, index_length);
+  return scan_result(c, index_length);
 }
 
 int wahgpu_compute_column_length(wahgpu_ctx* c, const uint32_t* d_values,
@@ -1489,26 +1515,16 @@ int wahgpu_compute_column_length(wahgpu_ctx* c, const uint32_t* d_values,
   int rc = check_n(c, k, 0);
   if (rc) return rc;
   HIPCHK(c, hipSetDevice(c->device));
+  // fixed arenas keep their limit
   rc = arena_reserve(c, scan_scratch_bytes(k) + align_up(sizeof(wahgpu_counts)));
   if (rc) return rc;
-  ScanScratch s = carve_scan(c, k);
   wahgpu_counts* d_counts = take<wahgpu_counts>(c, 1);
-  wah::launch_fill32(s.base, s.words, 0, c->stream);
-  wah::launch_fill32(reinterpret_cast<uint32_t*>(d_counts), sizeof(wahgpu_counts) / 4, 0,
-                     c->stream);
   ORDERED(c);
-  wah::launch_colen(s.args, d_values, d_fills, k, d_keys, d_offsets, d_lengths, d_counts,
+  wah::launch_colen(scan_run(c), d_values, d_fills, k, d_keys, d_offsets, d_lengths, d_counts,
                     c->stream);
   LAUNCHCHK(c);
-  wahgpu_counts cc;
-  uint64_t unused;
   order_guard_.end();  // no host wait holds the device order
-  rc = read_scan_result(c, s.header, &unused);
-  if (rc) return rc;
-  rc = read_counts(c, d_counts, &cc);
-  if (rc) return rc;
-  *keycnt = cc.keycnt;
-  return WAHGPU_OK;
+  return scan_result(c, keycnt);
 }
 
 int wahgpu_stream_compaction(wahgpu_ctx* c, const uint32_t* d_data, const uint32_t* d_valid,
@@ -1518,15 +1534,13 @@ int wahgpu_stream_compaction(wahgpu_ctx* c, const uint32_t* d_data, const uint32
   int rc = check_n(c, n, 0);
   if (rc) return rc;
   HIPCHK(c, hipSetDevice(c->device));
-  rc = arena_reserve(c, scan_scratch_bytes(n));
+  rc = arena_reserve(c, scan_scratch_bytes(n));  // fixed arenas keep their limit
   if (rc) return rc;
-  ScanScratch s = carve_scan(c, n);
   ORDERED(c);
-  wah::launch_fill32(s.base, s.words, 0, c->stream);
-  wah::launch_compact(s.args, d_data, d_valid, n, 0, d_out, s.result, c->stream);
+  wah::launch_compact(scan_run(c), d_data, d_valid, n, 0, d_out, c->stream);
   LAUNCHCHK(c);
   order_guard_.end();  // no host wait holds the device order
-  return read_scan_result(c, s.header, count);
+  return scan_result(c, count);
 }
 
 int wahgpu_exclusive_scan(wahgpu_ctx* c, const uint32_t* d_in, uint64_t n, uint32_t* d_out) {
@@ -1535,12 +1549,10 @@ int wahgpu_exclusive_scan(wahgpu_ctx* c, const uint32_t* d_in, uint64_t n, uint3
   int rc = check_n(c, n, 0);
   if (rc) return rc;
   HIPCHK(c, hipSetDevice(c->device));
-  rc = arena_reserve(c, scan_scratch_bytes(n));
+  rc = arena_reserve(c, scan_scratch_bytes(n));  // fixed arenas keep their limit
   if (rc) return rc;
-  ScanScratch s = carve_scan(c, n);
   ORDERED(c);
-  wah::launch_fill32(s.base, s.words, 0, c->stream);
-  wah::launch_scan(s.args, d_in, nullptr, n, d_out, false, c->stream);
+  wah::launch_scan(scan_run(c), d_in, nullptr, n, d_out, false, c->stream);
   LAUNCHCHK(c);
   return WAHGPU_OK;
 }
@@ -1552,12 +1564,10 @@ int wahgpu_segmented_inclusive_scan(wahgpu_ctx* c, const uint32_t* d_in, const u
   int rc = check_n(c, n, 0);
   if (rc) return rc;
   HIPCHK(c, hipSetDevice(c->device));
-  rc = arena_reserve(c, scan_scratch_bytes(n));
+  rc = arena_reserve(c, scan_scratch_bytes(n));  // fixed arenas keep their limit
   if (rc) return rc;
-  ScanScratch s = carve_scan(c, n);
   ORDERED(c);
-  wah::launch_fill32(s.base, s.words, 0, c->stream);
-  wah::launch_scan(s.args, d_in, d_heads, n, d_out, true, c->stream);
+  wah::launch_scan(scan_run(c), d_in, d_heads, n, d_out, true, c->stream);
   LAUNCHCHK(c);
   return WAHGPU_OK;
 }
