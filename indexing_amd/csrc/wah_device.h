@@ -187,32 +187,6 @@ struct OpAdd {
   static __device__ __forceinline__ uint64_t identity() { return 0; }
   static __device__ __forceinline__ uint64_t combine(uint64_t a, uint64_t b) { return a + b; }
 };
-// uint32 sum that wraps mod 2^32 (the reference's uint32 scans).
-struct OpAdd32 {
-  static __device__ __forceinline__ uint64_t identity() { return 0; }
-  static __device__ __forceinline__ uint64_t combine(uint64_t a, uint64_t b) {
-    return (uint32_t)(a + b);
-  }
-};
-// Segmented OR: payload = heads (30 bits) << 32 | or-since-last-head (32).
-struct OpSegOr {
-  static __device__ __forceinline__ uint64_t identity() { return 0; }
-  static __device__ __forceinline__ uint64_t combine(uint64_t a, uint64_t b) {
-    uint64_t h = (a >> 32) + (b >> 32);
-    uint32_t x = (b >> 32) ? (uint32_t)b : ((uint32_t)a | (uint32_t)b);
-    return (h << 32) | x;
-  }
-};
-// Segmented sum: payload = has-head (bit 32) | sum-since-last-head (32).
-struct OpSegAdd {
-  static __device__ __forceinline__ uint64_t identity() { return 0; }
-  static __device__ __forceinline__ uint64_t combine(uint64_t a, uint64_t b) {
-    bool hb = (b >> 32) & 1u;
-    uint32_t x = hb ? (uint32_t)b : (uint32_t)a + (uint32_t)b;
-    return ((uint64_t)(((a >> 32) | (b >> 32)) & 1u) << 32) | x;
-  }
-};
-
 // Inclusive scan within a wave.
 template <class Op>
 __device__ __forceinline__ uint64_t wave_inclusive(uint64_t x) {
@@ -248,29 +222,10 @@ __device__ __forceinline__ uint64_t block_exclusive(uint64_t x, uint64_t* smem,
   return Op::combine(before, exc);
 }
 
-// Bounded wait on a look-back status word: returns the word once its flag is
-// set, or 0 after kSpinLimit polls (then *fault is raised and the caller
-// proceeds with a zero contribution, so every wave still finishes).
+// Every wait on a look-back status is bounded: after kSpinLimit polls it raises
+// *fault and proceeds with a zero contribution, so every wave still finishes.
 // Once any wait of the launch has given up, the others stop waiting too.
 constexpr uint32_t kSpinLimit = 1u << 18;
-
-template <class T, int SHIFT>
-__device__ __forceinline__ T wait_status_t(T* p, uint32_t* fault) {
-  T s;
-  for (uint32_t i = 0; i < kSpinLimit; ++i) {
-    if ((s = ld_agent(p)) >> SHIFT) return s;
-    if ((i & 1023u) == 1023u && ld_agent(fault)) return 0;
-    __builtin_amdgcn_s_sleep(1);
-  }
-  atomicOr(fault, 1u);
-  return 0;
-}
-__device__ __forceinline__ uint32_t wait_status(uint32_t* p, uint32_t* fault) {
-  return wait_status_t<uint32_t, 30>(p, fault);
-}
-__device__ __forceinline__ uint64_t wait_status(uint64_t* p, uint32_t* fault) {
-  return wait_status_t<uint64_t, 62>(p, fault);
-}
 
 // Exclusive prefix of one digit over the preceding tiles, reading up to
 // WAH_LOOKAHEAD predecessors per round trip (32-bit words: flag << 30 | count).
@@ -376,30 +331,6 @@ __device__ __forceinline__ void lookback_digits4(uint32_t* status, uint32_t tile
       __builtin_amdgcn_s_sleep(1);
     }
   }
-}
-
-// Decoupled look-back over 64-bit status words (flag << 62 | payload).
-// Called by one thread of the tile; publishes the tile's aggregate first so
-// later tiles can proceed, then walks back to the nearest inclusive prefix,
-// publishes its own prefix and returns the exclusive prefix of the tile.
-template <class Op>
-__device__ uint64_t lookback64(uint64_t* status, uint32_t tile, uint64_t agg, uint32_t* fault) {
-  constexpr uint64_t kMask = (1ull << 62) - 1;
-  if (tile == 0) {
-    st_agent(&status[0], ((uint64_t)kFlagPrefix << 62) | (agg & kMask));
-    return Op::identity();
-  }
-  st_agent(&status[tile], ((uint64_t)kFlagAgg << 62) | (agg & kMask));
-  uint64_t acc = Op::identity();
-  int64_t t = (int64_t)tile - 1;
-  while (t >= 0) {
-    uint64_t s = wait_status(&status[t], fault);
-    acc = Op::combine(s & kMask, acc);
-    if ((s >> 62) != kFlagAgg) break;  // prefix found (or gave up)
-    --t;
-  }
-  st_agent(&status[tile], ((uint64_t)kFlagPrefix << 62) | (Op::combine(acc, agg) & kMask));
-  return acc;
 }
 
 // Look-back for commutative sums, run by a whole wave: each round reads the

@@ -280,35 +280,28 @@ __host__ __device__ inline uint32_t hist_chunks_of(uint64_t n) {
   return (uint32_t)((n + kHistChunk - 1) / kHistChunk);
 }
 
-struct ScanArgs {
-  uint64_t* status;        // scan_status_words(n), zeroed
-  uint32_t* tile_counter;  // kLaneWords tile-counter lanes, zeroed
-  uint32_t* fault;         // zeroed; nonzero after a failed wait / bad index
-  uint32_t max_resident;
-};
-
 // State of the single-pass scans (wah_scan.hip), one per context: zero before
 // every launch, and zeroed again by the launch's last block.  The status words
 // (kScanStatusWords of them) follow it.
 struct ScanState {
-  uint32_t tiles[kLaneWords];  // per lane: word 0 the tile counter, word 1 its ended blocks
+  uint32_t tiles[kLaneWords];  // per lane: word 0 the tile counter, word 1 its ended
+                               // blocks, words 2 and 3 a maximum (the result's, if any)
   uint32_t done;               // lanes whose blocks have all ended
   uint32_t fault;
-  uint64_t result[2];
-  uint32_t pad[58];
+  uint64_t result;
+  uint64_t range[4];           // a range query's keys and words (k_q_range)
+  uint32_t pad[52];
 };
 static_assert(sizeof(ScanState) % 256 == 0, "status words follow at a line boundary");
-// Tiles of the longest scan with room to spare: 2^30 elements in tiles of
-// 8192 at most.
-constexpr uint64_t kScanStatusWords = 1ull << 18;
+// Tiles of the longest scan: two streams of 2^32 WAH words in decode tiles of
+// 4096.
+constexpr uint64_t kScanStatusWords = 1ull << 21;
 struct ScanRun {
   ScanState* state;
   uint64_t* status;
-  uint64_t* host;  // page-locked: fault, result[0], result[1] when the launch ends
+  uint64_t* host;  // page-locked: fault and result when the launch ends
   uint32_t cus;    // compute units of the device
 };
-
-uint64_t scan_status_words(uint64_t n);
 
 // Optional hook called between kernel groups of the fused build (timing).
 struct LaunchHook {
@@ -339,17 +332,23 @@ void launch_colen(const ScanRun& a, const uint32_t* vals, const uint32_t* fills,
 void launch_scan(const ScanRun& a, const uint32_t* in, const uint32_t* heads, uint64_t n,
                  uint32_t* out, bool segmented, hipStream_t s);
 
-// Query side (wah_query.hip): WAH streams -> row bitmaps -> WAH streams.
-void launch_decode(const ScanArgs& s, const uint32_t* words, const uint32_t* heads,
-                   uint64_t len, uint32_t* bitmap, uint64_t nrows, uint64_t* last_row,
+// Query side (wah_query.hip): WAH streams -> row bitmaps -> WAH streams.  The
+// bitmaps a decode ORs into are zero before it.
+struct DecodeStream {
+  const uint32_t* words;
+  uint64_t len;
+  uint32_t* bitmap;
+};
+// The result is the row after the last set row of stream a.
+void launch_decode(const ScanRun& s, const DecodeStream& a, const DecodeStream& b, uint64_t nrows,
                    hipStream_t st);
-void launch_mark_heads(const uint32_t* offsets, uint64_t a, uint64_t b, uint64_t w0,
-                       uint32_t* heads, hipStream_t st);
-void launch_key_range(const uint32_t* keys, const uint32_t* offsets, const uint32_t* lengths,
-                      uint64_t keycnt, uint32_t lo, uint32_t hi, uint64_t* range, hipStream_t st);
-uint64_t encode_tiles(uint64_t nrows);
-void launch_encode(const uint32_t* a, const uint32_t* b, int op, uint64_t nrows,
-                   uint64_t* tile_sum, uint32_t* out, uint64_t cap, uint64_t* len,
-                   hipStream_t st);
+// Zeroes the bitmap and decodes the keys in [lo, hi] into it; host[3] = keys,
+// host[4] = words of the range.
+void launch_range(const ScanRun& s, const uint32_t* keys, const uint32_t* offsets,
+                  const uint32_t* lengths, uint64_t keycnt, const uint32_t* words, uint32_t lo,
+                  uint32_t hi, uint32_t* bitmap, uint64_t nrows, hipStream_t st);
+// The result is the words of the stream (b null: of bitmap a alone).
+void launch_encode(const ScanRun& s, const uint32_t* a, const uint32_t* b, int op, uint64_t nrows,
+                   uint32_t* out, uint64_t cap, hipStream_t st);
 
 }  // namespace wah

@@ -12,36 +12,83 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
-#include "wah_device.h"
-#include "wah_kernels.h"
+#include <type_traits>
+
+#include "wah_scan.h"
 
 namespace wah {
 
 namespace {
 
-constexpr int kDecItems = 8;
-constexpr int kDecTile = kBlock * kDecItems;
-constexpr int kEncItems = 8;                  // chunks per thread
-constexpr int kEncTile = kBlock * kEncItems;  // chunks per tile
+// Decode tiles of 4096 words at two blocks per CU: two million words (2^27 rows
+// at density 0.01) take 18.9 us, 2048-word tiles 21.5, 8192-word ones 19.6, and
+// two streams of 6000 words 9.3, 10.1 and 14.8 us (a lane writes its words one
+// after another, so a short stream wants more lanes).
+constexpr int kDecRows = 2;
+constexpr uint32_t kDecTile = kScanTileOf<kDecRows>;  // words per decode tile
+// Resident blocks per CU.
+constexpr int kDecBlocks = 2;
+constexpr int kEncBlocks = 4;  // 20.2 us for 2^27 rows; 2 and 3 blocks 24.5, 23.1 us
+constexpr int query_waves_per_eu(int blocks) { return blocks * kScanWaves / 4; }
 
 __device__ __forceinline__ uint32_t word_chunks(uint32_t w) {
   return (w & 0x80000000u) ? 1u : (w & 0x3FFFFFFFu);
 }
 
-// ORs the 31 bits `bits` (bit b = row row0 + b) into the bitmap, dropping
-// rows at or past nrows.
-__device__ __forceinline__ void or_bits31(uint32_t* bitmap, uint64_t nrows, uint64_t row0,
-                                          uint32_t bits) {
-  if (row0 >= nrows || bits == 0) return;
+// ORs the payload of a literal at chunk c into the bitmap, dropping rows at or
+// past nrows (chunks = chunks of nrows rows; rows are below 2^32).
+__device__ __forceinline__ void or_literal(uint32_t* bitmap, uint64_t nrows, uint32_t chunks,
+                                           uint32_t c, uint32_t bits) {
+  if (c >= chunks) return;
+  const uint32_t row0 = 31u * c;
   if (nrows - row0 < 31) bits &= (1u << (uint32_t)(nrows - row0)) - 1u;
-  if (!bits) return;
-  const uint64_t wi = row0 >> 5;
-  const uint32_t sh = (uint32_t)(row0 & 31u);
+  const uint32_t wi = row0 >> 5, sh = row0 & 31u;
   const uint32_t lo = bits << sh;
   if (lo) atomicOr(&bitmap[wi], lo);
   if (sh > 1) {
     const uint32_t hi = bits >> (32u - sh);
     if (hi) atomicOr(&bitmap[wi + 1], hi);
+  }
+}
+
+// How a word beside a literal's bears on the bitmap words they may share: a
+// literal (its payload is in those words), a 0-fill (nothing is), or a word
+// that says nothing about the neighbouring chunk (a fill of no chunks, the end
+// of the stream) or sets rows by itself (a 1-fill).
+__device__ __forceinline__ bool beside_literal(uint32_t v) { return v & 0x80000000u; }
+__device__ __forceinline__ bool beside_open(uint32_t v) {
+  return !(v & 0x80000000u) && ((v & 0x40000000u) || !(v & 0x3FFFFFFFu));
+}
+
+// Writes the payload of a literal at chunk c of a single stream, between the
+// words before and after it.  A bitmap word holds rows of two chunks at most,
+// c and c + 1: where both are literals the later one writes the word with the
+// earlier one's rows, else the one that has rows there does, so every word is
+// stored once and no atomics are needed (device-scope ORs ran at 37 G/s, which
+// held a decode of 2^27 rows at 59 us).  Beside an open word the ORs stay.
+__device__ __forceinline__ void put_literal(uint32_t* bitmap, uint64_t nrows, uint32_t chunks,
+                                            uint32_t c, uint32_t bits, uint32_t before,
+                                            uint32_t after) {
+  if (c >= chunks) return;
+  const uint32_t row0 = 31u * c;
+  if (nrows - row0 < 31) bits &= (1u << (uint32_t)(nrows - row0)) - 1u;
+  const uint32_t wi = row0 >> 5, sh = row0 & 31u;
+  // rows shared with chunk c - 1: word wi (sh = 0: that chunk ends with a word)
+  uint32_t lo = 0;
+  if (sh) {
+    lo = bits << sh;
+    if (beside_literal(before)) lo |= (before & 0x7FFFFFFFu) >> (31u - sh);
+  }
+  // rows shared with chunk c + 1: word wi + 1, or wi when c starts it
+  const uint32_t hi = sh ? (sh > 1 ? bits >> (32u - sh) : 0u) : bits;
+  const uint32_t hw = sh ? wi + 1u : wi;
+  const bool take_hi = hi && !(beside_literal(after) && c + 1u < chunks);
+  if (beside_open(before) || beside_open(after)) {
+    if (lo) atomicOr(&bitmap[wi], lo);
+    if (take_hi) atomicOr(&bitmap[hw], hi);
+  } else {
+    if (lo) bitmap[wi] = lo;
+    if (take_hi) bitmap[hw] = hi;
   }
 }
 
@@ -58,357 +105,474 @@ __device__ void set_rows(uint32_t* bitmap, uint64_t nrows, uint64_t row0, uint64
   }
 }
 
-// Chunk count of word i, with the segment-start flag in bit 32.
-__device__ __forceinline__ uint64_t dec_elem(const uint32_t* words, const uint32_t* heads,
-                                             uint64_t i) {
-  return (uint64_t)word_chunks(words[i]) |
-         ((uint64_t)(i == 0 || (heads && heads[i] != 0u)) << 32);
+// Number of the ascending x[0 .. n) below v, by a whole wave: 64 probes per
+// round trip.
+__device__ __forceinline__ uint64_t wave_lower_bound(const uint32_t* __restrict__ x, uint64_t n,
+                                                     uint64_t v) {
+  const uint32_t l = lane_id();
+  uint64_t a = 0, e = n;  // answer in [a, e]
+  while (e > a) {
+    const uint64_t step = (e - a + kWave - 1) / kWave;
+    const uint64_t p = a + (l + 1) * step - 1;  // last element of the lane's strip
+    const bool below = p < e && x[p] < v;
+    const uint64_t whole = (uint64_t)__builtin_popcountll(ballot(below));  // strips all below v
+    a += whole * step;
+    if (step == 1) break;
+    e = a + step - 1 < e ? a + step - 1 : e;
+  }
+  return a;
 }
 
 }  // namespace
 
-// One pass over a stream of WAH words (a key's, or the concatenated streams
-// of several keys with heads[i] != 0 where a key starts): per word its first
-// chunk (segmented scan of chunk counts, decoupled look-back across tiles),
-// then its literal bits or 1-fill rows ORed into the row bitmap.
-__global__ __launch_bounds__(kBlock) void k_q_decode(const uint32_t* __restrict__ words,
-                                                     const uint32_t* __restrict__ heads,
-                                                     uint64_t len, uint32_t* __restrict__ bitmap,
-                                                     uint64_t nrows, uint64_t* status,
-                                                     uint32_t num_tiles, uint32_t* tile_counter,
-                                                     uint32_t lanes, uint32_t* fault,
-                                                     uint64_t* last_row) {
-  __shared__ uint64_t s_scan[kWaves];
-  __shared__ uint64_t s_prefix;
-  __shared__ uint32_t s_tile;
-  const int t = threadIdx.x;
-  uint32_t iter = 0;
-  for (;;) {
-    const uint32_t tile = next_tile(tile_counter, lanes, &s_tile, iter);
-    if (tile >= num_tiles) break;
-    const uint64_t g0 = (uint64_t)tile * kDecTile + (uint64_t)t * kDecItems;
-    uint64_t agg = OpSegAdd::identity();
+// One pass over WAH words: per word its first chunk (a scan of chunk counts,
+// with look-back across tiles), then its literal bits or 1-fill rows ORed into
+// the row bitmap (zero before).
+//   SEG false: two streams, q.words[0 .. len) of each into its own bitmap (the
+//     second may be empty), the second's tiles after the first's; the row
+//     after the last set row of the first is the result.
+//   SEG true: the concatenated streams of keys [range[0], range[1]), words
+//     range[2] .. range[3] of q.words, which k_q_range found; each key's words
+//     restart at chunk 0.  A tile finds the keys that start in it by a search
+//     of their offsets and marks them in LDS, so the words are read once and
+//     nothing else is (a flag array took a fill, a marking launch and 4 bytes
+//     per word).
+// What bounds it: sparse streams the atomic ORs (one per literal, each to a
+// line of its own), dense ones the words.
+template <bool SEG>
+__global__ __launch_bounds__(kScanThreads, query_waves_per_eu(kDecBlocks)) void k_q_decode(
+    DecodeStream qa, DecodeStream qb, const uint32_t* __restrict__ offsets, uint64_t nrows,
+    ScanState* st, uint64_t* status, uint64_t* host) {
+  __shared__ uint32_t s_sum[kScanWaves], s_head[kScanWaves];
+  __shared__ uint32_t s_mark[SEG ? kDecTile / 32 : 1];
+  __shared__ uint64_t s_key0;
+  __shared__ uint32_t s_prefix, s_tile;
+  const int l = threadIdx.x % kWave;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const uint32_t chunks = (uint32_t)((nrows + 30) / 31);
+  uint64_t key_a = 0, key_b = 0, w0 = 0;
+  if (SEG) {
+    key_a = st->range[0];
+    key_b = st->range[1];
+    w0 = st->range[2];
+    qa.words += w0;
+    qa.len = st->range[3] - w0;
+  }
+  const uint32_t tiles_a = (uint32_t)((qa.len + kDecTile - 1) / kDecTile);
+  const uint32_t tiles = tiles_a + (SEG ? 0u : (uint32_t)((qb.len + kDecTile - 1) / kDecTile));
+  uint64_t my_last = 0;  // row after the last set row of this thread's words (stream a)
+  for (uint32_t tile = scan_next_tile(st, &s_tile, true); tile < tiles;
+       tile = scan_next_tile(st, &s_tile, false)) {
+    const bool second = !SEG && tile >= tiles_a;
+    const DecodeStream q = second ? qb : qa;
+    const uint32_t first = second ? tiles_a : 0u;
+    const uint64_t base = (uint64_t)(tile - first) * kDecTile;
+    auto body = [&](auto full_tag) {
+      constexpr bool FULL = decltype(full_tag)::value;
+      W4 x[kDecRows], y[kDecRows];  // words; their first chunks
 #pragma unroll
-    for (int i = 0; i < kDecItems; ++i)
-      if (g0 + i < len) agg = OpSegAdd::combine(agg, dec_elem(words, heads, g0 + i));
-    uint64_t tile_agg;
-    const uint64_t ex = block_exclusive<OpSegAdd>(agg, s_scan, &tile_agg);
-    if (t == 0) s_prefix = lookback64<OpSegAdd>(status, tile, tile_agg, fault);
-    __syncthreads();
-    uint64_t run = OpSegAdd::combine(s_prefix, ex);
-    uint64_t my_last = 0;  // row after the last set row of this thread's words
+      for (int r = 0; r < kDecRows; ++r)
+        x[r] = load4<FULL>(q.words, base + row_at<kDecRows>(w, l, r), q.len);
+      uint32_t hb = 0;  // key starts, bit 4r + k
+      if (SEG) {
+        for (uint32_t i = threadIdx.x; i < kDecTile / 32; i += kScanThreads) s_mark[i] = 0;
+        if (w == 0) {
+          const uint64_t k0 = wave_lower_bound(offsets + key_a, key_b - key_a, w0 + base) + key_a;
+          if (l == 0) s_key0 = k0;
+        }
+        __syncthreads();
+        for (uint64_t k = s_key0 + threadIdx.x; k < key_b; k += kScanThreads) {
+          const uint64_t at = (uint64_t)offsets[k] - w0 - base;
+          if (at >= kDecTile) break;
+          atomicOr(&s_mark[at / 32], 1u << (at % 32));
+        }
+        __syncthreads();
 #pragma unroll
-    for (int i = 0; i < kDecItems; ++i) {
-      const uint64_t g = g0 + i;
-      if (g < len) {
-        const uint32_t w = words[g];
-        const uint64_t e = dec_elem(words, heads, g);
-        // first chunk of this word = inclusive sum before adding it
-        const uint32_t c0 = (e >> 32) ? 0u : (uint32_t)run;
-        run = OpSegAdd::combine(run, e);
-        const uint64_t row0 = 31ull * c0;
-        if (w & 0x80000000u) {
-          const uint32_t bits = w & 0x7FFFFFFFu;
-          or_bits31(bitmap, nrows, row0, bits);
-          if (bits) {
-            const uint64_t r = row0 + 32u - (uint32_t)__clz(bits);
-            my_last = r > my_last ? r : my_last;
-          }
-        } else if ((w & 0x40000000u) && (w & 0x3FFFFFFFu)) {
-          const uint64_t cnt = 31ull * (w & 0x3FFFFFFFu);
-          set_rows(bitmap, nrows, row0, cnt);
-          my_last = row0 + cnt > my_last ? row0 + cnt : my_last;
+        for (int r = 0; r < kDecRows; ++r) {
+          const uint32_t e = row_at<kDecRows>(w, l, r);
+          hb |= ((s_mark[e / 32] >> (e % 32)) & 15u) << (4 * r);
         }
       }
+      uint32_t run = 0;    // chunks of the wave's earlier rows
+      uint32_t start = 0;  // chunks before the open key's first word
+      uint32_t openm = 0;  // words whose key began before the wave
+      bool open = true;
+#pragma unroll
+      for (int r = 0; r < kDecRows; ++r) {
+        const uint32_t h4 = (hb >> (4 * r)) & 15u;
+        const uint32_t p1 = word_chunks(x[r].x), p2 = p1 + word_chunks(x[r].y),
+                       p3 = p2 + word_chunks(x[r].z), s = p3 + word_chunks(x[r].w);
+        const uint32_t inc = wave_incl_add(s);
+        const uint32_t ex = run + inc - s;
+        if (!SEG) {
+          y[r] = W4{ex, ex + p1, ex + p2, ex + p3};
+          run += readlane(inc, kWave - 1);
+          continue;
+        }
+        const uint32_t b = ex + (h4 & 8u ? p3 : h4 & 4u ? p2 : h4 & 2u ? p1 : 0u);
+        const uint64_t hm = ballot(h4 != 0u);
+        const uint64_t below = hm & ((1ull << l) - 1ull);
+        const uint32_t got = __shfl(b, below ? 63 - __builtin_clzll(below) : 0, kWave);
+        uint32_t cur = below ? got : start;
+        bool o = !below && open;
+        if (h4 & 1u) { cur = ex; o = false; }
+        y[r].x = ex - cur;
+        openm |= o ? 1u << (4 * r) : 0u;
+        if (h4 & 2u) { cur = ex + p1; o = false; }
+        y[r].y = ex + p1 - cur;
+        openm |= o ? 2u << (4 * r) : 0u;
+        if (h4 & 4u) { cur = ex + p2; o = false; }
+        y[r].z = ex + p2 - cur;
+        openm |= o ? 4u << (4 * r) : 0u;
+        if (h4 & 8u) { cur = ex + p3; o = false; }
+        y[r].w = ex + p3 - cur;
+        openm |= o ? 8u << (4 * r) : 0u;
+        run += readlane(inc, kWave - 1);
+        if (hm) {  // wave-uniform
+          start = readlane(b, 63 - __builtin_clzll(hm));
+          open = false;
+        }
+      }
+      if (l == 0) {
+        s_sum[w] = open ? run : run - start;
+        s_head[w] = open ? 0u : 1u;
+      }
+      __syncthreads();
+      uint32_t carry = 0, agg = 0;
+      bool closed = false, tile_closed = false;
+#pragma unroll
+      for (int i = 0; i < kScanWaves; ++i) {
+        if (i == w) {
+          carry = agg;
+          closed = tile_closed;
+        }
+        const bool h = SEG && s_head[i] != 0u;
+        agg = h ? s_sum[i] : agg + s_sum[i];
+        tile_closed |= h;
+      }
+      if (w == 0) {
+        uint32_t hi, p;
+        lookback2<kOpNone, kOpSum>(status, tile, 0u, agg, tile_closed, &st->fault, hi, p, first);
+        if (l == 0) s_prefix = p;
+      }
+      __syncthreads();
+      if (!closed) carry += s_prefix;
+      // the words before and after the wave's (a single stream's first word
+      // has a 0-fill before it, its last word an open one after it)
+      uint32_t wb = 1u, wa = 0u;
+      if (!SEG) {
+        const uint64_t b = base + row_at<kDecRows>(w, 0, 0), e = b + kDecRows * kRowElems;
+        if (b > 0 && b <= q.len) wb = q.words[b - 1];
+        if (e < q.len) wa = q.words[e];
+      }
+#pragma unroll
+      for (int r = 0; r < kDecRows; ++r) {
+        const uint32_t before =
+            SEG ? 0u : lane_before(x[r].w, r ? readlane(x[r ? r - 1 : 0].w, kWave - 1) : wb);
+        const uint32_t after =
+            SEG ? 0u
+                : lane_after(x[r].x, r + 1 < kDecRows
+                                         ? readlane(x[r + 1 < kDecRows ? r + 1 : r].x, 0)
+                                         : wa);
+        const uint32_t xs[4] = {x[r].x, x[r].y, x[r].z, x[r].w};
+        const uint32_t ys[4] = {y[r].x, y[r].y, y[r].z, y[r].w};
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const uint32_t c = ys[k] + (!SEG || ((openm >> (4 * r + k)) & 1u) ? carry : 0u);
+          const uint32_t v = xs[k];  // past the stream's end: 0, a fill of nothing
+          if (v & 0x80000000u) {
+            const uint32_t bits = v & 0x7FFFFFFFu;
+            if (SEG)
+              or_literal(q.bitmap, nrows, chunks, c, bits);
+            else
+              put_literal(q.bitmap, nrows, chunks, c, bits, k ? xs[k - 1] : before,
+                          k < 3 ? xs[k + 1] : after);
+            if (!SEG && !second && bits) {
+              const uint64_t end = 31ull * c + 32u - (uint32_t)__builtin_clz(bits);
+              my_last = end > my_last ? end : my_last;
+            }
+          } else if ((v & 0x40000000u) && (v & 0x3FFFFFFFu)) {
+            const uint64_t row0 = 31ull * c, cnt = 31ull * (v & 0x3FFFFFFFu);
+            set_rows(q.bitmap, nrows, row0, cnt);
+            if (!SEG && !second) my_last = row0 + cnt > my_last ? row0 + cnt : my_last;
+          }
+        }
+      }
+    };
+    if (base + kDecTile <= q.len) body(std::true_type{});
+    else body(std::false_type{});
+  }
+  if (!SEG) {
+    // the block's last row goes to its lane's word, once (8 waves of 1000
+    // blocks on one address took 90 us)
+    __shared__ uint64_t s_row[kScanWaves];
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) {
+      const uint64_t o = ((uint64_t)__shfl_xor((uint32_t)(my_last >> 32), d, kWave) << 32) |
+                         __shfl_xor((uint32_t)my_last, d, kWave);
+      my_last = o > my_last ? o : my_last;
     }
-    if (last_row && my_last) atomicMax((unsigned long long*)last_row, (unsigned long long)my_last);
+    if (l == 0) s_row[w] = my_last;
     __syncthreads();
+    if (threadIdx.x == 0) {
+#pragma unroll
+      for (int i = 1; i < kScanWaves; ++i) my_last = s_row[i] > my_last ? s_row[i] : my_last;
+      const uint32_t lane = blockIdx.x % tile_lanes(gridDim.x);
+      if (my_last)
+        atomicMax(reinterpret_cast<unsigned long long*>(&st->tiles[lane * kLaneStride + 2]),
+                  (unsigned long long)my_last);
+    }
   }
+  scan_finish(st, status, tiles, host);
 }
 
-// Marks the first word of each key k in [a, b) of an index: heads[offsets[k]
-// - w0] = 1 (heads zeroed before).
-__global__ __launch_bounds__(kBlock) void k_q_mark_heads(const uint32_t* __restrict__ offsets,
-                                                         uint64_t a, uint64_t b, uint64_t w0,
-                                                         uint32_t* __restrict__ heads) {
-  for (uint64_t k = a + (uint64_t)blockIdx.x * kBlock + threadIdx.x; k < b;
-       k += (uint64_t)gridDim.x * kBlock)
-    heads[offsets[k] - w0] = 1u;
-}
-
-// Locates the keys of an index in [lo, hi] (keys ascend): range[0] = first
-// key index >= lo, range[1] = first > hi, range[2] = first word of key
-// range[0], range[3] = one past the last word of key range[1] - 1.
-__global__ void k_q_key_range(const uint32_t* __restrict__ keys,
-                              const uint32_t* __restrict__ offsets,
-                              const uint32_t* __restrict__ lengths, uint64_t keycnt,
-                              uint32_t lo, uint32_t hi, uint64_t* __restrict__ range) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  uint64_t a = 0, e = keycnt;
-  while (a < e) {  // lower bound of lo
-    const uint64_t m = (a + e) / 2;
-    if (keys[m] < lo) a = m + 1;
-    else e = m;
+// Starts a range query: zeroes the row bitmap and locates the keys of the
+// index in [lo, hi] (keys ascend): range[0] = first key index >= lo, range[1]
+// = first > hi, range[2] = first word of key range[0], range[3] = one past the
+// last word of key range[1] - 1.  The number of keys goes to host[3].
+__global__ __launch_bounds__(kBlock) void k_q_range(const uint32_t* __restrict__ keys,
+                                                    const uint32_t* __restrict__ offsets,
+                                                    const uint32_t* __restrict__ lengths,
+                                                    uint64_t keycnt, uint32_t lo, uint32_t hi,
+                                                    uint32_t* __restrict__ bitmap, uint64_t words,
+                                                    ScanState* st, uint64_t* host) {
+  __shared__ uint64_t s_at[2];
+  const uint32_t t = threadIdx.x;
+  if (blockIdx.x == 0) {
+    if (t < 2 * kWave) {
+      const uint64_t v = t < kWave ? (uint64_t)lo : (uint64_t)hi + 1;
+      const uint64_t at = wave_lower_bound(keys, keycnt, v);
+      if (t % kWave == 0) s_at[t / kWave] = at;
+    }
+    __syncthreads();
+    if (t == 0) {
+      const uint64_t a = s_at[0], b = s_at[1];
+      st->range[0] = a;
+      st->range[1] = b;
+      st->range[2] = a < b ? offsets[a] : 0;
+      st->range[3] = a < b ? (uint64_t)offsets[b - 1] + lengths[b - 1] : 0;
+      __hip_atomic_store(&host[3], b - a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      __hip_atomic_store(&host[4], st->range[3] - st->range[2], __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_SYSTEM);
+    }
   }
-  uint64_t b = a;
-  e = keycnt;
-  while (b < e) {  // upper bound of hi
-    const uint64_t m = (b + e) / 2;
-    if (keys[m] <= hi) b = m + 1;
-    else e = m;
-  }
-  range[0] = a;
-  range[1] = b;
-  range[2] = a < b ? offsets[a] : 0;
-  range[3] = a < b ? (uint64_t)offsets[b - 1] + lengths[b - 1] : 0;
+  for (uint64_t i = (uint64_t)blockIdx.x * kBlock + t; i < words; i += (uint64_t)gridDim.x * kBlock)
+    bitmap[i] = 0;
 }
 
 // ---- encoding a row bitmap (or op(a, b) of two) into WAH words -------------
 
 namespace {
 
-// Payload of chunk c: rows 31 c .. 31 c + 30 of the bitmap (rows >= nrows
-// are zero).
-__device__ __forceinline__ uint32_t chunk_bits(const uint32_t* bm, uint64_t nrows, uint64_t c) {
-  const uint64_t r = 31ull * c;
-  if (r >= nrows) return 0u;
-  const uint64_t wi = r >> 5;
-  const uint32_t sh = (uint32_t)(r & 31u);
-  const uint64_t nwords = (nrows + 31) / 32;
-  uint64_t x = bm[wi];
-  if (wi + 1 < nwords) x |= (uint64_t)bm[wi + 1] << 32;
-  uint32_t bits = (uint32_t)(x >> sh) & 0x7FFFFFFFu;
-  if (nrows - r < 31) bits &= (1u << (uint32_t)(nrows - r)) - 1u;
-  return bits;
-}
+// A lane owns 8 consecutive chunks, 248 rows; a wave 512 chunks, which are
+// 15872 rows and so whole bitmap words (496); a tile 4096 chunks, 3968 words.
+constexpr int kEncItems = 8;
+constexpr uint32_t kEncTile = kScanThreads * kEncItems;
+constexpr uint32_t kEncWaveWords = kWave * kEncItems * 31 / 32;
+constexpr uint32_t kEncWords = kEncWaveWords * kScanWaves;
+static_assert(kWave * kEncItems * 31 % 32 == 0 && kEncWords % 4 == 0, "whole words per wave");
 
 __device__ __forceinline__ uint32_t combine_bits(int op, uint32_t a, uint32_t b) {
   switch (op) {
     case 0: return a & b;   // AND
     case 1: return a | b;   // OR
     case 2: return a ^ b;   // XOR
-    case 3: return a & ~b;  // AND NOT
-    default: return a;      // the first bitmap alone
+    default: return a & ~b; // AND NOT
   }
-}
-
-struct OpMax {
-  static __device__ __forceinline__ uint64_t identity() { return 0; }
-  static __device__ __forceinline__ uint64_t combine(uint64_t a, uint64_t b) {
-    return a > b ? a : b;
-  }
-};
-
-// Per thread: its kEncItems chunks' payloads, the words they emit counting a
-// fill only where the previous emitted chunk is this thread's own, and its
-// first and last emitted chunk (+1; 0 = none).
-struct ThreadChunks {
-  uint32_t bits[kEncItems];
-  uint32_t words;
-  uint64_t first, last;
-};
-
-__device__ __forceinline__ ThreadChunks thread_chunks(const uint32_t* a, const uint32_t* b,
-                                                      int op, uint64_t nrows, uint64_t chunks,
-                                                      uint64_t c0) {
-  ThreadChunks r;
-  r.words = 0;
-  r.first = r.last = 0;
-#pragma unroll
-  for (int i = 0; i < kEncItems; ++i) {
-    const uint64_t c = c0 + i;
-    uint32_t x = 0;
-    if (c < chunks) {
-      const uint32_t pa = chunk_bits(a, nrows, c);
-      x = b ? combine_bits(op, pa, chunk_bits(b, nrows, c)) : pa;
-    }
-    r.bits[i] = x;
-    if (x) {
-      // previous emitted chunk of this thread is r.last - 1: the fill
-      // c - r.last is a word when nonzero; the fill of the thread's first
-      // entry is counted by the caller
-      r.words += 1u + (r.last && c != r.last ? 1u : 0u);
-      if (!r.first) r.first = c + 1;
-      r.last = c + 1;
-    }
-  }
-  return r;
 }
 
 }  // namespace
 
-// Pass 1: per tile of kEncTile chunks, the words its entries emit except the
-// fill of its first entry, and its first and last emitted chunk (+1).
-__global__ __launch_bounds__(kBlock) void k_q_enc_count(const uint32_t* __restrict__ a,
-                                                        const uint32_t* __restrict__ b, int op,
-                                                        uint64_t nrows, uint64_t chunks,
-                                                        uint64_t* __restrict__ tile_sum) {
-  __shared__ uint64_t s_scan[kWaves];
-  const int t = threadIdx.x;
-  const uint64_t c0 = (uint64_t)blockIdx.x * kEncTile + (uint64_t)t * kEncItems;
-  const ThreadChunks tc = thread_chunks(a, b, op, nrows, chunks, c0);
-  // fill of this thread's first entry, when an earlier thread of the tile
-  // emitted: chunk gap to that thread's last entry
-  uint64_t tot;
-  const uint64_t prev = block_exclusive<OpMax>(tc.last, s_scan, &tot);
-  uint32_t w = tc.words;
-  if (tc.first && prev) w += (tc.first != prev + 1) ? 1u : 0u;
-  uint64_t wsum;
-  (void)block_exclusive<OpAdd>(w, s_scan, &wsum);
-  uint64_t first_any;
-  (void)block_exclusive<OpMax>(tc.first ? (uint64_t)(0xFFFFFFFFFFull - tc.first) : 0ull,
-                               s_scan, &first_any);
-  if (t == 0) {
-    tile_sum[3 * (uint64_t)blockIdx.x + 0] = wsum;
-    tile_sum[3 * (uint64_t)blockIdx.x + 1] = first_any ? 0xFFFFFFFFFFull - first_any : 0ull;
-    tile_sum[3 * (uint64_t)blockIdx.x + 2] = tot;
-  }
-}
-
-// Pass 2 (one block): per tile its first word and the last emitted chunk
-// (+1) before it; the total word count into *len (L).
-__global__ __launch_bounds__(1024) void k_q_enc_scan(uint64_t* __restrict__ tile_sum,
-                                                     uint32_t tiles, uint64_t* __restrict__ len) {
-  __shared__ uint64_t s_part[1024];
-  __shared__ uint64_t s_last[1024];
-  const uint32_t t = threadIdx.x;
-  const uint32_t per = (tiles + 1023) / 1024;
-  const uint32_t s0 = t * per < tiles ? t * per : tiles;
-  const uint32_t s1 = s0 + per < tiles ? s0 + per : tiles;
-  // strip summary: last emitted chunk of the strip
-  uint64_t last = 0;
-  for (uint32_t s = s0; s < s1; ++s) {
-    const uint64_t l = tile_sum[3 * (uint64_t)s + 2];
-    last = l > last ? l : last;
-  }
-  s_last[t] = last;
-  __syncthreads();
-  // exclusive max over strips (chunks ascend, so max = last nonempty)
-  if (t == 0) {
-    uint64_t m = 0;
-    for (uint32_t i = 0; i < 1024; ++i) {
-      const uint64_t x = s_last[i];
-      s_last[i] = m;
-      m = x > m ? x : m;
-    }
-  }
-  __syncthreads();
-  // strip words, with each tile's first fill against the last chunk before it
-  uint64_t prev = s_last[t], words = 0;
-  for (uint32_t s = s0; s < s1; ++s) {
-    const uint64_t w = tile_sum[3 * (uint64_t)s + 0];
-    const uint64_t f = tile_sum[3 * (uint64_t)s + 1];
-    const uint64_t l = tile_sum[3 * (uint64_t)s + 2];
-    // a key's first fill is its chunk (prev = 0 means chunk -1)
-    words += w + (f ? (f != prev + 1 ? 1u : 0u) : 0u);
-    prev = l > prev ? l : prev;
-  }
-  s_part[t] = words;
-  __syncthreads();
-  if (t == 0) {
-    uint64_t run = 0;
-    for (uint32_t i = 0; i < 1024; ++i) {
-      const uint64_t x = s_part[i];
-      s_part[i] = run;
-      run += x;
-    }
-    *len = run;
-  }
-  __syncthreads();
-  uint64_t pos = s_part[t];
-  prev = s_last[t];
-  for (uint32_t s = s0; s < s1; ++s) {
-    const uint64_t w = tile_sum[3 * (uint64_t)s + 0];
-    const uint64_t f = tile_sum[3 * (uint64_t)s + 1];
-    const uint64_t l = tile_sum[3 * (uint64_t)s + 2];
-    tile_sum[3 * (uint64_t)s + 0] = pos;   // first word of the tile
-    tile_sum[3 * (uint64_t)s + 1] = prev;  // last emitted chunk (+1) before it
-    pos += w + (f ? (f != prev + 1 ? 1u : 0u) : 0u);
-    prev = l > prev ? l : prev;
-  }
-}
-
-// Pass 3: each tile writes its words: per emitted chunk c a fill of
-// c - prev - 1 chunks when nonzero (prev = the previous emitted chunk, -1 at
-// the start), then the literal 0x80000000 | payload.  Words past cap are not
-// written (the caller compares L with cap).
-__global__ __launch_bounds__(kBlock) void k_q_enc_write(const uint32_t* __restrict__ a,
-                                                        const uint32_t* __restrict__ b, int op,
-                                                        uint64_t nrows, uint64_t chunks,
-                                                        const uint64_t* __restrict__ tile_sum,
-                                                        uint32_t* __restrict__ out, uint64_t cap) {
-  __shared__ uint64_t s_scan[kWaves];
-  const int t = threadIdx.x;
-  const uint64_t c0 = (uint64_t)blockIdx.x * kEncTile + (uint64_t)t * kEncItems;
-  const ThreadChunks tc = thread_chunks(a, b, op, nrows, chunks, c0);
-  uint64_t tot;
-  uint64_t prev = block_exclusive<OpMax>(tc.last, s_scan, &tot);
-  if (!prev) prev = tile_sum[3 * (uint64_t)blockIdx.x + 1];
-  uint32_t w = tc.words;
-  if (tc.first) w += (tc.first != prev + 1) ? 1u : 0u;
-  uint64_t wsum;
-  uint64_t pos = tile_sum[3 * (uint64_t)blockIdx.x + 0] + block_exclusive<OpAdd>(w, s_scan, &wsum);
+// One pass over a row bitmap (TWO: over a op b, combined word by word as they
+// are loaded): per nonempty chunk c a fill of the chunks skipped since the
+// last nonempty one, when there are any, then the literal.  Whether c has a
+// fill word depends on chunk c - 1 alone, so the word count of a tile is known
+// without its neighbours and the look-back is a plain sum of words, with the
+// maximum of the nonempty chunks beside it for the one fill per tile that
+// starts in an earlier tile.  The bitmap goes through LDS (a lane's 248 rows
+// start off its words), the words too.  Words past cap are not written.
+template <bool TWO>
+__global__ __launch_bounds__(kScanThreads, query_waves_per_eu(kEncBlocks)) void k_q_encode(
+    const uint32_t* __restrict__ a, const uint32_t* __restrict__ b, int op, uint64_t nrows,
+    uint32_t* __restrict__ out, uint64_t cap, ScanState* st, uint64_t* status, uint32_t tiles,
+    uint64_t* host) {
+  // the tile's bitmap words (one before them, one after), then its WAH words
+  __shared__ alignas(16) uint32_t s_buf[2 * kEncTile];
+  __shared__ uint32_t s_words[kScanWaves], s_first[kScanWaves], s_last[kScanWaves];
+  __shared__ uint32_t s_prefix, s_tile;
+  static_assert(kEncWords + 5 <= 2 * kEncTile, "the bitmap words fit");
+  uint32_t* const s_bits = s_buf + 4;  // 16-byte aligned, room for the word before
+  const int l = threadIdx.x % kWave;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const uint64_t nwords = (nrows + 31) / 32;
+  const uint32_t tail = (uint32_t)(nrows & 31u);  // rows of the last word (0: all 32)
+  for (uint32_t tile = scan_next_tile(st, &s_tile, true); tile < tiles;
+       tile = scan_next_tile(st, &s_tile, false)) {
+    const uint64_t wbase = (uint64_t)tile * kEncWords;
+    const uint32_t c0 = tile * kEncTile;  // chunks are below 2^28
+    auto load = [&](auto full_tag) {
+      constexpr bool FULL = decltype(full_tag)::value;
 #pragma unroll
-  for (int i = 0; i < kEncItems; ++i) {
-    const uint32_t x = tc.bits[i];
-    if (x) {
-      const uint64_t c1 = c0 + i + 1;  // chunk + 1
-      const uint64_t fill = c1 - prev - 1;
-      if (fill) {
-        if (pos < cap) out[pos] = (uint32_t)fill;
-        ++pos;
+      for (uint32_t h = 0; h < 2; ++h) {
+        const uint32_t qd = h * kScanThreads + threadIdx.x;
+        if (4 * qd < kEncWords) {
+          const uint64_t g = wbase + 4 * qd;
+          W4 x = load4<FULL>(a, g, nwords);
+          if (TWO) {
+            const W4 y = load4<FULL>(b, g, nwords);
+            x.x = combine_bits(op, x.x, y.x);
+            x.y = combine_bits(op, x.y, y.y);
+            x.z = combine_bits(op, x.z, y.z);
+            x.w = combine_bits(op, x.w, y.w);
+          }
+          if (!FULL && tail && nwords - 1 - g < 4) {  // rows past nrows
+            const uint32_t m = (1u << tail) - 1u;
+            const uint32_t k = (uint32_t)(nwords - 1 - g);
+            x.x &= k == 0 ? m : ~0u;
+            x.y &= k == 1 ? m : ~0u;
+            x.z &= k == 2 ? m : ~0u;
+            x.w &= k == 3 ? m : ~0u;
+          }
+          *reinterpret_cast<W4*>(&s_bits[4 * qd]) = x;
+        }
       }
-      if (pos < cap) out[pos] = 0x80000000u | x;
-      ++pos;
-      prev = c1;
+    };
+    if (wbase + kEncWords < nwords) load(std::true_type{});
+    else load(std::false_type{});
+    if (threadIdx.x == 0) {
+      uint32_t x = 0;
+      if (tile) {
+        x = a[wbase - 1];
+        if (TWO) x = combine_bits(op, x, b[wbase - 1]);
+      }
+      s_bits[-1] = x;
+      s_bits[kEncWords] = 0;
     }
+    __syncthreads();
+    // the lane's 248 rows from bit 0 of v[0] on, then its chunks
+    uint32_t e[kEncItems];
+    {
+      const uint32_t bit = (uint32_t)l * (kEncItems * 31u);
+      const uint32_t* p = s_bits + w * kEncWaveWords + (bit >> 5);
+      uint32_t x[9], v[8];
+#pragma unroll
+      for (int i = 0; i < 9; ++i) x[i] = p[i];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) v[i] = __builtin_amdgcn_alignbit(x[i + 1], x[i], bit & 31u);
+      e[0] = v[0] & 0x7FFFFFFFu;
+#pragma unroll
+      for (int i = 1; i < kEncItems; ++i)
+        e[i] = __builtin_amdgcn_alignbit(v[i], v[i - 1], 32u - (uint32_t)i) & 0x7FFFFFFFu;
+    }
+    uint32_t ne = 0;  // nonempty chunks of the lane
+#pragma unroll
+    for (int i = 0; i < kEncItems; ++i) ne |= e[i] ? 1u << i : 0u;
+    // the chunk before the lane's first: nonempty?  (before chunk 0: no fill)
+    const uint32_t before_wave = s_bits[(int)(w * kEncWaveWords) - 1] >> 1;
+    const uint32_t cw = c0 + (uint32_t)w * kWave * kEncItems;  // the wave's first chunk
+    const uint32_t pb = lane_before(ne >> (kEncItems - 1), cw == 0 || before_wave ? 1u : 0u);
+    const uint32_t fm = ne & ~(ne << 1 | pb);  // chunks whose literal follows a fill
+    const uint32_t cnt = (uint32_t)(__builtin_popcount(ne) + __builtin_popcount(fm));
+    const uint32_t inc = wave_incl_add(cnt);
+    // last nonempty chunk (+ 1) before the lane, within the wave
+    const uint64_t hm = ballot(ne != 0u);
+    const uint64_t below = hm & ((1ull << l) - 1ull);
+    const uint32_t top = 32u - (uint32_t)__builtin_clz(ne | 1u);
+    const int src = below ? 63 - __builtin_clzll(below) : 0;
+    const uint32_t got = __shfl(top, src, kWave);
+    uint32_t prev = below ? cw + (uint32_t)src * kEncItems + got : 0u;
+    {
+      const int lo = hm ? __builtin_ctzll(hm) : 0, hi = hm ? 63 - __builtin_clzll(hm) : 0;
+      const uint32_t low = (uint32_t)__builtin_ctz(ne | 0x100u);
+      const uint32_t f = readlane(low, lo), g = readlane(top, hi);
+      if (l == 0) {
+        s_words[w] = readlane(inc, kWave - 1);
+        s_first[w] = hm ? cw + (uint32_t)lo * kEncItems + f + 1u : 0u;  // chunk + 1
+        s_last[w] = hm ? cw + (uint32_t)hi * kEncItems + g : 0u;        // chunk + 1
+      }
+    }
+    __syncthreads();  // the bitmap words are consumed: s_buf takes the WAH words
+    uint32_t all = 0, wpos = 0, last = 0, wprev = 0, first = 0;
+#pragma unroll
+    for (int i = 0; i < kScanWaves; ++i) {
+      if (i == w) {
+        wpos = all;
+        wprev = last;
+      }
+      all += s_words[i];
+      if (!first) first = s_first[i];
+      if (s_last[i]) last = s_last[i];
+    }
+    if (!prev) prev = wprev;
+    uint32_t pos = wpos + inc - cnt;
+#pragma unroll
+    for (int i = 0; i < kEncItems; ++i) {
+      if ((ne >> i) & 1u) {
+        const uint32_t c = cw + (uint32_t)l * kEncItems + i;
+        if ((fm >> i) & 1u) {
+          // the tile's first entry takes its fill from the look-back, below
+          if (prev) s_buf[pos] = c - prev;
+          ++pos;
+        }
+        s_buf[pos++] = 0x80000000u | e[i];
+        prev = c + 1u;
+      }
+    }
+    if (w == 0) {
+      uint32_t ph, pw;
+      lookback2<kOpMax, kOpSum>(status, tile, last, all, false, &st->fault, ph, pw);
+      if (l == 0) {
+        s_prefix = pw;
+        // a first entry right after the tile before's last chunk (or chunk 0)
+        // has no fill and its literal stays
+        if (first && first - 1u != ph) s_buf[0] = first - 1u - ph;
+        if (tile == tiles - 1) st_agent(&st->result, (uint64_t)pw + all);
+      }
+    }
+    __syncthreads();
+    const uint64_t pre = s_prefix;
+    if (pre < cap) store_staged(s_buf, out + pre, cap - pre < all ? (uint32_t)(cap - pre) : all);
   }
+  scan_finish(st, status, tiles, host);
 }
 
 // ---- launchers ---------------------------------------------------------------
 
-uint64_t scan_status_words(uint64_t n) { return (n + kDecTile - 1) / kDecTile; }
-uint64_t encode_tiles(uint64_t nrows) {
-  const uint64_t chunks = (nrows + 30) / 31;
-  return (chunks + kEncTile - 1) / kEncTile;
-}
-
-void launch_decode(const ScanArgs& s, const uint32_t* words, const uint32_t* heads,
-                   uint64_t len, uint32_t* bitmap, uint64_t nrows, uint64_t* last_row,
+void launch_decode(const ScanRun& s, const DecodeStream& a, const DecodeStream& b, uint64_t nrows,
                    hipStream_t st) {
-  const uint32_t tiles = (uint32_t)((len + kDecTile - 1) / kDecTile);
+  const uint64_t tiles = (a.len + kDecTile - 1) / kDecTile + (b.len + kDecTile - 1) / kDecTile;
   if (!tiles) return;
-  const uint32_t grid = tiles < s.max_resident ? tiles : s.max_resident;
-  hipLaunchKernelGGL(k_q_decode, dim3(grid), dim3(kBlock), 0, st, words, heads, len, bitmap,
-                     nrows, s.status, tiles, s.tile_counter, tile_lanes(grid), s.fault, last_row);
+  const uint32_t most = s.cus * kDecBlocks;
+  hipLaunchKernelGGL(k_q_decode<false>, dim3(tiles < most ? (uint32_t)tiles : most),
+                     dim3(kScanThreads), 0, st, a, b, nullptr, nrows, s.state, s.status, s.host);
 }
 
-void launch_mark_heads(const uint32_t* offsets, uint64_t a, uint64_t b, uint64_t w0,
-                       uint32_t* heads, hipStream_t st) {
-  if (b <= a) return;
-  uint64_t g = (b - a + kBlock - 1) / kBlock;
-  if (g > 4096) g = 4096;
-  hipLaunchKernelGGL(k_q_mark_heads, dim3((uint32_t)g), dim3(kBlock), 0, st, offsets, a, b, w0,
-                     heads);
+void launch_range(const ScanRun& s, const uint32_t* keys, const uint32_t* offsets,
+                  const uint32_t* lengths, uint64_t keycnt, const uint32_t* words, uint32_t lo,
+                  uint32_t hi, uint32_t* bitmap, uint64_t nrows, hipStream_t st) {
+  const uint64_t bw = (nrows + 31) / 32;
+  uint64_t g = (bw + 4 * kBlock - 1) / (4 * kBlock);
+  g = g < 1 ? 1 : g > 4096 ? 4096 : g;
+  hipLaunchKernelGGL(k_q_range, dim3((uint32_t)g), dim3(kBlock), 0, st, keys, offsets, lengths,
+                     keycnt, lo, hi, bitmap, bw, s.state, s.host);
+  // the words of the range are known on the device only: a full grid
+  hipLaunchKernelGGL(k_q_decode<true>, dim3(s.cus * kDecBlocks), dim3(kScanThreads), 0, st,
+                     DecodeStream{words, 0, bitmap}, DecodeStream{nullptr, 0, nullptr}, offsets,
+                     nrows, s.state, s.status, s.host);
 }
 
-void launch_key_range(const uint32_t* keys, const uint32_t* offsets, const uint32_t* lengths,
-                      uint64_t keycnt, uint32_t lo, uint32_t hi, uint64_t* range, hipStream_t st) {
-  hipLaunchKernelGGL(k_q_key_range, dim3(1), dim3(64), 0, st, keys, offsets, lengths, keycnt, lo,
-                     hi, range);
-}
-
-void launch_encode(const uint32_t* a, const uint32_t* b, int op, uint64_t nrows,
-                   uint64_t* tile_sum, uint32_t* out, uint64_t cap, uint64_t* len,
-                   hipStream_t st) {
+void launch_encode(const ScanRun& s, const uint32_t* a, const uint32_t* b, int op, uint64_t nrows,
+                   uint32_t* out, uint64_t cap, hipStream_t st) {
   const uint64_t chunks = (nrows + 30) / 31;
-  const uint32_t tiles = (uint32_t)encode_tiles(nrows);
+  const uint32_t tiles = (uint32_t)((chunks + kEncTile - 1) / kEncTile);
   if (!tiles) return;
-  hipLaunchKernelGGL(k_q_enc_count, dim3(tiles), dim3(kBlock), 0, st, a, b, op, nrows, chunks,
-                     tile_sum);
-  hipLaunchKernelGGL(k_q_enc_scan, dim3(1), dim3(1024), 0, st, tile_sum, tiles, len);
-  hipLaunchKernelGGL(k_q_enc_write, dim3(tiles), dim3(kBlock), 0, st, a, b, op, nrows, chunks,
-                     tile_sum, out, cap);
+  const uint32_t most = s.cus * kEncBlocks, grid = tiles < most ? tiles : most;
+  if (b)
+    hipLaunchKernelGGL(k_q_encode<true>, dim3(grid), dim3(kScanThreads), 0, st, a, b, op, nrows,
+                       out, cap, s.state, s.status, tiles, s.host);
+  else
+    hipLaunchKernelGGL(k_q_encode<false>, dim3(grid), dim3(kScanThreads), 0, st, a, b, op, nrows,
+                       out, cap, s.state, s.status, tiles, s.host);
 }
 
 }  // namespace wah

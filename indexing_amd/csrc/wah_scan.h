@@ -83,27 +83,28 @@ constexpr int kOpMax = 2;
 constexpr int kOpOrSinceHi = 3;  // lo: OR from the last tile with hi != 0 on
 
 // Run by a whole wave: publishes the tile's (hi, lo) and returns the
-// combination over tiles 0 .. tile - 1, reading 64 predecessors per round
+// combination over tiles first .. tile - 1, reading 64 predecessors per round
 // trip.  closed: the tile's own values already are the inclusive prefix
-// (tile 0; a segmented sum whose tile starts a segment), so later tiles stop
-// there at once; else the inclusive prefix is published at the end.
+// (tile `first`; a segmented sum whose tile starts a segment), so later tiles
+// stop there at once; else the inclusive prefix is published at the end.
 template <int HI, int LO>
 __device__ __forceinline__ void lookback2(uint64_t* status, uint32_t tile, uint32_t hi,
                                           uint32_t lo, bool closed, uint32_t* fault,
-                                          uint32_t& pre_hi, uint32_t& pre_lo) {
+                                          uint32_t& pre_hi, uint32_t& pre_lo,
+                                          uint32_t first = 0) {
   constexpr uint64_t kHiMask = (1ull << 30) - 1;
   const uint32_t lane = lane_id();
   const uint64_t own = ((hi & kHiMask) << 32) | lo;
-  closed |= tile == 0;
+  closed |= tile == first;
   if (lane == 0)
     st_agent(&status[tile], ((uint64_t)(closed ? kFlagPrefix : kFlagAgg) << 62) | own);
   uint32_t ah = 0, al = 0;
   bool or_open = true;  // kOpOrSinceHi: no tile with hi != 0 met yet
   int64_t base = (int64_t)tile - 1;
   uint32_t spins = 0;
-  while (base >= 0) {
+  while (base >= (int64_t)first) {
     const int64_t idx = base - (int64_t)lane;
-    const uint64_t s = idx >= 0 ? ld_agent(&status[idx]) : ((uint64_t)kFlagPrefix << 62);
+    const uint64_t s = idx >= (int64_t)first ? ld_agent(&status[idx]) : ((uint64_t)kFlagPrefix << 62);
     const uint32_t f = (uint32_t)(s >> 62);
     const uint64_t pmask = ballot(f == kFlagPrefix);
     const uint64_t empty = ballot(f == 0);
@@ -188,19 +189,22 @@ __device__ __forceinline__ void scan_finish(ScanState* st, uint64_t* status, uin
   __syncthreads();
   if (!s_last) return;
   for (uint32_t i = threadIdx.x; i < tiles; i += blockDim.x) st_agent(&status[i], (uint64_t)0);
-  if (threadIdx.x < 2 * kTileLanes)
-    st_agent(&st->tiles[threadIdx.x / 2 * kLaneStride + threadIdx.x % 2], 0u);
   if (threadIdx.x == 0) {
     const uint64_t f = ld_agent(&st->fault);
+    uint64_t r = ld_agent(&st->result);
+    for (uint32_t i = 0; i < kTileLanes; ++i) {  // the lanes' maxima
+      const uint64_t m = ld_agent(reinterpret_cast<uint64_t*>(&st->tiles[i * kLaneStride + 2]));
+      r = m > r ? m : r;
+    }
     if (host) {
       __hip_atomic_store(&host[0], f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-      __hip_atomic_store(&host[1], ld_agent(&st->result[0]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-      __hip_atomic_store(&host[2], ld_agent(&st->result[1]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      __hip_atomic_store(&host[1], r, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
     st_agent(&st->fault, 0u);
     st_agent(&st->done, 0u);
-    st_agent(&st->result[0], (uint64_t)0);
-    st_agent(&st->result[1], (uint64_t)0);
+    st_agent(&st->result, (uint64_t)0);
+    for (uint32_t i = 0; i < kTileLanes; ++i)
+      for (uint32_t j = 0; j < 4; ++j) st_agent(&st->tiles[i * kLaneStride + j], 0u);
   }
 }
 

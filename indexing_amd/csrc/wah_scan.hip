@@ -275,7 +275,7 @@ __global__ __launch_bounds__(kScanThreads, waves_per_eu(kScanBlocks)) void k_com
       lookback2<kOpNone, kOpSum>(status, tile, 0u, all, false, &st->fault, h, p);
       if (l == 0) {
         s_prefix = p;
-        if (tile == tiles - 1) st_agent(&st->result[0], (uint64_t)p + all);
+        if (tile == tiles - 1) st_agent(&st->result, (uint64_t)p + all);
       }
     }
     __syncthreads();
@@ -449,7 +449,7 @@ __global__ __launch_bounds__(kScanThreads, waves_per_eu(kScanBlocks)) void k_mer
         if (l == 0) {
           s_pre_heads = ph;
           s_pre_or = po;
-          if (tile == tiles - 1) st_agent(&st->result[0], (uint64_t)ph + heads_all);
+          if (tile == tiles - 1) st_agent(&st->result, (uint64_t)ph + heads_all);
         }
       }
       // the first emitted run has index (heads before the tile) - 1 when it
@@ -563,8 +563,7 @@ __global__ __launch_bounds__(kScanThreads, waves_per_eu(kScanBlocks)) void k_col
           if (tile == tiles - 1) {
             counts->length = (uint64_t)pw + (all & 0xFFFFu);
             counts->keycnt = (uint64_t)ph + (all >> 16);
-            st_agent(&st->result[0], (uint64_t)ph + (all >> 16));
-            st_agent(&st->result[1], (uint64_t)pw + (all & 0xFFFFu));
+            st_agent(&st->result, (uint64_t)ph + (all >> 16));
           }
         }
       }

@@ -19,7 +19,6 @@
 #include "wahgpu.h"
 
 using wah::BuildArgs;
-using wah::ScanArgs;
 using wah::ScanRun;
 
 struct wahgpu_ctx {
@@ -298,31 +297,14 @@ void set_one(BuildArgs* a, uint64_t n, uint32_t rid_base, bool wide = false) {
   a->one = wah::Column{0, n, rid_base, 0u, 0u, 0u, 0u, wide ? 1u : 0u, 0u, 0u};
 }
 
-// Scan scratch, zeroed before use: tile-counter lanes (kLaneWords words),
-// then [fault u32, pad u32, result u64], then the u64 status words.
-struct ScanScratch {
-  uint32_t* base;
-  uint64_t words;
-  ScanArgs args;
-  uint32_t* header;  // fault, pad, result lo, result hi
-  uint64_t* result;
-};
-constexpr uint64_t kScanHeadWords = wah::kLaneWords + 8;
-uint64_t scan_scratch_bytes(uint64_t n) {
-  return align_up(kScanHeadWords * 4 + wah::scan_status_words(n) * 8);
-}
-ScanScratch carve_scan(wahgpu_ctx* c, uint64_t n) {
-  ScanScratch s;
-  uint64_t bytes = kScanHeadWords * 4 + wah::scan_status_words(n) * 8;
-  s.base = take<uint32_t>(c, bytes / 4);
-  s.words = bytes / 4;
-  s.args.tile_counter = s.base;
-  s.header = s.base + wah::kLaneWords;
-  s.args.fault = s.header;
-  s.result = reinterpret_cast<uint64_t*>(s.header + 2);
-  s.args.status = reinterpret_cast<uint64_t*>(s.base + kScanHeadWords);
-  s.args.max_resident = c->max_resident;
-  return s;
+// Scans keep their state in the context and take nothing from the arena, but a
+// fixed arena still bounds what a call on its context may ask for: bytes a scan
+// of n elements counts as, and the check.
+uint64_t scan_scratch_bytes(uint64_t n) { return align_up(2080 + (n + 2047) / 2048 * 8); }
+int arena_limit(wahgpu_ctx* c, uint64_t bytes) {
+  if (!c->fixed || bytes <= c->arena_cap) return WAHGPU_OK;
+  return fail(c, WAHGPU_ENOMEM, "arena of " + std::to_string(c->arena_cap) +
+                                    " bytes is too small for " + std::to_string(bytes));
 }
 
 int check_n(wahgpu_ctx* c, uint64_t n, uint32_t rid_base) {
@@ -345,31 +327,20 @@ int read_counts(wahgpu_ctx* c, const wahgpu_counts* d_counts, wahgpu_counts* out
   return WAHGPU_OK;
 }
 
-// Reads a scan scratch header [fault, pad, result] and its result.
-int read_scan_result(wahgpu_ctx* c, const uint32_t* header, uint64_t* out) {
-  HIPCHK(c, hipMemcpyAsync(c->pinned_counts, header, 16, hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
-  uint32_t hdr[4];
-  memcpy(hdr, c->pinned_counts, 16);
-  if (hdr[0])
-    return fail(c, WAHGPU_EHIP, "kernel reported fault " + std::to_string(hdr[0]) +
-                                    " (look-back wait gave up or index out of range)");
-  memcpy(out, &hdr[2], 8);
-  return WAHGPU_OK;
-}
-
 // The context's scan state, for launches on its stream (one after another).
-// Results land in scan_host; a launch of no elements writes nothing, so they
-// start at zero.
+// Results land in scan_host: fault and result, two more words of a range query
+// (3 and 4), and those of a decode whose encode follows (5 and 6).  A launch of
+// no elements writes nothing, so they start at zero.
+constexpr int kScanHostWords = 8, kDecodeSlot = 5;
 ScanRun scan_run(wahgpu_ctx* c) {
-  memset(c->scan_host, 0, 3 * sizeof(uint64_t));
+  memset(c->scan_host, 0, kScanHostWords * sizeof(uint64_t));
   return ScanRun{c->scan_state, reinterpret_cast<uint64_t*>(c->scan_state + 1), c->scan_host,
                  c->cus};
 }
-// Waits for the stream and reads the result of its last scan.
-int scan_result(wahgpu_ctx* c, uint64_t* out) {
+// Waits for the stream and reads the result of the scan that wrote `slot`.
+int scan_result(wahgpu_ctx* c, uint64_t* out, int slot = 0) {
   HIPCHK(c, hipStreamSynchronize(c->stream));
-  const volatile uint64_t* h = c->scan_host;
+  const volatile uint64_t* h = c->scan_host + slot;
   if (h[0])
     return fail(c, WAHGPU_EHIP, "kernel reported fault " + std::to_string(h[0]) +
                                     " (look-back wait gave up or index out of range)");
@@ -1317,7 +1288,7 @@ int wahgpu_build_staged(wahgpu_ctx* c, const uint32_t* values, uint64_t n, uint3
   HIPCHK(c, hipSetDevice(c->device));
   uint64_t nn = n ? n : 1;
   uint64_t bytes = build_scratch_bytes(caps_one(n, shape_for(c, n))) + align_up(nn * 4) * 12 + align_up(2 * nn * 4) +
-                   align_up(sizeof(wahgpu_counts)) + 4 * scan_scratch_bytes(2 * nn);  // fixed arenas keep their limit
+                   align_up(sizeof(wahgpu_counts)) + 4 * scan_scratch_bytes(2 * nn);
   rc = arena_reserve(c, bytes);
   if (rc) return rc;
   auto t0 = std::chrono::steady_clock::now();
@@ -1470,7 +1441,7 @@ int wahgpu_merge_lit_by_val_chids(wahgpu_ctx* c, const uint32_t* d_values,
   int rc = check_n(c, n, 0);
   if (rc) return rc;
   HIPCHK(c, hipSetDevice(c->device));
-  rc = arena_reserve(c, scan_scratch_bytes(n));  // fixed arenas keep their limit
+  rc = arena_limit(c, scan_scratch_bytes(n));
   if (rc) return rc;
   ORDERED(c);
   wah::launch_merge(scan_run(c), d_values, d_chids, d_lits, n, d_values_out, d_chids_out,
@@ -1497,7 +1468,7 @@ int wahgpu_fuse_fill_literals(wahgpu_ctx* c, const uint32_t* d_fills, const uint
   int rc = check_n(c, k, 0);
   if (rc) return rc;
   HIPCHK(c, hipSetDevice(c->device));
-  rc = arena_reserve(c, scan_scratch_bytes(k));  // fixed arenas keep their limit
+  rc = arena_limit(c, scan_scratch_bytes(k));
   if (rc) return rc;
   ORDERED(c);
   wah::launch_compact(scan_run(c), d_fills, d_lits, k, 1, d_index, c->stream);
@@ -1515,7 +1486,6 @@ int wahgpu_compute_column_length(wahgpu_ctx* c, const uint32_t* d_values,
   int rc = check_n(c, k, 0);
   if (rc) return rc;
   HIPCHK(c, hipSetDevice(c->device));
-  // fixed arenas keep their limit
   rc = arena_reserve(c, scan_scratch_bytes(k) + align_up(sizeof(wahgpu_counts)));
   if (rc) return rc;
   wahgpu_counts* d_counts = take<wahgpu_counts>(c, 1);
@@ -1534,7 +1504,7 @@ int wahgpu_stream_compaction(wahgpu_ctx* c, const uint32_t* d_data, const uint32
   int rc = check_n(c, n, 0);
   if (rc) return rc;
   HIPCHK(c, hipSetDevice(c->device));
-  rc = arena_reserve(c, scan_scratch_bytes(n));  // fixed arenas keep their limit
+  rc = arena_limit(c, scan_scratch_bytes(n));
   if (rc) return rc;
   ORDERED(c);
   wah::launch_compact(scan_run(c), d_data, d_valid, n, 0, d_out, c->stream);
@@ -1549,7 +1519,7 @@ int wahgpu_exclusive_scan(wahgpu_ctx* c, const uint32_t* d_in, uint64_t n, uint3
   int rc = check_n(c, n, 0);
   if (rc) return rc;
   HIPCHK(c, hipSetDevice(c->device));
-  rc = arena_reserve(c, scan_scratch_bytes(n));  // fixed arenas keep their limit
+  rc = arena_limit(c, scan_scratch_bytes(n));
   if (rc) return rc;
   ORDERED(c);
   wah::launch_scan(scan_run(c), d_in, nullptr, n, d_out, false, c->stream);
@@ -1564,7 +1534,7 @@ int wahgpu_segmented_inclusive_scan(wahgpu_ctx* c, const uint32_t* d_in, const u
   int rc = check_n(c, n, 0);
   if (rc) return rc;
   HIPCHK(c, hipSetDevice(c->device));
-  rc = arena_reserve(c, scan_scratch_bytes(n));  // fixed arenas keep their limit
+  rc = arena_limit(c, scan_scratch_bytes(n));
   if (rc) return rc;
   ORDERED(c);
   wah::launch_scan(scan_run(c), d_in, d_heads, n, d_out, true, c->stream);
@@ -1608,6 +1578,11 @@ int wah_build_batch_ws(wahgpu_ctx* c, const uint32_t* d_values, uint64_t values_
 namespace {
 constexpr uint64_t kMaxRows = 1ull << 32;  // rows are uint32 (src/cpu.cpp:182)
 uint64_t bitmap_words(uint64_t nrows) { return (nrows + 31) / 32; }
+// Arena bytes an encode counts as (see arena_limit).
+uint64_t encode_scratch_bytes(uint64_t nrows) {
+  const uint64_t chunks = (nrows + 30) / 31;
+  return align_up((chunks + 2047) / 2048 * 24);
+}
 }  // namespace
 
 int wahgpu_decode_device(wahgpu_ctx* c, const uint32_t* d_words, uint64_t len, uint64_t nrows,
@@ -1617,25 +1592,17 @@ int wahgpu_decode_device(wahgpu_ctx* c, const uint32_t* d_words, uint64_t len, u
   if (nrows > kMaxRows || len > ((uint64_t)1 << 32))
     return fail(c, WAHGPU_ERANGE, "more than 2^32 rows or words");
   HIPCHK(c, hipSetDevice(c->device));
-  int rc = arena_reserve(c, scan_scratch_bytes(len) + kAlign);
+  int rc = arena_limit(c, scan_scratch_bytes(len) + kAlign);
   if (rc) return rc;
-  ScanScratch sc = carve_scan(c, len);
-  uint64_t* d_last = take<uint64_t>(c, 2);
   ORDERED(c);
-  wah::launch_fill32(sc.base, sc.words, 0, c->stream);
-  wah::launch_fill32(reinterpret_cast<uint32_t*>(d_last), 4, 0, c->stream);
-  if (nrows) wah::launch_fill32(d_bitmap, bitmap_words(nrows), 0, c->stream);
-  wah::launch_decode(sc.args, d_words, nullptr, len, d_bitmap, nrows, d_last, c->stream);
+  wah::launch_fill32(d_bitmap, bitmap_words(nrows), 0, c->stream);
+  wah::launch_decode(scan_run(c), {d_words, len, d_bitmap}, {nullptr, 0, nullptr}, nrows, c->stream);
   LAUNCHCHK(c);
-  uint64_t unused;
+  uint64_t last = 0;
   order_guard_.end();  // no host wait holds the device order
-  rc = read_scan_result(c, sc.header, &unused);  // fault word (synchronizes)
+  rc = scan_result(c, &last);
   if (rc) return rc;
-  if (last_row) {
-    HIPCHK(c, hipMemcpyAsync(c->pinned_counts, d_last, 8, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    memcpy(last_row, c->pinned_counts, 8);
-  }
+  if (last_row) *last_row = last;
   return WAHGPU_OK;
 }
 
@@ -1648,36 +1615,24 @@ int wahgpu_query_range_device(wahgpu_ctx* c, const uint32_t* d_keys, const uint3
     return fail(c, WAHGPU_EINVAL, "null buffer");
   if (nrows > kMaxRows) return fail(c, WAHGPU_ERANGE, "more than 2^32 rows");
   HIPCHK(c, hipSetDevice(c->device));
-  if (nrows) wah::launch_fill32(d_bitmap, bitmap_words(nrows), 0, c->stream);
   if (keys_matched) *keys_matched = 0;
-  if (!keycnt || lo > hi) return WAHGPU_OK;
-  int rc = arena_reserve(c, align_up(4 * 8));
+  if (!keycnt || lo > hi) {
+    wah::launch_fill32(d_bitmap, bitmap_words(nrows), 0, c->stream);
+    return WAHGPU_OK;
+  }
+  int rc = arena_limit(c, align_up(4 * 8));
   if (rc) return rc;
-  uint64_t* d_range = take<uint64_t>(c, 4);
-  wah::launch_key_range(d_keys, d_offsets, d_lengths, keycnt, lo, hi, d_range, c->stream);
-  LAUNCHCHK(c);
-  uint64_t range[4];
-  HIPCHK(c, hipMemcpyAsync(c->pinned_counts, d_range, 32, hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
-  memcpy(range, c->pinned_counts, 32);
-  if (keys_matched) *keys_matched = range[1] - range[0];
-  const uint64_t w0 = range[2], len = range[3] - range[2];
-  if (range[1] <= range[0] || len == 0) return WAHGPU_OK;
-  // the selected keys' words are contiguous: decode them as one stream whose
-  // segments restart at each key's first word
-  rc = arena_reserve(c, scan_scratch_bytes(len) + align_up(len * 4));
-  if (rc) return rc;
-  ScanScratch sc = carve_scan(c, len);
-  uint32_t* heads = take<uint32_t>(c, len);
   ORDERED(c);
-  wah::launch_fill32(sc.base, sc.words, 0, c->stream);
-  wah::launch_fill32(heads, len, 0, c->stream);
-  wah::launch_mark_heads(d_offsets, range[0], range[1], w0, heads, c->stream);
-  wah::launch_decode(sc.args, d_words + w0, heads, len, d_bitmap, nrows, nullptr, c->stream);
+  wah::launch_range(scan_run(c), d_keys, d_offsets, d_lengths, keycnt, d_words, lo, hi, d_bitmap,
+                    nrows, c->stream);
   LAUNCHCHK(c);
   uint64_t unused;
   order_guard_.end();  // no host wait holds the device order
-  return read_scan_result(c, sc.header, &unused);
+  rc = scan_result(c, &unused);
+  if (rc) return rc;
+  if (keys_matched) *keys_matched = c->scan_host[3];
+  const uint64_t words = c->scan_host[4];
+  return words ? arena_limit(c, scan_scratch_bytes(words) + align_up(words * 4)) : WAHGPU_OK;
 }
 
 int wahgpu_encode_device(wahgpu_ctx* c, const uint32_t* d_bitmap, uint64_t nrows,
@@ -1688,16 +1643,14 @@ int wahgpu_encode_device(wahgpu_ctx* c, const uint32_t* d_bitmap, uint64_t nrows
   HIPCHK(c, hipSetDevice(c->device));
   *len = 0;
   if (!nrows) return WAHGPU_OK;
-  const uint64_t tiles = wah::encode_tiles(nrows);
-  int rc = arena_reserve(c, align_up(tiles * 24) + kAlign);
+  int rc = arena_limit(c, encode_scratch_bytes(nrows) + kAlign);
   if (rc) return rc;
-  uint64_t* tile_sum = take<uint64_t>(c, 3 * tiles);
-  uint64_t* d_len = take<uint64_t>(c, 1);
-  wah::launch_encode(d_bitmap, nullptr, 4, nrows, tile_sum, d_words, cap, d_len, c->stream);
+  ORDERED(c);
+  wah::launch_encode(scan_run(c), d_bitmap, nullptr, 0, nrows, d_words, cap, c->stream);
   LAUNCHCHK(c);
-  HIPCHK(c, hipMemcpyAsync(c->pinned_counts, d_len, 8, hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
-  memcpy(len, c->pinned_counts, 8);
+  order_guard_.end();  // no host wait holds the device order
+  rc = scan_result(c, len);
+  if (rc) return rc;
   if (*len > cap) return fail(c, WAHGPU_EINVAL, "output capacity too small: " +
                                                     std::to_string(*len) + " words");
   return WAHGPU_OK;
@@ -1715,33 +1668,26 @@ int wahgpu_combine_device(wahgpu_ctx* c, int op, const uint32_t* d_a, uint64_t l
   HIPCHK(c, hipSetDevice(c->device));
   *len = 0;
   if (!nrows) return WAHGPU_OK;
-  const uint64_t bw = bitmap_words(nrows), tiles = wah::encode_tiles(nrows);
+  const uint64_t bw = bitmap_words(nrows);
   int rc = arena_reserve(c, 2 * align_up(bw * 4) + scan_scratch_bytes(la) +
-                                scan_scratch_bytes(lb) + align_up(tiles * 24) + kAlign);
+                                scan_scratch_bytes(lb) + encode_scratch_bytes(nrows) + kAlign);
   if (rc) return rc;
   uint32_t* bm_a = take<uint32_t>(c, bw);
   uint32_t* bm_b = take<uint32_t>(c, bw);
-  ScanScratch sa = carve_scan(c, la), sb = carve_scan(c, lb);
-  uint64_t* tile_sum = take<uint64_t>(c, 3 * tiles);
-  uint64_t* d_len = take<uint64_t>(c, 1);
   ORDERED(c);
-  wah::launch_fill32(sa.base, sa.words, 0, c->stream);
-  wah::launch_fill32(sb.base, sb.words, 0, c->stream);
-  wah::launch_fill32(bm_a, bw, 0, c->stream);
-  wah::launch_fill32(bm_b, bw, 0, c->stream);
-  wah::launch_decode(sa.args, d_a, nullptr, la, bm_a, nrows, nullptr, c->stream);
-  wah::launch_decode(sb.args, d_b, nullptr, lb, bm_b, nrows, nullptr, c->stream);
-  wah::launch_encode(bm_a, bm_b, op, nrows, tile_sum, d_out, cap, d_len, c->stream);
+  wah::launch_fill32(bm_a, (uint64_t)(bm_b - bm_a) + bw, 0, c->stream);  // both, and the gap
+  ScanRun run = scan_run(c);
+  run.host += kDecodeSlot;  // the encode's results follow in the first slot
+  wah::launch_decode(run, {d_a, la, bm_a}, {d_b, lb, bm_b}, nrows, c->stream);
   LAUNCHCHK(c);
-  uint64_t unused;
+  run.host -= kDecodeSlot;
+  wah::launch_encode(run, bm_a, bm_b, op, nrows, d_out, cap, c->stream);
+  LAUNCHCHK(c);
   order_guard_.end();  // no host wait holds the device order
-  rc = read_scan_result(c, sa.header, &unused);
+  uint64_t unused;
+  rc = scan_result(c, &unused, kDecodeSlot);
+  if (!rc) rc = scan_result(c, len);
   if (rc) return rc;
-  rc = read_scan_result(c, sb.header, &unused);
-  if (rc) return rc;
-  HIPCHK(c, hipMemcpyAsync(c->pinned_counts, d_len, 8, hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
-  memcpy(len, c->pinned_counts, 8);
   if (*len > cap) return fail(c, WAHGPU_EINVAL, "output capacity too small: " +
                                                     std::to_string(*len) + " words");
   return WAHGPU_OK;

@@ -1,0 +1,124 @@
+"""Decode, encode and combine where their tiles end and where a literal meets
+words the builds never write: streams of a decode tile's words (4096) give or
+take one, bitmaps of an encode tile's chunks (4096) give or take a row, 1-fills
+and fills of no chunks beside literals, rows past nrows, and outputs one word
+short.  Whole numbers: results are equal or wrong.
+"""
+import numpy as np
+import pytest
+
+from indexing_amd import WahError
+from tests.test_gpu_query import bitmap_rows, canonical_words, rows_to_bitmap
+from tests.test_gpu_scan import dev, u32
+
+pytestmark = pytest.mark.gpu
+
+
+def decode_rows(words):
+    """Rows of a word stream, from the word format alone."""
+    rows, chunk = [], 0
+    for w in np.asarray(words, np.uint64).tolist():
+        if w & 0x80000000:
+            rows += [31 * chunk + b for b in range(31) if (w >> b) & 1]
+            chunk += 1
+        else:
+            n = w & 0x3FFFFFFF
+            if w & 0x40000000:
+                rows += range(31 * chunk, 31 * (chunk + n))
+            chunk += n
+    return np.array(rows, np.int64), chunk
+
+
+def stream(n, seed, odd):
+    """n words: literals in runs (their bitmap words are shared), 0-fills, and
+    if odd 1-fills, fills of no chunks and empty literals among them."""
+    rng = np.random.default_rng(seed)
+    lit = (rng.integers(0, 1 << 31, n) | 0x80000000).astype(np.uint32)
+    one = ((1 << rng.integers(0, 31, n)) | 0x80000000).astype(np.uint32)
+    fill = rng.integers(1, 40, n).astype(np.uint32)
+    pick = rng.random(n)
+    w = np.where(pick < 0.4, lit, np.where(pick < 0.7, one, fill))
+    if odd:
+        kind = rng.random(n)
+        w = np.where(kind < 0.05, fill | 0x40000000, w)
+        w = np.where((kind >= 0.05) & (kind < 0.10), np.uint32(0), w)
+        w = np.where((kind >= 0.10) & (kind < 0.15), np.uint32(0x80000000), w)
+        w = np.where((kind >= 0.15) & (kind < 0.18), np.uint32(0x40000000), w)
+    return w.astype(np.uint32)
+
+
+@pytest.mark.parametrize("odd", [False, True], ids=["canonical", "odd"])
+@pytest.mark.parametrize("n", [1, 2, 255, 256, 257, 511, 513, 4095, 4096, 4097, 12289])
+def test_decode_streams(ctx, n, odd):
+    words = stream(n, 10 * n + odd, odd)
+    rows, chunks = decode_rows(words)
+    for nrows in sorted({max(1, 31 * chunks), max(1, 31 * chunks - 17), max(1, 31 * chunks // 2),
+                         31 * chunks + 100, 1}):
+        print(f"[decode] n={n} odd={odd} nrows={nrows}", flush=True)
+        bm, last = ctx.decode_device(dev(words, n % 4), nrows)
+        assert np.array_equal(bitmap_rows(u32(bm), nrows), rows[rows < nrows])
+        assert not bitmap_rows(u32(bm), u32(bm).size * 32)[rows[rows < nrows].size:].size
+        assert last == (int(rows[-1]) + 1 if rows.size else 0)
+
+
+@pytest.mark.parametrize("chunks", [511, 512, 513, 4095, 4096, 4097, 8193])
+@pytest.mark.parametrize("extra", [-30, -1, 0, 1])
+def test_encode_at_tile_ends(ctx, chunks, extra):
+    n = 31 * chunks + extra
+    rng = np.random.default_rng(n)
+    # nothing, the last row alone, the first chunk of the last tile alone, dense
+    # up to the tile's end, scattered
+    for rows in ([], [n - 1], [min(n - 1, 31 * (chunks // 4096 * 4096))], np.arange(n),
+                 np.flatnonzero(rng.random(n) < 0.01), np.flatnonzero(rng.random(n) < 0.3)):
+        want = canonical_words(rows)
+        print(f"[encode] rows={n} set={len(rows)}", flush=True)
+        got = ctx.encode_device(dev(rows_to_bitmap(rows, n), n % 3), n)
+        assert np.array_equal(u32(got), want)
+        if want.size > 1:
+            with pytest.raises(WahError):
+                ctx.encode_device(dev(rows_to_bitmap(rows, n)), n, cap=want.size - 1)
+
+
+def test_encode_ignores_rows_past_the_end_and_writes_none_past_cap(ctx):
+    import ctypes
+
+    import torch
+
+    from indexing_amd import _ptr
+    n = 31 * 5000 + 7
+    bits = np.full((n + 31) // 32, 0xFFFFFFFF, np.uint32)
+    assert np.array_equal(u32(ctx.encode_device(dev(bits), n)), canonical_words(np.arange(n)))
+    out = torch.full((6000,), 7, dtype=torch.int32, device="cuda:0")
+    length = ctypes.c_uint64(0)
+    ctx._bind_stream()
+    rc = ctx._lib.wahgpu_encode_device(ctx._h, _ptr(dev(bits)), n, _ptr(out), 4990,
+                                       ctypes.byref(length))
+    assert rc != 0 and length.value == 5001
+    assert bool((out[4990:] == 7).all()) and bool((out[:4990] != 7).all())
+
+
+@pytest.mark.parametrize("op", ["and", "or", "xor", "andnot"])
+def test_combine_of_unequal_streams(ctx, op):
+    a, b = stream(4097, 1, True), stream(300, 2, False)
+    for x, y in ((a, b), (b, a), (a, b[:0]), (b[:0], a)):
+        (rx, cx), (ry, cy) = decode_rows(x), decode_rows(y)
+        n = 31 * max(cx, cy) - 5
+        sx, sy = (np.isin(np.arange(n), r) for r in (rx, ry))
+        want = {"and": sx & sy, "or": sx | sy, "xor": sx ^ sy, "andnot": sx & ~sy}[op]
+        got = ctx.combine_device(op, dev(x), dev(y), n, cap=2 * (n // 31 + 1))
+        assert np.array_equal(u32(got), canonical_words(np.flatnonzero(want)))
+
+
+@pytest.mark.parametrize("card", [2, 97, 5000])
+def test_range_over_many_keys_per_tile(ctx, card):
+    rng = np.random.default_rng(card)
+    n = 200_003
+    v = rng.integers(0, card, n).astype(np.uint32)
+    idx = ctx.build(v)
+    k, o, ln, w = (dev(x) for x in (idx.keys, idx.offsets, idx.lengths, idx.words))
+    for lo, hi in ((0, card), (card // 3, card // 2), (card - 1, card - 1), (card, card + 9),
+                   (1, 0xFFFFFFFF), (5, 4)):
+        bm, m = ctx.query_range_device(k, o, ln, w, lo, hi, n)
+        sel = (v >= lo) & (v <= hi)
+        assert np.array_equal(bitmap_rows(u32(bm), n), np.flatnonzero(sel))
+        assert m == np.unique(v[sel]).size
