@@ -202,13 +202,18 @@ __global__ __launch_bounds__(kScanThreads, query_waves_per_eu(kDecBlocks)) void 
         const uint32_t h4 = (hb >> (4 * r)) & 15u;
         const uint32_t p1 = word_chunks(x[r].x), p2 = p1 + word_chunks(x[r].y),
                        p3 = p2 + word_chunks(x[r].z), s = p3 + word_chunks(x[r].w);
-        const uint32_t inc = wave_incl_add(s);
-        const uint32_t ex = run + inc - s;
         if (!SEG) {
-          y[r] = W4{ex, ex + p1, ex + p2, ex + p3};
-          run += readlane(inc, kWave - 1);
+          // saturating: a literal far past nrows stays there
+          const uint32_t q1 = word_chunks(x[r].x), q2 = add_sat(q1, word_chunks(x[r].y)),
+                         q3 = add_sat(q2, word_chunks(x[r].z));
+          const uint32_t sat = wave_incl_add_sat(add_sat(q3, word_chunks(x[r].w)));
+          const uint32_t e0 = add_sat(run, lane_before(sat, 0u));
+          y[r] = W4{e0, add_sat(e0, q1), add_sat(e0, q2), add_sat(e0, q3)};
+          run = add_sat(run, readlane(sat, kWave - 1));
           continue;
         }
+        const uint32_t inc = wave_incl_add(s);
+        const uint32_t ex = run + inc - s;
         const uint32_t b = ex + (h4 & 8u ? p3 : h4 & 4u ? p2 : h4 & 2u ? p1 : 0u);
         const uint64_t hm = ballot(h4 != 0u);
         const uint64_t below = hm & ((1ull << l) - 1ull);
@@ -247,16 +252,17 @@ __global__ __launch_bounds__(kScanThreads, query_waves_per_eu(kDecBlocks)) void 
           closed = tile_closed;
         }
         const bool h = SEG && s_head[i] != 0u;
-        agg = h ? s_sum[i] : agg + s_sum[i];
+        agg = h ? s_sum[i] : SEG ? agg + s_sum[i] : add_sat(agg, s_sum[i]);
         tile_closed |= h;
       }
       if (w == 0) {
         uint32_t hi, p;
-        lookback2<kOpNone, kOpSum>(status, tile, 0u, agg, tile_closed, &st->fault, hi, p, first);
+        lookback2<kOpNone, SEG ? kOpSum : kOpSumSat>(status, tile, 0u, agg, tile_closed,
+                                                     &st->fault, hi, p, first);
         if (l == 0) s_prefix = p;
       }
       __syncthreads();
-      if (!closed) carry += s_prefix;
+      if (!closed) carry = SEG ? carry + s_prefix : add_sat(carry, s_prefix);
       // the words before and after the wave's (a single stream's first word
       // has a 0-fill before it, its last word an open one after it)
       uint32_t wb = 1u, wa = 0u;
@@ -278,7 +284,8 @@ __global__ __launch_bounds__(kScanThreads, query_waves_per_eu(kDecBlocks)) void 
         const uint32_t ys[4] = {y[r].x, y[r].y, y[r].z, y[r].w};
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
-          const uint32_t c = ys[k] + (!SEG || ((openm >> (4 * r + k)) & 1u) ? carry : 0u);
+          const uint32_t c = SEG ? ys[k] + ((openm >> (4 * r + k)) & 1u ? carry : 0u)
+                                 : add_sat(ys[k], carry);
           const uint32_t v = xs[k];  // past the stream's end: 0, a fill of nothing
           if (v & 0x80000000u) {
             const uint32_t bits = v & 0x7FFFFFFFu;

@@ -67,6 +67,19 @@ __device__ __forceinline__ uint32_t wave_max(uint32_t x) {
 __device__ __forceinline__ uint32_t wave_sum(uint32_t x) {
   return readlane(wave_incl_add(x), kWave - 1);
 }
+// Sums that stop at 2^32 - 1 instead of wrapping.
+__device__ __forceinline__ uint32_t add_sat(uint32_t a, uint32_t b) {
+  return __builtin_elementwise_add_sat(a, b);
+}
+__device__ __forceinline__ uint32_t wave_incl_add_sat(uint32_t x) {
+  x = add_sat(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xF, 0xF, true));   // row_shr:1
+  x = add_sat(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xF, 0xF, true));   // row_shr:2
+  x = add_sat(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xF, 0xF, true));   // row_shr:4
+  x = add_sat(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xF, 0xF, true));   // row_shr:8
+  x = add_sat(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x142, 0xA, 0xF, false));  // row_bcast:15
+  x = add_sat(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x143, 0xC, 0xF, false));  // row_bcast:31
+  return x;
+}
 // Lane l - 1's x (lane 0: first), lane l + 1's x (lane 63: last).
 __device__ __forceinline__ uint32_t lane_before(uint32_t x, uint32_t first) {
   return (uint32_t)__builtin_amdgcn_update_dpp((int)first, (int)x, 0x138, 0xF, 0xF, false);
@@ -81,6 +94,7 @@ constexpr int kOpNone = 0;
 constexpr int kOpSum = 1;
 constexpr int kOpMax = 2;
 constexpr int kOpOrSinceHi = 3;  // lo: OR from the last tile with hi != 0 on
+constexpr int kOpSumSat = 4;     // lo: sum, 2^32 - 1 at most
 
 // Run by a whole wave: publishes the tile's (hi, lo) and returns the
 // combination over tiles first .. tile - 1, reading 64 predecessors per round
@@ -122,6 +136,7 @@ __device__ __forceinline__ void lookback2(uint64_t* status, uint32_t tile, uint3
     const uint32_t h = take ? (uint32_t)((s >> 32) & kHiMask) : 0u;
     const uint32_t v = take ? (uint32_t)s : 0u;
     if (LO == kOpSum) al += wave_sum(v);
+    if (LO == kOpSumSat) al = add_sat(al, readlane(wave_incl_add_sat(v), kWave - 1));
     if (LO == kOpOrSinceHi && or_open) {
       const uint64_t hm = ballot(h != 0u);
       const uint64_t upto = hm ? (hm ^ (hm - 1)) : ~0ull;
@@ -141,6 +156,7 @@ __device__ __forceinline__ void lookback2(uint64_t* status, uint32_t tile, uint3
     if (HI == kOpSum) ih = ah + hi;
     if (HI == kOpMax) ih = hi > ah ? hi : ah;
     if (LO == kOpSum) il = al + lo;
+    if (LO == kOpSumSat) il = add_sat(al, lo);
     if (LO == kOpOrSinceHi) il = hi ? lo : al | lo;
     st_agent(&status[tile], ((uint64_t)kFlagPrefix << 62) | ((ih & kHiMask) << 32) | il);
   }

@@ -61,6 +61,13 @@ def test_decode_streams(ctx, n, odd):
         assert last == (int(rows[-1]) + 1 if rows.size else 0)
 
 
+def test_decode_drops_what_lies_past_every_row(ctx):
+    """Fills that sum past 2^32 chunks: what follows them lies past nrows."""
+    words = np.concatenate([[0x80000005], np.full(6, 0x3FFFFFFF), [0x80000003] * 5000])
+    bm, _ = ctx.decode_device(dev(words.astype(np.uint32)), 100_000)
+    assert bitmap_rows(u32(bm), 100_000).tolist() == [0, 2]
+
+
 @pytest.mark.parametrize("chunks", [511, 512, 513, 4095, 4096, 4097, 8193])
 @pytest.mark.parametrize("extra", [-30, -1, 0, 1])
 def test_encode_at_tile_ends(ctx, chunks, extra):
