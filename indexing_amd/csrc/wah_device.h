@@ -109,6 +109,16 @@ __device__ __forceinline__ uint32_t next_tile(uint32_t* counters, uint32_t lanes
   return *s_tile;
 #endif
 }
+// Group of a launch over `tiles` tiles: `group` where the blocks draw several
+// tiles each.  Where there is a block for every tile, the tiles are dealt to
+// the lanes in equal runs, so that each lane has as many tiles as blocks (a
+// grid of a multiple of the lanes): with runs of 8, 18 tiles lay in three
+// lanes of 2 or 3 blocks, which took them in turn while the other lanes'
+// blocks found nothing (a radix pass over 300,007 rows 41 us, over 2^20 rows
+// 14 us).
+__device__ __forceinline__ uint32_t tile_group(uint32_t tiles, uint32_t lanes, uint32_t group) {
+  return tiles <= gridDim.x ? (tiles + lanes - 1) / lanes : group;
+}
 // Counter lanes for a grid of `grid` blocks.
 __host__ __device__ __forceinline__ uint32_t tile_lanes(uint32_t grid) {
   return grid < kTileLanes ? (grid ? grid : 1u) : kTileLanes;

@@ -695,14 +695,12 @@ __global__ __launch_bounds__(THREADS, sort_waves_per_eu(ITEMS)) void k_onesweep(
   constexpr int TILE = THREADS * ITEMS;
   constexpr int WAVES = THREADS / kWave;
   static_assert(THREADS >= 256 && THREADS % 256 == 0, "one thread per digit");
-  static_assert(ITEMS <= 32, "participation bits");
   static_assert(TILE <= 65536, "LDS slots packed in 16 bits");
   __shared__ uint32_t s_stage[TILE];
   __shared__ uint32_t s_wcnt[WAVES][256];
   __shared__ uint32_t s_excl[256];
   __shared__ uint32_t s_glob[256];
   __shared__ uint32_t s_dsum[4];
-  __shared__ uint32_t s_tilen;
   __shared__ uint32_t s_tile;
 
   // pair mode: launch 0 reads the values (rids implicit); run mode: the run
@@ -728,7 +726,7 @@ __global__ __launch_bounds__(THREADS, sort_waves_per_eu(ITEMS)) void k_onesweep(
   for (;;) {
     for (int i = t; i < WAVES * 256; i += THREADS) (&s_wcnt[0][0])[i] = 0;
     const uint32_t tile = __builtin_amdgcn_readfirstlane(
-        next_tile(counter, lanes, &s_tile, iter, WAH_SORT_TILE_GROUP));
+        next_tile(counter, lanes, &s_tile, iter, tile_group(dims.sort_tiles, lanes, WAH_SORT_TILE_GROUP)));
     if (tile >= dims.sort_tiles) break;
     const uint32_t c = find_segment(&cols[0].sort_tile0, sizeof(Column) / 4, dims.ncols, tile);
     const ColState* col = &cs[c];
@@ -752,8 +750,12 @@ __global__ __launch_bounds__(THREADS, sort_waves_per_eu(ITEMS)) void k_onesweep(
     const bool narrow = col->narrow != 0u, src_narrow = narrow && !implicit && !(RUN && a == 0);
     if (t < 256) status_next[(uint64_t)tile * 256 + t] = 0;  // next launch's state
     const uint64_t wbase = base + (uint64_t)w * kWave * ITEMS + l;
-    // A full tile runs a straight-line body (no per-item guards), so the
-    // compiler can wait for the rid loads without draining the key stores.
+    // The body is straight-line, so the compiler can wait for the rid loads
+    // without draining the key stores, and the ranking atomics issue back to
+    // back.  A column's last tile runs it too: items past its end read the
+    // last one, count in a word of their own instead of a digit's, and keep
+    // their own index as their slot (they are the tile's last in input order,
+    // so those slots lie past tile_n), which nothing stores.
     // PACKED: launch 0 of a pair-mode column with keys < 2^16.  Its rids are
     // implicit (rid_base + column row), so one LDS word carries both the key
     // (high half) and the row's tile-local index (low half): one staging
@@ -764,45 +766,47 @@ __global__ __launch_bounds__(THREADS, sort_waves_per_eu(ITEMS)) void k_onesweep(
       // Keys only for now: the rids are loaded once the keys are staged, so
       // they never occupy registers during ranking and look-back.
       uint32_t key[ITEMS], rank[ITEMS];
-      const uint32_t nvalid =
-          FULL ? (uint32_t)ITEMS * kWave : (uint32_t)(n > wbase ? n - wbase : 0);
+      // item i of an array of the column (indices fit 32 bits): one base and
+      // immediate offsets in a whole tile; past the column its last item
+      // (first: the lane's first item, opaque per array so that the clamped
+      // indices are formed again instead of spilled across the ranking)
+      const uint32_t j0 = (uint32_t)wbase, jl = (uint32_t)n - 1u;
+      auto item = [&](const auto* col0, int i, uint32_t first) -> uint32_t {
+        if (FULL) return (uint32_t)(col0 + wbase)[i * kWave];
+        const uint32_t j = first + (uint32_t)(i * kWave);
+        return (uint32_t)col0[j < jl ? j : jl];
+      };
       if (src_narrow) {
-        const uint16_t* kp = reinterpret_cast<const uint16_t*>(src_keys + cd.off) + wbase;
+        const uint16_t* kp = reinterpret_cast<const uint16_t*>(src_keys + cd.off);
 #pragma unroll
-        for (int i = 0; i < ITEMS; ++i)
-          key[i] = FULL || (uint32_t)(i * kWave) < nvalid ? (uint32_t)kp[i * kWave] : 0u;
+        for (int i = 0; i < ITEMS; ++i) key[i] = item(kp, i, j0);
       } else {
-        const uint32_t* kp = src_keys + cd.off + wbase;  // one base, immediate offsets
+        const uint32_t* kp = src_keys + cd.off;
 #pragma unroll
-        for (int i = 0; i < ITEMS; ++i)
-          key[i] = FULL || (uint32_t)(i * kWave) < nvalid ? kp[i * kWave] : 0u;
+        for (int i = 0; i < ITEMS; ++i) key[i] = item(kp, i, j0);
       }
-      uint32_t part = 0;  // items this lane ranks
-#pragma unroll
-      for (int i = 0; i < ITEMS; ++i)
-        part |= (FULL || (uint32_t)(i * kWave) < nvalid ? 1u : 0u) << i;
+      const uint32_t tile_n = FULL ? (uint32_t)TILE : (uint32_t)(n - base);
       // Rank: peers = lanes with the same digit (8 ballots); rank = peers
       // below this lane + keys of that digit the wave ranked before.
 #pragma unroll
       for (int i = 0; i < ITEMS; ++i) {
-        if (FULL || ((part >> i) & 1u)) {
-          const uint32_t d = (key[i] >> shift) & 255u;
-          if (RANK == kRankAtomic) {
-            rank[i] = atomicAdd(&s_wcnt[w][d], 1u);
-          } else {
-            uint64_t peers = ballot(true);
+        const uint32_t d = (key[i] >> shift) & 255u;
+        const bool in = FULL || j0 + (uint32_t)(i * kWave) <= jl;
+        if (RANK == kRankAtomic) {
+          rank[i] = atomicAdd(in ? &s_wcnt[w][d] : &s_stage[t], 1u);
+        } else {
+          uint64_t peers = ballot(in);
 #pragma unroll
-            for (int b = 0; b < 8; ++b) {
-              const bool bit = (d >> b) & 1u;
-              const uint64_t bb = ballot(bit);
-              peers &= bit ? bb : ~bb;
-            }
-            const uint32_t cnt = (uint32_t)__popcll(peers);
-            const uint32_t below = mbcnt(peers);
-            const uint32_t prior = s_wcnt[w][d];
-            rank[i] = prior + below;
-            if (below == cnt - 1) s_wcnt[w][d] = prior + cnt;
+          for (int b = 0; b < 8; ++b) {
+            const bool bit = (d >> b) & 1u;
+            const uint64_t bb = ballot(bit);
+            peers &= bit ? bb : ~bb;
           }
+          const uint32_t cnt = (uint32_t)__popcll(peers);
+          const uint32_t below = mbcnt(peers);
+          const uint32_t prior = s_wcnt[w][d];
+          rank[i] = prior + below;
+          if (in && below == cnt - 1) s_wcnt[w][d] = prior + cnt;
         }
       }
       __syncthreads();
@@ -840,7 +844,6 @@ __global__ __launch_bounds__(THREADS, sort_waves_per_eu(ITEMS)) void k_onesweep(
         for (int i = 0; i < 4; ++i) before += i < w ? s_dsum[i] : 0u;
         const uint32_t ex = s_excl[t] + before;
         s_glob[t] -= ex;  // column index = s_glob[d] + local index
-        if (t == 255) s_tilen = ex + total;
         // each wave's first slot for digit t: one LDS read per key below
         uint32_t xw[WAVES];
 #pragma unroll
@@ -853,21 +856,19 @@ __global__ __launch_bounds__(THREADS, sort_waves_per_eu(ITEMS)) void k_onesweep(
         const uint32_t row0 = (uint32_t)(wbase - base);  // tile-local index of item 0
 #pragma unroll
         for (int i = 0; i < ITEMS; ++i) {
-          if (FULL || ((part >> i) & 1u)) {
-            const uint32_t d = (key[i] >> shift) & 255u;
-            s_stage[s_wcnt[w][d] + rank[i]] = key[i] << 16 | (row0 + (uint32_t)(i * kWave));
-          }
+          const uint32_t d = (key[i] >> shift) & 255u, row = row0 + (uint32_t)(i * kWave);
+          const uint32_t pos = s_wcnt[w][d] + rank[i];
+          s_stage[FULL || row < tile_n ? pos : row] = key[i] << 16 | row;
         }
         __syncthreads();
-        const uint32_t tile_n = FULL ? (uint32_t)TILE : s_tilen;
         uint16_t* dk16 = reinterpret_cast<uint16_t*>(dst_keys + cd.off);
         uint32_t* dr = dst_rids + cd.off;
         const uint32_t last = (uint32_t)(n_out - 1);  // stores stay in the column
         const uint32_t rid0 = cd.rid_base + (uint32_t)base;
         bool bad = false;
         // the staged words, then their digits' offsets, then the stores: each
-        // batch of LDS reads issues back to back (slots past tile_n read
-        // in-bounds stale words and store nothing)
+        // batch of LDS reads issues back to back (slots past tile_n hold the
+        // items past the column and store nothing)
         uint32_t xs[ITEMS], gs[ITEMS];
 #pragma unroll
         for (int j = 0; j < ITEMS; ++j) xs[j] = s_stage[(uint32_t)j * THREADS + t];
@@ -889,12 +890,11 @@ __global__ __launch_bounds__(THREADS, sort_waves_per_eu(ITEMS)) void k_onesweep(
       }
 #pragma unroll
       for (int i = 0; i < ITEMS; ++i) {
-        if (FULL || ((part >> i) & 1u)) {
-          const uint32_t d = (key[i] >> shift) & 255u;
-          const uint32_t pos = s_wcnt[w][d] + rank[i];
-          s_stage[pos] = key[i];
-          rank[i] = pos;  // keep the LDS slot for the rids
-        }
+        const uint32_t d = (key[i] >> shift) & 255u;
+        const uint32_t row = (uint32_t)(wbase - base) + (uint32_t)(i * kWave);
+        const uint32_t pos = FULL || row < tile_n ? s_wcnt[w][d] + rank[i] : row;
+        s_stage[pos] = key[i];
+        rank[i] = pos;  // keep the LDS slot for the rids
       }
       // LDS slots, two per register (a tile has at most 2^16 items)
       uint32_t slot2[(ITEMS + 1) / 2];
@@ -907,13 +907,12 @@ __global__ __launch_bounds__(THREADS, sort_waves_per_eu(ITEMS)) void k_onesweep(
 #pragma unroll
         for (int i = 0; i < ITEMS; ++i) rid[i] = cd.rid_base + (uint32_t)wbase + (uint32_t)(i * kWave);
       } else {
-        const uint32_t* rp = src_rids + cd.off + wbase;
+        const uint32_t* rp = src_rids + cd.off;
+        const uint32_t first = FULL ? j0 : opaque(j0);
 #pragma unroll
-        for (int i = 0; i < ITEMS; ++i)
-          rid[i] = FULL || (uint32_t)(i * kWave) < nvalid ? rp[i * kWave] : 0u;
+        for (int i = 0; i < ITEMS; ++i) rid[i] = item(rp, i, first);
       }
       __syncthreads();
-      const uint32_t tile_n = FULL ? (uint32_t)TILE : s_tilen;
       uint32_t* dk = dst_keys + cd.off;
       uint32_t* dr = dst_rids + cd.off;
       const uint32_t last = (uint32_t)(n_out - 1);  // stores stay in the column
@@ -923,8 +922,8 @@ __global__ __launch_bounds__(THREADS, sort_waves_per_eu(ITEMS)) void k_onesweep(
       uint32_t gq[ITEMS], kq[ITEMS];
       uint16_t* dk16 = reinterpret_cast<uint16_t*>(dk);
       // the staged keys, then their digits' offsets, then the stores: each
-      // batch of LDS reads issues back to back (slots past tile_n read
-      // in-bounds stale keys and store nothing)
+      // batch of LDS reads issues back to back (slots past tile_n hold the
+      // items past the column and store nothing)
 #pragma unroll
       for (int j = 0; j < ITEMS; ++j) kq[j] = s_stage[(uint32_t)j * THREADS + t];
 #pragma unroll
@@ -948,8 +947,13 @@ __global__ __launch_bounds__(THREADS, sort_waves_per_eu(ITEMS)) void k_onesweep(
       }
       __syncthreads();
 #pragma unroll
-      for (int i = 0; i < ITEMS; ++i)
-        if (FULL || ((part >> i) & 1u)) s_stage[(slot2[i / 2] >> (16 * (i % 2))) & 0xFFFFu] = rid[i];
+      for (int i = 0; i < ITEMS; ++i) s_stage[(slot2[i / 2] >> (16 * (i % 2))) & 0xFFFFu] = rid[i];
+      if (RUN) {  // literal bits: issued now, in flight while the rids go out
+        const uint32_t* lp = src_lits + cd.off;
+        const uint32_t first = FULL ? j0 : opaque(j0);
+#pragma unroll
+        for (int i = 0; i < ITEMS; ++i) rid[i] = item(lp, i, first);
+      }
       __syncthreads();
 #pragma unroll
       for (int j = 0; j < ITEMS; ++j) kq[j] = s_stage[(uint32_t)j * THREADS + t];
@@ -959,10 +963,9 @@ __global__ __launch_bounds__(THREADS, sort_waves_per_eu(ITEMS)) void k_onesweep(
       if (RUN) {
         // literal bits of each run item, moved along with its key and rid
         __syncthreads();
-        const uint32_t* lp = src_lits + cd.off + wbase;  // one base, immediate offsets
 #pragma unroll
         for (int i = 0; i < ITEMS; ++i)
-          if (FULL || ((part >> i) & 1u)) s_stage[(slot2[i / 2] >> (16 * (i % 2))) & 0xFFFFu] = lp[i * kWave];
+          s_stage[(slot2[i / 2] >> (16 * (i % 2))) & 0xFFFFu] = rid[i];
         __syncthreads();
         uint32_t* dl = dst_lits + cd.off;
 #pragma unroll
@@ -1155,7 +1158,7 @@ __global__ __launch_bounds__(kWideThreads, sort_waves_per_eu(kWideItems)) void k
   for (;;) {
     for (int i = t; i < WAVES * (int)kWideBins / 2; i += THREADS) (&s_cnt[0][0])[i] = 0;
     const uint32_t tile = __builtin_amdgcn_readfirstlane(
-        next_tile(counter, lanes, &s_tile, iter, WAH_SORT_TILE_GROUP));
+        next_tile(counter, lanes, &s_tile, iter, tile_group(dims.wide_tiles, lanes, WAH_SORT_TILE_GROUP)));
     if (tile >= dims.wide_tiles) break;
     const uint32_t c = find_segment(&cols[0].wide_tile0, sizeof(Column) / 4, dims.ncols, tile);
     const ColState* col = &cs[c];
@@ -1411,7 +1414,7 @@ __global__ __launch_bounds__(THREADS, tail_waves_per_eu(ITEMS)) void k_tail(
   for (;;) {
     const uint32_t tile = __builtin_amdgcn_readfirstlane(next_tile(
         &hdr->tiles[RUN ? kCounterRunTail : kCounterTail][0], lanes, &s_tile, iter,
-        WAH_TAIL_TILE_GROUP));
+        tile_group(dims.tail_tiles, lanes, WAH_TAIL_TILE_GROUP)));
     if (tile >= dims.tail_tiles) break;
     const uint32_t c = find_segment(&cols[0].tail_tile0, sizeof(Column) / 4, dims.ncols, tile);
     const Column cd = cols[c];
@@ -1853,6 +1856,12 @@ static uint32_t cap_grid(uint32_t work, uint32_t cap) {
   const uint32_t g = work < cap ? work : cap;
   return g ? g : 1u;
 }
+// Grid of a kernel that draws tiles: a whole number of blocks per counter lane
+// (see tile_group).
+static uint32_t tile_grid(uint32_t tiles, uint32_t cap) {
+  const uint32_t whole = tiles > kTileLanes ? (tiles + kTileLanes - 1) / kTileLanes * kTileLanes : tiles;
+  return cap_grid(whole, cap);
+}
 
 // Radix blocks resident per CU: the waves the register budget allows
 // (sort_waves_per_eu per SIMD) and the LDS of k_onesweep (staged keys,
@@ -1874,14 +1883,14 @@ constexpr uint32_t kWideBlocksPerCU = 2;
 // wide-digit launches when a column may take them).
 template <int T, int I>
 static void launch_radix(const BuildArgs& a, hipStream_t s, LaunchHook* hook) {
-  const uint32_t grid = cap_grid(a.sort_tiles_cap, WAH_STATIC_TILES
+  const uint32_t grid = tile_grid(a.sort_tiles_cap, WAH_STATIC_TILES
                                                        ? a.sort_tiles_cap
                                                        : a.max_resident / 4 * sort_blocks_per_cu<T, I>());
   hipLaunchKernelGGL(k_runcut, dim3(cap_grid(a.sort_tiles_cap, 2 * a.max_resident)), dim3(kBlock),
                      0, s, a.values, a.keysB, a.ridsB, a.litsB, a.desc, a.cs, a.hdr, a.tile_runs,
                      (uint32_t)(T * I));
   // wide digits: the histograms of the wide columns' digits and their offsets
-  const uint32_t wgrid = cap_grid(a.wide_tiles_cap, WAH_STATIC_TILES ? a.wide_tiles_cap
+  const uint32_t wgrid = tile_grid(a.wide_tiles_cap, WAH_STATIC_TILES ? a.wide_tiles_cap
                                                                     : a.max_resident / 4 * kWideBlocksPerCU);
   if (a.wide_tiles_cap) {
     uint64_t hb = (a.n_cap + 4 * kHistChunk - 1) / (4 * kHistChunk);
@@ -1952,7 +1961,7 @@ void launch_sort(const BuildArgs& a, hipStream_t s, LaunchHook* hook) {
 // Both tails of a long column, on 16384-item tiles.
 static void launch_long_tail(const BuildArgs& a, hipStream_t s) {
   const uint32_t grid =
-      cap_grid(a.tail_tiles_cap, WAH_STATIC_TILES ? a.tail_tiles_cap
+      tile_grid(a.tail_tiles_cap, WAH_STATIC_TILES ? a.tail_tiles_cap
                                                   : a.max_resident / 4 * kLongTailBlocksPerCU);
   const uint32_t lanes = WAH_TAIL_LANES ? WAH_TAIL_LANES : tile_lanes(grid);
   hipLaunchKernelGGL((k_tail<kLongTailThreads, kLongTailItems, false>), dim3(grid),
@@ -1968,7 +1977,7 @@ static void launch_long_tail(const BuildArgs& a, hipStream_t s) {
 // Both tails of other columns and of batches, on 8192-item tiles.
 static void launch_short_tail(const BuildArgs& a, hipStream_t s) {
   const uint32_t grid =
-      cap_grid(a.tail_tiles_cap, WAH_STATIC_TILES ? a.tail_tiles_cap
+      tile_grid(a.tail_tiles_cap, WAH_STATIC_TILES ? a.tail_tiles_cap
                                                   : a.max_resident / 4 * kTailBlocksPerCU);
   const uint32_t lanes = WAH_TAIL_LANES ? WAH_TAIL_LANES : tile_lanes(grid);
   hipLaunchKernelGGL((k_tail<kTailThreads, kTailItems, false>), dim3(grid), dim3(kTailThreads),
@@ -1978,7 +1987,7 @@ static void launch_short_tail(const BuildArgs& a, hipStream_t s) {
   // run mode: the same tiles as 512 threads x 16 items (fewer, longer lanes
   // suit its sparser items)
   const uint32_t rgrid =
-      cap_grid(a.tail_tiles_cap, WAH_STATIC_TILES ? a.tail_tiles_cap
+      tile_grid(a.tail_tiles_cap, WAH_STATIC_TILES ? a.tail_tiles_cap
                                                   : a.max_resident / 4 * kRunTailBlocksPerCU);
   const uint32_t rlanes = WAH_TAIL_LANES ? WAH_TAIL_LANES : tile_lanes(rgrid);
   hipLaunchKernelGGL((k_tail<kRunTailThreads, kRunTailItems, true>), dim3(rgrid),
