@@ -60,7 +60,9 @@ typedef struct wahgpu_counts {
                        pair per row, 1 = one item per run of equal values
                        inside a 31-row chunk (chosen when that sorts under
                        2/3 of the rows), 2 = pairs sorted with wide digits
-                       (see wahgpu_tuning); staged paths report 0        */
+                       (see wahgpu_tuning); staged paths report 0.  A
+                       column of at most 2^14 values reports 0 or 1 by the
+                       same rule, and one workgroup sorts its rows       */
 } wahgpu_counts;
 
 /* Microseconds per phase, the buckets `phases` prints (src/phases.cpp:714-1127). */
@@ -90,7 +92,8 @@ int wahgpu_find_device(const char* name);
  * separately, and no host wait holds the order).  Their look-back waits on tiles drawn by
  * workgroups placed on particular XCDs, and two such launches sharing the
  * device could each hold the CUs the other needs.  Copies and other work still
- * overlap them.  Calls made while their stream captures a graph are not
+ * overlap them, and so do builds of columns of at most 2^14 values, which one
+ * workgroup each does without waiting for another.  Calls made while their stream captures a graph are not
  * ordered: replay such graphs on one stream at a time. */
 int wahgpu_create(wahgpu_ctx** out, int device_ordinal, uint64_t arena_bytes);
 void wahgpu_destroy(wahgpu_ctx* ctx);
@@ -236,6 +239,9 @@ int wahgpu_graph_stats(const wahgpu_ctx* ctx, uint64_t* captures, uint64_t* repl
  *             those (a second histogram pass over its values, then one pass
  *             per wide digit, 512 x 16 tiles).  counts.mode reports 2 for it
  *             and counts.passes its wide passes.
+ * A column of at most 2^14 values that does not take wide digits is built by
+ * one workgroup and has no tiles (bucket 0's shape is timed by wahgpu_autotune
+ * all the same).
  * wahgpu_autotune times, on this device, synthetic batches of each bucket
  * (columns of 2^13, 2^15.5, 2^18.5, 2^22 and 2^26 values, 2^24 values per
  * bucket and one 2^26 column for the last): every shape with 8-bit digits on

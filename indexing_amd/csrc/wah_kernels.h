@@ -133,6 +133,10 @@ constexpr int kWideItems = 16;
 constexpr uint32_t kWideTile = kWideThreads * kWideItems;
 constexpr uint64_t kWideMinValues = 1u << 14;  // shorter columns keep 8-bit digits
 
+// Longest column that one workgroup builds (wah_small.hip): what its LDS holds.
+// One CU is still well ahead there (16000 rows 32 us, the general build 90).
+constexpr uint32_t kSmallMax = 1u << 14;
+
 // Which buffer a pass reads / writes.
 constexpr uint32_t kBufValues = 0;  // the input column, rids implicit (rid_base + i)
 constexpr uint32_t kBufA = 1;
@@ -312,6 +316,9 @@ struct LaunchHook {
 void launch_sort(const BuildArgs& a, hipStream_t s, LaunchHook* hook = nullptr);
 void launch_tail(const BuildArgs& a, hipStream_t s, LaunchHook* hook = nullptr);
 void launch_sort_finalize(const BuildArgs& a, hipStream_t s);
+// The whole build of columns of at most kSmallMax rows: the inline column, or
+// those of the descriptor (cols_cap at most).  Uses no scratch.
+void launch_small(const BuildArgs& a, hipStream_t s);
 // *ok must hold 1; stays 1 if LDS fetch-adds rank lanes in lane order here.
 void launch_rank_selftest(uint32_t* ok, hipStream_t s);
 void launch_fill32(uint32_t* p, uint64_t words, uint32_t v, hipStream_t s);

@@ -213,6 +213,11 @@ bool wide_ok(const wahgpu_ctx* c, uint64_t n) {
   const uint32_t d = c->force_digits ? (uint32_t)c->force_digits : c->tune_digits[bucket_of(n)];
   return d == 11u && n >= wah::kWideMinValues;
 }
+// One workgroup builds the column (the tuner's timed builds take the general
+// path, whose tile shapes they are for).
+bool small_ok(const wahgpu_ctx* c, uint64_t n) {
+  return n <= wah::kSmallMax && c->force_shape < 0 && !wide_ok(c, n);
+}
 uint32_t wide_tiles_of(uint64_t n) { return (uint32_t)((n + wah::kWideTile - 1) / wah::kWideTile); }
 
 Caps caps_one(uint64_t n, int shape, bool wide = false) {
@@ -577,6 +582,10 @@ struct EventHook : wah::LaunchHook {
   hipEvent_t* ev;
   int n = 0;
   void mark(hipStream_t s) override { (void)hipEventRecord(ev[n++], s); }
+  // a build of one launch: all of it counts as the first group
+  void rest(hipStream_t s) {
+    while (n <= WAHGPU_TIMING_GROUPS) mark(s);
+  }
 };
 }  // namespace
 
@@ -585,7 +594,10 @@ static int build_device_impl(wahgpu_ctx* c, const uint32_t* d_values, uint64_t n
                              uint32_t* d_lengths, uint32_t* d_words, wahgpu_counts* d_counts,
                              Marks* marks, char* scratch_base = nullptr) {
   BuildArgs a{};
-  if (scratch_base) {
+  const bool small = small_ok(c, n);
+  if (small) {
+    a.atomic_rank = c->atomic_rank;
+  } else if (scratch_base) {
     // carve from the caller's scratch instead of the arena
     char* const arena = c->arena;
     const uint64_t bump = c->bump;
@@ -611,6 +623,13 @@ static int build_device_impl(wahgpu_ctx* c, const uint32_t* d_values, uint64_t n
     hp = &hook;
     ++c->tcalls;
     hook.mark(c->stream);
+  }
+  if (small) {  // waits for no other workgroup, so it needs no device order
+    wah::launch_small(a, c->stream);
+    LAUNCHCHK(c);
+    if (marks) marks->mark(c->stream);
+    if (hp) hook.rest(c->stream);
+    return WAHGPU_OK;
   }
   ORDERED(c);
   wah::launch_sort(a, c->stream, hp);
@@ -663,7 +682,8 @@ int wahgpu_build_device(wahgpu_ctx* c, const uint32_t* d_values, uint64_t n, uin
   int rc = check_n(c, n, rid_base);
   if (rc) return rc;
   HIPCHK(c, hipSetDevice(c->device));
-  rc = arena_reserve(c, build_scratch_bytes(caps_for(c, n)));
+  const uint64_t scratch = build_scratch_bytes(caps_for(c, n));
+  rc = small_ok(c, n) ? arena_limit(c, scratch) : arena_reserve(c, scratch);
   if (rc) return rc;
   return build_device_impl(c, d_values, n, rid_base, d_keys, d_offsets, d_lengths, d_words,
                            d_counts, nullptr);
@@ -763,19 +783,22 @@ namespace {
 // radix tile shape, with their descriptor (dims + columns with tile and
 // chunk prefixes in that shape's tiles) in host memory.
 struct SubBatch {
-  int shape;
+  int shape;  // kSmallShape: columns of one workgroup each
   std::vector<char> desc;
   Caps caps;
 };
 
-// Validates the columns and splits them into sub-batches by tuned shape
-// (every compiled shape when `all_shapes`, empty ones included, so that a
-// captured graph fits any batch).  *shared = element-wise maximum of the
+constexpr int kSmallShape = wah::kRadixShapes;
+constexpr int kSubShapes = wah::kRadixShapes + 1;  // launch sets a batch may need
+
+// Validates the columns and splits them into sub-batches: the short ones, which
+// take a workgroup each, and the others by tuned shape (all of them when
+// `all_shapes`, empty ones included, so that a captured graph fits any batch).  *shared = element-wise maximum of the
 // sub-batches' caps (the scratch they share, one after another).
 int plan_batch(wahgpu_ctx* c, const wahgpu_column* cols, uint32_t ncols, uint64_t values_len,
                bool all_shapes, std::vector<SubBatch>* subs, Caps* shared) {
   uint64_t end = 0;
-  std::vector<uint32_t> members[wah::kRadixShapes];
+  std::vector<uint32_t> members[kSubShapes];
   for (uint32_t i = 0; i < ncols; ++i) {
     const wahgpu_column& col = cols[i];
     int rc = check_n(c, col.n, col.rid_base);
@@ -784,13 +807,14 @@ int plan_batch(wahgpu_ctx* c, const wahgpu_column* cols, uint32_t ncols, uint64_
       return fail(c, WAHGPU_EINVAL, "column " + std::to_string(i) +
                                         " overlaps the previous one or exceeds values_len");
     end = col.offset + col.n;
-    members[shape_for(c, col.n)].push_back(i);
+    members[small_ok(c, col.n) ? kSmallShape : shape_for(c, col.n)].push_back(i);
   }
   subs->clear();
   *shared = Caps{values_len, 0, 0, 0, 0};
-  bool tuned[wah::kRadixShapes] = {};
+  bool tuned[kSubShapes] = {};
   for (uint32_t b = 0; b < WAHGPU_TUNE_BUCKETS; ++b) tuned[c->tune_shape[b]] = true;
-  for (int sh = 0; sh < wah::kRadixShapes; ++sh) {
+  tuned[kSmallShape] = true;
+  for (int sh = 0; sh < kSubShapes; ++sh) {
     if (members[sh].empty() && !(all_shapes && tuned[sh])) continue;
     SubBatch sb;
     sb.shape = sh;
@@ -800,10 +824,10 @@ int plan_batch(wahgpu_ctx* c, const wahgpu_column* cols, uint32_t ncols, uint64_
     wah::Column* dc = wah::desc_cols(head);
     uint64_t st = 0, tt = 0, hc = 0, wt = 0;
     uint32_t ws = 0;  // columns that may take wide digits, each with a WideState
-    const uint32_t tile = wah::radix_tile(sh);
+    const uint32_t tile = wah::radix_tile(sh);  // (a short column's counts are bounds only)
     for (uint32_t j = 0; j < m; ++j) {
       const wahgpu_column& col = cols[members[sh][j]];
-      const bool wide = wide_ok(c, col.n);
+      const bool wide = sh != kSmallShape && wide_ok(c, col.n);
       dc[j] = wah::Column{col.offset, col.n, col.rid_base, (uint32_t)st, (uint32_t)tt,
                           (uint32_t)hc, members[sh][j], wide ? ws + 1u : 0u, (uint32_t)wt, 0u};
       st += wah::sort_tiles_of(col.n, tile);
@@ -950,6 +974,10 @@ int batch_device_impl(wahgpu_ctx* c, const uint32_t* d_values, uint64_t values_l
       }
       HIPCHK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
       for (const BuildArgs& a : args) {
+        if (a.shape == kSmallShape) {
+          wah::launch_small(a, c->stream);
+          continue;
+        }
         wah::launch_sort(a, c->stream);
         wah::launch_tail(a, c->stream);
       }
@@ -972,6 +1000,11 @@ int batch_device_impl(wahgpu_ctx* c, const uint32_t* d_values, uint64_t values_l
   }
   ORDERED(c);
   for (const BuildArgs& a : args) {
+    if (a.shape == kSmallShape) {
+      wah::launch_small(a, c->stream);
+      LAUNCHCHK(c);
+      continue;
+    }
     EventHook hook;
     EventHook* hp = nullptr;
     if (c->timing && c->tcalls < c->tmax && args.size() == 1) {
@@ -1558,7 +1591,7 @@ uint64_t wah_batch_acc_scratch(const wah_batch_acc* acc) {
   // one descriptor region per compiled tile shape: the most sub-batches
   const Caps k{acc->values, acc->cols, (uint32_t)acc->sort_tiles, (uint32_t)acc->tail_tiles,
                (uint32_t)acc->hist_chunks};
-  return build_scratch_bytes(k, wah::kRadixShapes);
+  return build_scratch_bytes(k, kSubShapes);
 }
 
 int wah_build_batch_ws(wahgpu_ctx* c, const uint32_t* d_values, uint64_t values_len,

@@ -1,5 +1,6 @@
-"""Radix and tail tiles of one column where their number and their ends change:
-one tile and a row, fewer tiles than the eight counter lanes, a number the
+"""Short columns, which one workgroup builds, at the sizes where its rows per
+thread change (1024, 4096, 8192, 16384), alone and in batches.  Radix and tail
+tiles of longer ones where their number and their ends change: one tile and a row, fewer tiles than the eight counter lanes, a number the
 lanes do not divide, as many tiles as blocks and one more, with last tiles of
 one row and of all but one, over even and skewed digits, in both sort modes and
 both rankings.  Against the oracle; whole numbers, so equal or wrong.
@@ -14,7 +15,7 @@ from tests.test_gpu_parity import assert_same
 pytestmark = pytest.mark.gpu
 
 T = 16384  # rows of a radix tile (the tail's is 8192)
-SIZES = [8193, T - 1, T, T + 1, 3 * T + 1, 9 * T - 1, 18 * T + 1, 65 * T - 1, 255 * T + 1,
+SIZES = [1, 2, 31, 63, 1023, 1024, 1025, 4095, 4096, 4097, 8191, 8192, 8193, T - 1, T, T + 1, 3 * T + 1, 9 * T - 1, 18 * T + 1, 65 * T - 1, 255 * T + 1,
          256 * T + 7]
 
 
@@ -45,7 +46,47 @@ def test_ballot_ranking(monkeypatch, kind):
     monkeypatch.setenv("WAHGPU_RANK", "match")
     with ia.Context(0) as c:
         assert c.rank_mode == 0
-        for n in (T + 1, 9 * T - 1, 65 * T - 1):
+        for n in (1, 1000, 4097, 8193, T, T + 1, 9 * T - 1, 65 * T - 1):
             v = column(kind, n)
             print(f"[tiles] match n={n} {kind}", flush=True)
             assert_same(c.build(v), oracle.build(v), f"{n} {kind}")
+
+
+@pytest.mark.parametrize("reserved", [False, True], ids=["eager", "graph"])
+def test_short_and_long_columns_in_one_batch(reserved):
+    """Short columns take a workgroup each beside the launch set of the longer
+    ones; a graph replays layouts with more, fewer and none of either."""
+    import torch
+
+    from tests.test_gpu_batch import per_column
+    kinds = ["u16", "u32", "top", "skew", "runs"]
+    layouts = [[1, 1000, 5000, 0, T, T + 1, 16000, 40000, 3], [7, 8192, 0, 1024] * 3,
+               [T + 5, 60000], [T, 0, 20011]]
+    total = max(sum(n + 3 for n in lay) for lay in layouts)
+    with ia.Context(0) as c:
+        if reserved:
+            c.batch_reserve(total, 16)
+        buf = torch.zeros(total, dtype=torch.int32, device="cuda:0")
+        out = None
+        for rep, lay in enumerate(layouts + layouts[:2]):
+            cols, refs, at = [], [], rep % 2
+            for i, n in enumerate(lay):
+                v = column(kinds[(i + rep) % 5], n) if n else np.zeros(0, np.uint32)
+                buf[at:at + n] = torch.from_numpy(v.view(np.int32))
+                cols.append((at, n, 1000 * i))
+                refs.append(oracle.build(v, rid_base=1000 * i))
+                at += n + i % 3  # offsets off the 16-byte grid
+            print(f"[batch] {lay} reserved={reserved}", flush=True)
+            d = torch.zeros(16 * 10, dtype=torch.int32, device="cuda:0") if out is None else out[4]
+            if out is None:
+                out = tuple(torch.zeros(m, dtype=torch.int32, device="cuda:0")
+                            for m in (total, total, total, 2 * total)) + (d,)
+            c.build_batch_device(buf, cols, out)
+            torch.cuda.synchronize()
+            counts = c.read_counts_batch(out[4], len(lay))
+            got = per_column(out, counts, [(o, n) for o, n, _ in cols])
+            for i, (g, r) in enumerate(zip(got, refs)):
+                assert counts[i].fault == 0
+                assert_same(g, r, f"layout {rep} column {i}")
+        if reserved:
+            assert c.graph_stats()[0] == 1
