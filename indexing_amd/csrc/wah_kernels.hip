@@ -23,8 +23,7 @@
 
 #include <type_traits>
 
-#include "wah_device.h"
-#include "wah_kernels.h"
+#include "wah_scan.h"
 
 namespace wah {
 
@@ -63,44 +62,6 @@ __global__ __launch_bounds__(kBlock) void k_begin(Header* __restrict__ hdr,
 // Block b takes a contiguous range of 4096-value chunks, accumulates in LDS
 // and folds into the column's histogram when the column changes.
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ void hist_add(uint32_t* h, uint32_t bin, bool valid) {
-  // A wave whose valid lanes all share the bin adds once (the high digits of
-  // small-range columns are constant); otherwise one LDS atomic per lane.
-  const uint32_t first = __builtin_amdgcn_readfirstlane(bin);
-  const uint64_t differ = ballot(valid && bin != first);
-  if (differ == 0) {
-    const uint64_t cnt = ballot(valid);
-    if (lane_id() == 0 && cnt) atomicAdd(&h[first], (uint32_t)__popcll(cnt));
-  } else if (valid) {
-    atomicAdd(&h[bin], 1u);
-  }
-}
-
-// Adds a value to the digit histograms, and to the repeat histograms when
-// it repeats its predecessor inside one chunk (rep).
-__device__ __forceinline__ void hist_value(uint32_t* h, uint32_t* hr, uint32_t v, bool valid,
-                                           bool rep) {
-  const uint32_t f = __builtin_amdgcn_readfirstlane(v);
-  if (ballot(valid && v != f) == 0) {  // one value across the wave (runs)
-    const uint32_t cnt = (uint32_t)__popcll(ballot(valid));
-    const uint32_t rc = (uint32_t)__popcll(ballot(rep));
-    if (lane_id() == 0 && cnt) {
-#pragma unroll
-      for (int p = 0; p < 4; ++p) {
-        atomicAdd(&h[p * 256 + ((f >> (8 * p)) & 255u)], cnt);
-        if (rc) atomicAdd(&hr[p * 256 + ((f >> (8 * p)) & 255u)], rc);
-      }
-    }
-    return;
-  }
-#pragma unroll
-  for (int p = 0; p < 4; ++p) hist_add(h, p * 256 + ((v >> (8 * p)) & 255u), valid);
-  if (ballot(rep)) {
-#pragma unroll
-    for (int p = 0; p < 4; ++p) hist_add(hr, p * 256 + ((v >> (8 * p)) & 255u), rep);
-  }
-}
-
 __device__ __forceinline__ void hist_flush(uint32_t* h, uint32_t* hr, uint32_t* s_max,
                                            uint32_t& vmax, ColState* col) {
   const int t = threadIdx.x;
@@ -164,27 +125,45 @@ __global__ __launch_bounds__(kBlock, 8) void k_histogram(
     }
     const Column cd = cols[col];
     const uint64_t lo = (uint64_t)(c - cd.hist_chunk0) * kHistChunk;
-    const uint32_t cnt = cd.n - lo < kHistChunk ? (uint32_t)(cd.n - lo) : kHistChunk;
+    // as a 32-bit minimum (a column holds fewer than 2^30 rows): written as a
+    // 64-bit compare and a select beside the branch on it, hipcc 7.2 selects
+    // on a stale condition bit
+    const uint32_t left = (uint32_t)(cd.n - lo);
+    const uint32_t cnt = __builtin_elementwise_min(left, kHistChunk);
     const uint32_t* src = values + cd.off + lo;
     // row of src[i] is rid_base + lo + i; a row repeats its predecessor when
     // it is not the first of the column or of a chunk and has its value
     const uint32_t row0 = cd.rid_base + (uint32_t)lo;
-    uint32_t reps = 0;  // rows of this chunk that repeat their predecessor
-    if (cnt == kHistChunk && ((uintptr_t)src % 16) == 0) {
-      // four 16-byte loads per thread, and per wave the value before each
-      // of its four 256-value spans (a uniform load), all issued before any
-      // is used: one memory latency per chunk
-      const uint4* v4 = reinterpret_cast<const uint4*>(src);
-      const uint32_t wv = __builtin_amdgcn_readfirstlane(t / kWave);
-      uint4 q[4];
+    const uint32_t wv = __builtin_amdgcn_readfirstlane(t / kWave);
+    const uint32_t w0 = wv * kWave * 4;  // the wave's first row of the chunk
+    // Whole chunks and a column's last, partial one run the same code: rows
+    // past the column take the value of the wave's first row (so they vary no
+    // digit) and are left out of the counts.  A wave with no row does nothing.
+    auto chunk = [&](auto full_tag) {
+      constexpr bool FULL = decltype(full_tag)::value;
+      // four 16-byte loads per thread (4-byte aligned ones do), and per wave
+      // the value before each of its four 256-value spans, all issued before
+      // any is used: one memory latency per chunk
+      W4 q[4];
+      if (FULL) {
 #pragma unroll
-      for (int u = 0; u < 4; ++u) q[u] = v4[u * kBlock + t];
+        for (int u = 0; u < 4; ++u) q[u] = reinterpret_cast<const W4u*>(src)[u * kBlock + t];
+      } else {  // one row at a time, past the end the last one: no branches
+        // (opaque: the indices are formed here, not kept across whole chunks)
+        const uint32_t end = cnt - 1u, t4 = 4u * opaque((uint32_t)t);
+        auto at = [&](uint32_t i) -> uint32_t { return src[i < end ? i : end]; };
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const uint32_t i0 = t4 + (uint32_t)(u * kBlock * 4);
+          q[u] = W4{at(i0), at(i0 + 1u), at(i0 + 2u), at(i0 + 3u)};
+        }
+      }
       // lane u < 4: the value before span u of the wave (one vector load)
       uint32_t wprev;
       {
         const uint32_t lu = lane_id();
         const uint32_t s0 = (lu * kBlock + wv * kWave) * 4;  // span's first index
-        wprev = lu < 4u && lo + s0 > 0 ? src[(int64_t)s0 - 1] : 0u;
+        wprev = lu < 4u && lo + s0 > 0 && (FULL || s0 < cnt) ? src[(int64_t)s0 - 1] : 0u;
       }
       __builtin_amdgcn_sched_barrier(0);
       // The wave's 1024 rows of the chunk (4 spans of 256).  A digit the same
@@ -196,6 +175,27 @@ __global__ __launch_bounds__(kBlock, 8) void k_histogram(
       // wave-uniform branch), so columns without repeats carry no per-row
       // conditions on their atomics.
       const uint32_t f0 = __builtin_amdgcn_readfirstlane(q[0].x);
+      uint32_t vm = 0xFFFFu;  // rows of the lane below the column's end: bit 4u + j
+      if (!FULL) {
+        vm = 0;
+        const uint32_t t4 = 4u * opaque((uint32_t)t);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const uint32_t i0 = t4 + (uint32_t)(u * kBlock * 4);
+          const uint32_t ok = i0 + 4 <= cnt ? 15u : i0 < cnt ? (1u << (cnt - i0)) - 1u : 0u;
+          vm |= ok << (4 * u);
+          q[u].x = ok & 1u ? q[u].x : f0;
+          q[u].y = ok & 2u ? q[u].y : f0;
+          q[u].z = ok & 4u ? q[u].z : f0;
+          q[u].w = ok & 8u ? q[u].w : f0;
+        }
+      }
+      // rows of span u of the wave, and of the wave
+      auto span_rows = [&](int u) -> uint32_t {
+        const uint32_t s0 = (uint32_t)(u * kBlock * 4) + w0;
+        return FULL || cnt >= s0 + 4u * kWave ? 4u * kWave : cnt > s0 ? cnt - s0 : 0u;
+      };
+      const uint32_t rows = span_rows(0) + span_rows(1) + span_rows(2) + span_rows(3);
       uint32_t x = 0;    // bits in which a value of the lane differs from its span's first
       uint32_t fx = 0;   // bits in which a span's first value differs from f0
       uint32_t one = 0;  // bit u: span u holds a single value
@@ -204,17 +204,15 @@ __global__ __launch_bounds__(kBlock, 8) void k_histogram(
       uint32_t m = (row0 + (uint32_t)t * 4u) % 31u;
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
-        const uint32_t i0 = (uint32_t)(u * kBlock + t) * 4;  // index of q[u].x in src
         // lane l-1's last value (DPP wave shift); lane 0 the value before the span
-        const uint32_t prev = (uint32_t)__builtin_amdgcn_update_dpp(
-            (int)readlane(wprev, u), (int)q[u].w, 0x138, 0xF, 0xF, false);
+        const uint32_t prev = lane_before(q[u].w, readlane(wprev, u));
         const uint32_t e[4] = {q[u].x, q[u].y, q[u].z, q[u].w};
         uint32_t mj = m;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           vmax = e[j] > vmax ? e[j] : vmax;
           const uint32_t pv = j == 0 ? prev : e[j - 1];
-          const bool rep = lo + i0 + j > 0 && mj != 0u && e[j] == pv;
+          const bool rep = lo + (uint32_t)(u * kBlock + t) * 4 + j > 0 && mj != 0u && e[j] == pv;
           rm |= rep ? 1u << (4 * u + j) : 0u;
           mj = mj == 30u ? 0u : mj + 1u;
         }
@@ -225,99 +223,76 @@ __global__ __launch_bounds__(kBlock, 8) void k_histogram(
         x |= xu;
         fx |= fu ^ f0;
       }
-      reps += (uint32_t)__builtin_popcount(rm);
+      if (!FULL) rm &= vm;
       // a bit varies over the 1024 rows iff it varies inside a span or
       // between the spans' first values
       const uint32_t vary = wave_or(x) | fx;
+      // runs of the wave's rows, added to their radix tile (a run-mode
+      // column's cut places its items from these counts); no block barrier,
+      // so the waves of a block stream their chunks independently
+      const uint32_t reps = readlane(wave_incl_add((uint32_t)__builtin_popcount(rm)), kWave - 1);
+      if (lane_id() == 0 && rows != reps)
+        atomicAdd(&tile_runs[cd.sort_tile0 + (uint32_t)(lo / sort_tile)], rows - reps);
       if (vary == 0u) {
         // every row of the chunk holds f0 (inside a run): lane p adds the
         // wave's rows, and its repeat rows, to digit p's bin of f0
-        const uint32_t rc = readlane(wave_incl_add((uint32_t)__builtin_popcount(rm)), kWave - 1);
         const uint32_t lp = lane_id();
         if (lp < 4u) {
           const uint32_t bin = lp * 256u + ((f0 >> (8u * lp)) & 255u);
-          atomicAdd(&h[bin], 16u * kWave);
-          if (rc) atomicAdd(&hr[bin], rc);
+          atomicAdd(&h[bin], rows);
+          if (reps) atomicAdd(&hr[bin], reps);
         }
-      } else {
+        return;
+      }
+#pragma unroll
+      for (int p = 0; p < 4; ++p) {
+        if (((vary >> (8 * p)) & 255u) == 0u) {
+          if (lane_id() == 0) atomicAdd(&h[p * 256 + ((q[0].x >> (8 * p)) & 255u)], rows);
+          continue;
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const uint32_t e[4] = {q[u].x, q[u].y, q[u].z, q[u].w};
+          if ((one >> u) & 1u) {
+            if (lane_id() == 0) atomicAdd(&h[p * 256 + ((e[0] >> (8 * p)) & 255u)], span_rows(u));
+          } else {
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+              if (FULL || ((vm >> (4 * u + j)) & 1u))
+                atomicAdd(&h[p * 256 + ((e[j] >> (8 * p)) & 255u)], 1u);
+          }
+        }
+      }
+      if (reps) {
+        uint32_t rcu[4];  // repeats of each span
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          rcu[u] = 0;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) rcu[u] += (uint32_t)__popcll(ballot((rm >> (4 * u + j)) & 1u));
+        }
 #pragma unroll
         for (int p = 0; p < 4; ++p) {
           if (((vary >> (8 * p)) & 255u) == 0u) {
-            if (lane_id() == 0) atomicAdd(&h[p * 256 + ((q[0].x >> (8 * p)) & 255u)], 16u * kWave);
+            if (lane_id() == 0) atomicAdd(&hr[p * 256 + ((q[0].x >> (8 * p)) & 255u)], reps);
             continue;
           }
 #pragma unroll
           for (int u = 0; u < 4; ++u) {
             const uint32_t e[4] = {q[u].x, q[u].y, q[u].z, q[u].w};
             if ((one >> u) & 1u) {
-              if (lane_id() == 0) atomicAdd(&h[p * 256 + ((e[0] >> (8 * p)) & 255u)], 4u * kWave);
+              if (lane_id() == 0 && rcu[u]) atomicAdd(&hr[p * 256 + ((e[0] >> (8 * p)) & 255u)], rcu[u]);
             } else {
 #pragma unroll
-              for (int j = 0; j < 4; ++j) atomicAdd(&h[p * 256 + ((e[j] >> (8 * p)) & 255u)], 1u);
-            }
-          }
-        }
-        if (ballot(rm != 0u)) {
-          uint32_t rcu[4], rc = 0;  // repeats of each span and of the wave
-#pragma unroll
-          for (int u = 0; u < 4; ++u) {
-            rcu[u] = 0;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) rcu[u] += (uint32_t)__popcll(ballot((rm >> (4 * u + j)) & 1u));
-            rc += rcu[u];
-          }
-#pragma unroll
-          for (int p = 0; p < 4; ++p) {
-            if (((vary >> (8 * p)) & 255u) == 0u) {
-              if (lane_id() == 0) atomicAdd(&hr[p * 256 + ((q[0].x >> (8 * p)) & 255u)], rc);
-              continue;
-            }
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-              const uint32_t e[4] = {q[u].x, q[u].y, q[u].z, q[u].w};
-              if ((one >> u) & 1u) {
-                if (lane_id() == 0 && rcu[u]) atomicAdd(&hr[p * 256 + ((e[0] >> (8 * p)) & 255u)], rcu[u]);
-              } else {
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-                  if ((rm >> (4 * u + j)) & 1u) atomicAdd(&hr[p * 256 + ((e[j] >> (8 * p)) & 255u)], 1u);
-              }
+              for (int j = 0; j < 4; ++j)
+                if ((rm >> (4 * u + j)) & 1u) atomicAdd(&hr[p * 256 + ((e[j] >> (8 * p)) & 255u)], 1u);
             }
           }
         }
       }
-    } else {
-      for (uint32_t b = 0; b < cnt; b += kBlock) {
-        const uint32_t i = b + t;
-        const bool valid = i < cnt;
-        const uint32_t v = valid ? src[i] : 0;
-        const bool has_prev = valid && lo + i > 0;
-        const uint32_t pv = has_prev ? src[(int64_t)i - 1] : 0u;
-        vmax = valid && v > vmax ? v : vmax;
-        const bool rep = has_prev && (row0 + i) % 31u != 0u && v == pv;
-        reps += rep ? 1u : 0u;
-        hist_value(h, hr, v, valid, rep);
-      }
-    }
-    // runs of the wave's rows, added to their radix tile (a run-mode
-    // column's cut places its items from these counts); no block barrier,
-    // so the waves of a block stream their chunks independently
-    reps = readlane(wave_incl_add(reps), kWave - 1);  // at most 4096
-    if ((t % kWave) == 0) {
-      // rows this wave covered: the fast path gives wave w rows 4 x 64 x
-      // {u * 256 + w * 64 ..}; the slow path row i to thread i % 256
-      const uint32_t w = t / kWave;
-      uint32_t rows = 0;
-      if (cnt == kHistChunk && ((uintptr_t)src % 16) == 0) {
-        rows = kHistChunk / kWaves;
-      } else {
-        for (uint32_t b = 0; b < cnt; b += kBlock) {
-          const uint32_t lo_i = b + w * kWave;
-          rows += cnt > lo_i ? (cnt - lo_i < (uint32_t)kWave ? cnt - lo_i : (uint32_t)kWave) : 0u;
-        }
-      }
-      if (rows - reps) atomicAdd(&tile_runs[cd.sort_tile0 + (uint32_t)(lo / sort_tile)], rows - reps);
-    }
+    };
+    if (cnt == kHistChunk) chunk(std::true_type{});
+    else if (w0 < cnt) chunk(std::false_type{});
   }
   hist_flush(h, hr, s_max, vmax, &cs[col]);
 }
@@ -334,23 +309,42 @@ __global__ __launch_bounds__(kBlock) void k_plan(const DescHead* __restrict__ de
                                                  WideState* __restrict__ wide) {
   __shared__ uint64_t s_scan[kWaves];
   __shared__ int s_trivial[4];
-  __shared__ uint32_t s_reps;
   __shared__ uint32_t s_wide;  // 1 + wide slot of a column that takes wide digits
-  const int t = threadIdx.x;
+  const int t = threadIdx.x, l = t % kWave;
+  const int w = __builtin_amdgcn_readfirstlane(t / kWave);
   const uint32_t ncols = desc->dims.ncols;
   for (uint32_t c = blockIdx.x; c < ncols; c += gridDim.x) {
     const uint64_t n = desc_cols(desc)[c].n;
     ColState* col = &cs[c];
-    if (t < 4) s_trivial[t] = 0;
-    if (t == 0) s_reps = 0;
-    __syncthreads();
-    atomicAdd(&s_reps, col->rep[0][t]);
-    __syncthreads();
+    // Wave p takes digit p, lane l its bins 4l .. 4l + 3: the digits' scans
+    // run side by side, with one barrier after them (one after another over
+    // the block, with two barriers each, they made the kernel 7 us of a
+    // build of 2^20 rows).
+    const uint4 hq = reinterpret_cast<const uint4*>(col->hist[w])[l];
+    const uint4 rq = reinterpret_cast<const uint4*>(col->rep[w])[l];
+    // every digit counts every repeat row once
+    const uint32_t reps = readlane(wave_incl_add(rq.x + rq.y + rq.z + rq.w), kWave - 1);
     // Run mode when it sorts under 2/3 of the rows (an item moves 12 bytes
     // per pass, a pair 8).
-    const uint64_t runs = n - s_reps;
+    const uint64_t runs = n - reps;
     const bool run_mode = !force_pair && n > 0 && 3 * runs < 2 * n;
     const uint64_t items = run_mode ? runs : n;
+    {
+      const uint32_t h[4] = {hq.x - (run_mode ? rq.x : 0u), hq.y - (run_mode ? rq.y : 0u),
+                             hq.z - (run_mode ? rq.z : 0u), hq.w - (run_mode ? rq.w : 0u)};
+      const uint32_t sum = h[0] + h[1] + h[2] + h[3];
+      uint4 ex;
+      ex.x = wave_incl_add(sum) - sum;
+      ex.y = ex.x + h[0];
+      ex.z = ex.y + h[1];
+      ex.w = ex.z + h[2];
+      reinterpret_cast<uint4*>(col->digit_offset[w])[l] = ex;
+      bool all = false;  // one digit holds every item
+#pragma unroll
+      for (int i = 0; i < 4; ++i) all |= (uint64_t)h[i] == items;
+      const bool trivial = ballot(all) != 0;
+      if (l == 0) s_trivial[w] = trivial;
+    }
     if (run_mode) {
       // where each radix tile's runs go: exclusive prefix of the runs per tile
       const Column cd = desc_cols(desc)[c];
@@ -399,13 +393,6 @@ __global__ __launch_bounds__(kBlock) void k_plan(const DescHead* __restrict__ de
           }
         }
       }
-    }
-    for (int p = 0; p < 4; ++p) {
-      const uint32_t h = col->hist[p][t] - (run_mode ? col->rep[p][t] : 0u);
-      uint64_t total;
-      const uint64_t ex = block_exclusive<OpAdd>(h, s_scan, &total);
-      col->digit_offset[p][t] = (uint32_t)ex;
-      if ((uint64_t)h == items) s_trivial[p] = 1;  // every item has digit t
     }
     __syncthreads();
     if (t == 0) {
@@ -1793,17 +1780,25 @@ __global__ __launch_bounds__(kBlock) void k_finish(const DescHead* __restrict__ 
       if (last && seg) atomicAdd((unsigned long long*)&counts[cols[c].index].k, (unsigned long long)seg);
     }
   }
-  for (uint32_t c = 0; c < ncols; ++c) {
+  // The blocks are dealt to the columns, `parts` of them to each; with more
+  // columns than blocks a block takes every gridDim-th.  (All blocks walking
+  // all columns cost a batch of 128 columns 90 us.)
+  if (ncols == 0) return;
+  const uint32_t parts = gridDim.x > ncols ? gridDim.x / ncols : 1u;
+  const uint32_t part = blockIdx.x / ncols;
+  if (part >= parts) return;
+  for (uint32_t c = blockIdx.x % ncols; c < ncols; c += gridDim.x) {
     const Column cd = cols[c];
     const uint64_t kc = counts[cd.index].keycnt;
     const uint64_t K = kc < cd.n ? kc : cd.n, L = counts[cd.index].length;
     const uint32_t* o = offsets + cd.off;
     uint32_t* len = lengths + cd.off;
-    for (uint64_t i = gt; i < K; i += gs) {
+    const uint32_t step = parts * kBlock;
+    for (uint32_t i = part * kBlock + threadIdx.x; i < K; i += step) {
       const uint32_t end = (i + 1 < K) ? o[i + 1] : (uint32_t)L;
       len[i] = end - o[i];
     }
-    if (gt == 0 && fault) counts[cd.index].fault = fault;
+    if (part == 0 && threadIdx.x == 0 && fault) counts[cd.index].fault = fault;
   }
 }
 
@@ -2002,8 +1997,9 @@ void launch_tail(const BuildArgs& a, hipStream_t s, LaunchHook* hook) {
   else
     launch_short_tail(a, s);
   if (hook) hook->mark(s);
-  uint64_t lg = (a.n_cap + kBlock - 1) / kBlock;
-  hipLaunchKernelGGL(k_finish, dim3(cap_grid(lg > 1024 ? 1024u : (uint32_t)lg, 1024)),
+  // blocks for up to 8 x 256 keys per column of a batch at a time
+  const uint64_t lg = (a.n_cap + kBlock - 1) / kBlock, most = a.cols_cap > 128u ? 8ull * a.cols_cap : 1024u;
+  hipLaunchKernelGGL(k_finish, dim3(cap_grid((uint32_t)(lg < most ? lg : most), 8192)),
                      dim3(kBlock), 0, s, a.desc, a.hdr, a.tile_entries, a.out_offsets,
                      a.out_lengths, a.counts);
 }
