@@ -86,12 +86,6 @@ constexpr int kTailTile = kTailThreads * kTailItems;  // sorted pairs per tail t
 #endif
 constexpr int kTailWavesPerEU = WAH_TAIL_WAVES_PER_EU;
 constexpr int kTailBlocksPerCU = kTailWavesPerEU * 4 * 64 / kTailThreads;
-// Run-mode tail: the same tiles as 16 items per thread (512 threads for the
-// 8192-item tile) at 4 waves per SIMD (128 VGPRs), two blocks per CU.
-constexpr int kRunTailItems = 16;
-constexpr int kRunTailThreads = kTailTile / kRunTailItems;
-constexpr int kRunTailBlocksPerCU = 4 * 4 * 64 / kRunTailThreads;
-static_assert(kRunTailThreads * kRunTailItems == kTailTile, "run tail tiles = pair tail tiles");
 // Long single columns (at least 2^WAH_LONG_TAIL_MIN_LOG2 values) take tail
 // tiles of 16384 items, 1024 threads x 16 at one block per CU (4 waves per
 // SIMD), in both modes: 2^28 uniform values, tail 0.95 ms against 0.99 ms in
@@ -267,7 +261,8 @@ struct BuildArgs {
   // Single column: k_begin writes the descriptor from these (no host copy).
   bool inline_desc;
   // The column is long: tail tiles of kLongTailTile items (one_dims counts
-  // them); tail_tiles_cap still bounds the kTailTile count.
+  // them; tail_tiles_cap still bounds the kTailTile count), and a launch per
+  // sort mode.
   bool long_tail;
   Dims one_dims;
   Column one;

@@ -673,7 +673,14 @@ __global__ __launch_bounds__(256) void k_rank_selftest(uint32_t* ok) {
 // order and written out in runs per digit.  Run mode moves (key, rid,
 // literal bits) items the run cut wrote to B: launch 0 reads B.
 // ---------------------------------------------------------------------------
-template <int THREADS, int ITEMS, bool RUN, int RANK>
+// MODES 0: the tiles of the pair-mode columns; 1: of the run-mode columns; 2:
+// of the former and then of the latter in one launch, where a mode without an
+// a-th pass costs a scalar load.  A launch per mode leaves half the radix
+// launches of a single column with nothing to do, 4 to 5 us each (2^20 rows
+// 77 us, in one launch 70); with both bodies in one kernel fewer scalar
+// registers are left per body, and from 2^24 rows on that costs more (2^28
+// rows: 2835 us, in one launch 2863).
+template <int THREADS, int ITEMS, int RANK, int MODES>
 __global__ __launch_bounds__(THREADS, sort_waves_per_eu(ITEMS)) void k_onesweep(
     uint32_t a, const uint32_t* __restrict__ values, uint32_t* keysA, uint32_t* ridsA,
     uint32_t* keysB, uint32_t* ridsB, uint32_t* litsA, uint32_t* litsB,
@@ -689,291 +696,14 @@ __global__ __launch_bounds__(THREADS, sort_waves_per_eu(ITEMS)) void k_onesweep(
   __shared__ uint32_t s_glob[256];
   __shared__ uint32_t s_dsum[4];
   __shared__ uint32_t s_tile;
-
-  // pair mode: launch 0 reads the values (rids implicit); run mode: the run
-  // cut wrote the items to B.  Then A -> B, B -> A, ...
-  const bool implicit = !RUN && a == 0;
-  const uint32_t* src_keys = implicit ? values : ((a % 2) ? keysA : keysB);
-  const uint32_t* src_rids = (a % 2) ? ridsA : ridsB;
-  const uint32_t* src_lits = (a % 2) ? litsA : litsB;
-  uint32_t* dst_keys = (a % 2) ? keysB : keysA;
-  uint32_t* dst_rids = (a % 2) ? ridsB : ridsA;
-  uint32_t* dst_lits = (a % 2) ? litsB : litsA;
-  uint32_t* status = status_base + (uint64_t)(a % 2) * status_stride;
-  uint32_t* status_next = status_base + (uint64_t)(1u - a % 2) * status_stride;
-  uint32_t* fault = &hdr->fault;
-  const Dims dims = desc->dims;
-  const Column* cols = desc_cols(desc);
-  const int t = threadIdx.x, l = t % kWave;
-  const int w = __builtin_amdgcn_readfirstlane(t / kWave);  // scalar: per-wave LDS addresses
-  if (hdr->max_active[RUN ? 1 : 0] <= a) return;  // no column has an a-th pass
-  uint32_t* counter = hdr->tiles[(RUN ? kCounterRun : 0) + a];
-
-  uint32_t iter = 0;
-  for (;;) {
-    for (int i = t; i < WAVES * 256; i += THREADS) (&s_wcnt[0][0])[i] = 0;
-    const uint32_t tile = __builtin_amdgcn_readfirstlane(
-        next_tile(counter, lanes, &s_tile, iter, tile_group(dims.sort_tiles, lanes, WAH_SORT_TILE_GROUP)));
-    if (tile >= dims.sort_tiles) break;
-    const uint32_t c = find_segment(&cols[0].sort_tile0, sizeof(Column) / 4, dims.ncols, tile);
-    const ColState* col = &cs[c];
-    const Column cd = cols[c];
-    const uint32_t first = cd.sort_tile0;
-    const uint64_t base = (uint64_t)(tile - first) * TILE;  // column-local
-    // elements: rows, or the run items of a run-mode column
-    const uint64_t n = RUN ? (uint64_t)col->items : cd.n;
-    const uint64_t n_out = n;
-    if (col->mode != (RUN ? kModeRun : kModePair) || col->wide || col->num_active <= a ||
-        base >= n) {
-      // other mode, already sorted, or past the run items; a block draws its
-      // tiles in increasing order, so past the last column's items it is done
-      if (RUN && c + 1 == dims.ncols && col->mode == kModeRun && base >= n) break;
-      __syncthreads();  // s_tile is read by every wave before it is rewritten
-      continue;
-    }
-    const uint32_t shift = col->shift[a];
-    // 16-bit keys: every pass writes them; the first reads the values (or
-    // the run cut's items) as 32-bit words
-    const bool narrow = col->narrow != 0u, src_narrow = narrow && !implicit && !(RUN && a == 0);
-    if (t < 256) status_next[(uint64_t)tile * 256 + t] = 0;  // next launch's state
-    const uint64_t wbase = base + (uint64_t)w * kWave * ITEMS + l;
-    // The body is straight-line, so the compiler can wait for the rid loads
-    // without draining the key stores, and the ranking atomics issue back to
-    // back.  A column's last tile runs it too: items past its end read the
-    // last one, count in a word of their own instead of a digit's, and keep
-    // their own index as their slot (they are the tile's last in input order,
-    // so those slots lie past tile_n), which nothing stores.
-    // PACKED: launch 0 of a pair-mode column with keys < 2^16.  Its rids are
-    // implicit (rid_base + column row), so one LDS word carries both the key
-    // (high half) and the row's tile-local index (low half): one staging
-    // round moves keys and rids.
-    auto sweep = [&](auto full_tag, auto packed_tag) {
-      constexpr bool FULL = decltype(full_tag)::value;
-      constexpr bool PACKED = decltype(packed_tag)::value;
-      // Keys only for now: the rids are loaded once the keys are staged, so
-      // they never occupy registers during ranking and look-back.
-      uint32_t key[ITEMS], rank[ITEMS];
-      // item i of an array of the column (indices fit 32 bits): one base and
-      // immediate offsets in a whole tile; past the column its last item
-      // (first: the lane's first item, opaque per array so that the clamped
-      // indices are formed again instead of spilled across the ranking)
-      const uint32_t j0 = (uint32_t)wbase, jl = (uint32_t)n - 1u;
-      auto item = [&](const auto* col0, int i, uint32_t first) -> uint32_t {
-        if (FULL) return (uint32_t)(col0 + wbase)[i * kWave];
-        const uint32_t j = first + (uint32_t)(i * kWave);
-        return (uint32_t)col0[j < jl ? j : jl];
-      };
-      if (src_narrow) {
-        const uint16_t* kp = reinterpret_cast<const uint16_t*>(src_keys + cd.off);
-#pragma unroll
-        for (int i = 0; i < ITEMS; ++i) key[i] = item(kp, i, j0);
-      } else {
-        const uint32_t* kp = src_keys + cd.off;
-#pragma unroll
-        for (int i = 0; i < ITEMS; ++i) key[i] = item(kp, i, j0);
-      }
-      const uint32_t tile_n = FULL ? (uint32_t)TILE : (uint32_t)(n - base);
-      // Rank: peers = lanes with the same digit (8 ballots); rank = peers
-      // below this lane + keys of that digit the wave ranked before.
-#pragma unroll
-      for (int i = 0; i < ITEMS; ++i) {
-        const uint32_t d = (key[i] >> shift) & 255u;
-        const bool in = FULL || j0 + (uint32_t)(i * kWave) <= jl;
-        if (RANK == kRankAtomic) {
-          rank[i] = atomicAdd(in ? &s_wcnt[w][d] : &s_stage[t], 1u);
-        } else {
-          uint64_t peers = ballot(in);
-#pragma unroll
-          for (int b = 0; b < 8; ++b) {
-            const bool bit = (d >> b) & 1u;
-            const uint64_t bb = ballot(bit);
-            peers &= bit ? bb : ~bb;
-          }
-          const uint32_t cnt = (uint32_t)__popcll(peers);
-          const uint32_t below = mbcnt(peers);
-          const uint32_t prior = s_wcnt[w][d];
-          rank[i] = prior + below;
-          if (in && below == cnt - 1) s_wcnt[w][d] = prior + cnt;
-        }
-      }
-      __syncthreads();
-      // Threads 0..255 own one digit each: wave prefixes, tile total,
-      // exclusive scan over digits, look-back.
-      uint32_t total = 0;
-      if (t < 256) {
-        const uint32_t goff = col->digit_offset[shift / 8][t];
-        // all the wave counts first (independent reads), then the prefixes:
-        // interleaved, each read would wait for the write before it
-        uint32_t xw[WAVES];
-#pragma unroll
-        for (int i = 0; i < WAVES; ++i) xw[i] = s_wcnt[i][t];
-#pragma unroll
-        for (int i = 0; i < WAVES; ++i) {
-          s_wcnt[i][t] = total;
-          total += xw[i];
-        }
-        uint32_t* my = &status[(uint64_t)tile * 256 + t];
-        st_agent(my, ((tile == first ? kFlagPrefix : kFlagAgg) << 30) | total);
-        const uint32_t inc = wave_incl_add(total);
-        if (l == kWave - 1) s_dsum[w] = inc;
-        s_excl[t] = inc - total;  // within this wave's 64 digits
-        uint32_t prev = 0;
-        if (tile > first) {
-          prev = lookback_digit(status + t, tile, first, 256, fault);
-          st_agent(my, (kFlagPrefix << 30) | (prev + total));
-        }
-        s_glob[t] = goff + prev;  // the tile-local offset is subtracted below
-      }
-      __syncthreads();
-      if (t < 256) {
-        uint32_t before = 0;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) before += i < w ? s_dsum[i] : 0u;
-        const uint32_t ex = s_excl[t] + before;
-        s_glob[t] -= ex;  // column index = s_glob[d] + local index
-        // each wave's first slot for digit t: one LDS read per key below
-        uint32_t xw[WAVES];
-#pragma unroll
-        for (int i = 0; i < WAVES; ++i) xw[i] = s_wcnt[i][t];
-#pragma unroll
-        for (int i = 0; i < WAVES; ++i) s_wcnt[i][t] = xw[i] + ex;
-      }
-      __syncthreads();
-      if constexpr (PACKED) {
-        const uint32_t row0 = (uint32_t)(wbase - base);  // tile-local index of item 0
-#pragma unroll
-        for (int i = 0; i < ITEMS; ++i) {
-          const uint32_t d = (key[i] >> shift) & 255u, row = row0 + (uint32_t)(i * kWave);
-          const uint32_t pos = s_wcnt[w][d] + rank[i];
-          s_stage[FULL || row < tile_n ? pos : row] = key[i] << 16 | row;
-        }
-        __syncthreads();
-        uint16_t* dk16 = reinterpret_cast<uint16_t*>(dst_keys + cd.off);
-        uint32_t* dr = dst_rids + cd.off;
-        const uint32_t last = (uint32_t)(n_out - 1);  // stores stay in the column
-        const uint32_t rid0 = cd.rid_base + (uint32_t)base;
-        bool bad = false;
-        // the staged words, then their digits' offsets, then the stores: each
-        // batch of LDS reads issues back to back (slots past tile_n hold the
-        // items past the column and store nothing)
-        uint32_t xs[ITEMS], gs[ITEMS];
-#pragma unroll
-        for (int j = 0; j < ITEMS; ++j) xs[j] = s_stage[(uint32_t)j * THREADS + t];
-#pragma unroll
-        for (int j = 0; j < ITEMS; ++j) gs[j] = s_glob[(xs[j] >> (16 + shift)) & 255u];
-#pragma unroll
-        for (int j = 0; j < ITEMS; ++j) {
-          const uint32_t q = (uint32_t)j * THREADS + t;
-          if (FULL || q < tile_n) {
-            const uint32_t g = gs[j] + q;
-            bad |= g > last;
-            const uint32_t gc = g < last ? g : last;
-            dk16[gc] = (uint16_t)(xs[j] >> 16);
-            dr[gc] = rid0 + (xs[j] & 0xFFFFu);
-          }
-        }
-        if (ballot(bad) && l == 0) atomicOr(fault, 2u);  // a scatter index past the column
-        return;
-      }
-#pragma unroll
-      for (int i = 0; i < ITEMS; ++i) {
-        const uint32_t d = (key[i] >> shift) & 255u;
-        const uint32_t row = (uint32_t)(wbase - base) + (uint32_t)(i * kWave);
-        const uint32_t pos = FULL || row < tile_n ? s_wcnt[w][d] + rank[i] : row;
-        s_stage[pos] = key[i];
-        rank[i] = pos;  // keep the LDS slot for the rids
-      }
-      // LDS slots, two per register (a tile has at most 2^16 items)
-      uint32_t slot2[(ITEMS + 1) / 2];
-#pragma unroll
-      for (int i = 0; i < ITEMS; i += 2)
-        slot2[i / 2] = (rank[i] & 0xFFFFu) | (i + 1 < ITEMS ? rank[i + 1 < ITEMS ? i + 1 : i] << 16 : 0u);
-      // rids: issued now, in flight while the keys go out
-      uint32_t rid[ITEMS];
-      if (implicit) {
-#pragma unroll
-        for (int i = 0; i < ITEMS; ++i) rid[i] = cd.rid_base + (uint32_t)wbase + (uint32_t)(i * kWave);
-      } else {
-        const uint32_t* rp = src_rids + cd.off;
-        const uint32_t first = FULL ? j0 : opaque(j0);
-#pragma unroll
-        for (int i = 0; i < ITEMS; ++i) rid[i] = item(rp, i, first);
-      }
-      __syncthreads();
-      uint32_t* dk = dst_keys + cd.off;
-      uint32_t* dr = dst_rids + cd.off;
-      const uint32_t last = (uint32_t)(n_out - 1);  // stores stay in the column
-      bool bad = false;
-      // destination of each slot this thread stores, kept for the rids (and
-      // literal bits): the digit comes from the staged key
-      uint32_t gq[ITEMS], kq[ITEMS];
-      uint16_t* dk16 = reinterpret_cast<uint16_t*>(dk);
-      // the staged keys, then their digits' offsets, then the stores: each
-      // batch of LDS reads issues back to back (slots past tile_n hold the
-      // items past the column and store nothing)
-#pragma unroll
-      for (int j = 0; j < ITEMS; ++j) kq[j] = s_stage[(uint32_t)j * THREADS + t];
-#pragma unroll
-      for (int j = 0; j < ITEMS; ++j) gq[j] = s_glob[(kq[j] >> shift) & 255u];
-#pragma unroll
-      for (int j = 0; j < ITEMS; ++j) {
-        const uint32_t q = (uint32_t)j * THREADS + t;
-        const uint32_t g = gq[j] + q;
-        const bool in = FULL || q < tile_n;
-        bad |= in && g > last;
-        gq[j] = in && g < last ? g : last;
-      }
-      if (narrow) {
-#pragma unroll
-        for (int j = 0; j < ITEMS; ++j)
-          if (FULL || (uint32_t)j * THREADS + t < tile_n) dk16[gq[j]] = (uint16_t)kq[j];
-      } else {
-#pragma unroll
-        for (int j = 0; j < ITEMS; ++j)
-          if (FULL || (uint32_t)j * THREADS + t < tile_n) dk[gq[j]] = kq[j];
-      }
-      __syncthreads();
-#pragma unroll
-      for (int i = 0; i < ITEMS; ++i) s_stage[(slot2[i / 2] >> (16 * (i % 2))) & 0xFFFFu] = rid[i];
-      if (RUN) {  // literal bits: issued now, in flight while the rids go out
-        const uint32_t* lp = src_lits + cd.off;
-        const uint32_t first = FULL ? j0 : opaque(j0);
-#pragma unroll
-        for (int i = 0; i < ITEMS; ++i) rid[i] = item(lp, i, first);
-      }
-      __syncthreads();
-#pragma unroll
-      for (int j = 0; j < ITEMS; ++j) kq[j] = s_stage[(uint32_t)j * THREADS + t];
-#pragma unroll
-      for (int j = 0; j < ITEMS; ++j)
-        if (FULL || (uint32_t)j * THREADS + t < tile_n) dr[gq[j]] = kq[j];
-      if (RUN) {
-        // literal bits of each run item, moved along with its key and rid
-        __syncthreads();
-#pragma unroll
-        for (int i = 0; i < ITEMS; ++i)
-          s_stage[(slot2[i / 2] >> (16 * (i % 2))) & 0xFFFFu] = rid[i];
-        __syncthreads();
-        uint32_t* dl = dst_lits + cd.off;
-#pragma unroll
-        for (int j = 0; j < ITEMS; ++j) kq[j] = s_stage[(uint32_t)j * THREADS + t];
-#pragma unroll
-        for (int j = 0; j < ITEMS; ++j)
-          if (FULL || (uint32_t)j * THREADS + t < tile_n) dl[gq[j]] = kq[j];
-      }
-      if (ballot(bad) && l == 0) atomicOr(fault, 2u);  // a scatter index past the column
-    };
-    auto dispatch = [&](auto packed_tag) {
-      if (base + TILE <= n) sweep(std::true_type{}, packed_tag);
-      else sweep(std::false_type{}, packed_tag);
-    };
-    if constexpr (!RUN) {
-      if (implicit && narrow) dispatch(std::true_type{});
-      else dispatch(std::false_type{});
-    } else {
-      dispatch(std::false_type{});
-    }
-    __syncthreads();
+  if constexpr (MODES != 1) {
+    constexpr bool RUN = false;
+#include "radix_tiles.inl"
+  }
+  if constexpr (MODES == 2) __syncthreads();  // the last draw is read before the next mode's first
+  if constexpr (MODES != 0) {
+    constexpr bool RUN = true;
+#include "radix_tiles.inl"
   }
 }
 
@@ -1367,7 +1097,9 @@ __device__ __forceinline__ SortedView sorted_view(const ColState* col, const Col
 // are exchanged in LDS.  Words are staged in LDS at tile-local positions and
 // stored contiguously.
 // ---------------------------------------------------------------------------
-template <int THREADS, int ITEMS, bool RUN>
+// MODES as in k_onesweep: one mode's tiles per launch for long columns, both in
+// one launch for the others.
+template <int THREADS, int ITEMS, int MODES>
 __global__ __launch_bounds__(THREADS, tail_waves_per_eu(ITEMS)) void k_tail(
     const DescHead* __restrict__ desc, const ColState* __restrict__ cs, Header* __restrict__ hdr,
     const uint32_t* values, const uint32_t* keysA, const uint32_t* ridsA,
@@ -1388,356 +1120,14 @@ __global__ __launch_bounds__(THREADS, tail_waves_per_eu(ITEMS)) void k_tail(
   __shared__ uint32_t s_wlead[WAVES + 1];  // [w]: lead bits of wave w; [WAVES]: of the next tile
   __shared__ uint64_t s_prefix;
   __shared__ uint32_t s_tile;
-  const Dims dims = desc->dims;
-  const Column* cols = desc_cols(desc);
-  // the wave index in a scalar register: per-wave LDS addresses stay out of
-  // the 64 vector registers
-  const int t = threadIdx.x, l = t % kWave;
-  const int w = __builtin_amdgcn_readfirstlane(t / kWave);
-  uint32_t* fault = &hdr->fault;
-  if (hdr->mode_cols[RUN ? 1 : 0] == 0) return;  // no column in this mode
-
-  uint32_t iter = 0;
-  for (;;) {
-    const uint32_t tile = __builtin_amdgcn_readfirstlane(next_tile(
-        &hdr->tiles[RUN ? kCounterRunTail : kCounterTail][0], lanes, &s_tile, iter,
-        tile_group(dims.tail_tiles, lanes, WAH_TAIL_TILE_GROUP)));
-    if (tile >= dims.tail_tiles) break;
-    const uint32_t c = find_segment(&cols[0].tail_tile0, sizeof(Column) / 4, dims.ncols, tile);
-    const Column cd = cols[c];
-    const uint32_t first_tile = cd.tail_tile0;
-    // column-local indices fit 32 bits: a column holds fewer than 2^30 items
-    const uint32_t base = (tile - first_tile) * (uint32_t)TILE;
-    // items: rows, or the runs of a run-mode column (fewer than its tiles)
-    const uint32_t n = RUN ? (uint32_t)cs[c].items : (uint32_t)cd.n;
-    if (cs[c].mode != (RUN ? kModeRun : kModePair) || base >= n) {
-      if (RUN && c + 1 == dims.ncols && cs[c].mode == kModeRun) break;  // past the last items
-      __syncthreads();  // s_tile is read by every wave before it is rewritten
-      continue;
-    }
-    // the tile's body, compiled once per key width (16-bit keys load 8 per
-    // 16 bytes); the column's width picks one
-    // and once for whole aligned tiles (16-byte loads, no per-item checks,
-    // and no control-flow merge with the per-item loads of partial tiles)
-    const SortedView sv0 =
-        sorted_view(&cs[c], cd, values, keysA, ridsA, keysB, ridsB, litsA, litsB);
-    const bool aligned = (((uintptr_t)sv0.keys | (uintptr_t)sv0.rids |
-                           (RUN ? (uintptr_t)sv0.lits : (uintptr_t)0)) % 16) == 0;
-    auto body = [&](auto narrow_tag, auto full_tag) {
-    constexpr bool NARROW = decltype(narrow_tag)::value;
-    constexpr bool FULL = decltype(full_tag)::value;
-    const uint32_t rid_base = cd.rid_base;
-    SortedView sv = sv0;
-    sv.narrow = NARROW;
-    const uint32_t j0 = base + (uint32_t)t * ITEMS;  // the lane's first item
-    const uint32_t nv =
-        FULL ? (uint32_t)ITEMS
-             : (n > j0 ? (n - j0 < (uint32_t)ITEMS ? n - j0 : (uint32_t)ITEMS) : 0u);
-
-    // Loads the tile needs besides its own items, issued before them so that
-    // one memory latency covers all: the item before the wave (lane 0's
-    // predecessor; wave-uniform) and, for the last wave, the 32 items after
-    // the tile (the run that crosses its end).
-    // Branch-free: out-of-range indices read item 0 and are masked later
-    // (an implicit-rid column's rids array is the unused ping-pong buffer).
-    const uint32_t gw = base + (uint32_t)(w * kWave * ITEMS);
-    const bool have_pred = gw > 0 && gw <= n;
-    const uint32_t gp = have_pred ? gw - 1 : 0u;
-    uint32_t k0 = sv.key(gp), r0 = sv.rids[gp];
-    const uint32_t gn0 = base + (uint32_t)TILE + (uint32_t)l;
-    const bool nv_next = w == WAVES - 1 && l < 32 && gn0 < n;
-    const uint32_t gn = nv_next ? gn0 : 0u;
-    uint32_t kk = 0, rr = 0, ll = 0;
-    if (w == WAVES - 1) {
-      kk = sv.key(gn);
-      rr = sv.rids[gn];
-      if (RUN) ll = sv.lits[gn];
-    }
-
-    // ---- items of the lane: key, chid, literal bits (0 past the column)
-    uint32_t key[ITEMS], ch[ITEMS], b[ITEMS];
-    if constexpr (FULL) {
-      if (NARROW) {  // 8 keys per 16-byte load
-#pragma unroll
-        for (int q = 0; q < ITEMS / 8; ++q) {
-          const uint4 k8 = reinterpret_cast<const uint4*>(reinterpret_cast<const uint16_t*>(sv.keys) + j0)[q];
-          const uint32_t w4[4] = {k8.x, k8.y, k8.z, k8.w};
-#pragma unroll
-          for (int h = 0; h < 4; ++h) {
-            key[8 * q + 2 * h] = w4[h] & 0xFFFFu;
-            key[8 * q + 2 * h + 1] = w4[h] >> 16;
-          }
-        }
-      }
-#pragma unroll
-      for (int q = 0; q < ITEMS / 4; ++q) {
-        if (!NARROW) {
-          const uint4 k4 = reinterpret_cast<const uint4*>(sv.keys + j0)[q];
-          key[4 * q] = k4.x; key[4 * q + 1] = k4.y; key[4 * q + 2] = k4.z; key[4 * q + 3] = k4.w;
-        }
-        // loaded either way (an implicit-rid column reads the unused
-        // buffer), so the loads are not split by a branch
-        const uint4 r4 = reinterpret_cast<const uint4*>(sv.rids + j0)[q];
-        ch[4 * q] = r4.x; ch[4 * q + 1] = r4.y; ch[4 * q + 2] = r4.z; ch[4 * q + 3] = r4.w;
-        if (RUN) {
-          const uint4 l4 = reinterpret_cast<const uint4*>(sv.lits + j0)[q];
-          b[4 * q] = l4.x; b[4 * q + 1] = l4.y; b[4 * q + 2] = l4.z; b[4 * q + 3] = l4.w;
-        }
-      }
-    } else {
-#pragma unroll
-      for (int i = 0; i < ITEMS; ++i) {
-        const bool v = (uint32_t)i < nv;
-        const uint32_t g = j0 + i;
-        key[i] = v ? sv.key(g) : 0u;
-        ch[i] = v ? (sv.implicit ? rid_base + g : sv.rids[g]) : 0u;
-        if (RUN) b[i] = v ? sv.lits[g] : 0u;
-      }
-    }
-    if (FULL && sv.implicit) {
-#pragma unroll
-      for (int i = 0; i < ITEMS; ++i) ch[i] = rid_base + j0 + (uint32_t)i;
-    }
-    // ch[] held rids so far: chunk id q = rid / 31 and the literal bit
-    // rid % 31 = (rid + q) & 31 (rid + q = 32q + rid % 31).  Rows below 2^31
-    // (every column with rid_base + n <= 2^31) divide by a multiply-high,
-    // exact there (it first fails at 2369637147); the others by the
-    // compiler's full 32-bit division.
-    auto chunks = [&](auto fast_tag) {
-      constexpr bool FAST = decltype(fast_tag)::value;
-#pragma unroll
-      for (int i = 0; i < ITEMS; ++i) {
-        const uint32_t r = ch[i];
-        const uint32_t q = FAST ? __umulhi(r, 0x84210843u) >> 4 : r / 31u;
-        ch[i] = q;
-        if (!RUN) b[i] = (uint32_t)i < nv ? 1u << ((r + q) & 31u) : 0u;
-      }
-    };
-    if ((uint64_t)rid_base + cd.n <= (1ull << 31)) chunks(std::true_type{});
-    else chunks(std::false_type{});
-    // predecessor of the lane's first item: lane l-1's last, or for lane 0
-    // the item before the wave (one load per wave)
-    uint32_t pk, pc;
-    {
-      // first use of the side loads, tied to the tile's own (so that no
-      // arithmetic on them is placed, with its wait, before those loads)
-      k0 = __builtin_amdgcn_readfirstlane(k0);
-      r0 = __builtin_amdgcn_readfirstlane(r0);
-      asm volatile("" : "+s"(k0), "+s"(r0) : "v"(key[ITEMS - 1]), "v"(ch[ITEMS - 1]));
-      if (!have_pred) k0 = r0 = 0u;
-      else if (sv.implicit) r0 = rid_base + gp;
-      const uint32_t c0 = r0 / 31u;
-      pk = (uint32_t)__builtin_amdgcn_update_dpp((int)k0, (int)key[ITEMS - 1], 0x138, 0xF, 0xF, false);
-      pc = (uint32_t)__builtin_amdgcn_update_dpp((int)c0, (int)ch[ITEMS - 1], 0x138, 0xF, 0xF, false);
-    }
-    // ---- entry and key starts, fills, counts
-    const bool colfirst = base == 0 && t == 0;
-    uint32_t f[ITEMS];
-    uint32_t stm = 0, khm = 0, fm = 0;  // per item: entry start, key start, nonzero fill
-#pragma unroll
-    for (int i = 0; i < ITEMS; ++i) {
-      const uint32_t kp = i ? key[i - 1] : pk, cp = i ? ch[i - 1] : pc;
-      const bool v = (uint32_t)i < nv;
-      const bool kh = v && (key[i] != kp || (i == 0 && colfirst));
-      const bool st = kh || (v && ch[i] != cp);
-      f[i] = st ? (kh ? ch[i] : ch[i] - cp - 1u) : 0u;
-      stm |= st ? 1u << i : 0u;
-      khm |= kh ? 1u << i : 0u;
-      fm |= f[i] != 0u ? 1u << i : 0u;
-    }
-    // From here on an item's flags are read back from these bits: the
-    // compiler would otherwise keep each item's compare masks (64-bit scalar
-    // pairs) alive to the staging and spill them to VGPR lanes.
-    stm = opaque(stm);
-    khm = opaque(khm);
-    fm = opaque(fm);
-    const uint32_t nwords = (uint32_t)(__builtin_popcount(stm) + __builtin_popcount(fm));
-    // lead bits: items before the lane's first stop (entry start or end of items)
-    const uint32_t stops = stm | (~0u << nv & kAll);
-    const uint32_t fs = stops ? (uint32_t)__builtin_ctz(stops) : (uint32_t)ITEMS;
-    uint32_t lead = 0;
-#pragma unroll
-    for (int i = 0; i < ITEMS; ++i) lead |= (uint32_t)i < fs ? b[i] : 0u;
-    // continuation of the lane's last run inside the wave: leads of lanes
-    // l+1 .. the next lane with a stop (at most 4 lanes on)
-    const uint64_t hsm = ballot(stops != 0u);
-    const uint64_t above = l == kWave - 1 ? 0ull : hsm >> (l + 1);
-    const uint32_t dist = above ? (uint32_t)__builtin_ctzll(above) + 1u : 64u;
-    uint32_t cont = 0;
-    {
-      uint32_t sh = lead;
-#pragma unroll
-      for (uint32_t s = 1; s <= 4; ++s) {
-        sh = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)sh, 0x130, 0xF, 0xF, false);  // wave_shl:1
-        cont |= s <= dist ? sh : 0u;
-      }
-    }
-    // wave lead: lane 0's items before its first stop and, without one, the
-    // lanes after it
-    {
-      const uint32_t wl = readlane(stops ? lead : lead | cont, 0);
-      if (l == 0) s_wlead[w] = wl;
-    }
-    // next tile's lead: the run that crosses the tile end (last wave, 32 items)
-    if (w == WAVES - 1) {
-      const bool v = nv_next;
-      if (sv.implicit) rr = rid_base + gn;
-      uint32_t cc = 0, bb = 0;
-      if (!v) kk = 0u;
-      if (v) {
-        cc = rr / 31u;
-        bb = RUN ? ll : 1u << (rr - cc * 31u);
-      }
-      const uint32_t kl = readlane(key[ITEMS - 1], kWave - 1), cl = readlane(ch[ITEMS - 1], kWave - 1);
-      const uint32_t kq = (uint32_t)__builtin_amdgcn_update_dpp((int)kl, (int)kk, 0x138, 0xF, 0xF, false);
-      const uint32_t cq = (uint32_t)__builtin_amdgcn_update_dpp((int)cl, (int)cc, 0x138, 0xF, 0xF, false);
-      const uint64_t sm = ballot(!v || kk != kq || cc != cq);  // lanes 32.. always stop
-      const int fh = __builtin_ctzll(sm);
-      const uint32_t tl = wave_or(l < fh ? bb : 0u);
-      if (l == 0) s_wlead[WAVES] = tl;
-    }
-    // tile-local word and key offsets: one wave scan of (keys << 16 | words)
-    const uint32_t packed = ((uint32_t)__builtin_popcount(khm) << 16) | nwords;
-    const uint32_t inc = wave_incl_add(packed);
-    if (l == kWave - 1) s_wtot[w] = inc;
-    {
-      // entries of the tile (k of the column is their sum, formed by k_finish)
-      const uint32_t e = readlane(wave_incl_add((uint32_t)__builtin_popcount(stm)), kWave - 1);
-      if (l == 0) s_went[w] = e;
-    }
-    __syncthreads();
-
-    // ---- literals: reverse sweep along the lane, seeded with the bits the
-    // lane's last run picks up from the lanes (wave, tile) after it
-    if (above == 0) cont |= s_wlead[w + 1];
-    if (nv < (uint32_t)ITEMS) cont = 0;  // the run ends with the items
-    uint32_t woff, tot;
-    {
-      // wave totals: one LDS read per lane and a wave scan
-      const uint32_t lo = opaque((uint32_t)l);
-      const uint32_t x = lo < WAVES ? s_wtot[lo] : 0u;
-      const uint32_t xi = wave_incl_add(x);
-      woff = readlane(xi - x, __builtin_amdgcn_readfirstlane(w));
-      tot = readlane(xi, WAVES - 1);
-    }
-    const uint32_t lpos = woff + inc - packed;  // (keys << 16 | words) before the lane
-    if (w == 0) {
-      const uint64_t tile_agg = ((uint64_t)(tot >> 16) << 31) | (tot & 0xFFFFu);
-      const uint64_t pre = lookback_wave_sum<WAH_TAIL_LOOKBACK_SLOTS>(status, tile, first_tile,
-                                                                      tile_agg, fault);
-      const uint32_t lo = opaque((uint32_t)l);
-      const uint32_t e = readlane(wave_incl_add(lo < WAVES ? s_went[lo] : 0u), kWave - 1);
-      if (l == 0) {
-        s_prefix = pre;
-        tile_entries[tile] = e;
-      }
-    }
-    {
-      // from the lane's last word back: [fill,] literal of each entry start
-      uint32_t carry = cont;
-      uint32_t pos = (lpos & 0xFFFFu) + nwords;
-#pragma unroll
-      for (int i = ITEMS - 1; i >= 0; --i) {
-        const bool st = (stm >> i) & 1u, fw = (fm >> i) & 1u;
-        carry |= b[i];
-        pos -= st ? 1u : 0u;
-        if (st) s_words[pos + (pos >> 4)] = 0x80000000u | carry;
-        pos -= fw ? 1u : 0u;
-        if (fw) s_words[pos + (pos >> 4)] = f[i];
-        carry = st ? 0u : carry;
-      }
-    }
-    uint32_t kv[ITEMS];
-    if (khm) {
-      // key starts: the values (the lane's keys read again, all at once:
-      // the lines are still in L2) and the position of each key's first word
-      if (nv == (uint32_t)ITEMS && aligned && !NARROW) {
-#pragma unroll
-        for (int q = 0; q < ITEMS / 4; ++q) {
-          const uint4 k4 = reinterpret_cast<const uint4*>(sv.keys + j0)[q];
-          kv[4 * q] = k4.x; kv[4 * q + 1] = k4.y; kv[4 * q + 2] = k4.z; kv[4 * q + 3] = k4.w;
-        }
-      } else if (nv == (uint32_t)ITEMS && aligned) {
-#pragma unroll
-        for (int q = 0; q < ITEMS / 8; ++q) {
-          const uint4 k8 = reinterpret_cast<const uint4*>(reinterpret_cast<const uint16_t*>(sv.keys) + j0)[q];
-          const uint32_t w4[4] = {k8.x, k8.y, k8.z, k8.w};
-#pragma unroll
-          for (int h = 0; h < 4; ++h) {
-            kv[8 * q + 2 * h] = w4[h] & 0xFFFFu;
-            kv[8 * q + 2 * h + 1] = w4[h] >> 16;
-          }
-        }
-      } else {
-#pragma unroll
-        for (int i = 0; i < ITEMS; ++i) kv[i] = (uint32_t)i < nv ? sv.key(j0 + i) : 0u;
-      }
-    }
-    __syncthreads();  // words staged, prefix published
-    const uint64_t pre = s_prefix;
-    const uint32_t Wpre = (uint32_t)(pre & 0x7FFFFFFFu), Kpre = (uint32_t)(pre >> 31);
-    uint32_t* out_keys = keys_out + cd.off;
-    uint32_t* out_offsets = offsets_out + cd.off;
-    uint32_t* out_words = words_out + 2 * cd.off;
-    if (khm) {
-      bool bad = false;
-#pragma unroll
-      for (int i = 0; i < ITEMS; ++i) {
-        if ((khm >> i) & 1u) {
-          const uint32_t below = (1u << i) - 1u;
-          const uint32_t kg = Kpre + (lpos >> 16) + __builtin_popcount(khm & below);
-          const uint32_t wp = (lpos & 0xFFFFu) + __builtin_popcount(stm & below) +
-                              __builtin_popcount(fm & below);
-          bad |= kg >= n;
-          const uint32_t kc = kg < n ? kg : n - 1u;  // stores stay in the column
-          out_keys[kc] = kv[i];
-          out_offsets[kc] = Wpre + wp;
-        }
-      }
-      if (bad) atomicOr(fault, 2u);
-    }
-    const uint32_t Wt = tot & 0xFFFFu;
-    if ((uint64_t)Wpre + Wt <= 2ull * n) {
-      // single words up to the first 16-byte boundary, then 4 words per
-      // 16-byte store, then the rest
-      uint32_t* ow = out_words + Wpre;
-      const uint32_t head0 = (4u - (uint32_t)(((uintptr_t)ow >> 2) & 3u)) & 3u;
-      const uint32_t head = head0 < Wt ? head0 : Wt;
-      const uint32_t quads = (Wt - head) / 4u;
-      const uint32_t tt = opaque((uint32_t)t);
-      if (tt < head) ow[tt] = s_words[tt + (tt >> 4)];
-      for (uint32_t qd = tt; qd < quads; qd += THREADS) {
-        const uint32_t j = head + 4u * qd;
-        uint4 v;
-        v.x = s_words[j + (j >> 4)];
-        v.y = s_words[j + 1u + ((j + 1u) >> 4)];
-        v.z = s_words[j + 2u + ((j + 2u) >> 4)];
-        v.w = s_words[j + 3u + ((j + 3u) >> 4)];
-        *reinterpret_cast<uint4*>(ow + j) = v;  // 16-byte aligned: j - head is a multiple of 4
-      }
-      for (uint32_t j = head + 4u * quads + tt; j < Wt; j += THREADS) ow[j] = s_words[j + (j >> 4)];
-    } else {
-      for (uint32_t j = opaque((uint32_t)t); j < Wt; j += THREADS) {
-        const uint32_t o = Wpre + j;
-        if (o < 2 * n) out_words[o] = s_words[j + (j >> 4)];
-        else atomicOr(fault, 2u);
-      }
-    }
-    if (base + TILE >= n && t == 0) {  // the column's last tile
-      counts[cd.index].length = (uint64_t)Wpre + Wt;
-      counts[cd.index].keycnt = (uint64_t)Kpre + (tot >> 16);
-    }
-    };
-    const bool full = base + TILE <= n && aligned;
-    if (cs[c].narrow) {
-      if (full) body(std::true_type{}, std::true_type{});
-      else body(std::true_type{}, std::false_type{});
-    } else {
-      if (full) body(std::false_type{}, std::true_type{});
-      else body(std::false_type{}, std::false_type{});
-    }
-    // the next tile's first barrier (in next_tile) orders these LDS reads
-    // before its writes
+  if constexpr (MODES != 1) {
+    constexpr bool RUN = false;
+#include "tail_tiles.inl"
+  }
+  if constexpr (MODES == 2) __syncthreads();  // the last draw is read before the next mode's first
+  if constexpr (MODES != 0) {
+    constexpr bool RUN = true;
+#include "tail_tiles.inl"
   }
 }
 
@@ -1881,7 +1271,8 @@ static void launch_radix(const BuildArgs& a, hipStream_t s, LaunchHook* hook) {
   const uint32_t grid = tile_grid(a.sort_tiles_cap, WAH_STATIC_TILES
                                                        ? a.sort_tiles_cap
                                                        : a.max_resident / 4 * sort_blocks_per_cu<T, I>());
-  hipLaunchKernelGGL(k_runcut, dim3(cap_grid(a.sort_tiles_cap, 2 * a.max_resident)), dim3(kBlock),
+  if (!a.force_pair)
+    hipLaunchKernelGGL(k_runcut, dim3(cap_grid(a.sort_tiles_cap, 2 * a.max_resident)), dim3(kBlock),
                      0, s, a.values, a.keysB, a.ridsB, a.litsB, a.desc, a.cs, a.hdr, a.tile_runs,
                      (uint32_t)(T * I));
   // wide digits: the histograms of the wide columns' digits and their offsets
@@ -1897,22 +1288,19 @@ static void launch_radix(const BuildArgs& a, hipStream_t s, LaunchHook* hook) {
   }
   if (hook) hook->mark(s);
   // each launch runs the a-th pass of pair-mode columns, then of run-mode
-  // columns; a kernel with no such column returns at once
+  // columns
   for (uint32_t p = 0; p < 4; ++p) {
-    if (a.atomic_rank) {
-      hipLaunchKernelGGL((k_onesweep<T, I, false, kRankAtomic>), dim3(grid), dim3(T), 0, s, p,
-                         a.values, a.keysA, a.ridsA, a.keysB, a.ridsB, a.litsA, a.litsB, a.desc,
-                         a.cs, a.hdr, a.sort_status, a.sort_status_stride, tile_lanes(grid));
-      hipLaunchKernelGGL((k_onesweep<T, I, true, kRankAtomic>), dim3(grid), dim3(T), 0, s, p,
-                         a.values, a.keysA, a.ridsA, a.keysB, a.ridsB, a.litsA, a.litsB, a.desc,
-                         a.cs, a.hdr, a.sort_status, a.sort_status_stride, tile_lanes(grid));
+    auto sweep = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3(grid), dim3(T), 0, s, p, a.values, a.keysA, a.ridsA, a.keysB,
+                         a.ridsB, a.litsA, a.litsB, a.desc, a.cs, a.hdr, a.sort_status,
+                         a.sort_status_stride, tile_lanes(grid));
+    };
+    if (!a.long_tail && !a.force_pair) {
+      sweep(a.atomic_rank ? k_onesweep<T, I, kRankAtomic, 2> : k_onesweep<T, I, kRankMatch, 2>);
     } else {
-      hipLaunchKernelGGL((k_onesweep<T, I, false, kRankMatch>), dim3(grid), dim3(T), 0, s, p,
-                         a.values, a.keysA, a.ridsA, a.keysB, a.ridsB, a.litsA, a.litsB, a.desc,
-                         a.cs, a.hdr, a.sort_status, a.sort_status_stride, tile_lanes(grid));
-      hipLaunchKernelGGL((k_onesweep<T, I, true, kRankMatch>), dim3(grid), dim3(T), 0, s, p,
-                         a.values, a.keysA, a.ridsA, a.keysB, a.ridsB, a.litsA, a.litsB, a.desc,
-                         a.cs, a.hdr, a.sort_status, a.sort_status_stride, tile_lanes(grid));
+      sweep(a.atomic_rank ? k_onesweep<T, I, kRankAtomic, 0> : k_onesweep<T, I, kRankMatch, 0>);
+      if (!a.force_pair)
+        sweep(a.atomic_rank ? k_onesweep<T, I, kRankAtomic, 1> : k_onesweep<T, I, kRankMatch, 1>);
     }
     if (a.wide_tiles_cap && p < (uint32_t)kWidePasses) {
       if (a.atomic_rank)
@@ -1953,49 +1341,25 @@ void launch_sort(const BuildArgs& a, hipStream_t s, LaunchHook* hook) {
   static_assert(kRadixShapes == 6, "a case per compiled shape");
 }
 
-// Both tails of a long column, on 16384-item tiles.
-static void launch_long_tail(const BuildArgs& a, hipStream_t s) {
-  const uint32_t grid =
-      tile_grid(a.tail_tiles_cap, WAH_STATIC_TILES ? a.tail_tiles_cap
-                                                  : a.max_resident / 4 * kLongTailBlocksPerCU);
-  const uint32_t lanes = WAH_TAIL_LANES ? WAH_TAIL_LANES : tile_lanes(grid);
-  hipLaunchKernelGGL((k_tail<kLongTailThreads, kLongTailItems, false>), dim3(grid),
-                     dim3(kLongTailThreads), 0, s, a.desc, a.cs, a.hdr, a.values, a.keysA,
-                     a.ridsA, a.keysB, a.ridsB, a.litsA, a.litsB, a.out_keys, a.out_offsets,
-                     a.out_words, a.tail_status, a.tile_entries, lanes, a.counts);
-  hipLaunchKernelGGL((k_tail<kLongTailThreads, kLongTailItems, true>), dim3(grid),
-                     dim3(kLongTailThreads), 0, s, a.desc, a.cs, a.hdr, a.values, a.keysA,
-                     a.ridsA, a.keysB, a.ridsB, a.litsA, a.litsB, a.out_keys, a.out_offsets,
-                     a.out_words, a.tail_status, a.tile_entries, lanes, a.counts);
-}
-
-// Both tails of other columns and of batches, on 8192-item tiles.
-static void launch_short_tail(const BuildArgs& a, hipStream_t s) {
-  const uint32_t grid =
-      tile_grid(a.tail_tiles_cap, WAH_STATIC_TILES ? a.tail_tiles_cap
-                                                  : a.max_resident / 4 * kTailBlocksPerCU);
-  const uint32_t lanes = WAH_TAIL_LANES ? WAH_TAIL_LANES : tile_lanes(grid);
-  hipLaunchKernelGGL((k_tail<kTailThreads, kTailItems, false>), dim3(grid), dim3(kTailThreads),
-                     0, s, a.desc, a.cs, a.hdr, a.values, a.keysA, a.ridsA, a.keysB, a.ridsB,
-                     a.litsA, a.litsB, a.out_keys, a.out_offsets, a.out_words, a.tail_status,
-                     a.tile_entries, lanes, a.counts);
-  // run mode: the same tiles as 512 threads x 16 items (fewer, longer lanes
-  // suit its sparser items)
-  const uint32_t rgrid =
-      tile_grid(a.tail_tiles_cap, WAH_STATIC_TILES ? a.tail_tiles_cap
-                                                  : a.max_resident / 4 * kRunTailBlocksPerCU);
-  const uint32_t rlanes = WAH_TAIL_LANES ? WAH_TAIL_LANES : tile_lanes(rgrid);
-  hipLaunchKernelGGL((k_tail<kRunTailThreads, kRunTailItems, true>), dim3(rgrid),
-                     dim3(kRunTailThreads), 0, s, a.desc, a.cs, a.hdr, a.values, a.keysA, a.ridsA,
-                     a.keysB, a.ridsB, a.litsA, a.litsB, a.out_keys, a.out_offsets, a.out_words,
-                     a.tail_status, a.tile_entries, rlanes, a.counts);
+// The tails of a long column, on 16384-item tiles, or of other columns and of
+// batches, on 8192-item tiles.
+template <int T, int I, int MODES>
+static void launch_tail_tiles(const BuildArgs& a, uint32_t blocks_per_cu, hipStream_t s) {
+  const uint32_t grid = tile_grid(
+      a.tail_tiles_cap, WAH_STATIC_TILES ? a.tail_tiles_cap : a.max_resident / 4 * blocks_per_cu);
+  hipLaunchKernelGGL((k_tail<T, I, MODES>), dim3(grid), dim3(T), 0, s, a.desc, a.cs, a.hdr,
+                     a.values, a.keysA, a.ridsA, a.keysB, a.ridsB, a.litsA, a.litsB, a.out_keys,
+                     a.out_offsets, a.out_words, a.tail_status, a.tile_entries,
+                     WAH_TAIL_LANES ? WAH_TAIL_LANES : tile_lanes(grid), a.counts);
 }
 
 void launch_tail(const BuildArgs& a, hipStream_t s, LaunchHook* hook) {
-  if (a.long_tail)
-    launch_long_tail(a, s);
-  else
-    launch_short_tail(a, s);
+  if (a.long_tail) {
+    launch_tail_tiles<kLongTailThreads, kLongTailItems, 0>(a, kLongTailBlocksPerCU, s);
+    launch_tail_tiles<kLongTailThreads, kLongTailItems, 1>(a, kLongTailBlocksPerCU, s);
+  } else {
+    launch_tail_tiles<kTailThreads, kTailItems, 2>(a, kTailBlocksPerCU, s);
+  }
   if (hook) hook->mark(s);
   // blocks for up to 8 x 256 keys per column of a batch at a time
   const uint64_t lg = (a.n_cap + kBlock - 1) / kBlock, most = a.cols_cap > 128u ? 8ull * a.cols_cap : 1024u;
