@@ -138,8 +138,11 @@ constexpr uint32_t kBufB = 2;
 
 constexpr uint32_t kLaneWords = 8 * 64;     // tile-counter lanes of one kernel
 constexpr uint32_t kHistChunk = 4096;       // values per histogram work item
+constexpr uint32_t kCutTiles = 4096;        // k_runcut: whole radix tiles from here on
 constexpr bool radix_tiles_whole_chunks(int sh = 0) {
-  return sh == kRadixShapes || (radix_tile(sh) % kHistChunk == 0 && radix_tiles_whole_chunks(sh + 1));
+  return sh == kRadixShapes || (radix_tile(sh) % kHistChunk == 0 &&
+                                  radix_tile(sh) / kHistChunk * 4 <= 64 &&
+                                  radix_tiles_whole_chunks(sh + 1));
 }
 static_assert(radix_tiles_whole_chunks(), "radix tiles hold whole histogram chunks");
 
@@ -231,7 +234,8 @@ struct WideState {
 struct BuildArgs {
   const uint32_t* values;            // concatenated input
   uint32_t *keysA, *ridsA, *keysB, *ridsB;
-  uint32_t *litsA, *litsB;           // run mode: literal bits of each item
+  uint32_t *litsA, *litsB;           // run mode: literal bits of each item; before the
+                                     // first pass litsA holds the runs of each chunk's waves
   DescHead* desc;                    // device descriptor
   Header* hdr;
   ColState* cs;                      // cols_cap entries

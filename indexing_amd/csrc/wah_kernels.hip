@@ -91,7 +91,7 @@ __global__ __launch_bounds__(kBlock, 8) void k_histogram(
     const uint32_t* __restrict__ values, const DescHead* __restrict__ desc,
     ColState* __restrict__ cs, uint32_t* __restrict__ status0,
     uint64_t* __restrict__ tail_status, uint32_t* __restrict__ tile_entries,
-    uint32_t* __restrict__ tile_runs, uint32_t sort_tile) {
+    uint32_t* __restrict__ tile_runs, uint32_t sort_tile, uint32_t* __restrict__ chunk_runs) {
   __shared__ uint32_t h[4 * 256];
   __shared__ uint32_t hr[4 * 256];
   __shared__ uint32_t s_max[kWaves];
@@ -227,12 +227,20 @@ __global__ __launch_bounds__(kBlock, 8) void k_histogram(
       // a bit varies over the 1024 rows iff it varies inside a span or
       // between the spans' first values
       const uint32_t vary = wave_or(x) | fx;
-      // runs of the wave's rows, added to their radix tile (a run-mode
-      // column's cut places its items from these counts); no block barrier,
-      // so the waves of a block stream their chunks independently
+      // runs of the wave's rows, added to their radix tile and, where the cut
+      // goes by chunks (see k_runcut), kept in the wave's word of the chunk's
+      // four: a run-mode column's cut places its items from them.  The words
+      // are the column's part of a literal buffer that nothing holds yet; a
+      // wave without rows has none, so they end before the column's.  No
+      // block barrier, so the waves of a block stream their chunks
+      // independently.
       const uint32_t reps = readlane(wave_incl_add((uint32_t)__builtin_popcount(rm)), kWave - 1);
-      if (lane_id() == 0 && rows != reps)
-        atomicAdd(&tile_runs[cd.sort_tile0 + (uint32_t)(lo / sort_tile)], rows - reps);
+      if (lane_id() == 0) {
+        if (dims.sort_tiles < kCutTiles)
+          chunk_runs[cd.off + lo / (kHistChunk / 4) + wv] = rows - reps;
+        if (rows != reps)
+          atomicAdd(&tile_runs[cd.sort_tile0 + (uint32_t)(lo / sort_tile)], rows - reps);
+      }
       if (vary == 0u) {
         // every row of the chunk holds f0 (inside a run): lane p adds the
         // wave's rows, and its repeat rows, to digit p's bin of f0
@@ -451,10 +459,17 @@ __global__ __launch_bounds__(kBlock) void k_plan(const DescHead* __restrict__ de
 // (a row starts one unless it repeats its predecessor's value inside the
 // same 31-row chunk) and writes one item per run, in row order, to buffer B:
 // value, rid of its first row, literal bits of its rows.  An ordered stream
-// compaction without look-back: the histogram counted the runs of each
-// radix tile and k_plan turned the counts into per-tile offsets.  A block
-// takes whole radix tiles (static grid stride) and walks each in steps of
-// kBlock x 16 rows with a running offset.  Lane t owns 16 consecutive rows
+// compaction without look-back: the histogram counted the runs of each radix
+// tile, k_plan turned the counts into offsets, and a block takes whole units
+// (static grid stride) and walks a unit in steps of one chunk of the
+// histogram with a running offset.  A unit is a radix tile where there are
+// kCutTiles or more: one for every block that runs.  With fewer, blocks that
+// walk a 16384-row tile in four steps leave the chip idle (the cut of 128
+// columns of 2^17 rows, and of one of 2^20, took 30 us); there a unit is one
+// chunk, placed by its tile's offset and the runs that the histogram kept for
+// the tile's earlier chunks (15 us; 128 columns of 2^17 rows build in 481 us,
+// 492 before).  Chunks everywhere cost a column of 2^28 rows 10 us more.
+// Lane t owns 16 consecutive rows
 // (16-byte loads); a run is at most 31 rows, so the run of a lane's last
 // start ends within the next two lanes (or the next wave's first two, or
 // the rows past the step, exchanged in LDS).  Items are staged in LDS and
@@ -462,11 +477,13 @@ __global__ __launch_bounds__(kBlock) void k_plan(const DescHead* __restrict__ de
 // ---------------------------------------------------------------------------
 constexpr int kCutRows = 16;                    // rows per lane
 constexpr int kCutStep = kBlock * kCutRows;     // rows per block step
+static_assert(kCutStep == (int)kHistChunk, "a chunk of the histogram per block step");
 __global__ __launch_bounds__(kBlock, 8) void k_runcut(
     const uint32_t* __restrict__ values, uint32_t* __restrict__ keysB,
     uint32_t* __restrict__ ridsB, uint32_t* __restrict__ litsB,
     const DescHead* __restrict__ desc, const ColState* __restrict__ cs,
-    Header* __restrict__ hdr, const uint32_t* __restrict__ tile_runs, uint32_t sort_tile) {
+    Header* __restrict__ hdr, const uint32_t* __restrict__ tile_runs, uint32_t sort_tile,
+    const uint32_t* __restrict__ chunk_runs) {
   constexpr int R = kCutRows;
   constexpr uint32_t kAll = (1u << R) - 1u;
   __shared__ uint32_t s_stage[kCutStep];
@@ -477,27 +494,39 @@ __global__ __launch_bounds__(kBlock, 8) void k_runcut(
   const int t = threadIdx.x, l = t % kWave;
   const int w = __builtin_amdgcn_readfirstlane(t / kWave);  // scalar: per-wave LDS addresses
   if (hdr->mode_cols[1] == 0) return;  // no run-mode column
-  for (uint32_t tile = blockIdx.x; tile < dims.sort_tiles; tile += gridDim.x) {
-    const uint32_t c = find_segment(&cols[0].sort_tile0, sizeof(Column) / 4, dims.ncols, tile);
+  const bool whole = dims.sort_tiles >= kCutTiles;
+  const uint32_t units = whole ? dims.sort_tiles : dims.hist_chunks;
+  const uint32_t unit_rows = whole ? sort_tile : kHistChunk;
+  const uint32_t* unit0 = whole ? &cols[0].sort_tile0 : &cols[0].hist_chunk0;
+  for (uint32_t u = blockIdx.x; u < units; u += gridDim.x) {
+    const uint32_t c = find_segment(unit0, sizeof(Column) / 4, dims.ncols, u);
     const ColState* col = &cs[c];
     if (col->mode != kModeRun) continue;  // block-uniform, no LDS touched
     const Column cd = cols[c];
     // column-local rows fit 32 bits (a column holds fewer than 2^30)
     const uint32_t n = (uint32_t)cd.n;
-    const uint32_t t0 = (tile - cd.sort_tile0) * sort_tile;
-    const uint32_t t1 = t0 + sort_tile < n ? t0 + sort_tile : n;
+    const uint32_t t0 = (u - (whole ? cd.sort_tile0 : cd.hist_chunk0)) * unit_rows;
+    const uint32_t t1 = t0 + unit_rows < n ? t0 + unit_rows : n;
     const uint32_t* vp = values + cd.off;
-    const bool aligned = ((uintptr_t)vp % 16) == 0;
     const uint32_t items = col->items;
-    uint32_t off = tile_runs[tile];  // runs of the column's earlier rows
+    // runs of the column's earlier rows: those before the radix tile, and the
+    // words of the tile's earlier chunks (a lane a word: no tile has more
+    // than 64)
+    const uint32_t tlo = t0 - t0 % sort_tile;
+    uint32_t off = tile_runs[cd.sort_tile0 + t0 / sort_tile];
+    if (tlo != t0) {  // block-uniform
+      const bool in = (uint32_t)l < (t0 - tlo) / (kHistChunk / 4);
+      const uint32_t x = in ? chunk_runs[cd.off + tlo / (kHistChunk / 4) + l] : 0u;
+      off += readlane(wave_incl_add(x), kWave - 1);
+    }
     for (uint32_t lo = t0; lo < t1; lo += kCutStep) {
       const uint32_t j0 = lo + (uint32_t)t * R;  // the lane's first row
       const uint32_t nv = t1 > j0 ? (t1 - j0 < (uint32_t)R ? t1 - j0 : (uint32_t)R) : 0u;
       uint32_t v[R];
-      if (lo + kCutStep <= t1 && aligned) {
+      if (lo + kCutStep <= t1) {
 #pragma unroll
         for (int q = 0; q < R / 4; ++q) {
-          const uint4 x = reinterpret_cast<const uint4*>(vp + j0)[q];
+          const W4 x = reinterpret_cast<const W4u*>(vp + j0)[q];
           v[4 * q] = x.x; v[4 * q + 1] = x.y; v[4 * q + 2] = x.z; v[4 * q + 3] = x.w;
         }
       } else {
@@ -570,7 +599,7 @@ __global__ __launch_bounds__(kBlock, 8) void k_runcut(
       const uint32_t k0 = woff + inc - cnt;  // items of the step before the lane
       if (off + tot > items) {
         if (t == 0) atomicOr(&hdr->fault, 2u);
-        return;  // block-uniform: tile_runs disagree with the items
+        return;  // block-uniform: the chunks' runs disagree with the items
       }
       // the item of start i: round 0 its value, 1 its rid, 2 its literal bits
       auto item = [&](int round, int i) -> uint32_t {
@@ -1272,9 +1301,9 @@ static void launch_radix(const BuildArgs& a, hipStream_t s, LaunchHook* hook) {
                                                        ? a.sort_tiles_cap
                                                        : a.max_resident / 4 * sort_blocks_per_cu<T, I>());
   if (!a.force_pair)
-    hipLaunchKernelGGL(k_runcut, dim3(cap_grid(a.sort_tiles_cap, 2 * a.max_resident)), dim3(kBlock),
-                     0, s, a.values, a.keysB, a.ridsB, a.litsB, a.desc, a.cs, a.hdr, a.tile_runs,
-                     (uint32_t)(T * I));
+    hipLaunchKernelGGL(k_runcut, dim3(cap_grid(a.hist_chunks_cap, 2 * a.max_resident)),
+                       dim3(kBlock), 0, s, a.values, a.keysB, a.ridsB, a.litsB, a.desc, a.cs,
+                       a.hdr, a.tile_runs, (uint32_t)(T * I), a.litsA);
   // wide digits: the histograms of the wide columns' digits and their offsets
   const uint32_t wgrid = tile_grid(a.wide_tiles_cap, WAH_STATIC_TILES ? a.wide_tiles_cap
                                                                     : a.max_resident / 4 * kWideBlocksPerCU);
@@ -1323,8 +1352,7 @@ void launch_sort(const BuildArgs& a, hipStream_t s, LaunchHook* hook) {
   if (hb > a.hist_chunks_cap) hb = a.hist_chunks_cap;
   hipLaunchKernelGGL(k_histogram, dim3(cap_grid((uint32_t)hb, kHistMaxBlocks)), dim3(kBlock), 0,
                      s, a.values, a.desc, a.cs, a.sort_status, a.tail_status, a.tile_entries,
-                     a.tile_runs,
-                     radix_tile(a.shape));
+                     a.tile_runs, radix_tile(a.shape), a.litsA);
   hipLaunchKernelGGL(k_plan, dim3(cap_grid(a.cols_cap, 1024)), dim3(kBlock), 0, s, a.desc, a.cs,
                      a.hdr, a.tile_runs, a.counts, (int)a.force_pair, radix_tile(a.shape), a.wide);
   switch (a.shape) {

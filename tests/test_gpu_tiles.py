@@ -52,6 +52,21 @@ def test_ballot_ranking(monkeypatch, kind):
             assert_same(c.build(v), oracle.build(v), f"{n} {kind}")
 
 
+@pytest.mark.parametrize("shape", [0, 1, 4])
+@pytest.mark.parametrize("tiles", [4094, 4095, 4096])
+def test_run_cut_units(shape, tiles):
+    """The cut of a run-mode column goes by chunks below 4096 radix tiles and
+    by tiles from there on; a last tile of one row and of all but one."""
+    from indexing_amd import _native as N
+    rows = {0: T, 1: T // 2, 4: T // 4}[shape]
+    with ia.Context(0) as c:
+        c.set_tuning([shape] * N.TUNE_BUCKETS)
+        for n in (tiles * rows + 1, (tiles + 1) * rows - 1):
+            v = column("runs", n)
+            print(f"[tiles] cut shape={shape} n={n}", flush=True)
+            assert_same(c.build(v, rid_base=7), oracle.build(v, rid_base=7, threads=8), f"{n}")
+
+
 @pytest.mark.parametrize("reserved", [False, True], ids=["eager", "graph"])
 def test_short_and_long_columns_in_one_batch(reserved):
     """Short columns take a workgroup each beside the launch set of the longer
