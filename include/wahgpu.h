@@ -247,8 +247,11 @@ int wahgpu_graph_stats(const wahgpu_ctx* ctx, uint64_t* captures, uint64_t* repl
  * bucket and one 2^26 column for the last): every shape with 8-bit digits on
  * uniform values with 2^12 distinct (ms), then the fastest shape with 8-bit
  * and with wide digits on uniform values with 2^10 distinct (digit_ms), and
- * keeps the fastest of each per bucket in the context.  The default table is
- * shape 0 and 8-bit digits everywhere. */
+ * keeps the fastest of each per bucket in the context.  The default table
+ * reads shape 0 and 8-bit digits everywhere; a context whose table was never
+ * set takes 8-bit digits and tile shapes by a built-in rule (smaller tiles for
+ * columns of up to 2^21 values and batches of such, unless its arena is
+ * fixed).  The results do not depend on any of this. */
 #define WAHGPU_TUNE_BUCKETS 5
 #define WAHGPU_TUNE_SHAPES 6
 typedef struct wahgpu_tuning {

@@ -54,6 +54,7 @@ struct wahgpu_ctx {
   bool atomic_rank = false;  // radix ranking by LDS fetch-add (self-tested)
   // radix tile shape per column-length bucket (wahgpu_autotune / set_tuning)
   uint32_t tune_shape[WAHGPU_TUNE_BUCKETS] = {0, 0, 0, 0, 0};
+  bool tuned = false;  // a table was installed; until then single_shape / batch_shape choose
   double tune_ms[WAHGPU_TUNE_BUCKETS][WAHGPU_TUNE_SHAPES] = {};
   int force_shape = -1;  // autotune runs: every column in this shape
   // radix digit width per bucket: 8, or 11 = wide digits allowed (when they
@@ -204,8 +205,30 @@ uint32_t bucket_of(uint64_t n) {
     if (n < (1ull << kBucketLog2[b])) return b;
   return WAHGPU_TUNE_BUCKETS - 1;
 }
+// Radix tile shape of a context without a tuning table.  A short column has
+// too few 16384-row tiles (shape 0) for the chip's 256 CUs, so it takes 4096
+// (shape 4) or 8192 rows (shape 1) a tile; from 2^21 rows on the longer runs
+// per digit of a large tile are worth more.  Times in us, shape 0 / 1 / 4,
+// 32-bit uniform values: 10^5 rows 88 / 80 / 77, 500000 98 / 92 / 91, 2^20
+// 114 / 109 / 110, 3 * 2^19 120 / 117 / 124, 2^21 131 / 128 / 138, 2400000
+// 145 / 151 / 160, 2^23 281 / 294 / 332; values in runs: 2^20 118 / 95 / 80.
+// A fixed arena may hold just what shape 0 needs (smaller tiles have more
+// look-back state) and keeps it.
+int single_shape(const wahgpu_ctx* c, uint64_t n) {
+  return c->fixed ? 0 : n < (1ull << 20) ? 4 : n <= (1ull << 21) ? 1 : 0;
+}
+// The one shape of a batch's launch set, by the mean length of its columns:
+// they fill the chip together, so the tile only has to be short against a
+// column.  Shape 0 / 1 / 4: 128 columns of 2^12 to 2^20 values 480 / 470 /
+// 500, 32 of 2^17 to 2^20 289 / 281 / 289, 8 of 2^20 172 / 171 / 179, 40 of
+// 2^19 to 2^22 811 / 825 / 941, 8 of 2^22 407 / 415 / 477.
+int batch_shape(const wahgpu_ctx* c, uint64_t values, uint64_t cols) {
+  return !c->fixed && values / (cols ? cols : 1) < (1ull << 20) ? 1 : 0;
+}
 int shape_for(const wahgpu_ctx* c, uint64_t n) {
-  return c->force_shape >= 0 ? c->force_shape : (int)c->tune_shape[bucket_of(n)];
+  return c->force_shape >= 0 ? c->force_shape
+         : c->tuned          ? (int)c->tune_shape[bucket_of(n)]
+                             : single_shape(c, n);
 }
 
 // A column of n values may take wide digits (k_plan decides from its values).
@@ -792,13 +815,27 @@ constexpr int kSmallShape = wah::kRadixShapes;
 constexpr int kSubShapes = wah::kRadixShapes + 1;  // launch sets a batch may need
 
 // Validates the columns and splits them into sub-batches: the short ones, which
-// take a workgroup each, and the others by tuned shape (all of them when
-// `all_shapes`, empty ones included, so that a captured graph fits any batch).  *shared = element-wise maximum of the
+// take a workgroup each, and the others by tile shape (all that the context
+// may use when `all_shapes`, empty ones included, so that a captured graph fits
+// any batch of the reservation).  *shared = element-wise maximum of the
 // sub-batches' caps (the scratch they share, one after another).
 int plan_batch(wahgpu_ctx* c, const wahgpu_column* cols, uint32_t ncols, uint64_t values_len,
                bool all_shapes, std::vector<SubBatch>* subs, Caps* shared) {
   uint64_t end = 0;
   std::vector<uint32_t> members[kSubShapes];
+  // a captured graph has to fit any batch of the reservation, so its shape
+  // goes by the reservation
+  const bool table = c->tuned || c->force_shape >= 0;
+  uint64_t values = c->res_values, columns = c->res_cols;
+  if (!all_shapes) {
+    values = columns = 0;
+    for (uint32_t i = 0; i < ncols; ++i)
+      if (!small_ok(c, cols[i].n)) {
+        values += cols[i].n;
+        ++columns;
+      }
+  }
+  const int rule = batch_shape(c, values, columns);
   for (uint32_t i = 0; i < ncols; ++i) {
     const wahgpu_column& col = cols[i];
     int rc = check_n(c, col.n, col.rid_base);
@@ -807,12 +844,13 @@ int plan_batch(wahgpu_ctx* c, const wahgpu_column* cols, uint32_t ncols, uint64_
       return fail(c, WAHGPU_EINVAL, "column " + std::to_string(i) +
                                         " overlaps the previous one or exceeds values_len");
     end = col.offset + col.n;
-    members[small_ok(c, col.n) ? kSmallShape : shape_for(c, col.n)].push_back(i);
+    members[small_ok(c, col.n) ? kSmallShape : table ? shape_for(c, col.n) : rule].push_back(i);
   }
   subs->clear();
   *shared = Caps{values_len, 0, 0, 0, 0};
   bool tuned[kSubShapes] = {};
-  for (uint32_t b = 0; b < WAHGPU_TUNE_BUCKETS; ++b) tuned[c->tune_shape[b]] = true;
+  for (uint32_t b = 0; b < WAHGPU_TUNE_BUCKETS; ++b)
+    tuned[table ? (int)c->tune_shape[b] : rule] = true;
   tuned[kSmallShape] = true;
   for (int sh = 0; sh < kSubShapes; ++sh) {
     if (members[sh].empty() && !(all_shapes && tuned[sh])) continue;
@@ -1172,6 +1210,7 @@ int wahgpu_set_tuning(wahgpu_ctx* c, const wahgpu_tuning* in) {
     c->tune_shape[b] = in->shape[b];
     c->tune_digits[b] = in->digit_bits[b] == 11 ? 11u : 8u;
   }
+  c->tuned = true;
   return WAHGPU_OK;
 }
 
@@ -1298,6 +1337,7 @@ int wahgpu_autotune(wahgpu_ctx* c, wahgpu_tuning* out) {
   cleanup();
   if (rc != WAHGPU_OK && !fault_msg.empty()) return fail(c, rc, fault_msg);
   if (rc != WAHGPU_OK) return rc == WAHGPU_EHIP ? fail(c, rc, "autotune: build failed") : rc;
+  c->tuned = true;
   return out ? wahgpu_get_tuning(c, out) : WAHGPU_OK;
 }
 

@@ -52,6 +52,53 @@ def test_ballot_ranking(monkeypatch, kind):
             assert_same(c.build(v), oracle.build(v), f"{n} {kind}")
 
 
+@pytest.mark.parametrize("kind", ["u32", "top", "runs"])
+def test_untuned_shape(ctx, kind):
+    """A context without a tuning table takes its tile shape from the column's
+    length: where it changes; and the shape that a table of zeros keeps."""
+    from indexing_amd import _native as N
+    for n in (2**20 - 1, 2**20, 2**21, 2**21 + 1):
+        v = column(kind, n)
+        print(f"[tiles] untuned n={n} {kind}", flush=True)
+        assert_same(ctx.build(v), oracle.build(v, threads=8), f"{n} {kind}")
+    with ia.Context(0) as c:
+        c.set_tuning([0] * N.TUNE_BUCKETS)
+        for n in (T + 1, 9 * T - 1, 18 * T + 1):
+            v = column(kind, n)
+            print(f"[tiles] table n={n} {kind}", flush=True)
+            assert_same(c.build(v), oracle.build(v), f"{n} {kind}")
+
+
+@pytest.mark.parametrize("reserve", [0, 2**22, 2**24], ids=["eager", "short", "long"])
+def test_untuned_batch_shape(reserve):
+    """A batch's one shape goes by the mean length of its columns, a graph's by
+    that of the reservation."""
+    import torch
+
+    from tests.test_gpu_batch import per_column
+    lens = [2**20 - 1, 2**20 + 1, 20001, 5] if reserve != 2**24 else [2**21 + 3, 17, T + 1, 40000]
+    cols, refs, at = [], [], 0
+    for i, n in enumerate(lens):
+        cols.append((at, n, i))
+        refs.append(oracle.build(column("u32", n), rid_base=i, threads=8))
+        at += (n + 63) // 64 * 64
+    buf = torch.zeros(at, dtype=torch.int32, device="cuda:0")
+    for o, n, _ in cols:
+        buf[o:o + n] = torch.from_numpy(column("u32", n).view(np.int32))
+    with ia.Context(0) as c:
+        if reserve:
+            c.batch_reserve(reserve, 8)
+        out = None
+        for _ in range(3):
+            out = c.build_batch_device(buf, cols) if out is None else \
+                c.build_batch_device(buf, cols, out)
+            counts = c.read_counts_batch(out[4], len(lens))
+            got = per_column(out, counts, [(o, n) for o, n, _ in cols])
+            for i, (g, r) in enumerate(zip(got, refs)):
+                assert counts[i].fault == 0
+                assert_same(g, r, f"reserve {reserve} column {i}")
+
+
 @pytest.mark.parametrize("shape", [0, 1, 4])
 @pytest.mark.parametrize("tiles", [4094, 4095, 4096])
 def test_run_cut_units(shape, tiles):
