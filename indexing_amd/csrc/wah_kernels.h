@@ -293,7 +293,8 @@ struct ScanState {
   uint32_t fault;
   uint64_t result;
   uint64_t range[4];           // a range query's keys and words (k_q_range)
-  uint32_t pad[52];
+  uint32_t slice_span;         // chunks per slice of its bitmap (0: not by slices)
+  uint32_t pad[51];
 };
 static_assert(sizeof(ScanState) % 256 == 0, "status words follow at a line boundary");
 // Tiles of the longest scan: two streams of 2^32 WAH words in decode tiles of
@@ -349,10 +350,13 @@ struct DecodeStream {
 void launch_decode(const ScanRun& s, const DecodeStream& a, const DecodeStream& b, uint64_t nrows,
                    hipStream_t st);
 // Zeroes the bitmap and decodes the keys in [lo, hi] into it; host[3] = keys,
-// host[4] = words of the range.
+// host[4] = words of the range.  table: scratch of table_cap entries for a
+// range that decodes by slices (range_table_entries at most are used).
+uint64_t range_table_entries(uint64_t keycnt, uint64_t nrows, uint32_t cus);
 void launch_range(const ScanRun& s, const uint32_t* keys, const uint32_t* offsets,
                   const uint32_t* lengths, uint64_t keycnt, const uint32_t* words, uint32_t lo,
-                  uint32_t hi, uint32_t* bitmap, uint64_t nrows, hipStream_t st);
+                  uint32_t hi, uint32_t* bitmap, uint64_t nrows, uint64_t* table,
+                  uint64_t table_cap, hipStream_t st);
 // The result is the words of the stream (b null: of bitmap a alone).
 void launch_encode(const ScanRun& s, const uint32_t* a, const uint32_t* b, int op, uint64_t nrows,
                    uint32_t* out, uint64_t cap, hipStream_t st);

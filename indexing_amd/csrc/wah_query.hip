@@ -125,6 +125,206 @@ __device__ __forceinline__ uint64_t wave_lower_bound(const uint32_t* __restrict_
 
 }  // namespace
 
+namespace {
+
+// Slices of a range's bitmap, one block each: as many as CUs or a multiple of
+// that (264 of 8192 chunks took 44 us for 2^26 rows, 256 of 8480 35: 8 CUs had
+// two), of up to kSliceMax chunks.  A range of an index of 2^22 rows or more
+// (below that the ORs it replaces take about what its launch does) decodes by
+// slices if its words are kSliceWords or more per entry of the table: a wave
+// works through a slice's part of a key in steps of 128 words, full or not.
+// Slices / ORs: 18 words per entry (2800 keys of 2^26 rows) 179 / 283 us, 15
+// (1800 of 2^24) 125 / 156, 13 (12000 of 2^26) 614 / 782, 10 (1000 of 2^26)
+// 83 / 81, 8 (410 of 2^22) 52 / 45; 130 (410 of 2^26) 84 / 281.
+constexpr uint32_t kSliceMax = 10240;
+constexpr int kSliceThreads = 1024;
+constexpr uint64_t kSliceMinRows = 1ull << 22;
+constexpr uint64_t kSliceWords = 12;
+// Chunks per slice: a multiple of 32, so that a slice is whole bitmap words.
+uint32_t slice_span_of(uint64_t nrows, uint32_t cus) {
+  if (nrows < kSliceMinRows) return 0;
+  const uint64_t chunks = (nrows + 30) / 31, each = (uint64_t)cus * kSliceMax;
+  const uint64_t slices = (chunks + each - 1) / each * cus;
+  return (uint32_t)((chunks + slices * 32 - 1) / (slices * 32)) * 32;
+}
+uint64_t slices_of(uint64_t nrows, uint32_t span) { return ((nrows + 30) / 31 + span - 1) / span; }
+static_assert(kSliceMax % 32 == 0, "a slice's span is rounded up to it at most");
+
+}  // namespace
+
+namespace {
+
+constexpr int kEnterRows = 4;  // tiles of 8192 words
+constexpr uint32_t kEnterTile = kScanTileOf<kEnterRows>;
+
+// A range that decodes by slices: one pass over its words, as k_q_decode<true>
+// makes it (per key a scan of chunk counts, with look-back), that writes where
+// each key's words enter each slice: table[slice * keys + key] = first chunk <<
+// 32 | word + 1 of the word whose chunks hold the slice's first.  A lane needs
+// the first chunk of its four words only, and looks for a slice's start among
+// all of their chunks at once; a tile in which no key starts, which is most of
+// them, skips everything about keys.
+// (54 MB of words take 31 us.)
+__device__ __forceinline__ void enter_slices(const uint32_t* __restrict__ words,
+                                             const uint32_t* __restrict__ offsets, uint32_t span,
+                                             uint32_t slices, uint64_t* __restrict__ table,
+                                             ScanState* st, uint64_t* status, uint64_t* host) {
+  __shared__ uint32_t s_sum[kScanWaves], s_head[kScanWaves];
+  __shared__ uint32_t s_mark[kEnterTile / 32];
+  __shared__ uint64_t s_key0, s_key1;
+  __shared__ uint32_t s_prefix, s_tile;
+  const uint32_t recip = 0xFFFFFFFFu / span + 1u;  // 2^32 / span, rounded up
+  const int l = threadIdx.x % kWave;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const uint64_t key_a = st->range[0], key_b = st->range[1], w0 = st->range[2];
+  const uint64_t len = st->range[3] - w0;
+  const uint32_t keys = (uint32_t)(key_b - key_a);
+  words += w0;
+  const uint32_t tiles = (uint32_t)((len + kEnterTile - 1) / kEnterTile);
+  for (uint32_t tile = scan_next_tile(st, &s_tile, true); tile < tiles;
+       tile = scan_next_tile(st, &s_tile, false)) {
+    const uint64_t base = (uint64_t)tile * kEnterTile;
+    W4 x[kEnterRows];
+    if (base + kEnterTile <= len) {
+#pragma unroll
+      for (int r = 0; r < kEnterRows; ++r)
+        x[r] = load4<true>(words, base + row_at<kEnterRows>(w, l, r), len);
+    } else {
+#pragma unroll
+      for (int r = 0; r < kEnterRows; ++r)
+        x[r] = load4<false>(words, base + row_at<kEnterRows>(w, l, r), len);
+    }
+    if (w < 2) {  // the keys that start in the tile: [s_key0, s_key1)
+      const uint64_t k = wave_lower_bound(offsets + key_a, key_b - key_a,
+                                          w0 + base + (w ? kEnterTile : 0u)) + key_a;
+      if (l == 0) *(w ? &s_key1 : &s_key0) = k;
+    }
+    __syncthreads();
+    const uint64_t key0 = s_key0, key1 = s_key1;
+    const bool heads = key0 < key1;  // block-uniform
+    uint32_t hb = 0;                 // key starts, bit 4r + k
+    if (heads) {
+      for (uint32_t i = threadIdx.x; i < kEnterTile / 32; i += kScanThreads) s_mark[i] = 0;
+      __syncthreads();
+      for (uint64_t k = key0 + threadIdx.x; k < key1; k += kScanThreads) {
+        const uint64_t at = (uint64_t)offsets[k] - w0 - base;
+        if (at >= kEnterTile) break;
+        atomicOr(&s_mark[at / 32], 1u << (at % 32));
+      }
+      __syncthreads();
+#pragma unroll
+      for (int r = 0; r < kEnterRows; ++r) {
+        const uint32_t e = row_at<kEnterRows>(w, l, r);
+        hb |= ((s_mark[e / 32] >> (e % 32)) & 15u) << (4 * r);
+      }
+    }
+    uint32_t q[kEnterRows];  // first chunk of the lane's four words, from its key's start or
+    uint32_t openm = 0;      // (bit r) from the wave's
+    uint32_t run = 0;        // chunks of the wave's earlier rows
+    uint32_t start = 0;      // chunks before the open key's first word
+    bool open = true;
+#pragma unroll
+    for (int r = 0; r < kEnterRows; ++r) {
+      const uint32_t p1 = word_chunks(x[r].x), p2 = p1 + word_chunks(x[r].y),
+                     p3 = p2 + word_chunks(x[r].z), s = p3 + word_chunks(x[r].w);
+      const uint32_t inc = wave_incl_add(s);
+      const uint32_t ex = run + inc - s;
+      run += readlane(inc, kWave - 1);
+      q[r] = ex - start;
+      openm |= open ? 1u << r : 0u;
+      if (heads) {
+        const uint32_t h4 = (hb >> (4 * r)) & 15u;
+        const uint32_t b = ex + (h4 & 8u ? p3 : h4 & 4u ? p2 : h4 & 2u ? p1 : 0u);
+        const uint64_t hm = ballot(h4 != 0u);
+        const uint64_t below = hm & ((1ull << l) - 1ull);
+        const uint32_t got = __shfl(b, below ? 63 - __builtin_clzll(below) : 0, kWave);
+        if (below) {
+          q[r] = ex - got;
+          openm &= ~(1u << r);
+        }
+        if (hm) {  // wave-uniform
+          start = readlane(b, 63 - __builtin_clzll(hm));
+          open = false;
+        }
+      }
+    }
+    if (l == 0) {
+      s_sum[w] = open ? run : run - start;
+      s_head[w] = open ? 0u : 1u;
+    }
+    __syncthreads();
+    uint32_t carry = 0, agg = 0;
+    bool closed = false, tile_closed = false;
+#pragma unroll
+    for (int i = 0; i < kScanWaves; ++i) {
+      if (i == w) {
+        carry = agg;
+        closed = tile_closed;
+      }
+      const bool h = s_head[i] != 0u;
+      agg = h ? s_sum[i] : agg + s_sum[i];
+      tile_closed |= h;
+    }
+    if (w == 0) {
+      uint32_t hi, p;
+      lookback2<kOpNone, kOpSum>(status, tile, 0u, agg, tile_closed, &st->fault, hi, p);
+      if (l == 0) s_prefix = p;
+    }
+    __syncthreads();
+    if (!closed) carry += s_prefix;
+#pragma unroll
+    for (int r = 0; r < kEnterRows; ++r) {
+      const uint64_t at = base + row_at<kEnterRows>(w, l, r);
+      // Slices that start in [c, c + n): p1 .. p3 part the chunks between the
+      // four words at `word` on.
+      auto enter = [&](uint32_t c, uint32_t n, uint32_t p1, uint32_t p2, uint32_t p3,
+                       uint64_t word) {
+        uint32_t sl = __umulhi(c, recip), d = c - sl * span;  // sl may be one too many
+        if ((int32_t)d < 0) {
+          d += span;
+          --sl;
+        }
+        if (d) {  // the next slice starts after c
+          d = span - d;
+          ++sl;
+        }
+        for (; d < n && sl < slices; d += span, ++sl) {
+          const uint32_t k = (d >= p1) + (d >= p2) + (d >= p3);
+          const uint32_t pk = k == 3 ? p3 : k == 2 ? p2 : k == 1 ? p1 : 0u;
+          // the word's key: the last that starts at or before it
+          uint64_t lo = key0, hi = key1;
+          while (lo < hi) {
+            const uint64_t mid = (lo + hi) / 2;
+            if ((uint64_t)offsets[mid] <= w0 + word + k) lo = mid + 1;
+            else hi = mid;
+          }
+          const uint64_t key = lo - 1 - key_a;
+          if (key < keys)
+            table[(uint64_t)sl * keys + key] = (uint64_t)(c + pk) << 32 | (word + k + 1);
+        }
+      };
+      const uint32_t n0 = word_chunks(x[r].x), n1 = word_chunks(x[r].y),
+                     n2 = word_chunks(x[r].z), n3 = word_chunks(x[r].w);
+      uint32_t c = q[r] + ((openm >> r) & 1u ? carry : 0u);
+      const uint32_t h4 = (hb >> (4 * r)) & 15u;
+      if (!ballot(h4 != 0u)) {  // wave-uniform: no key starts in the row
+        enter(c, n0 + n1 + n2 + n3, n0, n0 + n1, n0 + n1 + n2, at);
+      } else {
+#pragma unroll 1
+        for (int k = 0; k < 4; ++k) {
+          if ((h4 >> k) & 1u) c = 0;
+          const uint32_t n = k == 0 ? n0 : k == 1 ? n1 : k == 2 ? n2 : n3;
+          enter(c, n, ~0u, ~0u, ~0u, at + k);
+          c += n;
+        }
+      }
+    }
+  }
+  scan_finish(st, status, tiles, host);
+}
+
+}  // namespace
+
 // One pass over WAH words: per word its first chunk (a scan of chunk counts,
 // with look-back across tiles), then its literal bits or 1-fill rows ORed into
 // the row bitmap (zero before).
@@ -138,11 +338,13 @@ __device__ __forceinline__ uint64_t wave_lower_bound(const uint32_t* __restrict_
 //     nothing else is (a flag array took a fill, a marking launch and 4 bytes
 //     per word).
 // What bounds it: sparse streams the atomic ORs (one per literal, each to a
-// line of its own), dense ones the words.
+// line of its own), dense ones the words.  A range of many words per key goes
+// by slices instead (enter_slices, then k_q_slices).
 template <bool SEG>
 __global__ __launch_bounds__(kScanThreads, query_waves_per_eu(kDecBlocks)) void k_q_decode(
     DecodeStream qa, DecodeStream qb, const uint32_t* __restrict__ offsets, uint64_t nrows,
-    ScanState* st, uint64_t* status, uint64_t* host) {
+    uint64_t* __restrict__ table, uint32_t slices, ScanState* st, uint64_t* status,
+    uint64_t* host) {
   __shared__ uint32_t s_sum[kScanWaves], s_head[kScanWaves];
   __shared__ uint32_t s_mark[SEG ? kDecTile / 32 : 1];
   __shared__ uint64_t s_key0;
@@ -152,6 +354,10 @@ __global__ __launch_bounds__(kScanThreads, query_waves_per_eu(kDecBlocks)) void 
   const uint32_t chunks = (uint32_t)((nrows + 30) / 31);
   uint64_t key_a = 0, key_b = 0, w0 = 0;
   if (SEG) {
+    if (const uint32_t span = st->slice_span) {  // the range decodes by slices
+      enter_slices(qa.words, offsets, span, slices, table, st, status, host);
+      return;
+    }
     key_a = st->range[0];
     key_b = st->range[1];
     w0 = st->range[2];
@@ -333,38 +539,179 @@ __global__ __launch_bounds__(kScanThreads, query_waves_per_eu(kDecBlocks)) void 
   scan_finish(st, status, tiles, host);
 }
 
-// Starts a range query: zeroes the row bitmap and locates the keys of the
-// index in [lo, hi] (keys ascend): range[0] = first key index >= lo, range[1]
-// = first > hi, range[2] = first word of key range[0], range[3] = one past the
-// last word of key range[1] - 1.  The number of keys goes to host[3].
-__global__ __launch_bounds__(kBlock) void k_q_range(const uint32_t* __restrict__ keys,
-                                                    const uint32_t* __restrict__ offsets,
-                                                    const uint32_t* __restrict__ lengths,
-                                                    uint64_t keycnt, uint32_t lo, uint32_t hi,
-                                                    uint32_t* __restrict__ bitmap, uint64_t words,
-                                                    ScanState* st, uint64_t* host) {
+// Starts a range query: locates the keys of the index in [lo, hi] (keys
+// ascend): range[0] = first key index >= lo, range[1] = first > hi, range[2] =
+// first word of key range[0], range[3] = one past the last word of key
+// range[1] - 1; the number of keys goes to host[3], of words to host[4].  Then
+// zeroes the row bitmap, or, for a range that decodes by slices, their table.
+// SLICES: whether it does is decided here, so every block locates the keys.
+template <bool SLICES>
+__global__ __launch_bounds__(kBlock) void k_q_range(
+    const uint32_t* __restrict__ keys, const uint32_t* __restrict__ offsets,
+    const uint32_t* __restrict__ lengths, uint64_t keycnt, uint32_t lo, uint32_t hi,
+    uint32_t* __restrict__ bitmap, uint64_t words, uint64_t* __restrict__ table,
+    uint64_t table_cap, uint32_t slices, uint32_t slice_span, ScanState* st, uint64_t* host) {
   __shared__ uint64_t s_at[2];
   const uint32_t t = threadIdx.x;
-  if (blockIdx.x == 0) {
+  uint64_t entries = 0;
+  if (SLICES || blockIdx.x == 0) {
     if (t < 2 * kWave) {
       const uint64_t v = t < kWave ? (uint64_t)lo : (uint64_t)hi + 1;
       const uint64_t at = wave_lower_bound(keys, keycnt, v);
       if (t % kWave == 0) s_at[t / kWave] = at;
     }
     __syncthreads();
-    if (t == 0) {
-      const uint64_t a = s_at[0], b = s_at[1];
+    const uint64_t a = s_at[0], b = s_at[1];
+    const uint64_t w0 = a < b ? offsets[a] : 0;
+    const uint64_t w1 = a < b ? (uint64_t)offsets[b - 1] + lengths[b - 1] : 0;
+    if (SLICES) {
+      entries = (b - a) * slices;  // below 2^60: table_cap bounds it
+      if (w1 < w0 || w1 - w0 >= 1ull << 31 || w1 - w0 < kSliceWords * entries ||
+          entries > table_cap)
+        entries = 0;
+    }
+    if (blockIdx.x == 0 && t == 0) {
       st->range[0] = a;
       st->range[1] = b;
-      st->range[2] = a < b ? offsets[a] : 0;
-      st->range[3] = a < b ? (uint64_t)offsets[b - 1] + lengths[b - 1] : 0;
+      st->range[2] = w0;
+      st->range[3] = w1;
+      st->slice_span = entries ? slice_span : 0u;
       __hip_atomic_store(&host[3], b - a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-      __hip_atomic_store(&host[4], st->range[3] - st->range[2], __ATOMIC_RELAXED,
-                         __HIP_MEMORY_SCOPE_SYSTEM);
+      __hip_atomic_store(&host[4], w1 - w0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
   }
-  for (uint64_t i = (uint64_t)blockIdx.x * kBlock + t; i < words; i += (uint64_t)gridDim.x * kBlock)
-    bitmap[i] = 0;
+  const uint64_t i0 = (uint64_t)blockIdx.x * kBlock + t, step = (uint64_t)gridDim.x * kBlock;
+  if (SLICES && entries) {
+    for (uint64_t i = i0; i < entries; i += step) table[i] = 0;
+    return;
+  }
+  for (uint64_t i = i0; i < words; i += step) bitmap[i] = 0;
+}
+
+// Decodes a range by slices of the bitmap, one block each, from the table of
+// where each key's words enter the slice (first chunk << 32 | word + 1, 0:
+// nowhere): the block ORs the literals of its part of every key into LDS and
+// stores the slice once.  The ORs of 6.7 million literals (a tenth of 4096
+// keys, 2^26 rows) took 260 us as device-scope atomics, which run at 25 G/s
+// however they are spread; here the same words take 32 us, and 33 us before for
+// the table.  Bound by the instructions per step (about 100 for 128 words, of
+// which a key has 124 in a slice), not by the loads: with one, two or three
+// steps loaded ahead it takes the same.
+__global__ __launch_bounds__(kSliceThreads) void k_q_slices(
+    const uint32_t* __restrict__ words, const uint32_t* __restrict__ offsets,
+    const uint64_t* __restrict__ table, uint32_t* __restrict__ bitmap, uint64_t nrows,
+    const ScanState* __restrict__ st) {
+  constexpr uint32_t kWavesHere = kSliceThreads / kWave;
+  constexpr uint32_t kStep = 2 * kWave;  // words per step of a wave
+  constexpr int kAhead = 2;
+  __shared__ alignas(16) uint32_t s_bits[kSliceMax / 32 * 31];
+  const uint32_t span = st->slice_span;  // the slice's chunks
+  if (!span) return;  // block-uniform
+  const uint32_t l = threadIdx.x % kWave;
+  const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const uint32_t bw = span / 32 * 31;  // the slice's bitmap words
+  const uint32_t slice = blockIdx.x, slices = gridDim.x;
+  const uint32_t first = slice * span;
+  const uint64_t key_a = st->range[0], w0 = st->range[2], w1 = st->range[3];
+  const uint32_t keys = (uint32_t)(st->range[1] - key_a);
+  const uint64_t total = w1 - w0;
+  words += w0;
+  for (uint32_t i = threadIdx.x; i < bw; i += kSliceThreads) s_bits[i] = 0;
+  __syncthreads();
+  auto literal = [&](uint32_t c, uint32_t bits) {
+    const uint32_t rel = c - first;
+    if (rel >= span) return;
+    const uint32_t row = 31u * rel, wi = row >> 5, sh = row & 31u;
+    atomicOr(&s_bits[wi], bits << sh);
+    const uint32_t hi = (uint32_t)(((uint64_t)bits << sh) >> 32);
+    if (hi) atomicOr(&s_bits[wi + 1], hi);
+  };
+  auto ones = [&](uint32_t c, uint32_t n) {  // a 1-fill's part of the slice
+    const uint32_t a = c > first ? c - first : 0u;
+    const uint64_t e = (uint64_t)c + n < first ? 0u : (uint64_t)c + n - first;
+    for (uint32_t i = a; i < span && i < e; ++i) literal(first + i, 0x7FFFFFFFu);
+  };
+  for (uint32_t k0 = 0; k0 < keys; k0 += kSliceThreads) {
+    // lane l holds one key of the wave's 64: its words of the slice
+    const uint32_t k = k0 + w + kWavesHere * l;
+    uint32_t from = 0, to = 0, at = 0;
+    if (k < keys) {
+      const uint64_t e = table[(uint64_t)slice * keys + k];
+      const uint64_t f = slice + 1 < slices ? table[(uint64_t)(slice + 1) * keys + k] : 0;
+      uint64_t end = k + 1 < keys ? (uint64_t)offsets[key_a + k + 1] - w0 : total;
+      if (end > total) end = total;
+      if (f && (uint32_t)f < end) end = (uint32_t)f;  // with the word that enters the next slice
+      if (e && (uint32_t)e <= end) {
+        from = (uint32_t)e - 1u;
+        to = (uint32_t)end;
+        at = (uint32_t)(e >> 32);
+      }
+    }
+    uint64_t left = ballot(from < to);
+    // the steps of the wave's keys, one after another; a step's words are
+    // loaded while the steps before it are worked on (kAhead of them take
+    // turns: a copy from one to the next would wait for its loads)
+    uint32_t pos = 0, stop = 0;  // uniform
+    struct Step {
+      uint2 x;        // words 2l, 2l + 1 (past the key's end: fills of nothing)
+      uint32_t c;     // first chunk
+      bool on, same;  // there is one; it goes on where the last one ended
+    };
+    auto next = [&]() -> Step {
+      Step q;
+      q.c = 0;
+      q.same = stop - pos > kStep;
+      if (q.same) {
+        pos += kStep;
+      } else if (left) {
+        const int j = __builtin_ctzll(left);
+        left &= left - 1;
+        pos = readlane(from, j);
+        stop = readlane(to, j);
+        q.c = readlane(at, j);
+      } else {
+        pos = stop = 0;
+      }
+      q.on = stop != 0;
+      const uint32_t i = pos + 2 * l;
+      q.x = uint2{0u, 0u};
+      if (i < stop) q.x.x = words[i];
+      if (i + 1 < stop) q.x.y = words[i + 1];
+      return q;
+    };
+    Step q[kAhead];
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) q[i] = next();
+    uint32_t base = 0;
+    for (bool on = true; on;) {
+#pragma unroll
+      for (int i = 0; i < kAhead; ++i) {
+        const Step p = q[i];
+        on = p.on;
+        if (!on) break;
+        if (!p.same) base = p.c;
+        const uint32_t n0 = word_chunks(p.x.x), n1 = word_chunks(p.x.y);
+        const uint32_t inc = wave_incl_add(n0 + n1);
+        const uint32_t c0 = base + inc - n0 - n1;
+        if (p.x.x & 0x80000000u) literal(c0, p.x.x & 0x7FFFFFFFu);
+        if (p.x.y & 0x80000000u) literal(c0 + n0, p.x.y & 0x7FFFFFFFu);
+        if (ballot(p.x.x >> 30 == 1u || p.x.y >> 30 == 1u)) {  // 1-fills, which builds never write
+          if (p.x.x >> 30 == 1u) ones(c0, n0);
+          if (p.x.y >> 30 == 1u) ones(c0 + n0, n1);
+        }
+        base += readlane(inc, kWave - 1);
+        q[i] = next();
+      }
+    }
+  }
+  __syncthreads();
+  const uint64_t nwords = (nrows + 31) / 32, out = (uint64_t)slice * bw;
+  const uint32_t tail = (uint32_t)(nrows & 31u);
+  for (uint32_t i = threadIdx.x; i < bw && out + i < nwords; i += kSliceThreads) {
+    uint32_t v = s_bits[i];
+    if (tail && out + i == nwords - 1) v &= (1u << tail) - 1u;
+    bitmap[out + i] = v;
+  }
 }
 
 // ---- encoding a row bitmap (or op(a, b) of two) into WAH words -------------
@@ -551,21 +898,44 @@ void launch_decode(const ScanRun& s, const DecodeStream& a, const DecodeStream& 
   if (!tiles) return;
   const uint32_t most = s.cus * kDecBlocks;
   hipLaunchKernelGGL(k_q_decode<false>, dim3(tiles < most ? (uint32_t)tiles : most),
-                     dim3(kScanThreads), 0, st, a, b, nullptr, nrows, s.state, s.status, s.host);
+                     dim3(kScanThreads), 0, st, a, b, nullptr, nrows, nullptr, 0u,
+                     s.state, s.status, s.host);
+}
+
+uint64_t range_table_entries(uint64_t keycnt, uint64_t nrows, uint32_t cus) {
+  const uint32_t span = slice_span_of(nrows, cus);
+  if (!span) return 0;
+  const uint64_t all = keycnt * slices_of(nrows, span);
+  const uint64_t most = 2 * nrows / kSliceWords;  // (a row takes two words at most)
+  return all < most ? all : most;
 }
 
 void launch_range(const ScanRun& s, const uint32_t* keys, const uint32_t* offsets,
                   const uint32_t* lengths, uint64_t keycnt, const uint32_t* words, uint32_t lo,
-                  uint32_t hi, uint32_t* bitmap, uint64_t nrows, hipStream_t st) {
+                  uint32_t hi, uint32_t* bitmap, uint64_t nrows, uint64_t* table,
+                  uint64_t table_cap, hipStream_t st) {
   const uint64_t bw = (nrows + 31) / 32;
   uint64_t g = (bw + 4 * kBlock - 1) / (4 * kBlock);
-  g = g < 1 ? 1 : g > 4096 ? 4096 : g;
-  hipLaunchKernelGGL(k_q_range, dim3((uint32_t)g), dim3(kBlock), 0, st, keys, offsets, lengths,
-                     keycnt, lo, hi, bitmap, bw, s.state, s.host);
+  const uint32_t span = table_cap ? slice_span_of(nrows, s.cus) : 0u;
+  const uint32_t slices = span ? (uint32_t)slices_of(nrows, span) : 0u;
+  if (span) {
+    g = g < 1 ? 1 : g > 1024 ? 1024 : g;
+    hipLaunchKernelGGL(k_q_range<true>, dim3((uint32_t)g), dim3(kBlock), 0, st, keys, offsets,
+                       lengths, keycnt, lo, hi, bitmap, bw, table, table_cap, slices, span,
+                       s.state, s.host);
+  } else {
+    g = g < 1 ? 1 : g > 4096 ? 4096 : g;
+    hipLaunchKernelGGL(k_q_range<false>, dim3((uint32_t)g), dim3(kBlock), 0, st, keys, offsets,
+                       lengths, keycnt, lo, hi, bitmap, bw, table, table_cap, slices, span,
+                       s.state, s.host);
+  }
   // the words of the range are known on the device only: a full grid
   hipLaunchKernelGGL(k_q_decode<true>, dim3(s.cus * kDecBlocks), dim3(kScanThreads), 0, st,
                      DecodeStream{words, 0, bitmap}, DecodeStream{nullptr, 0, nullptr}, offsets,
-                     nrows, s.state, s.status, s.host);
+                     nrows, table, slices, s.state, s.status, s.host);
+  if (span)
+    hipLaunchKernelGGL(k_q_slices, dim3(slices), dim3(kSliceThreads), 0, st, words, offsets, table,
+                       bitmap, nrows, s.state);
 }
 
 void launch_encode(const ScanRun& s, const uint32_t* a, const uint32_t* b, int op, uint64_t nrows,

@@ -1695,9 +1695,14 @@ int wahgpu_query_range_device(wahgpu_ctx* c, const uint32_t* d_keys, const uint3
   }
   int rc = arena_limit(c, align_up(4 * 8));
   if (rc) return rc;
+  // a table for a decode by slices, where the arena has or gets the room; the
+  // query does without it otherwise
+  uint64_t entries = wah::range_table_entries(keycnt, nrows, c->cus);
+  if (c->fixed) entries = std::min<uint64_t>(entries, c->arena_cap / 8);
+  else if (arena_reserve(c, entries * 8)) entries = 0;
   ORDERED(c);
   wah::launch_range(scan_run(c), d_keys, d_offsets, d_lengths, keycnt, d_words, lo, hi, d_bitmap,
-                    nrows, c->stream);
+                    nrows, reinterpret_cast<uint64_t*>(c->arena), entries, c->stream);
   LAUNCHCHK(c);
   uint64_t unused;
   order_guard_.end();  // no host wait holds the device order

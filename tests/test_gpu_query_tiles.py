@@ -129,3 +129,69 @@ def test_range_over_many_keys_per_tile(ctx, card):
         sel = (v >= lo) & (v <= hi)
         assert np.array_equal(bitmap_rows(u32(bm), n), np.flatnonzero(sel))
         assert m == np.unique(v[sel]).size
+
+
+SLICED = 1 << 22  # rows from which a range may decode by slices of the bitmap
+
+
+@pytest.mark.parametrize("arena", [0, 1 << 12, 1 << 30], ids=["grows", "no-room", "room"])
+@pytest.mark.parametrize("n", [SLICED - 1, SLICED, SLICED + 31 * 1024 - 17, 2 * SLICED + 5,
+                               31 * 8192 * 256 - 1, 31 * 8192 * 256 + 1])
+def test_range_by_slices(n, arena):
+    """Ranges of few and many words per key and slice, on either side of where
+    the slices' size and the way of decoding change."""
+    import torch
+
+    import indexing_amd as ia
+    with ia.Context(0) as c:
+        g = torch.Generator(device="cuda:0").manual_seed(n)
+        for card in (3, 100, 3000):
+            v = torch.randint(0, card, (n,), device="cuda:0", generator=g, dtype=torch.int32)
+            v[n // 3:n // 2] = 0  # slices that most keys skip
+            v[-1] = card - 1
+            with ia.Context(0, arena_bytes=arena) as q:
+                k, o, ln, w, counts = c.build_device(v)
+                m, L = c.read_counts(counts).keycnt, c.read_counts(counts).length
+                for lo, hi in ((0, card), (card // 3, card // 2), (card - 1, card - 1), (1, 1)):
+                    print(f"[range] n={n} card={card} [{lo}, {hi}]", flush=True)
+                    try:
+                        bm, keys = q.query_range_device(k[:m], o[:m], ln[:m], w[:L], lo, hi, n)
+                    except WahError:
+                        assert arena == 1 << 12  # the words' own limit
+                        continue
+                    sel = (v >= lo) & (v <= hi)
+                    pad = torch.zeros((n + 31) // 32 * 32, dtype=torch.int64, device="cuda:0")
+                    pad[:n] = sel
+                    want = (pad.view(-1, 32) << torch.arange(32, device="cuda:0")).sum(1)
+                    assert bool((bm.to(torch.int64) & 0xFFFFFFFF == want).all())
+                    assert keys == int(torch.unique(v[sel]).numel())
+
+
+@pytest.mark.parametrize("seed", [1, 2])
+def test_range_by_slices_of_words_that_builds_never_write(ctx, seed):
+    """1-fills and fills over several slices, fills of no chunks, empty
+    literals and a key without words."""
+    rng = np.random.default_rng(seed)
+    n = SLICED + 1000
+    chunks = (n + 30) // 31
+    streams = []
+    for k in range(40):
+        w = stream(12000 + 517 * k, 100 * seed + k, True)
+        if k % 5 == 1:  # a fill over several slices, of ones or not
+            w[rng.integers(w.size)] = np.uint32(5000 | (0x40000000 if k % 2 else 0))
+        if k == 7:
+            w = w[:0]
+        streams.append(w)
+    words = np.concatenate(streams)
+    lengths = np.array([s.size for s in streams], np.uint32)
+    offsets = (np.cumsum(lengths) - lengths).astype(np.uint32)
+    keys = np.arange(40, dtype=np.uint32) * 3
+    rows = [decode_rows(s)[0] for s in streams]
+    assert max(int(r[-1]) for r in rows if r.size) > n and chunks > 130 * 1024
+    d = [dev(x) for x in (keys, offsets, lengths, words)]
+    for lo, hi in ((0, 200), (20, 22), (21, 21), (30, 90)):
+        bm, m = ctx.query_range_device(*d, lo, hi, n)
+        take = [i for i in range(40) if lo <= 3 * i <= hi]
+        want = np.unique(np.concatenate([rows[i] for i in take])) if take else np.zeros(0, np.int64)
+        assert np.array_equal(bitmap_rows(u32(bm), n), want[want < n])
+        assert m == len(take)
