@@ -13,6 +13,7 @@ the HIP kernels; without the built library the import of a GPU entry point
 raises (there is no CPU fallback).
 """
 import ctypes
+import threading
 from dataclasses import dataclass, field
 
 import numpy as np
@@ -66,6 +67,11 @@ def device_count():
     return c.value
 
 
+# Longest column whose results Context.build receives in page-locked memory that
+# the context keeps (5 words a value, up to the next power of two: 80 MiB).
+_STAGE_MAX = 1 << 22
+
+
 class Context:
     """One HIP stream plus a pooled device arena (wahgpu_create)."""
 
@@ -78,11 +84,14 @@ class Context:
         self._h = h
         self.device = device
         self.use_torch_stream = use_torch_stream
+        self._stage = None
+        self._stage_lock = threading.Lock()
 
     def close(self):
         if getattr(self, "_h", None):
             self._lib.wahgpu_destroy(self._h)
             self._h = None
+        self._stage = None
 
     def __del__(self):
         try:
@@ -146,10 +155,35 @@ class Context:
         v = _as_u32(values)
         n = v.size
         cap = max(n, 1)
-        keys = np.empty(cap, np.uint32)
-        offs = np.empty(cap, np.uint32)
-        lens = np.empty(cap, np.uint32)
-        words = np.empty(2 * cap, np.uint32)
+        staged_out = n <= _STAGE_MAX and self._stage_lock.acquire(blocking=False)
+        try:
+            buf = self._staging(cap) if staged_out else None
+            if buf is None:
+                buf = (np.empty(cap, np.uint32), np.empty(cap, np.uint32),
+                       np.empty(cap, np.uint32), np.empty(2 * cap, np.uint32))
+            return self._build_into(v, cap, buf, rid_base, staged, timed)
+        finally:
+            if staged_out:
+                self._stage_lock.release()
+
+    def _staging(self, cap):
+        """Page-locked keys, offsets, lengths and words of a column of cap values:
+        arrays on a block that the context keeps, or None if there is none to be
+        had.  Results copied to fresh pageable memory cost a fault per page and the
+        runtime's own staging (300007 values: 304 us of the build's 359; 216 into
+        page-locked memory)."""
+        if self._stage is None or self._stage.size < 5 * cap:
+            self._stage = None  # the old block first
+            try:
+                self._stage = pinned_empty(5 << max(14, (cap - 1).bit_length()))
+            except WahError:
+                return None
+        s = self._stage
+        return s[:cap], s[cap:2 * cap], s[2 * cap:3 * cap], s[3 * cap:5 * cap]
+
+    def _build_into(self, v, cap, buf, rid_base, staged, timed):
+        n = v.size
+        keys, offs, lens, words = buf
         c = N.Counts()
         t = N.PhaseTimes()
         vp = v.ctypes.data_as(ctypes.c_void_p)
@@ -567,13 +601,14 @@ class _PinnedBlock:
 
     def __init__(self, nbytes):
         self.ptr = ctypes.c_void_p()
-        rc = N.lib().wahgpu_host_alloc(int(nbytes), ctypes.byref(self.ptr))
+        self._lib = N.lib()  # at interpreter exit the module's names may be gone
+        rc = self._lib.wahgpu_host_alloc(int(nbytes), ctypes.byref(self.ptr))
         if rc != N.OK:
             raise WahError(rc, f"pinned allocation of {nbytes} bytes failed")
 
     def __del__(self):
         if self.ptr:
-            N.lib().wahgpu_host_free(self.ptr)
+            self._lib.wahgpu_host_free(self.ptr)
             self.ptr = None
 
 

@@ -152,3 +152,26 @@ def test_short_and_long_columns_in_one_batch(reserved):
                 assert_same(g, r, f"layout {rep} column {i}")
         if reserved:
             assert c.graph_stats()[0] == 1
+
+
+def test_host_results_are_the_callers_own(monkeypatch):
+    """Context.build hands out copies of what it keeps: an index stays as it was
+    while the context builds others, longer than the kept memory's bound and
+    shorter, from several threads, and after the context is closed."""
+    from concurrent.futures import ThreadPoolExecutor
+    monkeypatch.setattr(ia, "_STAGE_MAX", 30000)
+    lens = [1, 20000, 16384, 0, 16385, 30000, 30001, 70001, 5]
+    cols = [column("skew", n) for n in lens]
+    with ia.Context(0) as c:
+        got = [c.build(v) for v in cols]
+        assert c._stage_lock.acquire(blocking=False)  # as if another call held the memory
+        got.append(c.build(cols[1]))
+        c._stage_lock.release()
+    with ThreadPoolExecutor(3) as pool:
+        def run(v):
+            with ia.Context(0) as own:
+                own.build(cols[-1])
+                return own.build(v)
+        got += pool.map(run, cols)
+    for g, v in zip(got, cols + [cols[1]] + cols):
+        assert_same(g, oracle.build(v), f"{v.size}")
