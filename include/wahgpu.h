@@ -62,7 +62,8 @@ typedef struct wahgpu_counts {
                        2/3 of the rows), 2 = pairs sorted with wide digits
                        (see wahgpu_tuning); staged paths report 0.  A
                        column of at most 2^14 values reports 0 or 1 by the
-                       same rule, and one workgroup sorts its rows       */
+                       same rule; one workgroup sorts its rows, except in
+                       a batch of few such beside much longer ones       */
 } wahgpu_counts;
 
 /* Microseconds per phase, the buckets `phases` prints (src/phases.cpp:714-1127). */

@@ -813,6 +813,15 @@ struct SubBatch {
 
 constexpr int kSmallShape = wah::kRadixShapes;
 constexpr int kSubShapes = wah::kRadixShapes + 1;  // launch sets a batch may need
+// Short columns join the launch set of a batch's longer ones where they are one
+// for two CUs at most and the long ones have this many rows for each: there a
+// few tiles more per pass cost less than the launch of one workgroup per column,
+// which takes as long as its longest column (34 us at 2^14 rows).  Joined / apart,
+// us: 64 columns of 2^12 to 2^17 rows 164 / 193, 20 of 2^8 to 2^20 136 / 154, 100
+// of 2^4 to 2^18 174 / 186, 128 of 2^12 to 2^20 467 / 474; more short columns
+// (half of 512 of 2^10 to 2^18) 500 / 474, little beside them (100 of 2^9 to
+// 2^14.2) 143 / 129.
+constexpr uint64_t kJoinRows = 1u << 15;
 
 // Validates the columns and splits them into sub-batches: the short ones, which
 // take a workgroup each, and the others by tile shape (all that the context
@@ -826,16 +835,18 @@ int plan_batch(wahgpu_ctx* c, const wahgpu_column* cols, uint32_t ncols, uint64_
   // a captured graph has to fit any batch of the reservation, so its shape
   // goes by the reservation
   const bool table = c->tuned || c->force_shape >= 0;
-  uint64_t values = c->res_values, columns = c->res_cols;
-  if (!all_shapes) {
-    values = columns = 0;
-    for (uint32_t i = 0; i < ncols; ++i)
-      if (!small_ok(c, cols[i].n)) {
-        values += cols[i].n;
-        ++columns;
-      }
+  uint64_t longs = 0, nlong = 0, nshort = 0;  // values and columns
+  for (uint32_t i = 0; i < ncols; ++i) {
+    if (small_ok(c, cols[i].n)) {
+      nshort += cols[i].n > 0;
+    } else {
+      longs += cols[i].n;
+      ++nlong;
+    }
   }
-  const int rule = batch_shape(c, values, columns);
+  const int rule = all_shapes ? batch_shape(c, c->res_values, c->res_cols)
+                              : batch_shape(c, longs, nlong);
+  const bool join = nshort <= c->cus / 2 && nshort * kJoinRows <= longs;
   for (uint32_t i = 0; i < ncols; ++i) {
     const wahgpu_column& col = cols[i];
     int rc = check_n(c, col.n, col.rid_base);
@@ -845,6 +856,16 @@ int plan_batch(wahgpu_ctx* c, const wahgpu_column* cols, uint32_t ncols, uint64_
                                         " overlaps the previous one or exceeds values_len");
     end = col.offset + col.n;
     members[small_ok(c, col.n) ? kSmallShape : table ? shape_for(c, col.n) : rule].push_back(i);
+  }
+  if (join) {
+    std::vector<uint32_t> rest;
+    for (uint32_t i : members[kSmallShape]) {
+      auto& m = members[table ? shape_for(c, cols[i].n) : rule];
+      if (m.empty() || !cols[i].n) rest.push_back(i);
+      else m.push_back(i);
+    }
+    members[kSmallShape].swap(rest);
+    for (int sh = 0; sh < kSmallShape; ++sh) std::sort(members[sh].begin(), members[sh].end());
   }
   subs->clear();
   *shared = Caps{values_len, 0, 0, 0, 0};

@@ -175,3 +175,44 @@ def test_host_results_are_the_callers_own(monkeypatch):
         got += pool.map(run, cols)
     for g, v in zip(got, cols + [cols[1]] + cols):
         assert_same(g, oracle.build(v), f"{v.size}")
+
+
+@pytest.mark.parametrize("shape", [None, 3], ids=["untuned", "table"])
+@pytest.mark.parametrize("reserved", [False, True], ids=["eager", "graph"])
+def test_short_columns_join_the_long_ones(reserved, shape):
+    """Few short columns beside long ones take part in their launch set, more
+    of them or with less beside them do not; one graph replays all of these."""
+    import torch
+
+    from indexing_amd import _native as N
+    from tests.test_gpu_batch import per_column
+    layouts = [[5, 2**16, 0, 1], [5, 2**16 - 1, 1, 0], [16384, 7, 2**18, 0, 16383, 1, 1025],
+               [3, 300000] + [4] * 8 + [9] * 200, [40] * 128 + [2**22], [40] * 129 + [2**22]]
+    with ia.Context(0) as c:
+        if shape is not None:
+            c.set_tuning([shape] * N.TUNE_BUCKETS)
+        total = 2**22 + 130 * 64
+        if reserved:
+            c.batch_reserve(total, 256)
+        buf = torch.zeros(total, dtype=torch.int32, device="cuda:0")
+        out = None
+        for rep, lay in enumerate(layouts):
+            cols, at = [], 0
+            for i, n in enumerate(lay):
+                v = column(("u16", "skew", "runs")[i % 3], n) if n else np.zeros(0, np.uint32)
+                buf[at:at + n] = torch.from_numpy(v.view(np.int32))
+                cols.append((at, n, i, v))
+                at += (n + 63) // 64 * 64
+            spec = [(o, n, r) for o, n, r, _ in cols]
+            if out is None:
+                out = tuple(torch.zeros(m, dtype=torch.int32, device="cuda:0")
+                            for m in (total, total, total, 2 * total, 256 * 10))
+            c.build_batch_device(buf, spec, out)
+            torch.cuda.synchronize()
+            counts = c.read_counts_batch(out[4], len(lay))
+            got = per_column(out, counts, [(o, n) for o, n, _ in spec])
+            for i, (g, col) in enumerate(zip(got, cols)):
+                assert counts[i].fault == 0
+                assert_same(g, oracle.build(col[3], rid_base=i), f"layout {rep} column {i}")
+        if reserved:
+            assert c.graph_stats()[0] == 1
