@@ -1348,7 +1348,14 @@ static void launch_radix(const BuildArgs& a, hipStream_t s, LaunchHook* hook) {
 void launch_sort(const BuildArgs& a, hipStream_t s, LaunchHook* hook) {
   hipLaunchKernelGGL(k_begin, dim3(64), dim3(kBlock), 0, s, a.hdr, a.cs, a.cols_cap,
                      a.tile_runs, a.sort_tiles_cap, a.desc, (int)a.inline_desc, a.one_dims, a.one);
-  uint64_t hb = (a.n_cap + 4 * kHistChunk - 1) / (4 * kHistChunk);
+  // Two chunks per block: 2^20 values 64.2 us, with four 67.0 and with one 65.3;
+  // 2^18 zipf values 63.9, with four 71.4; 128 columns of 2^12 to 2^20 values
+  // 449, 465 and 450.  Longer single columns take four: there the adds of each
+  // block's bins to the column's count (5 million ids 201.7 us, with two 203.4).
+  // (At most 1024 blocks: 2^25 uniform values 442 -> 431 us, but 2^26 in runs
+  // 248 -> 260 and 2^25 zipf ones 491 -> 495.)
+  const uint64_t hist_rows = (!a.inline_desc || a.n_cap <= (1u << 21) ? 2 : 4) * kHistChunk;
+  uint64_t hb = (a.n_cap + hist_rows - 1) / hist_rows;
   if (hb > a.hist_chunks_cap) hb = a.hist_chunks_cap;
   hipLaunchKernelGGL(k_histogram, dim3(cap_grid((uint32_t)hb, kHistMaxBlocks)), dim3(kBlock), 0,
                      s, a.values, a.desc, a.cs, a.sort_status, a.tail_status, a.tile_entries,
