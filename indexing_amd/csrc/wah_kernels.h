@@ -39,9 +39,9 @@ namespace wah {
 constexpr int kSortThreads = WAH_SORT_THREADS;  // threads of a radix-pass block
 constexpr int kSortItems = WAH_SORT_ITEMS;      // keys per thread in a radix pass
 constexpr int kSortTile = kSortThreads * kSortItems;
-// Radix tile shapes compiled in: threads per block x keys per thread (shape
-// 0 is the default).  A build runs one shape per column, chosen per
-// column-length bucket by the tuning table.  Fewer keys per thread make more,
+// Radix tile shapes compiled in: threads per block x keys per thread.  A build
+// runs one shape per column, chosen per column-length bucket by the tuning
+// table, or by column and batch length where none was set.  Fewer keys per thread make more,
 // smaller tiles (more blocks in flight, more look-back steps); more keys per
 // thread the reverse.  Every tile is a whole number of the histogram's
 // 4096-row chunks (and of the run cut's 4096-row steps), which count and cut

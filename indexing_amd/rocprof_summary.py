@@ -83,17 +83,23 @@ def calib_scale(path, counter, nbytes):
     return nbytes / (best * 1024.0) if best else None
 
 
+def _run_only(label):
+    """The run-mode instantiation of a radix pass or a tail (last template
+    argument: 0 pair, 1 run, 2 both)."""
+    return ", 1>" in label
+
+
 def byte_model(label, n, L, K, narrow):
     """(algorithmic bytes, bytes moved by design) of one launch, or None."""
     kb = 2.0 if narrow else 4.0
     if "k_histogram" in label:
         return 4.0 * n, 4.0 * n
-    if "k_onesweep" in label and "true" not in label:
+    if "k_onesweep" in label and not _run_only(label):
         i = int(label.rsplit(" ", 1)[1])
         if i == 0:
             return 12.0 * n, (4.0 + kb + 4.0) * n
         return 16.0 * n, 2.0 * (kb + 4.0) * n
-    if "k_tail" in label and "true" not in label:
+    if "k_tail" in label and not _run_only(label):
         return 8.0 * n + 4.0 * L + 8.0 * K, (kb + 4.0) * n + 4.0 * L + 8.0 * K
     if "k_finish" in label:
         return 4.0 * K, 4.0 * K
