@@ -35,6 +35,8 @@ struct wahgpu_ctx {
   wahgpu_counts* pinned_counts = nullptr;  // host-pinned landing slot
   // state of the single-pass scans: zero between launches (see ScanState)
   wah::ScanState* scan_state = nullptr;
+  uint64_t* table = nullptr;  // of a range by slices (range_table), table_cap entries
+  uint64_t table_cap = 0;
   uint64_t* scan_host = nullptr;  // host-pinned: fault and results of a scan
   uint32_t cus = 256;
   // per-kernel timing (wahgpu_timing_begin/end)
@@ -558,6 +560,7 @@ void wahgpu_destroy(wahgpu_ctx* c) {
   if (c->desc_stage) (void)hipHostFree(c->desc_stage);
   if (c->arena) (void)hipFree(c->arena);
   if (c->scan_state) (void)hipFree(c->scan_state);
+  if (c->table) (void)hipFree(c->table);
   if (c->scan_host) (void)hipHostFree(c->scan_host);
   if (c->pinned_counts) (void)hipHostFree(c->pinned_counts);
   if (c->own_stream) (void)hipStreamDestroy(c->own_stream);
@@ -1700,6 +1703,36 @@ int wahgpu_decode_device(wahgpu_ctx* c, const uint32_t* d_words, uint64_t len, u
   return WAHGPU_OK;
 }
 
+namespace {
+// Scratch for the table of a range that decodes by slices: `want` entries, or
+// fewer (*got), down to none; the query does without it then.  A fixed arena
+// serves what it holds.  Else the context keeps a buffer of its own, so that a
+// query never moves the arena, which a caller's captured builds may point into.
+uint64_t* range_table(wahgpu_ctx* c, uint64_t want, uint64_t* got) {
+  if (c->fixed) {
+    *got = std::min<uint64_t>(want, c->arena_cap / 8);
+    return reinterpret_cast<uint64_t*>(c->arena);
+  }
+  if (want > c->table_cap) {
+    if (c->table) {
+      if (hipStreamSynchronize(c->stream) == hipSuccess) (void)hipFree(c->table);
+      else return *got = 0, nullptr;
+    }
+    c->table = nullptr;
+    c->table_cap = 0;
+    const uint64_t cap = (want * 8 + (2u << 20) - 1) / (2u << 20) * (2u << 20);
+    if (hipMalloc(&c->table, cap) != hipSuccess) {
+      (void)hipGetLastError();
+      c->table = nullptr;
+      return *got = 0, nullptr;
+    }
+    c->table_cap = cap / 8;
+  }
+  *got = want;
+  return c->table;
+}
+}  // namespace
+
 int wahgpu_query_range_device(wahgpu_ctx* c, const uint32_t* d_keys, const uint32_t* d_offsets,
                               const uint32_t* d_lengths, uint64_t keycnt,
                               const uint32_t* d_words, uint32_t lo, uint32_t hi, uint64_t nrows,
@@ -1716,14 +1749,11 @@ int wahgpu_query_range_device(wahgpu_ctx* c, const uint32_t* d_keys, const uint3
   }
   int rc = arena_limit(c, align_up(4 * 8));
   if (rc) return rc;
-  // a table for a decode by slices, where the arena has or gets the room; the
-  // query does without it otherwise
-  uint64_t entries = wah::range_table_entries(keycnt, nrows, c->cus);
-  if (c->fixed) entries = std::min<uint64_t>(entries, c->arena_cap / 8);
-  else if (arena_reserve(c, entries * 8)) entries = 0;
+  uint64_t entries = 0;
+  uint64_t* table = range_table(c, wah::range_table_entries(keycnt, nrows, c->cus), &entries);
   ORDERED(c);
   wah::launch_range(scan_run(c), d_keys, d_offsets, d_lengths, keycnt, d_words, lo, hi, d_bitmap,
-                    nrows, reinterpret_cast<uint64_t*>(c->arena), entries, c->stream);
+                    nrows, table, entries, c->stream);
   LAUNCHCHK(c);
   uint64_t unused;
   order_guard_.end();  // no host wait holds the device order
