@@ -26,7 +26,7 @@
   for (;;) {
     for (int i = t; i < WAVES * 256; i += THREADS) (&s_wcnt[0][0])[i] = 0;
     const uint32_t tile = __builtin_amdgcn_readfirstlane(
-        next_tile(counter, lanes, &s_tile, iter, tile_group(dims.sort_tiles, lanes, WAH_SORT_TILE_GROUP)));
+        next_tile(counter, lanes, &s_tile, iter, tile_group(dims.sort_tiles, gridDim.x, lanes, WAH_SORT_TILE_GROUP)));
     if (tile >= dims.sort_tiles) break;
     const uint32_t c = find_segment(&cols[0].sort_tile0, sizeof(Column) / 4, dims.ncols, tile);
     const ColState* col = &cs[c];

@@ -13,7 +13,7 @@
   for (;;) {
     const uint32_t tile = __builtin_amdgcn_readfirstlane(next_tile(
         &hdr->tiles[RUN ? kCounterRunTail : kCounterTail][0], lanes, &s_tile, iter,
-        tile_group(dims.tail_tiles, lanes, WAH_TAIL_TILE_GROUP)));
+        tile_group(dims.tail_tiles, gridDim.x, lanes, WAH_TAIL_TILE_GROUP)));
     if (tile >= dims.tail_tiles) break;
     const uint32_t c = find_segment(&cols[0].tail_tile0, sizeof(Column) / 4, dims.ncols, tile);
     const Column cd = cols[c];

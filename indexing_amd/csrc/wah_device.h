@@ -6,6 +6,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "wah_tiles.h"
+
 namespace wah {
 
 constexpr int kWave = 64;
@@ -62,7 +64,8 @@ __device__ __forceinline__ uint64_t shfl64(uint64_t x, int src) {
   return ((uint64_t)hi << 32) | lo;
 }
 
-// Tile scheduling for the single-pass kernels.  Tiles are handed out by
+// Tile scheduling for the single-pass kernels (wah_tiles.h has the rules; the
+// scans' own is in wah_scan.h).  Tiles are handed out by
 // `lanes` counters (one per 256-byte line, kLaneStride words apart): block b
 // draws from counter b % lanes and gets tiles lane, lane + lanes, ... in
 // increasing order.  A global atomic on one address costs ~11 ns on MI355X
@@ -78,15 +81,6 @@ __device__ __forceinline__ uint64_t shfl64(uint64_t x, int src) {
 #ifndef WAH_STATIC_TILES
 #define WAH_STATIC_TILES 0
 #endif
-constexpr uint32_t kTileLanes = 8;
-constexpr uint32_t kLaneStride = 64;
-//
-// With group > 1 a lane's j-th draw is tile (j / group) * group * lanes +
-// lane * group + j % group: runs of `group` consecutive tiles go to one lane.
-// Workgroups are dispatched to the 8 XCDs round robin, so lane = block % 8
-// is the XCD, and neighbouring tiles then write the cache lines they share
-// (the ends of their output runs) through one L2, which merges them.  A
-// lane's draws still ascend, so the argument above holds.
 __device__ __forceinline__ uint32_t next_tile(uint32_t* counters, uint32_t lanes,
                                               uint32_t* s_tile, uint32_t& iter,
                                               uint32_t group = 1) {
@@ -102,26 +96,11 @@ __device__ __forceinline__ uint32_t next_tile(uint32_t* counters, uint32_t lanes
   if (threadIdx.x == 0) {
     const uint32_t lane = blockIdx.x % lanes;
     const uint32_t j = atomicAdd(&counters[lane * kLaneStride], 1u);
-    *s_tile = group == 1 ? j * lanes + lane
-                         : (j / group) * group * lanes + lane * group + j % group;
+    *s_tile = drawn_tile(j, lanes, lane, group);
   }
   __syncthreads();
   return *s_tile;
 #endif
-}
-// Group of a launch over `tiles` tiles: `group` where the blocks draw several
-// tiles each.  Where there is a block for every tile, the tiles are dealt to
-// the lanes in equal runs, so that each lane has as many tiles as blocks (a
-// grid of a multiple of the lanes): with runs of 8, 18 tiles lay in three
-// lanes of 2 or 3 blocks, which took them in turn while the other lanes'
-// blocks found nothing (a radix pass over 300,007 rows 41 us, over 2^20 rows
-// 14 us).
-__device__ __forceinline__ uint32_t tile_group(uint32_t tiles, uint32_t lanes, uint32_t group) {
-  return tiles <= gridDim.x ? (tiles + lanes - 1) / lanes : group;
-}
-// Counter lanes for a grid of `grid` blocks.
-__host__ __device__ __forceinline__ uint32_t tile_lanes(uint32_t grid) {
-  return grid < kTileLanes ? (grid ? grid : 1u) : kTileLanes;
 }
 
 // Asynchronous copy of 16 bytes per lane from global memory straight into

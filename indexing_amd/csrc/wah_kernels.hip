@@ -904,7 +904,7 @@ __global__ __launch_bounds__(kWideThreads, sort_waves_per_eu(kWideItems)) void k
   for (;;) {
     for (int i = t; i < WAVES * (int)kWideBins / 2; i += THREADS) (&s_cnt[0][0])[i] = 0;
     const uint32_t tile = __builtin_amdgcn_readfirstlane(
-        next_tile(counter, lanes, &s_tile, iter, tile_group(dims.wide_tiles, lanes, WAH_SORT_TILE_GROUP)));
+        next_tile(counter, lanes, &s_tile, iter, tile_group(dims.wide_tiles, gridDim.x, lanes, WAH_SORT_TILE_GROUP)));
     if (tile >= dims.wide_tiles) break;
     const uint32_t c = find_segment(&cols[0].wide_tile0, sizeof(Column) / 4, dims.ncols, tile);
     const ColState* col = &cs[c];

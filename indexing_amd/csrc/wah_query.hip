@@ -181,8 +181,8 @@ __device__ __forceinline__ void enter_slices(const uint32_t* __restrict__ words,
   const uint32_t keys = (uint32_t)(key_b - key_a);
   words += w0;
   const uint32_t tiles = (uint32_t)((len + kEnterTile - 1) / kEnterTile);
-  for (uint32_t tile = scan_next_tile(st, &s_tile, true); tile < tiles;
-       tile = scan_next_tile(st, &s_tile, false)) {
+  for (uint32_t tile = scan_next_tile(st, &s_tile, tiles, true); tile < tiles;
+       tile = scan_next_tile(st, &s_tile, tiles, false)) {
     const uint64_t base = (uint64_t)tile * kEnterTile;
     W4 x[kEnterRows];
     if (base + kEnterTile <= len) {
@@ -367,8 +367,8 @@ __global__ __launch_bounds__(kScanThreads, query_waves_per_eu(kDecBlocks)) void 
   const uint32_t tiles_a = (uint32_t)((qa.len + kDecTile - 1) / kDecTile);
   const uint32_t tiles = tiles_a + (SEG ? 0u : (uint32_t)((qb.len + kDecTile - 1) / kDecTile));
   uint64_t my_last = 0;  // row after the last set row of this thread's words (stream a)
-  for (uint32_t tile = scan_next_tile(st, &s_tile, true); tile < tiles;
-       tile = scan_next_tile(st, &s_tile, false)) {
+  for (uint32_t tile = scan_next_tile(st, &s_tile, tiles, true); tile < tiles;
+       tile = scan_next_tile(st, &s_tile, tiles, false)) {
     const bool second = !SEG && tile >= tiles_a;
     const DecodeStream q = second ? qb : qa;
     const uint32_t first = second ? tiles_a : 0u;
@@ -760,8 +760,8 @@ __global__ __launch_bounds__(kScanThreads, query_waves_per_eu(kEncBlocks)) void 
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const uint64_t nwords = (nrows + 31) / 32;
   const uint32_t tail = (uint32_t)(nrows & 31u);  // rows of the last word (0: all 32)
-  for (uint32_t tile = scan_next_tile(st, &s_tile, true); tile < tiles;
-       tile = scan_next_tile(st, &s_tile, false)) {
+  for (uint32_t tile = scan_next_tile(st, &s_tile, tiles, true); tile < tiles;
+       tile = scan_next_tile(st, &s_tile, tiles, false)) {
     const uint64_t wbase = (uint64_t)tile * kEncWords;
     const uint32_t c0 = tile * kEncTile;  // chunks are below 2^28
     auto load = [&](auto full_tag) {

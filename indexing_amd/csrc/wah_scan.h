@@ -165,16 +165,18 @@ __device__ __forceinline__ void lookback2(uint64_t* status, uint32_t tile, uint3
 }
 
 // ---- tiles and the state of a launch ---------------------------------------
-// A block's first tile is its own index (the lane it draws from hands out
-// lane, lane + 8, ... and starts past its blocks), so only a launch with more
-// tiles than blocks draws at all.
-__device__ __forceinline__ uint32_t scan_next_tile(ScanState* st, uint32_t* s_tile, bool first) {
-  const uint32_t lanes = tile_lanes(gridDim.x);
-  if (first) return blockIdx.x;
+// The block's next tile (`tiles` or more: none), by the rules of wah_tiles.h.  A
+// launch with a block for every tile draws nothing: its blocks know their tile
+// and that there is no other.
+__device__ __forceinline__ uint32_t scan_next_tile(ScanState* st, uint32_t* s_tile, uint32_t tiles,
+                                                   bool first) {
+  if (!scan_draws(tiles, gridDim.x)) return first ? blockIdx.x : tiles;
+  // (opaque: the draw's address is formed here, not kept in registers across a tile)
+  uint32_t b = blockIdx.x;
+  asm volatile("" : "+s"(b));
   if (threadIdx.x == 0) {
-    const uint32_t lane = blockIdx.x % lanes;
-    const uint32_t own = (gridDim.x - lane + lanes - 1) / lanes;  // blocks of the lane
-    *s_tile = (own + atomicAdd(&st->tiles[lane * kLaneStride], 1u)) * lanes + lane;
+    const uint32_t lanes = tile_lanes(gridDim.x), lane = b % lanes;
+    *s_tile = drawn_tile(atomicAdd(&st->tiles[lane * kLaneStride], 1u), lanes, lane);
   }
   __syncthreads();
   const uint32_t tile = __builtin_amdgcn_readfirstlane(*s_tile);

@@ -14,11 +14,10 @@ namespace wah {
 
 namespace {
 
-// Rows per tile and blocks per CU of each kernel.  All blocks of a launch are
-// resident (the look-back needs that): the registers and LDS of a block allow
-// that many.  What a tile costs besides its bytes is one look-back (its wait
-// is for the tiles just before it), so the largest tiles that leave two blocks
-// per CU are the fastest: 2^24 elements, 16384-element tiles at two blocks
+// Rows per tile and blocks per CU of each kernel.  A launch has no more blocks
+// than the registers and LDS of a block let the device hold at once.  What a
+// tile costs besides its bytes is one look-back (its wait is for the tiles just
+// before it), so the largest tiles that leave two blocks per CU are the fastest: 2^24 elements, 16384-element tiles at two blocks
 // per CU against 8192 at four and 4096 at four: scan 31.7 / 35.8 / 46.9 us,
 // compaction 40.2 / 42.6 / 51.4 us, fuse (half the elements) 20.6 / 22.7 /
 // 28.9 us on 2^22.  The segmented scan and the column lengths hold more
@@ -56,8 +55,8 @@ __global__ __launch_bounds__(kScanThreads, waves_per_eu(kScanBlocks)) void k_sca
   __shared__ uint32_t s_prefix, s_tile;
   const int l = threadIdx.x % kWave;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-  for (uint32_t tile = scan_next_tile(st, &s_tile, true); tile < tiles;
-       tile = scan_next_tile(st, &s_tile, false)) {
+  for (uint32_t tile = scan_next_tile(st, &s_tile, tiles, true); tile < tiles;
+       tile = scan_next_tile(st, &s_tile, tiles, false)) {
     const uint64_t base = (uint64_t)tile * TILE;
     auto body = [&](auto full_tag) {
       constexpr bool FULL = decltype(full_tag)::value;
@@ -116,8 +115,8 @@ __global__ __launch_bounds__(kScanThreads, waves_per_eu(kScanBlocks)) void k_seg
   __shared__ uint32_t s_prefix, s_tile;
   const int l = threadIdx.x % kWave;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-  for (uint32_t tile = scan_next_tile(st, &s_tile, true); tile < tiles;
-       tile = scan_next_tile(st, &s_tile, false)) {
+  for (uint32_t tile = scan_next_tile(st, &s_tile, tiles, true); tile < tiles;
+       tile = scan_next_tile(st, &s_tile, tiles, false)) {
     const uint64_t base = (uint64_t)tile * TILE;
     auto body = [&](auto full_tag) {
       constexpr bool FULL = decltype(full_tag)::value;
@@ -229,8 +228,8 @@ __global__ __launch_bounds__(kScanThreads, waves_per_eu(kScanBlocks)) void k_com
   __shared__ uint32_t s_prefix, s_tile;
   const int l = threadIdx.x % kWave;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-  for (uint32_t tile = scan_next_tile(st, &s_tile, true); tile < tiles;
-       tile = scan_next_tile(st, &s_tile, false)) {
+  for (uint32_t tile = scan_next_tile(st, &s_tile, tiles, true); tile < tiles;
+       tile = scan_next_tile(st, &s_tile, tiles, false)) {
     const uint64_t base = (uint64_t)tile * TILE;
     uint32_t all;
     auto body = [&](auto full_tag) {
@@ -307,8 +306,8 @@ __global__ __launch_bounds__(kScanThreads, waves_per_eu(kScanBlocks)) void k_mer
   __shared__ uint32_t s_pre_heads, s_pre_or, s_tile;
   const int l = threadIdx.x % kWave;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-  for (uint32_t tile = scan_next_tile(st, &s_tile, true); tile < tiles;
-       tile = scan_next_tile(st, &s_tile, false)) {
+  for (uint32_t tile = scan_next_tile(st, &s_tile, tiles, true); tile < tiles;
+       tile = scan_next_tile(st, &s_tile, tiles, false)) {
     const uint64_t base = (uint64_t)tile * TILE;
     auto body = [&](auto full_tag) {
       constexpr bool FULL = decltype(full_tag)::value;
@@ -513,8 +512,8 @@ __global__ __launch_bounds__(kScanThreads, waves_per_eu(kScanBlocks)) void k_col
   __shared__ uint32_t s_keys, s_words, s_tile;
   const int l = threadIdx.x % kWave;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-  for (uint32_t tile = scan_next_tile(st, &s_tile, true); tile < tiles;
-       tile = scan_next_tile(st, &s_tile, false)) {
+  for (uint32_t tile = scan_next_tile(st, &s_tile, tiles, true); tile < tiles;
+       tile = scan_next_tile(st, &s_tile, tiles, false)) {
     const uint64_t base = (uint64_t)tile * TILE;
     auto body = [&](auto full_tag) {
       constexpr bool FULL = decltype(full_tag)::value;
