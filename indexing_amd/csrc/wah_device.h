@@ -211,10 +211,10 @@ __device__ __forceinline__ uint64_t block_exclusive(uint64_t x, uint64_t* smem,
   return Op::combine(before, exc);
 }
 
-// Every wait on a look-back status is bounded: after kSpinLimit polls it raises
-// *fault and proceeds with a zero contribution, so every wave still finishes.
-// Once any wait of the launch has given up, the others stop waiting too.
-constexpr uint32_t kSpinLimit = 1u << 18;
+// Every wait on a look-back status is bounded: after kSpinLimit polls
+// (wah_tiles.h) it raises *fault and proceeds with a zero contribution, so every
+// wave still finishes.  Once any wait of the launch has given up, the others
+// stop waiting too.
 
 // Exclusive prefix of one digit over the preceding tiles, reading up to
 // WAH_LOOKAHEAD predecessors per round trip (32-bit words: flag << 30 | count).

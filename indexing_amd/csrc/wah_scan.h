@@ -115,7 +115,7 @@ __device__ __forceinline__ void lookback2(uint64_t* status, uint32_t tile, uint3
   uint32_t ah = 0, al = 0;
   bool or_open = true;  // kOpOrSinceHi: no tile with hi != 0 met yet
   int64_t base = (int64_t)tile - 1;
-  uint32_t spins = 0;
+  ScanWait wait;
   while (base >= (int64_t)first) {
     const int64_t idx = base - (int64_t)lane;
     const uint64_t s = idx >= (int64_t)first ? ld_agent(&status[idx]) : ((uint64_t)kFlagPrefix << 62);
@@ -125,11 +125,12 @@ __device__ __forceinline__ void lookback2(uint64_t* status, uint32_t tile, uint3
     // lanes up to the nearest prefix, all of which have to be there
     const uint64_t need = pmask ? (pmask ^ (pmask - 1)) : ~0ull;
     if (empty & need) {
-      if (++spins >= kSpinLimit) {
+      if (wait.poll(empty & need)) {
         if (lane == 0) atomicOr(fault, 1u);
         break;
       }
-      if ((spins & 1023u) == 0 && ld_agent(fault)) break;
+      if ((wait.polls & 1023u) == 0 && ld_agent(fault)) break;
+      __builtin_amdgcn_s_sleep(1);
       continue;
     }
     const bool take = (need >> lane) & 1u;
@@ -150,6 +151,7 @@ __device__ __forceinline__ void lookback2(uint64_t* status, uint32_t tile, uint3
     }
     if (pmask) break;
     base -= kWave;
+    wait.next_window();
   }
   if (!closed && lane == 0) {
     uint32_t ih = 0, il = 0;

@@ -47,4 +47,28 @@ constexpr uint32_t tile_group(uint32_t tiles, uint32_t grid, uint32_t lanes, uin
 // work on another stream may withhold for as long as it runs.
 constexpr bool scan_draws(uint32_t tiles, uint32_t grid) { return tiles > grid; }
 
+// Polls of a look-back wait that see nothing new before it gives up.
+constexpr uint32_t kSpinLimit = 1u << 18;
+
+// The wait of a scan's look-back: `waiting` is the set of tiles of its window
+// that it still waits for.  The limit counts from the last change of that set
+// (a tile published, or the next window), not over the whole walk, so tiles that
+// come slowly one after another are waited for as long as each of them may take.
+struct ScanWait {
+  uint32_t polls = 0;
+  uint64_t waiting = 0;
+  // One more poll that found `now` unpublished; true: give up.
+  constexpr bool poll(uint64_t now) {
+    if (now != waiting) {
+      waiting = now;
+      polls = 0;
+    }
+    return ++polls >= kSpinLimit;
+  }
+  constexpr void next_window() {
+    waiting = 0;
+    polls = 0;
+  }
+};
+
 }  // namespace wah

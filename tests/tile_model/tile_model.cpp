@@ -6,6 +6,10 @@
 // launch must finish every tile once, whatever is withheld, as long as each XCD
 // keeps one slot.
 //
+// Then the wait of the scans' look-back: predecessors that come one after another,
+// each short of the limit, are waited for however many there are, in one window
+// of 64 and over several; one that never comes is given up at the limit.
+//
 // Argument: "shipped", or "indexed" for the rule that these kernels must not
 // have (a block's first tile is its index even where it stays for more), which
 // the model has to see stall.
@@ -84,6 +88,35 @@ bool run(const Launch& L, const std::vector<uint32_t>& slots) {
   return finished == L.tiles;
 }
 
+// A walk over `windows` windows of which each tile comes `gap` polls after the one
+// before (never, from tile `lost` on).  Polls until it ended or gave up.
+bool walk(uint32_t windows, uint32_t gap, uint32_t lost, uint64_t* polls) {
+  wah::ScanWait wait;
+  *polls = 0;
+  for (uint32_t w = 0; w < windows; ++w) {
+    uint64_t empty = ~0ull;
+    for (uint32_t t = 0; t < 64; ++t) {
+      const bool never = w * 64 + t >= lost;
+      for (uint64_t p = 0; never || p < gap; ++p, ++*polls)
+        if (wait.poll(empty)) return false;
+      empty &= empty - 1;
+    }
+    wait.next_window();
+  }
+  return true;
+}
+
+int waits() {
+  uint64_t polls = 0;
+  int bad = 0;
+  bad += !walk(1, wah::kSpinLimit - 1, ~0u, &polls);      // 63 limits in one window
+  bad += !walk(3, wah::kSpinLimit / 2, ~0u, &polls);      // over three
+  bad += walk(1, 0, 0, &polls) || polls != wah::kSpinLimit - 1;  // (the last poll gives up)
+  bad += walk(2, 5, 70, &polls) || polls != 70 * 5 + wah::kSpinLimit - 1;
+  if (bad) printf("%d waits wrong\n", bad);
+  return bad;
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -107,5 +140,5 @@ int main(int argc, char** argv) {
     }
   }
   printf("%u of %u launches stalled\n", stalls, runs);
-  return stalls != 0;
+  return stalls != 0 || waits() != 0;
 }
