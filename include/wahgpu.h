@@ -376,7 +376,11 @@ int wahgpu_compute_column_length(wahgpu_ctx* ctx, const uint32_t* d_values,
                                  uint32_t* d_keys, uint32_t* d_offsets,
                                  uint32_t* d_lengths, uint64_t* keycnt);
 
-/* ---- primitives -------------------------------------------------------- */
+/* ---- primitives ---------------------------------------------------------
+ * The two scans are asynchronous.  One whose look-back gives up (see
+ * wahgpu_create: another launch of this kind on the device, outside the
+ * library's order) is reported, once and as WAHGPU_EHIP, by the next call on the
+ * context that waits for a result, or by wahgpu_synchronize. */
 /* include/stream_compaction.cl:68-160: keep d_data[i] where d_valid[i] != 0,
  * in order; returns the count (the kernel's result[0]). */
 int wahgpu_stream_compaction(wahgpu_ctx* ctx, const uint32_t* d_data,

@@ -304,6 +304,8 @@ struct ScanRun {
   ScanState* state;
   uint64_t* status;
   uint64_t* host;  // page-locked: fault and result when the launch ends
+  uint64_t* kept;  // page-locked: fault of a launch whose end no call waits for (its
+                   // nonzero faults only, so a later good one leaves it)
   uint32_t cus;    // compute units of the device
 };
 

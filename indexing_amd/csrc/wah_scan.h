@@ -187,14 +187,15 @@ __device__ __forceinline__ uint32_t scan_next_tile(ScanState* st, uint32_t* s_ti
 }
 
 // End of a block.  The last block of the launch hands the fault word and the
-// result to the host (host: page-locked memory, or null) and zeroes the state
+// result to the host (host: page-locked memory; where it is null nobody waits
+// for the launch, and a fault goes to *kept) and zeroes the state
 // for the next launch, so no launch needs a fill before it.  Every wave first
 // waits for its own stores and atomics: a status published late would
 // otherwise land on the zeroed state.  The blocks count themselves per lane
 // and the lanes' last blocks count the lanes, since atomics on one address
 // take about 11 ns each.
 __device__ __forceinline__ void scan_finish(ScanState* st, uint64_t* status, uint32_t tiles,
-                                            uint64_t* host) {
+                                            uint64_t* host, uint64_t* kept = nullptr) {
   __shared__ uint32_t s_last;
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
   __syncthreads();
@@ -219,6 +220,8 @@ __device__ __forceinline__ void scan_finish(ScanState* st, uint64_t* status, uin
     if (host) {
       __hip_atomic_store(&host[0], f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
       __hip_atomic_store(&host[1], r, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    } else if (f) {
+      __hip_atomic_store(kept, f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
     st_agent(&st->fault, 0u);
     st_agent(&st->done, 0u);

@@ -49,7 +49,7 @@ __device__ __forceinline__ uint32_t waves_before(const uint32_t* s_tot, int w, u
 template <int ROWS>
 __global__ __launch_bounds__(kScanThreads, waves_per_eu(kScanBlocks)) void k_scan(
     const uint32_t* in, uint64_t n, uint32_t* out, ScanState* st, uint64_t* status,
-    uint32_t tiles) {
+    uint32_t tiles, uint64_t* kept) {
   constexpr uint32_t TILE = kScanTileOf<ROWS>;
   __shared__ uint32_t s_tot[kScanWaves];
   __shared__ uint32_t s_prefix, s_tile;
@@ -95,7 +95,7 @@ __global__ __launch_bounds__(kScanThreads, waves_per_eu(kScanBlocks)) void k_sca
     if (base + TILE <= n) body(std::true_type{});
     else body(std::false_type{});
   }
-  scan_finish(st, status, tiles, nullptr);
+  scan_finish(st, status, tiles, nullptr, kept);
 }
 
 // Segmented inclusive sum scan (include/segmented_scan.cl): restarts where
@@ -108,7 +108,7 @@ __global__ __launch_bounds__(kScanThreads, waves_per_eu(kScanBlocks)) void k_sca
 // nothing from before it.  2^24 elements: 39.4 us (5.1 TB/s; was 230 us).
 __global__ __launch_bounds__(kScanThreads, waves_per_eu(kScanBlocks)) void k_segscan(
     const uint32_t* in, const uint32_t* heads, uint64_t n, uint32_t* out, ScanState* st,
-    uint64_t* status, uint32_t tiles) {
+    uint64_t* status, uint32_t tiles, uint64_t* kept) {
   constexpr int ROWS = kSegRows;
   constexpr uint32_t TILE = kScanTileOf<ROWS>;
   __shared__ uint32_t s_sum[kScanWaves], s_head[kScanWaves];
@@ -207,7 +207,7 @@ __global__ __launch_bounds__(kScanThreads, waves_per_eu(kScanBlocks)) void k_seg
     if (base + TILE <= n) body(std::true_type{});
     else body(std::false_type{});
   }
-  scan_finish(st, status, tiles, nullptr);
+  scan_finish(st, status, tiles, nullptr, kept);
 }
 
 // Order-preserving compaction.  FUSE false: keep a[i] where b[i] != 0
@@ -630,13 +630,13 @@ void launch_scan(const ScanRun& a, const uint32_t* in, const uint32_t* heads, ui
   const Tiles t = tiles_of(n, segmented ? kSegRows : small ? kSmallRows : kScanRows, a);
   if (segmented)
     hipLaunchKernelGGL(k_segscan, dim3(t.grid), dim3(kScanThreads), 0, s, in, heads, n, out,
-                       a.state, a.status, t.count);
+                       a.state, a.status, t.count, a.kept);
   else if (small)
     hipLaunchKernelGGL(k_scan<kSmallRows>, dim3(t.grid), dim3(kScanThreads), 0, s, in, n, out,
-                       a.state, a.status, t.count);
+                       a.state, a.status, t.count, a.kept);
   else
     hipLaunchKernelGGL(k_scan<kScanRows>, dim3(t.grid), dim3(kScanThreads), 0, s, in, n, out,
-                       a.state, a.status, t.count);
+                       a.state, a.status, t.count, a.kept);
 }
 
 void launch_compact(const ScanRun& a, const uint32_t* data, const uint32_t* valid, uint64_t n,

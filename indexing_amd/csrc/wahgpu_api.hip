@@ -37,7 +37,7 @@ struct wahgpu_ctx {
   wah::ScanState* scan_state = nullptr;
   uint64_t* table = nullptr;  // of a range by slices (range_table), table_cap entries
   uint64_t table_cap = 0;
-  uint64_t* scan_host = nullptr;  // host-pinned: fault and results of a scan
+  uint64_t* scan_host = nullptr;  // host-pinned: fault and results of a scan (kScanHostWords)
   uint32_t cus = 256;
   // per-kernel timing (wahgpu_timing_begin/end)
   std::vector<hipEvent_t> tev;  // max_calls x (WAHGPU_TIMING_GROUPS + 1)
@@ -346,10 +346,29 @@ int check_n(wahgpu_ctx* c, uint64_t n, uint32_t rid_base) {
   return WAHGPU_OK;
 }
 
+// Words of scan_host: fault and result of a scan, two more words of a range query
+// (3 and 4), those of a decode whose encode follows (5 and 6), and the fault that
+// an asynchronous scan left, kept until a call that waits reports it.
+constexpr int kScanHostWords = 8, kDecodeSlot = 5, kKeptSlot = 7;
+
+// Waits for the stream; reports the fault of an earlier scan that nobody waited
+// for, whose sums are then wrong, once.
+int wait_stream(wahgpu_ctx* c) {
+  HIPCHK(c, hipStreamSynchronize(c->stream));
+  volatile uint64_t* kept = c->scan_host + kKeptSlot;
+  if (const uint64_t f = *kept) {
+    *kept = 0;
+    return fail(c, WAHGPU_EHIP, "an earlier exclusive or segmented scan reported fault " +
+                                    std::to_string(f) + " (look-back wait gave up); its sums are wrong");
+  }
+  return WAHGPU_OK;
+}
+
 int read_counts(wahgpu_ctx* c, const wahgpu_counts* d_counts, wahgpu_counts* out) {
   HIPCHK(c, hipMemcpyAsync(c->pinned_counts, d_counts, sizeof(wahgpu_counts),
                            hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
+  const int rc = wait_stream(c);
+  if (rc) return rc;
   *out = *c->pinned_counts;
   if (out->fault)
     return fail(c, WAHGPU_EHIP, "kernel reported fault " + std::to_string(out->fault) +
@@ -358,18 +377,17 @@ int read_counts(wahgpu_ctx* c, const wahgpu_counts* d_counts, wahgpu_counts* out
 }
 
 // The context's scan state, for launches on its stream (one after another).
-// Results land in scan_host: fault and result, two more words of a range query
-// (3 and 4), and those of a decode whose encode follows (5 and 6).  A launch of
-// no elements writes nothing, so they start at zero.
-constexpr int kScanHostWords = 8, kDecodeSlot = 5;
+// Results land in scan_host.  A launch of no elements writes nothing, so they
+// start at zero.
 ScanRun scan_run(wahgpu_ctx* c) {
-  memset(c->scan_host, 0, kScanHostWords * sizeof(uint64_t));
+  memset(c->scan_host, 0, kKeptSlot * sizeof(uint64_t));
   return ScanRun{c->scan_state, reinterpret_cast<uint64_t*>(c->scan_state + 1), c->scan_host,
-                 c->cus};
+                 c->scan_host + kKeptSlot, c->cus};
 }
 // Waits for the stream and reads the result of the scan that wrote `slot`.
 int scan_result(wahgpu_ctx* c, uint64_t* out, int slot = 0) {
-  HIPCHK(c, hipStreamSynchronize(c->stream));
+  const int rc = wait_stream(c);
+  if (rc) return rc;
   const volatile uint64_t* h = c->scan_host + slot;
   if (h[0])
     return fail(c, WAHGPU_EHIP, "kernel reported fault " + std::to_string(h[0]) +
@@ -498,12 +516,13 @@ int wahgpu_create(wahgpu_ctx** out, int device_ordinal, uint64_t arena_bytes) {
   }
   c->stream = c->own_stream;
   const uint64_t scan_bytes = sizeof(wah::ScanState) + wah::kScanStatusWords * 8;
-  if (hipHostMalloc(reinterpret_cast<void**>(&c->scan_host), 64, hipHostMallocDefault) != hipSuccess ||
+  if (hipHostMalloc(reinterpret_cast<void**>(&c->scan_host), kScanHostWords * 8, hipHostMallocDefault) != hipSuccess ||
       hipMalloc(&c->scan_state, scan_bytes) != hipSuccess) {
     (void)hipGetLastError();
     wahgpu_destroy(c);
     return WAHGPU_EHIP;
   }
+  memset(c->scan_host, 0, kScanHostWords * 8);
   wah::launch_fill32(reinterpret_cast<uint32_t*>(c->scan_state), scan_bytes / 4, 0, c->stream);
   if (noalloc_lookup(c, device_ordinal) != WAHGPU_OK) {
     (void)hipGetLastError();
@@ -597,8 +616,7 @@ int wahgpu_rank_mode(const wahgpu_ctx* c) { return c && c->atomic_rank ? 1 : 0; 
 
 int wahgpu_synchronize(wahgpu_ctx* c) {
   if (!c) return WAHGPU_EINVAL;
-  HIPCHK(c, hipStreamSynchronize(c->stream));
-  return WAHGPU_OK;
+  return wait_stream(c);
 }
 
 // ---- fused build ---------------------------------------------------------
@@ -1145,7 +1163,8 @@ int wahgpu_build_batch(wahgpu_ctx* c, const uint32_t* const* values, const uint6
   std::vector<wahgpu_counts> hc(ncols);
   HIPCHK(c, hipMemcpyAsync(hc.data(), d_counts, ncols * sizeof(wahgpu_counts),
                            hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
+  rc = wait_stream(c);
+  if (rc) return rc;
   for (uint32_t i = 0; i < ncols; ++i) {
     const wahgpu_counts& k = hc[i];
     wahgpu_result& r = results[i];

@@ -1,0 +1,102 @@
+"""Host code of the C ABI (indexing_amd/csrc/wahgpu_api.hip) on the CPU: compiled
+with g++ against tests/api_harness, whose launchers compute nothing but hand the
+host what a test scripts, a given fault among it.  What the entry points do with
+that, how much memory they take, and what they refuse.
+"""
+import ctypes
+import os
+import shutil
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+HARNESS = os.path.join(ROOT, "tests", "api_harness")
+CSRC = os.path.join(ROOT, "indexing_amd", "csrc")
+OK, EHIP = 0, -3
+U64, VP = ctypes.c_uint64, ctypes.c_void_p
+
+
+def u64(x):
+    return U64(int(x))
+
+
+@pytest.fixture(scope="module")
+def lib(tmp_path_factory):
+    if shutil.which("g++") is None:
+        pytest.skip("g++ not installed")
+    so = str(tmp_path_factory.mktemp("api") / "libapi.so")
+    r = subprocess.run(["g++", "-shared", "-fPIC", "-std=c++17", "-O1", "-g", "-Wall", "-I" + HARNESS,
+                        "-I" + os.path.join(ROOT, "include"), "-I" + CSRC,
+                        "-x", "c++", os.path.join(CSRC, "wahgpu_api.hip"),
+                        os.path.join(HARNESS, "fake_gpu.cpp"), os.path.join(CSRC, "wah_host.cpp"),
+                        "-o", so], capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr[-4000:]
+    x = ctypes.CDLL(so)
+    x.fake_log.restype = ctypes.c_char_p
+    x.fake_device_bytes.restype = U64
+    x.wahgpu_last_error.restype = ctypes.c_char_p
+    x.wahgpu_stream.restype = VP
+    return x
+
+
+class Ctx:
+    """A context and one buffer that stands for every device pointer."""
+
+    def __init__(self, lib, arena=0):
+        self.lib, self.h = lib, VP()
+        self.buf = VP(256)  # (the launchers read nothing)
+        assert lib.wahgpu_create(ctypes.byref(self.h), 0, u64(arena)) == OK
+        lib.fake_reset()
+
+    def close(self):
+        self.lib.wahgpu_destroy(self.h)
+
+    def call(self, name, *args):
+        """An entry point; integers are 64-bit, None is the buffer."""
+        conv = [self.buf if a is None else u64(a) if isinstance(a, int) else a for a in args]
+        return getattr(self.lib, "wahgpu_" + name)(self.h, *conv)
+
+    def script(self, name, fault=0, result=0, extra=(0, 0), ends=True):
+        self.lib.fake_script(name.encode(), int(ends), u64(fault), u64(result), u64(extra[0]),
+                             u64(extra[1]))
+
+    def log(self):
+        return self.lib.fake_log().decode().splitlines()
+
+    def error(self):
+        return self.lib.wahgpu_last_error(self.h).decode()
+
+
+@pytest.fixture
+def ctx(lib):
+    c = Ctx(lib)
+    yield c
+    c.close()
+
+
+@pytest.mark.parametrize("segmented", [False, True])
+@pytest.mark.parametrize("next_call", ["synchronize", "compaction", "build"])
+def test_fault_of_an_asynchronous_scan_is_reported(ctx, segmented, next_call):
+    """A scan that nobody waits for and that gave up: the next call that waits
+    says so, once."""
+    out = U64(77)
+    counts = (ctypes.c_uint64 * 8)()
+
+    def waits():
+        if next_call == "synchronize":
+            return ctx.call("synchronize")
+        if next_call == "compaction":
+            return ctx.call("stream_compaction", None, None, 100, None, ctypes.byref(out))
+        return ctx.call("build", (ctypes.c_uint32 * 4)(), 4, ctypes.c_uint32(0), None, None, None,
+                        100, None, 100, counts, VP())
+
+    ctx.script("scan", fault=1)
+    if segmented:
+        assert ctx.call("segmented_inclusive_scan", None, None, 100, None) == OK
+    else:
+        assert ctx.call("exclusive_scan", None, 100, None) == OK
+    assert ctx.call("exclusive_scan", None, 100, None) == OK  # a good one takes nothing back
+    assert waits() == EHIP
+    assert "earlier" in ctx.error() and "scan" in ctx.error()
+    assert waits() == OK
