@@ -94,8 +94,13 @@ int wahgpu_find_device(const char* name);
  * workgroups placed on particular XCDs, and two such launches sharing the
  * device could each hold the CUs the other needs.  Copies and other work still
  * overlap them, and so do builds of columns of at most 2^14 values, which one
- * workgroup each does without waiting for another.  Calls made while their stream captures a graph are not
- * ordered: replay such graphs on one stream at a time. */
+ * workgroup each does without waiting for another.
+ * Calls made while their stream captures a graph are not ordered: replay such
+ * graphs on one stream at a time, and not while calls of this library run on
+ * another stream of the device; a wait of theirs that gives up then is a
+ * reported fault.  A captured scan has its state to itself and clears it in
+ * every replay, so calls of the context that overlap a replay spoil neither it
+ * nor any later call. */
 int wahgpu_create(wahgpu_ctx** out, int device_ordinal, uint64_t arena_bytes);
 void wahgpu_destroy(wahgpu_ctx* ctx);
 const char* wahgpu_last_error(const wahgpu_ctx* ctx);

@@ -285,7 +285,10 @@ __host__ __device__ inline uint32_t hist_chunks_of(uint64_t n) {
 
 // State of the single-pass scans (wah_scan.hip), one per context: zero before
 // every launch, and zeroed again by the launch's last block.  The status words
-// (kScanStatusWords of them) follow it.
+// (kScanStatusWords of them) follow it.  Launches that are captured into a graph
+// use another one, kGraphStatusWords long, which the graph zeroes first: replays
+// are outside the order of the context's calls, and blocks of two launches that
+// counted themselves in one state would leave it spoiled for every later call.
 struct ScanState {
   uint32_t tiles[kLaneWords];  // per lane: word 0 the tile counter, word 1 its ended
                                // blocks, words 2 and 3 a maximum (the result's, if any)
@@ -300,6 +303,9 @@ static_assert(sizeof(ScanState) % 256 == 0, "status words follow at a line bound
 // Tiles of the longest scan: two streams of 2^32 WAH words in decode tiles of
 // 4096.
 constexpr uint64_t kScanStatusWords = 1ull << 21;
+// Tiles of the longest scan that can be captured: 2^30 elements in segmented
+// tiles of 8192.
+constexpr uint64_t kGraphStatusWords = 1ull << 17;
 struct ScanRun {
   ScanState* state;
   uint64_t* status;
@@ -307,6 +313,7 @@ struct ScanRun {
   uint64_t* kept;  // page-locked: fault of a launch whose end no call waits for (its
                    // nonzero faults only, so a later good one leaves it)
   uint32_t cus;    // compute units of the device
+  bool captured;   // the state is the graphs': zero it first (launch_scan)
 };
 
 // Optional hook called between kernel groups of the fused build (timing).

@@ -613,6 +613,9 @@ __global__ __launch_bounds__(kBlock) void k_lengths(const uint32_t* __restrict__
 // ---- launchers ---------------------------------------------------------------
 
 namespace {
+static_assert(WAHGPU_MAX_VALUES <= kGraphStatusWords * kScanTileOf<kSegRows> &&
+                  kSegRows <= kScanRows && kSmallScan / kScanTileOf<kSmallRows> <= kGraphStatusWords,
+              "a captured scan's status words fit");
 struct Tiles {
   uint32_t count, grid;
 };
@@ -628,6 +631,8 @@ void launch_scan(const ScanRun& a, const uint32_t* in, const uint32_t* heads, ui
   if (!n) return;
   const bool small = n < kSmallScan;
   const Tiles t = tiles_of(n, segmented ? kSegRows : small ? kSmallRows : kScanRows, a);
+  if (a.captured)  // the status words follow the state
+    launch_fill32(reinterpret_cast<uint32_t*>(a.state), sizeof(ScanState) / 4 + 2ull * t.count, 0, s);
   if (segmented)
     hipLaunchKernelGGL(k_segscan, dim3(t.grid), dim3(kScanThreads), 0, s, in, heads, n, out,
                        a.state, a.status, t.count, a.kept);

@@ -35,6 +35,7 @@ struct wahgpu_ctx {
   wahgpu_counts* pinned_counts = nullptr;  // host-pinned landing slot
   // state of the single-pass scans: zero between launches (see ScanState)
   wah::ScanState* scan_state = nullptr;
+  wah::ScanState* graph_state = nullptr;  // the same for captured scans (scan_run_async)
   uint64_t* table = nullptr;  // of a range by slices (range_table), table_cap entries
   uint64_t table_cap = 0;
   uint64_t* scan_host = nullptr;  // host-pinned: fault and results of a scan (kScanHostWords)
@@ -382,7 +383,20 @@ int read_counts(wahgpu_ctx* c, const wahgpu_counts* d_counts, wahgpu_counts* out
 ScanRun scan_run(wahgpu_ctx* c) {
   memset(c->scan_host, 0, kKeptSlot * sizeof(uint64_t));
   return ScanRun{c->scan_state, reinterpret_cast<uint64_t*>(c->scan_state + 1), c->scan_host,
-                 c->scan_host + kKeptSlot, c->cus};
+                 c->scan_host + kKeptSlot, c->cus, false};
+}
+// The same for a scan that nobody waits for; one that its stream captures takes
+// the graphs' state.
+int scan_run_async(wahgpu_ctx* c, ScanRun* run) {
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  HIPCHK(c, hipStreamIsCapturing(c->stream, &cs));
+  *run = scan_run(c);
+  if (cs != hipStreamCaptureStatusNone) {
+    run->state = c->graph_state;
+    run->status = reinterpret_cast<uint64_t*>(c->graph_state + 1);
+    run->captured = true;
+  }
+  return WAHGPU_OK;
 }
 // Waits for the stream and reads the result of the scan that wrote `slot`.
 int scan_result(wahgpu_ctx* c, uint64_t* out, int slot = 0) {
@@ -517,7 +531,8 @@ int wahgpu_create(wahgpu_ctx** out, int device_ordinal, uint64_t arena_bytes) {
   c->stream = c->own_stream;
   const uint64_t scan_bytes = sizeof(wah::ScanState) + wah::kScanStatusWords * 8;
   if (hipHostMalloc(reinterpret_cast<void**>(&c->scan_host), kScanHostWords * 8, hipHostMallocDefault) != hipSuccess ||
-      hipMalloc(&c->scan_state, scan_bytes) != hipSuccess) {
+      hipMalloc(&c->scan_state, scan_bytes) != hipSuccess ||
+      hipMalloc(&c->graph_state, sizeof(wah::ScanState) + wah::kGraphStatusWords * 8) != hipSuccess) {
     (void)hipGetLastError();
     wahgpu_destroy(c);
     return WAHGPU_EHIP;
@@ -579,6 +594,7 @@ void wahgpu_destroy(wahgpu_ctx* c) {
   if (c->desc_stage) (void)hipHostFree(c->desc_stage);
   if (c->arena) (void)hipFree(c->arena);
   if (c->scan_state) (void)hipFree(c->scan_state);
+  if (c->graph_state) (void)hipFree(c->graph_state);
   if (c->table) (void)hipFree(c->table);
   if (c->scan_host) (void)hipHostFree(c->scan_host);
   if (c->pinned_counts) (void)hipHostFree(c->pinned_counts);
@@ -1638,7 +1654,10 @@ int wahgpu_exclusive_scan(wahgpu_ctx* c, const uint32_t* d_in, uint64_t n, uint3
   rc = arena_limit(c, scan_scratch_bytes(n));
   if (rc) return rc;
   ORDERED(c);
-  wah::launch_scan(scan_run(c), d_in, nullptr, n, d_out, false, c->stream);
+  ScanRun run;
+  rc = scan_run_async(c, &run);
+  if (rc) return rc;
+  wah::launch_scan(run, d_in, nullptr, n, d_out, false, c->stream);
   LAUNCHCHK(c);
   return WAHGPU_OK;
 }
@@ -1653,7 +1672,10 @@ int wahgpu_segmented_inclusive_scan(wahgpu_ctx* c, const uint32_t* d_in, const u
   rc = arena_limit(c, scan_scratch_bytes(n));
   if (rc) return rc;
   ORDERED(c);
-  wah::launch_scan(scan_run(c), d_in, d_heads, n, d_out, true, c->stream);
+  ScanRun run;
+  rc = scan_run_async(c, &run);
+  if (rc) return rc;
+  wah::launch_scan(run, d_in, d_heads, n, d_out, true, c->stream);
   LAUNCHCHK(c);
   return WAHGPU_OK;
 }

@@ -158,7 +158,7 @@ namespace wah {
 // A launch of at least one tile on scan state: its last block's results.
 static void scan(const char* name, const ScanRun& a, uint64_t n, bool waits) {
   if (!n) return;
-  note("%s n=%llu state=%p", name, (unsigned long long)n, (void*)a.state);
+  note("%s n=%llu state=%p captured=%d", name, (unsigned long long)n, (void*)a.state, a.captured);
   const Script s = next(name);
   if (!s.ends) return;
   if (waits) {

@@ -100,3 +100,24 @@ def test_fault_of_an_asynchronous_scan_is_reported(ctx, segmented, next_call):
     assert waits() == EHIP
     assert "earlier" in ctx.error() and "scan" in ctx.error()
     assert waits() == OK
+
+
+@pytest.mark.parametrize("segmented", [False, True])
+def test_captured_scans_have_a_state_of_their_own(ctx, segmented):
+    """Replays are outside the order of the context's calls: they share no
+    counters with them, and clear their own."""
+    def scan():
+        if segmented:
+            return ctx.call("segmented_inclusive_scan", None, None, 1000, None)
+        return ctx.call("exclusive_scan", None, 1000, None)
+    stream = VP(ctx.lib.wahgpu_stream(ctx.h))
+    assert scan() == OK
+    ctx.lib.fake_capture(stream, 1)
+    assert scan() == OK
+    ctx.lib.fake_capture(stream, 0)
+    assert scan() == OK
+    assert ctx.call("stream_compaction", None, None, 1000, None, ctypes.byref(U64())) == OK
+    before, held, after, other = [x for x in ctx.log() if "state=" in x]
+    state = [x.split("state=")[1].split()[0] for x in (before, held, after, other)]
+    assert state[0] == state[2] == state[3] != state[1]
+    assert ["captured=1" in x for x in (before, held, after, other)] == [False, True, False, False]

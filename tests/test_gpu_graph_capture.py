@@ -50,3 +50,43 @@ def test_build_captured_and_replayed(noalloc):
             assert_same(got, oracle.build(v), f"replay {rep}")
     finally:
         c.close()
+
+
+@pytest.mark.parametrize("segmented", [False, True], ids=["scan", "segmented"])
+def test_scan_replayed_beside_the_contexts_own_work(ctx, segmented):
+    """Replays on one stream while the context scans and compacts on another:
+    every result is right, and so are those after it.  (Few tiles: all blocks of
+    both have a place, so no wait depends on the order.)"""
+    import torch
+    n = 100_003
+    rng = np.random.default_rng(11)
+    data = rng.integers(0, 1 << 32, n, dtype=np.uint64).astype(np.uint32)
+    heads = (rng.random(n) < 0.001).astype(np.uint32)
+    src, flags = dev(data), dev(heads)
+    replayed, own = torch.cuda.Stream(), torch.cuda.Stream()
+
+    def scan():
+        return ctx.segmented_inclusive_scan(src, flags) if segmented else ctx.exclusive_scan(src)
+    want = oracle.segmented_inclusive_scan(data, heads) if segmented else oracle.exclusive_scan(data)
+    with torch.cuda.stream(replayed):
+        scan()
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=replayed):
+            out = scan()
+    torch.cuda.synchronize()
+    for rep in range(10):
+        print(f"[replay] {rep} segmented={segmented}", flush=True)
+        out.zero_()
+        torch.cuda.synchronize()
+        with torch.cuda.stream(replayed):
+            for _ in range(8):
+                g.replay()
+        with torch.cuda.stream(own):
+            for _ in range(4):
+                eager = scan()
+                kept = ctx.stream_compaction(src, flags)
+                assert np.array_equal(kept.cpu().numpy().view(np.uint32), data[heads != 0])
+        torch.cuda.synchronize()
+        for got in (out, eager):
+            assert np.array_equal(got.cpu().numpy().view(np.uint32), want)
