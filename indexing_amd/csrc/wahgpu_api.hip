@@ -351,6 +351,16 @@ int check_n(wahgpu_ctx* c, uint64_t n, uint32_t rid_base) {
 // (3 and 4), those of a decode whose encode follows (5 and 6), and the fault that
 // an asynchronous scan left, kept until a call that waits reports it.
 constexpr int kScanHostWords = 8, kDecodeSlot = 5, kKeptSlot = 7;
+constexpr uint64_t kScanStateBytes = sizeof(wah::ScanState) + wah::kScanStatusWords * 8;
+
+// A scan that is over and whose last block has not reported: its launch shared
+// the state with another one, or found it spoiled.
+constexpr uint64_t kScanUnended = 1ull << 32;
+
+// After a fault: the state may not be what the next launch needs.
+void reset_scan_state(wahgpu_ctx* c) {
+  wah::launch_fill32(reinterpret_cast<uint32_t*>(c->scan_state), kScanStateBytes / 4, 0, c->stream);
+}
 
 // Waits for the stream; reports the fault of an earlier scan that nobody waited
 // for, whose sums are then wrong, once.
@@ -359,6 +369,7 @@ int wait_stream(wahgpu_ctx* c) {
   volatile uint64_t* kept = c->scan_host + kKeptSlot;
   if (const uint64_t f = *kept) {
     *kept = 0;
+    reset_scan_state(c);
     return fail(c, WAHGPU_EHIP, "an earlier exclusive or segmented scan reported fault " +
                                     std::to_string(f) + " (look-back wait gave up); its sums are wrong");
   }
@@ -379,9 +390,10 @@ int read_counts(wahgpu_ctx* c, const wahgpu_counts* d_counts, wahgpu_counts* out
 
 // The context's scan state, for launches on its stream (one after another).
 // Results land in scan_host.  A launch of no elements writes nothing, so they
-// start at zero.
-ScanRun scan_run(wahgpu_ctx* c) {
+// start at zero; `launched`: there are some, so a fault word comes.
+ScanRun scan_run(wahgpu_ctx* c, bool launched) {
   memset(c->scan_host, 0, kKeptSlot * sizeof(uint64_t));
+  c->scan_host[0] = launched ? kScanUnended : 0;
   return ScanRun{c->scan_state, reinterpret_cast<uint64_t*>(c->scan_state + 1), c->scan_host,
                  c->scan_host + kKeptSlot, c->cus, false};
 }
@@ -390,7 +402,7 @@ ScanRun scan_run(wahgpu_ctx* c) {
 int scan_run_async(wahgpu_ctx* c, ScanRun* run) {
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   HIPCHK(c, hipStreamIsCapturing(c->stream, &cs));
-  *run = scan_run(c);
+  *run = scan_run(c, false);
   if (cs != hipStreamCaptureStatusNone) {
     run->state = c->graph_state;
     run->status = reinterpret_cast<uint64_t*>(c->graph_state + 1);
@@ -403,9 +415,13 @@ int scan_result(wahgpu_ctx* c, uint64_t* out, int slot = 0) {
   const int rc = wait_stream(c);
   if (rc) return rc;
   const volatile uint64_t* h = c->scan_host + slot;
-  if (h[0])
-    return fail(c, WAHGPU_EHIP, "kernel reported fault " + std::to_string(h[0]) +
-                                    " (look-back wait gave up or index out of range)");
+  if (const uint64_t f = h[0]) {
+    reset_scan_state(c);
+    return fail(c, WAHGPU_EHIP,
+                f == kScanUnended ? std::string("the scan's blocks did not end as one launch")
+                                  : "kernel reported fault " + std::to_string(f) +
+                                        " (look-back wait gave up or index out of range)");
+  }
   *out = h[1];
   return WAHGPU_OK;
 }
@@ -529,16 +545,15 @@ int wahgpu_create(wahgpu_ctx** out, int device_ordinal, uint64_t arena_bytes) {
     return WAHGPU_EHIP;
   }
   c->stream = c->own_stream;
-  const uint64_t scan_bytes = sizeof(wah::ScanState) + wah::kScanStatusWords * 8;
   if (hipHostMalloc(reinterpret_cast<void**>(&c->scan_host), kScanHostWords * 8, hipHostMallocDefault) != hipSuccess ||
-      hipMalloc(&c->scan_state, scan_bytes) != hipSuccess ||
+      hipMalloc(&c->scan_state, kScanStateBytes) != hipSuccess ||
       hipMalloc(&c->graph_state, sizeof(wah::ScanState) + wah::kGraphStatusWords * 8) != hipSuccess) {
     (void)hipGetLastError();
     wahgpu_destroy(c);
     return WAHGPU_EHIP;
   }
   memset(c->scan_host, 0, kScanHostWords * 8);
-  wah::launch_fill32(reinterpret_cast<uint32_t*>(c->scan_state), scan_bytes / 4, 0, c->stream);
+  reset_scan_state(c);
   if (noalloc_lookup(c, device_ordinal) != WAHGPU_OK) {
     (void)hipGetLastError();
     wahgpu_destroy(c);
@@ -1463,7 +1478,7 @@ int wahgpu_build_staged(wahgpu_ctx* c, const uint32_t* values, uint64_t n, uint3
     wah::launch_chunks(s_rids, n, chids, lits, c->stream);
     LAUNCHCHK(c);
     m.mark(c->stream);  // 3 chunks + literals
-    wah::launch_merge(scan_run(c), s_keys, chids, lits, n, mv, mc, ml, c->stream);
+    wah::launch_merge(scan_run(c, n > 0), s_keys, chids, lits, n, mv, mc, ml, c->stream);
     LAUNCHCHK(c);
   }
   uint64_t k = 0;
@@ -1475,7 +1490,7 @@ int wahgpu_build_staged(wahgpu_ctx* c, const uint32_t* values, uint64_t n, uint3
     wah::launch_fills(mv, mc, k, fills, c->stream);
     LAUNCHCHK(c);
     m.mark(c->stream);  // 5 fills
-    wah::launch_compact(scan_run(c), fills, ml, k, 1, index, c->stream);
+    wah::launch_compact(scan_run(c, k > 0), fills, ml, k, 1, index, c->stream);
     LAUNCHCHK(c);
   }
   uint64_t L = 0;
@@ -1484,7 +1499,8 @@ int wahgpu_build_staged(wahgpu_ctx* c, const uint32_t* values, uint64_t n, uint3
   m.mark(c->stream);  // 6 fuse
   {
     ORDERED(c);
-    wah::launch_colen(scan_run(c), mv, fills, k, o_keys, o_offsets, o_lengths, d_counts, c->stream);
+    wah::launch_colen(scan_run(c, k > 0), mv, fills, k, o_keys, o_offsets, o_lengths, d_counts,
+                      c->stream);
     LAUNCHCHK(c);
   }
   wahgpu_counts cc;
@@ -1576,7 +1592,7 @@ int wahgpu_merge_lit_by_val_chids(wahgpu_ctx* c, const uint32_t* d_values,
   rc = arena_limit(c, scan_scratch_bytes(n));
   if (rc) return rc;
   ORDERED(c);
-  wah::launch_merge(scan_run(c), d_values, d_chids, d_lits, n, d_values_out, d_chids_out,
+  wah::launch_merge(scan_run(c, n > 0), d_values, d_chids, d_lits, n, d_values_out, d_chids_out,
                     d_lits_out, c->stream);
   LAUNCHCHK(c);
   order_guard_.end();  // no host wait holds the device order
@@ -1603,7 +1619,7 @@ int wahgpu_fuse_fill_literals(wahgpu_ctx* c, const uint32_t* d_fills, const uint
   rc = arena_limit(c, scan_scratch_bytes(k));
   if (rc) return rc;
   ORDERED(c);
-  wah::launch_compact(scan_run(c), d_fills, d_lits, k, 1, d_index, c->stream);
+  wah::launch_compact(scan_run(c, k > 0), d_fills, d_lits, k, 1, d_index, c->stream);
   LAUNCHCHK(c);
   order_guard_.end();  // no host wait holds the device order
   return scan_result(c, index_length);
@@ -1622,7 +1638,7 @@ int wahgpu_compute_column_length(wahgpu_ctx* c, const uint32_t* d_values,
   if (rc) return rc;
   wahgpu_counts* d_counts = take<wahgpu_counts>(c, 1);
   ORDERED(c);
-  wah::launch_colen(scan_run(c), d_values, d_fills, k, d_keys, d_offsets, d_lengths, d_counts,
+  wah::launch_colen(scan_run(c, k > 0), d_values, d_fills, k, d_keys, d_offsets, d_lengths, d_counts,
                     c->stream);
   LAUNCHCHK(c);
   order_guard_.end();  // no host wait holds the device order
@@ -1639,7 +1655,7 @@ int wahgpu_stream_compaction(wahgpu_ctx* c, const uint32_t* d_data, const uint32
   rc = arena_limit(c, scan_scratch_bytes(n));
   if (rc) return rc;
   ORDERED(c);
-  wah::launch_compact(scan_run(c), d_data, d_valid, n, 0, d_out, c->stream);
+  wah::launch_compact(scan_run(c, n > 0), d_data, d_valid, n, 0, d_out, c->stream);
   LAUNCHCHK(c);
   order_guard_.end();  // no host wait holds the device order
   return scan_result(c, count);
@@ -1734,7 +1750,7 @@ int wahgpu_decode_device(wahgpu_ctx* c, const uint32_t* d_words, uint64_t len, u
   if (rc) return rc;
   ORDERED(c);
   wah::launch_fill32(d_bitmap, bitmap_words(nrows), 0, c->stream);
-  wah::launch_decode(scan_run(c), {d_words, len, d_bitmap}, {nullptr, 0, nullptr}, nrows, c->stream);
+  wah::launch_decode(scan_run(c, len > 0), {d_words, len, d_bitmap}, {nullptr, 0, nullptr}, nrows, c->stream);
   LAUNCHCHK(c);
   uint64_t last = 0;
   order_guard_.end();  // no host wait holds the device order
@@ -1793,7 +1809,7 @@ int wahgpu_query_range_device(wahgpu_ctx* c, const uint32_t* d_keys, const uint3
   uint64_t entries = 0;
   uint64_t* table = range_table(c, wah::range_table_entries(keycnt, nrows, c->cus), &entries);
   ORDERED(c);
-  wah::launch_range(scan_run(c), d_keys, d_offsets, d_lengths, keycnt, d_words, lo, hi, d_bitmap,
+  wah::launch_range(scan_run(c, true), d_keys, d_offsets, d_lengths, keycnt, d_words, lo, hi, d_bitmap,
                     nrows, table, entries, c->stream);
   LAUNCHCHK(c);
   uint64_t unused;
@@ -1816,7 +1832,7 @@ int wahgpu_encode_device(wahgpu_ctx* c, const uint32_t* d_bitmap, uint64_t nrows
   int rc = arena_limit(c, encode_scratch_bytes(nrows) + kAlign);
   if (rc) return rc;
   ORDERED(c);
-  wah::launch_encode(scan_run(c), d_bitmap, nullptr, 0, nrows, d_words, cap, c->stream);
+  wah::launch_encode(scan_run(c, true), d_bitmap, nullptr, 0, nrows, d_words, cap, c->stream);
   LAUNCHCHK(c);
   order_guard_.end();  // no host wait holds the device order
   rc = scan_result(c, len);
@@ -1846,7 +1862,8 @@ int wahgpu_combine_device(wahgpu_ctx* c, int op, const uint32_t* d_a, uint64_t l
   uint32_t* bm_b = take<uint32_t>(c, bw);
   ORDERED(c);
   wah::launch_fill32(bm_a, (uint64_t)(bm_b - bm_a) + bw, 0, c->stream);  // both, and the gap
-  ScanRun run = scan_run(c);
+  ScanRun run = scan_run(c, true);
+  if (la + lb) c->scan_host[kDecodeSlot] = kScanUnended;
   run.host += kDecodeSlot;  // the encode's results follow in the first slot
   wah::launch_decode(run, {d_a, la, bm_a}, {d_b, lb, bm_b}, nrows, c->stream);
   LAUNCHCHK(c);

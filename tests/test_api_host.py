@@ -121,3 +121,52 @@ def test_captured_scans_have_a_state_of_their_own(ctx, segmented):
     state = [x.split("state=")[1].split()[0] for x in (before, held, after, other)]
     assert state[0] == state[2] == state[3] != state[1]
     assert ["captured=1" in x for x in (before, held, after, other)] == [False, True, False, False]
+
+
+# entry point -> (launcher, arguments): one of each kind that waits
+WAITING = {
+    "merge_lit_by_val_chids": ("merge", lambda o: (None,) * 3 + (100,) + (None,) * 3 + (o,)),
+    "fuse_fill_literals": ("compact", lambda o: (None, None, 100, None, o)),
+    "compute_column_length": ("colen", lambda o: (None, None, 100, None, None, None, o)),
+    "stream_compaction": ("compact", lambda o: (None, None, 100, None, o)),
+    "decode_device": ("decode", lambda o: (None, 100, 3100, None, o)),
+    "encode_device": ("encode", lambda o: (None, 3100, None, 100, o)),
+}
+
+
+@pytest.mark.parametrize("ends", [True, False], ids=["fault", "unended"])
+@pytest.mark.parametrize("name", WAITING)
+def test_scan_state_is_cleared_after_a_fault(ctx, name, ends):
+    """A launch that reports a fault, or whose last block never came because the
+    state was not its own: an error, and a state the next launch can use."""
+    kernel, args = WAITING[name]
+    out = U64(77)
+    ctx.script(kernel, fault=2, result=5, ends=ends)
+    assert ctx.call(name, *args(ctypes.byref(out))) == EHIP
+    state = next(x for x in ctx.log() if x.startswith(kernel)).split("state=")[1].split()[0]
+    at = [i for i, x in enumerate(ctx.log()) if x.startswith(kernel)][-1]
+    words = [int(x.split("words=")[1]) for x in ctx.log()[at:] if x.startswith(f"fill {state} ")]
+    assert words and words[0] > 1000  # the counters and every status word
+    ctx.script(kernel, result=42)
+    assert ctx.call(name, *args(ctypes.byref(out))) == OK and out.value == 42
+
+
+@pytest.mark.parametrize("slot", ["decode", "encode"])
+@pytest.mark.parametrize("ends", [True, False], ids=["fault", "unended"])
+def test_combine_reports_either_half(ctx, slot, ends):
+    out = U64(0)
+    args = (ctypes.c_int(0), None, 50, None, 0, 3100, None, 100, ctypes.byref(out))
+    ctx.script(slot, fault=1, ends=ends)
+    assert ctx.call("combine_device", *args) == EHIP
+    ctx.script("encode", result=7)
+    assert ctx.call("combine_device", *args) == OK and out.value == 7
+
+
+def test_launches_of_nothing_wait_for_no_result(ctx):
+    out = U64(77)
+    assert ctx.call("stream_compaction", None, None, 0, None, ctypes.byref(out)) == OK
+    assert out.value == 0
+    assert ctx.call("decode_device", None, 0, 100, None, ctypes.byref(out)) == OK
+    ctx.script("encode", result=3)
+    assert ctx.call("combine_device", ctypes.c_int(1), None, 0, None, 0, 100, None, 9,
+                    ctypes.byref(out)) == OK and out.value == 3
