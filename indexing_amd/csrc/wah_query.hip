@@ -29,6 +29,7 @@ constexpr uint32_t kDecTile = kScanTileOf<kDecRows>;  // words per decode tile
 // Resident blocks per CU.
 constexpr int kDecBlocks = 2;
 constexpr int kEncBlocks = 4;  // 20.2 us for 2^27 rows; 2 and 3 blocks 24.5, 23.1 us
+static_assert(kRangeWords / kDecTile <= kScanStatusWords, "a status word per tile of any range");
 constexpr int query_waves_per_eu(int blocks) { return blocks * kScanWaves / 4; }
 
 __device__ __forceinline__ uint32_t word_chunks(uint32_t w) {
@@ -542,15 +543,18 @@ __global__ __launch_bounds__(kScanThreads, query_waves_per_eu(kDecBlocks)) void 
 // Starts a range query: locates the keys of the index in [lo, hi] (keys
 // ascend): range[0] = first key index >= lo, range[1] = first > hi, range[2] =
 // first word of key range[0], range[3] = one past the last word of key
-// range[1] - 1; the number of keys goes to host[3], of words to host[4].  Then
-// zeroes the row bitmap, or, for a range that decodes by slices, their table.
+// range[1] - 1; the number of keys goes to host[3], of words to host[4].  A range
+// of more than most_words words, which one whose offsets descend has too, takes
+// no words: the caller reports it.  Then zeroes the row bitmap, or, for a range
+// that decodes by slices, their table.
 // SLICES: whether it does is decided here, so every block locates the keys.
 template <bool SLICES>
 __global__ __launch_bounds__(kBlock) void k_q_range(
     const uint32_t* __restrict__ keys, const uint32_t* __restrict__ offsets,
     const uint32_t* __restrict__ lengths, uint64_t keycnt, uint32_t lo, uint32_t hi,
-    uint32_t* __restrict__ bitmap, uint64_t words, uint64_t* __restrict__ table,
-    uint64_t table_cap, uint32_t slices, uint32_t slice_span, ScanState* st, uint64_t* host) {
+    uint64_t most_words, uint32_t* __restrict__ bitmap, uint64_t words,
+    uint64_t* __restrict__ table, uint64_t table_cap, uint32_t slices, uint32_t slice_span,
+    ScanState* st, uint64_t* host) {
   __shared__ uint64_t s_at[2];
   const uint32_t t = threadIdx.x;
   uint64_t entries = 0;
@@ -561,23 +565,23 @@ __global__ __launch_bounds__(kBlock) void k_q_range(
       if (t % kWave == 0) s_at[t / kWave] = at;
     }
     __syncthreads();
-    const uint64_t a = s_at[0], b = s_at[1];
+    const uint64_t a = s_at[0], b = s_at[1] > a ? s_at[1] : a;  // (keys that descend: none)
     const uint64_t w0 = a < b ? offsets[a] : 0;
     const uint64_t w1 = a < b ? (uint64_t)offsets[b - 1] + lengths[b - 1] : 0;
+    const uint64_t found = w1 - w0;  // 2^33 at least if w1 < w0
+    const uint64_t len = found <= most_words ? found : 0;
     if (SLICES) {
       entries = (b - a) * slices;  // below 2^60: table_cap bounds it
-      if (w1 < w0 || w1 - w0 >= 1ull << 31 || w1 - w0 < kSliceWords * entries ||
-          entries > table_cap)
-        entries = 0;
+      if (len >= 1ull << 31 || len < kSliceWords * entries || entries > table_cap) entries = 0;
     }
     if (blockIdx.x == 0 && t == 0) {
       st->range[0] = a;
       st->range[1] = b;
       st->range[2] = w0;
-      st->range[3] = w1;
+      st->range[3] = w0 + len;
       st->slice_span = entries ? slice_span : 0u;
       __hip_atomic_store(&host[3], b - a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-      __hip_atomic_store(&host[4], w1 - w0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      __hip_atomic_store(&host[4], found, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
   }
   const uint64_t i0 = (uint64_t)blockIdx.x * kBlock + t, step = (uint64_t)gridDim.x * kBlock;
@@ -911,9 +915,9 @@ uint64_t range_table_entries(uint64_t keycnt, uint64_t nrows, uint32_t cus) {
 }
 
 void launch_range(const ScanRun& s, const uint32_t* keys, const uint32_t* offsets,
-                  const uint32_t* lengths, uint64_t keycnt, const uint32_t* words, uint32_t lo,
-                  uint32_t hi, uint32_t* bitmap, uint64_t nrows, uint64_t* table,
-                  uint64_t table_cap, hipStream_t st) {
+                  const uint32_t* lengths, uint64_t keycnt, const uint32_t* words,
+                  uint64_t most_words, uint32_t lo, uint32_t hi, uint32_t* bitmap, uint64_t nrows,
+                  uint64_t* table, uint64_t table_cap, hipStream_t st) {
   const uint64_t bw = (nrows + 31) / 32;
   uint64_t g = (bw + 4 * kBlock - 1) / (4 * kBlock);
   const uint32_t span = table_cap ? slice_span_of(nrows, s.cus) : 0u;
@@ -921,12 +925,12 @@ void launch_range(const ScanRun& s, const uint32_t* keys, const uint32_t* offset
   if (span) {
     g = g < 1 ? 1 : g > 1024 ? 1024 : g;
     hipLaunchKernelGGL(k_q_range<true>, dim3((uint32_t)g), dim3(kBlock), 0, st, keys, offsets,
-                       lengths, keycnt, lo, hi, bitmap, bw, table, table_cap, slices, span,
+                       lengths, keycnt, lo, hi, most_words, bitmap, bw, table, table_cap, slices, span,
                        s.state, s.host);
   } else {
     g = g < 1 ? 1 : g > 4096 ? 4096 : g;
     hipLaunchKernelGGL(k_q_range<false>, dim3((uint32_t)g), dim3(kBlock), 0, st, keys, offsets,
-                       lengths, keycnt, lo, hi, bitmap, bw, table, table_cap, slices, span,
+                       lengths, keycnt, lo, hi, most_words, bitmap, bw, table, table_cap, slices, span,
                        s.state, s.host);
   }
   // the words of the range are known on the device only: a full grid

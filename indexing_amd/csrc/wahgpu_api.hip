@@ -1809,8 +1809,8 @@ int wahgpu_query_range_device(wahgpu_ctx* c, const uint32_t* d_keys, const uint3
   uint64_t entries = 0;
   uint64_t* table = range_table(c, wah::range_table_entries(keycnt, nrows, c->cus), &entries);
   ORDERED(c);
-  wah::launch_range(scan_run(c, true), d_keys, d_offsets, d_lengths, keycnt, d_words, lo, hi, d_bitmap,
-                    nrows, table, entries, c->stream);
+  wah::launch_range(scan_run(c, true), d_keys, d_offsets, d_lengths, keycnt, d_words,
+                    wah::kRangeWords, lo, hi, d_bitmap, nrows, table, entries, c->stream);
   LAUNCHCHK(c);
   uint64_t unused;
   order_guard_.end();  // no host wait holds the device order
@@ -1818,6 +1818,8 @@ int wahgpu_query_range_device(wahgpu_ctx* c, const uint32_t* d_keys, const uint3
   if (rc) return rc;
   if (keys_matched) *keys_matched = c->scan_host[3];
   const uint64_t words = c->scan_host[4];
+  if (words > wah::kRangeWords)
+    return fail(c, WAHGPU_EINVAL, "the offsets of the range descend");
   return words ? arena_limit(c, scan_scratch_bytes(words) + align_up(words * 4)) : WAHGPU_OK;
 }
 

@@ -13,7 +13,7 @@ import pytest
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 HARNESS = os.path.join(ROOT, "tests", "api_harness")
 CSRC = os.path.join(ROOT, "indexing_amd", "csrc")
-OK, EHIP = 0, -3
+OK, EINVAL, ENOMEM, EHIP = 0, -1, -2, -3
 U64, VP = ctypes.c_uint64, ctypes.c_void_p
 
 
@@ -170,3 +170,19 @@ def test_launches_of_nothing_wait_for_no_result(ctx):
     ctx.script("encode", result=3)
     assert ctx.call("combine_device", ctypes.c_int(1), None, 0, None, 0, 100, None, 9,
                     ctypes.byref(out)) == OK and out.value == 3
+
+
+def query(ctx, keycnt=40, nrows=100_000, keys=None):
+    return ctx.call("query_range_device", None, None, None, keycnt, None, ctypes.c_uint32(0),
+                    ctypes.c_uint32(9), nrows, None, ctypes.byref(U64() if keys is None else keys))
+
+
+def test_range_whose_offsets_descend_is_refused(ctx):
+    """Its word count is negative: refused, never a launch over 2^64 words."""
+    for words in (-1, -2048, -(2**32 - 1)):
+        keys = U64()
+        ctx.script("range", extra=(3, 2**64 + words))
+        assert query(ctx, keys=keys) == EINVAL and keys.value == 3
+    assert all(" most=%d " % 2**33 in x for x in ctx.log() if x.startswith("range"))
+    ctx.script("range", extra=(3, 2**33 - 2))
+    assert query(ctx) == OK

@@ -195,3 +195,42 @@ def test_range_by_slices_of_words_that_builds_never_write(ctx, seed):
         want = np.unique(np.concatenate([rows[i] for i in take])) if take else np.zeros(0, np.int64)
         assert np.array_equal(bitmap_rows(u32(bm), n), want[want < n])
         assert m == len(take)
+
+
+@pytest.mark.parametrize("n", [100_000, SLICED + 31], ids=["small", "sliced"])
+@pytest.mark.parametrize("drop", [1, 2047, 5000, 1 << 31])
+def test_range_whose_offsets_descend_is_refused(ctx, n, drop):
+    """An index whose last key of the range ends before its first one begins:
+    refused with an empty bitmap (nothing of it is decoded); the same index in
+    order decodes."""
+    import ctypes
+
+    import torch
+
+    from indexing_amd import _ptr
+    words = dev(np.full(8000, 0x80000001, np.uint32))
+    keys = dev(np.arange(3, dtype=np.uint32))
+    lengths = dev(np.array([10, 10, 7], np.uint32))
+    first = drop + 7  # the last key ends `drop` words before it
+    good = [0, 10, 20]
+    bitmap = torch.full(((n + 31) // 32,), -1, dtype=torch.int32, device="cuda:0")
+    found = ctypes.c_uint64(0)
+    for offsets in ([first, 5, 0], good):
+        ctx._bind_stream()
+        print(f"[descend] n={n} offsets={offsets}", flush=True)
+        rc = ctx._lib.wahgpu_query_range_device(
+            ctx._h, _ptr(keys), _ptr(dev(np.array(offsets, np.uint32))), _ptr(lengths), 3,
+            _ptr(words), 0, 9, n, _ptr(bitmap), ctypes.byref(found))
+        assert found.value == 3
+        if offsets is good:
+            assert rc == 0 and np.array_equal(bitmap_rows(u32(bitmap), n), 31 * np.arange(10))
+        else:
+            assert rc == -1 and not bool(bitmap.any())
+
+
+def test_keys_that_descend_match_none(ctx):
+    words = dev(np.full(100, 0x80000001, np.uint32))
+    keys, offsets = dev(np.array([9, 5, 1], np.uint32)), dev(np.array([0, 1, 2], np.uint32))
+    for lo, hi in ((6, 7), (2, 3), (0, 9)):
+        bm, m = ctx.query_range_device(keys, offsets, dev(np.ones(3)), words, lo, hi, 1000)
+        assert 0 <= m <= 3 and set(bitmap_rows(u32(bm), 1000).tolist()) <= {0}
