@@ -1761,6 +1761,21 @@ int wahgpu_decode_device(wahgpu_ctx* c, const uint32_t* d_words, uint64_t len, u
 }
 
 namespace {
+// Arena bytes a range of `words` words counts as (see arena_limit), and the most
+// words that the arena allows: the device leaves a longer range undecoded, so a
+// call that is refused for its length has not written what it was refused.
+uint64_t range_bytes(uint64_t words) { return scan_scratch_bytes(words) + align_up(words * 4); }
+uint64_t range_words_limit(const wahgpu_ctx* c) {
+  uint64_t lo = 0, hi = wah::kRangeWords;  // the answer is in [lo, hi]
+  if (!c->fixed || range_bytes(hi) <= c->arena_cap) return hi;
+  while (lo < hi) {
+    const uint64_t mid = (lo + hi + 1) / 2;
+    if (range_bytes(mid) <= c->arena_cap) lo = mid;
+    else hi = mid - 1;
+  }
+  return lo;
+}
+
 // Scratch for the table of a range that decodes by slices: `want` entries, or
 // fewer (*got), down to none; the query does without it then.  A fixed arena
 // serves what it holds.  Else the context keeps a buffer of its own, so that a
@@ -1806,11 +1821,12 @@ int wahgpu_query_range_device(wahgpu_ctx* c, const uint32_t* d_keys, const uint3
   }
   int rc = arena_limit(c, align_up(4 * 8));
   if (rc) return rc;
+  const uint64_t most = range_words_limit(c);
   uint64_t entries = 0;
   uint64_t* table = range_table(c, wah::range_table_entries(keycnt, nrows, c->cus), &entries);
   ORDERED(c);
   wah::launch_range(scan_run(c, true), d_keys, d_offsets, d_lengths, keycnt, d_words,
-                    wah::kRangeWords, lo, hi, d_bitmap, nrows, table, entries, c->stream);
+                    most, lo, hi, d_bitmap, nrows, table, entries, c->stream);
   LAUNCHCHK(c);
   uint64_t unused;
   order_guard_.end();  // no host wait holds the device order
@@ -1820,7 +1836,7 @@ int wahgpu_query_range_device(wahgpu_ctx* c, const uint32_t* d_keys, const uint3
   const uint64_t words = c->scan_host[4];
   if (words > wah::kRangeWords)
     return fail(c, WAHGPU_EINVAL, "the offsets of the range descend");
-  return words ? arena_limit(c, scan_scratch_bytes(words) + align_up(words * 4)) : WAHGPU_OK;
+  return words > most ? arena_limit(c, range_bytes(words)) : WAHGPU_OK;
 }
 
 int wahgpu_encode_device(wahgpu_ctx* c, const uint32_t* d_bitmap, uint64_t nrows,

@@ -35,6 +35,7 @@ def lib(tmp_path_factory):
     x = ctypes.CDLL(so)
     x.fake_log.restype = ctypes.c_char_p
     x.fake_device_bytes.restype = U64
+    x.wahgpu_arena_bytes.restype = U64
     x.wahgpu_last_error.restype = ctypes.c_char_p
     x.wahgpu_stream.restype = VP
     return x
@@ -186,3 +187,27 @@ def test_range_whose_offsets_descend_is_refused(ctx):
     assert all(" most=%d " % 2**33 in x for x in ctx.log() if x.startswith("range"))
     ctx.script("range", extra=(3, 2**33 - 2))
     assert query(ctx) == OK
+
+
+@pytest.mark.parametrize("arena", [256, 4096, 8192, 1 << 20, (1 << 30) + 77, 1 << 36])
+def test_range_on_a_fixed_arena_is_refused_before_it_decodes(lib, arena):
+    """The device gets the most words that the arena allows (4 bytes each and 8
+    per 2048 of them, in blocks of 256), so a longer range decodes nothing."""
+    c = Ctx(lib, arena)
+    cap = int(lib.wahgpu_arena_bytes(c.h))
+
+    def needs(words):
+        up = lambda x: (x + 255) // 256 * 256  # noqa: E731
+        return up(2080 + (words + 2047) // 2048 * 8) + up(4 * words)
+    for words in (1, 5):
+        c.script("range", extra=(1, words))
+    query(c)
+    most = int(c.log()[-1].split("most=")[1].split()[0])
+    assert most == 2**33 or needs(most + 1) > cap
+    assert most == 0 or needs(most) <= cap
+    lib.fake_reset()
+    for words, want in ((0, OK), (most, OK), (most + 1, ENOMEM if most < 2**33 else EINVAL)):
+        keys = U64()
+        c.script("range", extra=(1, words))
+        assert query(c, keys=keys) == want and keys.value == 1
+    c.close()

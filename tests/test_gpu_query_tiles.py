@@ -234,3 +234,36 @@ def test_keys_that_descend_match_none(ctx):
     for lo, hi in ((6, 7), (2, 3), (0, 9)):
         bm, m = ctx.query_range_device(keys, offsets, dev(np.ones(3)), words, lo, hi, 1000)
         assert 0 <= m <= 3 and set(bitmap_rows(u32(bm), 1000).tolist()) <= {0}
+
+
+@pytest.mark.parametrize("n", [2_000_003, SLICED + 31], ids=["small", "sliced"])
+def test_range_on_a_fixed_arena_is_whole_or_untouched(ctx, n):
+    """In an arena of the bytes that a range's words count as, it decodes; in one
+    a step (2 MiB) short of them, or of a step, the call is refused with the
+    bitmap empty and the keys counted."""
+    import ctypes
+
+    import torch
+
+    import indexing_amd as ia
+    from indexing_amd import _ptr
+    step = 2 << 20
+    rng = np.random.default_rng(n)
+    v = rng.integers(0, 60, n).astype(np.uint32)
+    idx = ctx.build(v)
+    k, o, ln, w = (dev(x) for x in (idx.keys, idx.offsets, idx.lengths, idx.words))
+    words = int(idx.lengths[5:41].sum())
+    need = -(-(2080 + -(-words // 2048) * 8) // 256) * 256 + -(-4 * words // 256) * 256
+    assert need > step
+    for arena, room in ((need, True), (need // step * step, need % step == 0), (step, False)):
+        with ia.Context(0, arena_bytes=arena) as q:
+            bitmap = torch.full(((n + 31) // 32,), -1, dtype=torch.int32, device="cuda:0")
+            found = ctypes.c_uint64(0)
+            q._bind_stream()
+            print(f"[fixed] n={n} need={need} arena={q.arena_bytes()}", flush=True)
+            rc = q._lib.wahgpu_query_range_device(q._h, _ptr(k), _ptr(o), _ptr(ln), k.numel(),
+                                                  _ptr(w), 5, 40, n, _ptr(bitmap),
+                                                  ctypes.byref(found))
+            assert found.value == 36 and (rc == 0) == room
+            want = np.flatnonzero((v >= 5) & (v <= 40)) if room else np.zeros(0, np.int64)
+            assert np.array_equal(bitmap_rows(u32(bitmap), n), want)
