@@ -360,14 +360,14 @@ void launch_decode(const ScanRun& s, const DecodeStream& a, const DecodeStream& 
                    hipStream_t st);
 // Zeroes the bitmap and decodes the keys in [lo, hi] into it; host[3] = keys,
 // host[4] = words of the range, of which nothing is decoded if they are more than
-// most_words (kRangeWords at most: what the status words hold).  table: scratch of table_cap entries for a
-// range that decodes by slices (range_table_entries at most are used).
-uint64_t range_table_entries(uint64_t keycnt, uint64_t nrows, uint32_t cus);
+// most_words (kRangeWords at most: what the status words hold).  table: scratch of
+// table_cap entries for a range that decodes by slices; grow: one that needs more
+// (range_wants of wah_slices.h) decodes nothing.
 constexpr uint64_t kRangeWords = 1ull << 33;  // 32-bit offset plus 32-bit length
 void launch_range(const ScanRun& s, const uint32_t* keys, const uint32_t* offsets,
                   const uint32_t* lengths, uint64_t keycnt, const uint32_t* words,
                   uint64_t most_words, uint32_t lo, uint32_t hi, uint32_t* bitmap, uint64_t nrows,
-                  uint64_t* table, uint64_t table_cap, hipStream_t st);
+                  uint64_t* table, uint64_t table_cap, bool grow, hipStream_t st);
 // The result is the words of the stream (b null: of bitmap a alone).
 void launch_encode(const ScanRun& s, const uint32_t* a, const uint32_t* b, int op, uint64_t nrows,
                    uint32_t* out, uint64_t cap, hipStream_t st);

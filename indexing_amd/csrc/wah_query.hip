@@ -15,6 +15,7 @@
 #include <type_traits>
 
 #include "wah_scan.h"
+#include "wah_slices.h"
 
 namespace wah {
 
@@ -128,33 +129,7 @@ __device__ __forceinline__ uint64_t wave_lower_bound(const uint32_t* __restrict_
 
 namespace {
 
-// Slices of a range's bitmap, one block each: as many as CUs or a multiple of
-// that (264 of 8192 chunks took 44 us for 2^26 rows, 256 of 8480 35: 8 CUs had
-// two), of up to kSliceMax chunks.  A range of an index of 2^22 rows or more
-// (below that the ORs it replaces take about what its launch does) decodes by
-// slices if its words are kSliceWords or more per entry of the table: a wave
-// works through a slice's part of a key in steps of 128 words, full or not.
-// Slices / ORs: 18 words per entry (2800 keys of 2^26 rows) 179 / 283 us, 15
-// (1800 of 2^24) 125 / 156, 13 (12000 of 2^26) 614 / 782, 10 (1000 of 2^26)
-// 83 / 81, 8 (410 of 2^22) 52 / 45; 130 (410 of 2^26) 84 / 281.
-constexpr uint32_t kSliceMax = 10240;
 constexpr int kSliceThreads = 1024;
-constexpr uint64_t kSliceMinRows = 1ull << 22;
-constexpr uint64_t kSliceWords = 12;
-// Chunks per slice: a multiple of 32, so that a slice is whole bitmap words.
-uint32_t slice_span_of(uint64_t nrows, uint32_t cus) {
-  if (nrows < kSliceMinRows) return 0;
-  const uint64_t chunks = (nrows + 30) / 31, each = (uint64_t)cus * kSliceMax;
-  const uint64_t slices = (chunks + each - 1) / each * cus;
-  return (uint32_t)((chunks + slices * 32 - 1) / (slices * 32)) * 32;
-}
-uint64_t slices_of(uint64_t nrows, uint32_t span) { return ((nrows + 30) / 31 + span - 1) / span; }
-static_assert(kSliceMax % 32 == 0, "a slice's span is rounded up to it at most");
-
-}  // namespace
-
-namespace {
-
 constexpr int kEnterRows = 4;  // tiles of 8192 words
 constexpr uint32_t kEnterTile = kScanTileOf<kEnterRows>;
 
@@ -546,7 +521,9 @@ __global__ __launch_bounds__(kScanThreads, query_waves_per_eu(kDecBlocks)) void 
 // range[1] - 1; the number of keys goes to host[3], of words to host[4].  A range
 // of more than most_words words, which one whose offsets descend has too, takes
 // no words: the caller reports it.  Then zeroes the row bitmap, or, for a range
-// that decodes by slices, their table.
+// that decodes by slices, their table; one whose table would be larger than
+// table_cap takes no words either if `grow`, and leaves the bitmap: the caller
+// comes back with a table of that size.
 // SLICES: whether it does is decided here, so every block locates the keys.
 template <bool SLICES>
 __global__ __launch_bounds__(kBlock) void k_q_range(
@@ -554,10 +531,11 @@ __global__ __launch_bounds__(kBlock) void k_q_range(
     const uint32_t* __restrict__ lengths, uint64_t keycnt, uint32_t lo, uint32_t hi,
     uint64_t most_words, uint32_t* __restrict__ bitmap, uint64_t words,
     uint64_t* __restrict__ table, uint64_t table_cap, uint32_t slices, uint32_t slice_span,
-    ScanState* st, uint64_t* host) {
+    bool grow, ScanState* st, uint64_t* host) {
   __shared__ uint64_t s_at[2];
   const uint32_t t = threadIdx.x;
   uint64_t entries = 0;
+  bool later = false;  // with a larger table
   if (SLICES || blockIdx.x == 0) {
     if (t < 2 * kWave) {
       const uint64_t v = t < kWave ? (uint64_t)lo : (uint64_t)hi + 1;
@@ -569,10 +547,14 @@ __global__ __launch_bounds__(kBlock) void k_q_range(
     const uint64_t w0 = a < b ? offsets[a] : 0;
     const uint64_t w1 = a < b ? (uint64_t)offsets[b - 1] + lengths[b - 1] : 0;
     const uint64_t found = w1 - w0;  // 2^33 at least if w1 < w0
-    const uint64_t len = found <= most_words ? found : 0;
+    uint64_t len = found <= most_words ? found : 0;
     if (SLICES) {
-      entries = (b - a) * slices;  // below 2^60: table_cap bounds it
-      if (len >= 1ull << 31 || len < kSliceWords * entries || entries > table_cap) entries = 0;
+      entries = slice_entries(b - a, len, slices);
+      if (entries > table_cap) {
+        later = grow;
+        entries = 0;
+        if (later) len = 0;
+      }
     }
     if (blockIdx.x == 0 && t == 0) {
       st->range[0] = a;
@@ -585,6 +567,7 @@ __global__ __launch_bounds__(kBlock) void k_q_range(
     }
   }
   const uint64_t i0 = (uint64_t)blockIdx.x * kBlock + t, step = (uint64_t)gridDim.x * kBlock;
+  if (later) return;
   if (SLICES && entries) {
     for (uint64_t i = i0; i < entries; i += step) table[i] = 0;
     return;
@@ -906,18 +889,10 @@ void launch_decode(const ScanRun& s, const DecodeStream& a, const DecodeStream& 
                      s.state, s.status, s.host);
 }
 
-uint64_t range_table_entries(uint64_t keycnt, uint64_t nrows, uint32_t cus) {
-  const uint32_t span = slice_span_of(nrows, cus);
-  if (!span) return 0;
-  const uint64_t all = keycnt * slices_of(nrows, span);
-  const uint64_t most = 2 * nrows / kSliceWords;  // (a row takes two words at most)
-  return all < most ? all : most;
-}
-
 void launch_range(const ScanRun& s, const uint32_t* keys, const uint32_t* offsets,
                   const uint32_t* lengths, uint64_t keycnt, const uint32_t* words,
                   uint64_t most_words, uint32_t lo, uint32_t hi, uint32_t* bitmap, uint64_t nrows,
-                  uint64_t* table, uint64_t table_cap, hipStream_t st) {
+                  uint64_t* table, uint64_t table_cap, bool grow, hipStream_t st) {
   const uint64_t bw = (nrows + 31) / 32;
   uint64_t g = (bw + 4 * kBlock - 1) / (4 * kBlock);
   const uint32_t span = table_cap ? slice_span_of(nrows, s.cus) : 0u;
@@ -926,12 +901,12 @@ void launch_range(const ScanRun& s, const uint32_t* keys, const uint32_t* offset
     g = g < 1 ? 1 : g > 1024 ? 1024 : g;
     hipLaunchKernelGGL(k_q_range<true>, dim3((uint32_t)g), dim3(kBlock), 0, st, keys, offsets,
                        lengths, keycnt, lo, hi, most_words, bitmap, bw, table, table_cap, slices, span,
-                       s.state, s.host);
+                       grow, s.state, s.host);
   } else {
     g = g < 1 ? 1 : g > 4096 ? 4096 : g;
     hipLaunchKernelGGL(k_q_range<false>, dim3((uint32_t)g), dim3(kBlock), 0, st, keys, offsets,
                        lengths, keycnt, lo, hi, most_words, bitmap, bw, table, table_cap, slices, span,
-                       s.state, s.host);
+                       grow, s.state, s.host);
   }
   // the words of the range are known on the device only: a full grid
   hipLaunchKernelGGL(k_q_decode<true>, dim3(s.cus * kDecBlocks), dim3(kScanThreads), 0, st,

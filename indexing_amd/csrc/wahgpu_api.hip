@@ -16,6 +16,7 @@
 
 #include "wah_internal.h"
 #include "wah_kernels.h"
+#include "wah_slices.h"
 #include "wahgpu.h"
 
 using wah::BuildArgs;
@@ -1776,13 +1777,14 @@ uint64_t range_words_limit(const wahgpu_ctx* c) {
   return lo;
 }
 
-// Scratch for the table of a range that decodes by slices: `want` entries, or
-// fewer (*got), down to none; the query does without it then.  A fixed arena
-// serves what it holds.  Else the context keeps a buffer of its own, so that a
+// Scratch for the table of a range that decodes by slices: `want` entries or more
+// (*got), or none; the query does without it then.  A fixed arena
+// serves what it holds (a range that it allows needs less: 8 bytes per
+// kSliceWords words).  Else the context keeps a buffer of its own, so that a
 // query never moves the arena, which a caller's captured builds may point into.
 uint64_t* range_table(wahgpu_ctx* c, uint64_t want, uint64_t* got) {
   if (c->fixed) {
-    *got = std::min<uint64_t>(want, c->arena_cap / 8);
+    *got = c->arena_cap / 8;
     return reinterpret_cast<uint64_t*>(c->arena);
   }
   if (want > c->table_cap) {
@@ -1800,7 +1802,7 @@ uint64_t* range_table(wahgpu_ctx* c, uint64_t want, uint64_t* got) {
     }
     c->table_cap = cap / 8;
   }
-  *got = want;
+  *got = c->table_cap;
   return c->table;
 }
 }  // namespace
@@ -1822,16 +1824,24 @@ int wahgpu_query_range_device(wahgpu_ctx* c, const uint32_t* d_keys, const uint3
   int rc = arena_limit(c, align_up(4 * 8));
   if (rc) return rc;
   const uint64_t most = range_words_limit(c);
+  // The table has a size for most ranges at first; one that needs more comes
+  // back for its own, without one if that is not to be had.
   uint64_t entries = 0;
-  uint64_t* table = range_table(c, wah::range_table_entries(keycnt, nrows, c->cus), &entries);
-  ORDERED(c);
-  wah::launch_range(scan_run(c, true), d_keys, d_offsets, d_lengths, keycnt, d_words,
-                    most, lo, hi, d_bitmap, nrows, table, entries, c->stream);
-  LAUNCHCHK(c);
-  uint64_t unused;
-  order_guard_.end();  // no host wait holds the device order
-  rc = scan_result(c, &unused);
-  if (rc) return rc;
+  uint64_t* table = range_table(c, wah::range_table_first(keycnt, nrows, c->cus), &entries);
+  for (bool grow = table && !c->fixed;; grow = false) {
+    {
+      ORDERED(c);
+      wah::launch_range(scan_run(c, true), d_keys, d_offsets, d_lengths, keycnt, d_words, most, lo,
+                        hi, d_bitmap, nrows, table, entries, grow, c->stream);
+      LAUNCHCHK(c);
+    }  // no host wait holds the device order
+    uint64_t unused;
+    rc = scan_result(c, &unused);
+    if (rc) return rc;
+    const uint64_t want = wah::range_wants(c->scan_host[3], c->scan_host[4], nrows, c->cus);
+    if (!grow || want <= entries) break;
+    table = range_table(c, want, &entries);
+  }
   if (keys_matched) *keys_matched = c->scan_host[3];
   const uint64_t words = c->scan_host[4];
   if (words > wah::kRangeWords)

@@ -210,14 +210,11 @@ void launch_decode(const ScanRun& s, const DecodeStream& a, const DecodeStream& 
                    hipStream_t) {
   scan("decode", s, a.len + b.len, true);
 }
-uint64_t range_table_entries(uint64_t keycnt, uint64_t nrows, uint32_t) {
-  return nrows < (1ull << 22) ? 0 : keycnt * 256;
-}
 void launch_range(const ScanRun& s, const uint32_t*, const uint32_t*, const uint32_t*, uint64_t,
                   const uint32_t*, uint64_t most_words, uint32_t, uint32_t, uint32_t*,
-                  uint64_t nrows, uint64_t*, uint64_t table_cap, hipStream_t) {
-  note("range nrows=%llu most=%llu table=%llu", (unsigned long long)nrows,
-       (unsigned long long)most_words, (unsigned long long)table_cap);
+                  uint64_t nrows, uint64_t* table, uint64_t table_cap, bool grow, hipStream_t) {
+  note("range nrows=%llu most=%llu table=%llu grow=%d", (unsigned long long)nrows,
+       (unsigned long long)most_words, table ? (unsigned long long)table_cap : 0ull, grow);
   const Script x = next("range");
   s.host[3] = x.extra[0];
   s.host[4] = x.extra[1];

@@ -211,3 +211,48 @@ def test_range_on_a_fixed_arena_is_refused_before_it_decodes(lib, arena):
         c.script("range", extra=(1, words))
         assert query(c, keys=keys) == want and keys.value == 1
     c.close()
+
+
+def launched(ctx):
+    """Table entries and `grow` of the range launches so far."""
+    lines = [x for x in ctx.log() if x.startswith("range")]
+    return [(int(x.split("table=")[1].split()[0]), int(x.split("grow=")[1])) for x in lines]
+
+
+def test_range_table_is_bounded_by_what_ranges_need(ctx):
+    """An index of many keys and rows: a query brings 8 MB whatever its range
+    could need, and keeps more only for a range that decodes by it."""
+    start = ctx.lib.fake_device_bytes()
+    for extra in ((3, 100), (10**6, 5 * 10**7), (0, 0)):  # few words, few per key and slice, none
+        ctx.script("range", extra=extra)
+        assert query(ctx, keycnt=10**8, nrows=2**32) == OK
+    assert launched(ctx) == [(2**20, 1)] * 3
+    assert ctx.lib.fake_device_bytes() - start == 8 << 20
+
+
+def test_range_comes_back_for_a_larger_table(ctx):
+    nrows, keys = 2**24, 5000
+    slices = 256  # one per CU up to 10240 chunks each
+    words = 13 * keys * slices
+    start = ctx.lib.fake_device_bytes()
+    for _ in range(2):  # the launch that finds it too small, then the one that decodes
+        ctx.script("range", extra=(keys, words))
+    assert query(ctx, keycnt=2 * keys, nrows=nrows) == OK
+    (first, grow), (second, again) = launched(ctx)
+    assert (first, grow, again) == (2**20, 1, 0) and second >= 0.99 * keys * slices
+    held = ctx.lib.fake_device_bytes() - start
+    assert held == 8 * second < words  # 8 bytes for 13 words
+    ctx.script("range", extra=(keys, words))  # the table is kept
+    assert query(ctx, keycnt=2 * keys, nrows=nrows) == OK
+    assert launched(ctx)[2:] == [(second, 1)]
+
+
+def test_range_does_without_a_table_it_cannot_have(ctx):
+    keys, words = U64(), 13 * 256 * 9000
+    ctx.script("range", extra=(1, 1))
+    assert query(ctx, keycnt=10**6, nrows=2**24) == OK  # the first one is there
+    ctx.lib.fake_most_bytes(u64(9 << 20))
+    for _ in range(2):
+        ctx.script("range", extra=(9000, words))
+    assert query(ctx, keycnt=10**6, nrows=2**24, keys=keys) == OK and keys.value == 9000
+    assert launched(ctx)[1:] == [(2**20, 1), (0, 0)]

@@ -267,3 +267,25 @@ def test_range_on_a_fixed_arena_is_whole_or_untouched(ctx, n):
             assert found.value == 36 and (rc == 0) == room
             want = np.flatnonzero((v >= 5) & (v <= 40)) if room else np.zeros(0, np.int64)
             assert np.array_equal(bitmap_rows(u32(bitmap), n), want)
+
+
+@pytest.mark.parametrize("arena", [0, 1 << 28], ids=["grows", "fixed"])
+def test_range_of_more_keys_than_the_first_table_holds(arena):
+    """5000 keys of 2^24 rows need 1.28 million entries, the first table has 2^20:
+    the range comes back for its own; narrower ones before and after it."""
+    import torch
+
+    import indexing_amd as ia
+    n, card = 1 << 24, 5003
+    g = torch.Generator(device="cuda:0").manual_seed(5)
+    v = torch.randint(0, card, (n,), device="cuda:0", generator=g, dtype=torch.int32)
+    with ia.Context(0) as c, ia.Context(0, arena_bytes=arena) as q:
+        k, o, ln, w, counts = c.build_device(v)
+        m, L = c.read_counts(counts).keycnt, c.read_counts(counts).length
+        for lo, hi in ((7, 300), (2, 5001), (2, 5001), (4000, 4800), (17, 17)):
+            print(f"[range] card={card} arena={arena} [{lo}, {hi}]", flush=True)
+            bm, keys = q.query_range_device(k[:m], o[:m], ln[:m], w[:L], lo, hi, n)
+            sel = ((v >= lo) & (v <= hi)).to(torch.int64).view(-1, 32)
+            want = (sel << torch.arange(32, device="cuda:0")).sum(1)
+            assert bool((bm.to(torch.int64) & 0xFFFFFFFF == want).all())
+            assert keys == hi - lo + 1
