@@ -285,8 +285,8 @@ __host__ __device__ inline uint32_t hist_chunks_of(uint64_t n) {
 
 // State of the single-pass scans (wah_scan.hip), one per context: zero before
 // every launch, and zeroed again by the launch's last block.  The status words
-// (kScanStatusWords of them) follow it.  Launches that are captured into a graph
-// use another one, kGraphStatusWords long, which the graph zeroes first: replays
+// (the context's scan_words) follow it.  Launches that are captured into a graph
+// use another one, which the graph zeroes first: replays
 // are outside the order of the context's calls, and blocks of two launches that
 // counted themselves in one state would leave it spoiled for every later call.
 struct ScanState {
@@ -300,12 +300,11 @@ struct ScanState {
   uint32_t pad[51];
 };
 static_assert(sizeof(ScanState) % 256 == 0, "status words follow at a line boundary");
-// Tiles of the longest scan: two streams of 2^32 WAH words in decode tiles of
-// 4096.
-constexpr uint64_t kScanStatusWords = 1ull << 21;
-// Tiles of the longest scan that can be captured: 2^30 elements in segmented
-// tiles of 8192.
-constexpr uint64_t kGraphStatusWords = 1ull << 17;
+// Status words a context starts with, and those of its graphs' state: a word per
+// tile of the longest scan, 2^30 elements in segmented tiles of 8192.  Only a
+// decode or range of more than 2^29 words needs more.
+constexpr uint64_t kScanStatusWords = 1ull << 17;
+constexpr uint64_t kDecodeTileWords = 4096;  // words per status word of a decode or range
 struct ScanRun {
   ScanState* state;
   uint64_t* status;
@@ -360,7 +359,7 @@ void launch_decode(const ScanRun& s, const DecodeStream& a, const DecodeStream& 
                    hipStream_t st);
 // Zeroes the bitmap and decodes the keys in [lo, hi] into it; host[3] = keys,
 // host[4] = words of the range, of which nothing is decoded if they are more than
-// most_words (kRangeWords at most: what the status words hold).  table: scratch of
+// most_words (kDecodeTileWords per status word at most).  table: scratch of
 // table_cap entries for a range that decodes by slices; grow: one that needs more
 // (range_wants of wah_slices.h) decodes nothing.
 constexpr uint64_t kRangeWords = 1ull << 33;  // 32-bit offset plus 32-bit length

@@ -30,7 +30,7 @@ constexpr uint32_t kDecTile = kScanTileOf<kDecRows>;  // words per decode tile
 // Resident blocks per CU.
 constexpr int kDecBlocks = 2;
 constexpr int kEncBlocks = 4;  // 20.2 us for 2^27 rows; 2 and 3 blocks 24.5, 23.1 us
-static_assert(kRangeWords / kDecTile <= kScanStatusWords, "a status word per tile of any range");
+static_assert(kDecTile == kDecodeTileWords, "what the host counts status words by");
 constexpr int query_waves_per_eu(int blocks) { return blocks * kScanWaves / 4; }
 
 __device__ __forceinline__ uint32_t word_chunks(uint32_t w) {
@@ -132,6 +132,7 @@ namespace {
 constexpr int kSliceThreads = 1024;
 constexpr int kEnterRows = 4;  // tiles of 8192 words
 constexpr uint32_t kEnterTile = kScanTileOf<kEnterRows>;
+static_assert(kEnterTile >= kDecTile, "a range has no more of these");
 
 // A range that decodes by slices: one pass over its words, as k_q_decode<true>
 // makes it (per key a scan of chunk counts, with look-back), that writes where
@@ -709,6 +710,7 @@ namespace {
 // 15872 rows and so whole bitmap words (496); a tile 4096 chunks, 3968 words.
 constexpr int kEncItems = 8;
 constexpr uint32_t kEncTile = kScanThreads * kEncItems;
+static_assert(((1ull << 32) + 30) / 31 <= kScanStatusWords * kEncTile, "2^32 rows");
 constexpr uint32_t kEncWaveWords = kWave * kEncItems * 31 / 32;
 constexpr uint32_t kEncWords = kEncWaveWords * kScanWaves;
 static_assert(kWave * kEncItems * 31 % 32 == 0 && kEncWords % 4 == 0, "whole words per wave");

@@ -613,9 +613,14 @@ __global__ __launch_bounds__(kBlock) void k_lengths(const uint32_t* __restrict__
 // ---- launchers ---------------------------------------------------------------
 
 namespace {
-static_assert(WAHGPU_MAX_VALUES <= kGraphStatusWords * kScanTileOf<kSegRows> &&
-                  kSegRows <= kScanRows && kSmallScan / kScanTileOf<kSmallRows> <= kGraphStatusWords,
-              "a captured scan's status words fit");
+constexpr int least(int a, int b) { return a < b ? a : b; }
+static_assert(WAHGPU_MAX_VALUES <=
+                      kScanStatusWords *
+                          kScanTileOf<least(least(kScanRows, kCompactRows),
+                                            least(least(kFuseRows, kSegRows),
+                                                  least(kMergeRows, kColenRows)))> &&
+                  kSmallScan / kScanTileOf<kSmallRows> <= kScanStatusWords,
+              "a status word per tile of every scan");
 struct Tiles {
   uint32_t count, grid;
 };

@@ -36,6 +36,7 @@ struct wahgpu_ctx {
   wahgpu_counts* pinned_counts = nullptr;  // host-pinned landing slot
   // state of the single-pass scans: zero between launches (see ScanState)
   wah::ScanState* scan_state = nullptr;
+  uint64_t scan_words = 0;                // its status words (scan_reserve)
   wah::ScanState* graph_state = nullptr;  // the same for captured scans (scan_run_async)
   uint64_t* table = nullptr;  // of a range by slices (range_table), table_cap entries
   uint64_t table_cap = 0;
@@ -352,7 +353,7 @@ int check_n(wahgpu_ctx* c, uint64_t n, uint32_t rid_base) {
 // (3 and 4), those of a decode whose encode follows (5 and 6), and the fault that
 // an asynchronous scan left, kept until a call that waits reports it.
 constexpr int kScanHostWords = 8, kDecodeSlot = 5, kKeptSlot = 7;
-constexpr uint64_t kScanStateBytes = sizeof(wah::ScanState) + wah::kScanStatusWords * 8;
+uint64_t scan_state_bytes(uint64_t words) { return sizeof(wah::ScanState) + words * 8; }
 
 // A scan that is over and whose last block has not reported: its launch shared
 // the state with another one, or found it spoiled.
@@ -360,7 +361,28 @@ constexpr uint64_t kScanUnended = 1ull << 32;
 
 // After a fault: the state may not be what the next launch needs.
 void reset_scan_state(wahgpu_ctx* c) {
-  wah::launch_fill32(reinterpret_cast<uint32_t*>(c->scan_state), kScanStateBytes / 4, 0, c->stream);
+  wah::launch_fill32(reinterpret_cast<uint32_t*>(c->scan_state), scan_state_bytes(c->scan_words) / 4,
+                     0, c->stream);
+}
+// Scan state of `words` status words at least.
+int scan_reserve(wahgpu_ctx* c, uint64_t words) {
+  if (words <= c->scan_words) return WAHGPU_OK;
+  HIPCHK(c, hipStreamSynchronize(c->stream));
+  wah::ScanState* more = nullptr;
+  if (hipMalloc(&more, scan_state_bytes(words)) != hipSuccess) {
+    (void)hipGetLastError();
+    return fail(c, WAHGPU_ENOMEM, "hipMalloc of " + std::to_string(scan_state_bytes(words)) +
+                                      " bytes failed");
+  }
+  if (c->scan_state) (void)hipFree(c->scan_state);
+  c->scan_state = more;
+  c->scan_words = words;
+  reset_scan_state(c);
+  LAUNCHCHK(c);
+  return WAHGPU_OK;
+}
+uint64_t decode_tiles(uint64_t words) {
+  return (words + wah::kDecodeTileWords - 1) / wah::kDecodeTileWords;
 }
 
 // Waits for the stream; reports the fault of an earlier scan that nobody waited
@@ -547,14 +569,13 @@ int wahgpu_create(wahgpu_ctx** out, int device_ordinal, uint64_t arena_bytes) {
   }
   c->stream = c->own_stream;
   if (hipHostMalloc(reinterpret_cast<void**>(&c->scan_host), kScanHostWords * 8, hipHostMallocDefault) != hipSuccess ||
-      hipMalloc(&c->scan_state, kScanStateBytes) != hipSuccess ||
-      hipMalloc(&c->graph_state, sizeof(wah::ScanState) + wah::kGraphStatusWords * 8) != hipSuccess) {
+      scan_reserve(c, wah::kScanStatusWords) != WAHGPU_OK ||
+      hipMalloc(&c->graph_state, scan_state_bytes(wah::kScanStatusWords)) != hipSuccess) {
     (void)hipGetLastError();
     wahgpu_destroy(c);
     return WAHGPU_EHIP;
   }
   memset(c->scan_host, 0, kScanHostWords * 8);
-  reset_scan_state(c);
   if (noalloc_lookup(c, device_ordinal) != WAHGPU_OK) {
     (void)hipGetLastError();
     wahgpu_destroy(c);
@@ -1749,6 +1770,8 @@ int wahgpu_decode_device(wahgpu_ctx* c, const uint32_t* d_words, uint64_t len, u
   HIPCHK(c, hipSetDevice(c->device));
   int rc = arena_limit(c, scan_scratch_bytes(len) + kAlign);
   if (rc) return rc;
+  rc = scan_reserve(c, decode_tiles(len));
+  if (rc) return rc;
   ORDERED(c);
   wah::launch_fill32(d_bitmap, bitmap_words(nrows), 0, c->stream);
   wah::launch_decode(scan_run(c, len > 0), {d_words, len, d_bitmap}, {nullptr, 0, nullptr}, nrows, c->stream);
@@ -1823,12 +1846,14 @@ int wahgpu_query_range_device(wahgpu_ctx* c, const uint32_t* d_keys, const uint3
   }
   int rc = arena_limit(c, align_up(4 * 8));
   if (rc) return rc;
-  const uint64_t most = range_words_limit(c);
-  // The table has a size for most ranges at first; one that needs more comes
-  // back for its own, without one if that is not to be had.
+  // The table and the status words have a size for most ranges at first; one
+  // that needs more of either has decoded nothing and comes back for its own,
+  // without a table if that is not to be had.
+  const uint64_t limit = range_words_limit(c);
+  uint64_t most = std::min(limit, c->scan_words * wah::kDecodeTileWords);
   uint64_t entries = 0;
   uint64_t* table = range_table(c, wah::range_table_first(keycnt, nrows, c->cus), &entries);
-  for (bool grow = table && !c->fixed;; grow = false) {
+  for (bool grow = table && !c->fixed;;) {
     {
       ORDERED(c);
       wah::launch_range(scan_run(c, true), d_keys, d_offsets, d_lengths, keycnt, d_words, most, lo,
@@ -1838,15 +1863,23 @@ int wahgpu_query_range_device(wahgpu_ctx* c, const uint32_t* d_keys, const uint3
     uint64_t unused;
     rc = scan_result(c, &unused);
     if (rc) return rc;
-    const uint64_t want = wah::range_wants(c->scan_host[3], c->scan_host[4], nrows, c->cus);
+    if (keys_matched) *keys_matched = c->scan_host[3];
+    const uint64_t found = c->scan_host[4];
+    if (found > most && found <= limit) {
+      rc = scan_reserve(c, decode_tiles(found));
+      if (rc) return rc;
+      most = std::min(limit, c->scan_words * wah::kDecodeTileWords);
+      continue;
+    }
+    const uint64_t want = wah::range_wants(c->scan_host[3], found, nrows, c->cus);
     if (!grow || want <= entries) break;
     table = range_table(c, want, &entries);
+    grow = false;
   }
-  if (keys_matched) *keys_matched = c->scan_host[3];
   const uint64_t words = c->scan_host[4];
   if (words > wah::kRangeWords)
     return fail(c, WAHGPU_EINVAL, "the offsets of the range descend");
-  return words > most ? arena_limit(c, range_bytes(words)) : WAHGPU_OK;
+  return words > limit ? arena_limit(c, range_bytes(words)) : WAHGPU_OK;
 }
 
 int wahgpu_encode_device(wahgpu_ctx* c, const uint32_t* d_bitmap, uint64_t nrows,
@@ -1885,6 +1918,8 @@ int wahgpu_combine_device(wahgpu_ctx* c, int op, const uint32_t* d_a, uint64_t l
   const uint64_t bw = bitmap_words(nrows);
   int rc = arena_reserve(c, 2 * align_up(bw * 4) + scan_scratch_bytes(la) +
                                 scan_scratch_bytes(lb) + encode_scratch_bytes(nrows) + kAlign);
+  if (rc) return rc;
+  rc = scan_reserve(c, decode_tiles(la) + decode_tiles(lb));
   if (rc) return rc;
   uint32_t* bm_a = take<uint32_t>(c, bw);
   uint32_t* bm_b = take<uint32_t>(c, bw);

@@ -289,3 +289,37 @@ def test_range_of_more_keys_than_the_first_table_holds(arena):
             want = (sel << torch.arange(32, device="cuda:0")).sum(1)
             assert bool((bm.to(torch.int64) & 0xFFFFFFFF == want).all())
             assert keys == hi - lo + 1
+
+
+def test_streams_of_more_words_than_a_context_starts_with():
+    """More than 2^29 words (0-fills of a chunk with literals among them): a decode
+    and ranges on either side of the slices grow the context's status words; the
+    scans before and after it are as ever."""
+    import torch
+
+    import indexing_amd as ia
+    total, half = (1 << 29) + 3 * 4096 + 5, (1 << 28) + 777
+    words = torch.ones(total, dtype=torch.int32, device="cuda:0")
+    at = torch.cat([torch.arange(0, 4000, 7), torch.tensor([40_000, 135_290, total - 1])])
+    lit = -0x80000000 + (1 << 30) + 1  # rows 0 and 30 of the chunk
+    words[at.to("cuda:0")] = lit
+    second = torch.tensor([3, 40_001, 135_299])  # of the second key
+    words[(half + second).to("cuda:0")] = lit
+
+    def rows(*chunks):
+        r = torch.cat([torch.cat([31 * c, 31 * c + 30]) for c in chunks])
+        return np.unique(r.numpy())
+    small = dev(np.arange(5000))
+    with ia.Context(0) as c:
+        for nrows in (100_000, SLICED + 5):
+            print(f"[long] decode and range, nrows={nrows}", flush=True)
+            assert int(c.exclusive_scan(small)[-1]) == 4999 * 4998 // 2
+            bm, last = c.decode_device(words, nrows)
+            want = rows(at)
+            assert np.array_equal(bitmap_rows(u32(bm), nrows), want[want < nrows])
+            assert last == 31 * total
+            keys, offsets = dev(np.array([4, 9])), dev(np.array([0, half]))
+            bm, m = c.query_range_device(keys, offsets, dev(np.array([half, total - half])), words,
+                                         0, 10, nrows)
+            want = rows(at[at < half], second)
+            assert m == 2 and np.array_equal(bitmap_rows(u32(bm), nrows), want[want < nrows])
