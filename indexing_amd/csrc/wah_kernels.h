@@ -168,9 +168,10 @@ static_assert(sizeof(Column) == 48, "descriptor layout");
 struct Dims {
   uint32_t ncols, sort_tiles, tail_tiles, hist_chunks;
   uint32_t wide_tiles;  // kWideTile tiles of the columns that may take wide digits
-  uint32_t pad;
+  uint32_t shorts;      // columns that one workgroup each builds
 };
-// Device descriptor: dims, padding, then ncols Columns.
+// Device descriptor: dims, padding, then ncols Columns, then the short ones (in
+// one region, so that a batch of both needs no more scratch than one of either).
 struct DescHead {
   Dims dims;
   uint32_t pad[2];
@@ -256,6 +257,7 @@ struct BuildArgs {
   // Upper bounds the grids are sized for (a captured graph replays any batch
   // within them; the kernels read the actual sizes from the descriptor).
   uint32_t cols_cap, sort_tiles_cap, tail_tiles_cap, hist_chunks_cap;
+  uint32_t shorts_cap;                  // short columns of the descriptor (launch_small)
   uint32_t wide_slots_cap, wide_tiles_cap;  // 0: no column may take wide digits
   uint64_t n_cap;
   // Every column sorts (value, rid) pairs (the stage API needs them).
@@ -325,7 +327,7 @@ void launch_sort(const BuildArgs& a, hipStream_t s, LaunchHook* hook = nullptr);
 void launch_tail(const BuildArgs& a, hipStream_t s, LaunchHook* hook = nullptr);
 void launch_sort_finalize(const BuildArgs& a, hipStream_t s);
 // The whole build of columns of at most kSmallMax rows: the inline column, or
-// those of the descriptor (cols_cap at most).  Uses no scratch.
+// the descriptor's short ones (shorts_cap at most).  Uses no scratch.
 void launch_small(const BuildArgs& a, hipStream_t s);
 // *ok must hold 1; stays 1 if LDS fetch-adds rank lanes in lane order here.
 void launch_rank_selftest(uint32_t* ok, hipStream_t s);

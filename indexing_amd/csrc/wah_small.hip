@@ -260,7 +260,7 @@ __device__ __forceinline__ void small_build(SmallShared& sh, const Column& cd, b
 
 }  // namespace
 
-// Block c builds column c of the descriptor (desc null: column `one`).
+// Block c builds short column c of the descriptor (desc null: column `one`).
 __global__ __launch_bounds__(kThreads, 4) void k_small(
     const DescHead* __restrict__ desc, Column one, int atomic_rank,
     const uint32_t* __restrict__ values, uint32_t* out_keys, uint32_t* out_offsets,
@@ -268,8 +268,8 @@ __global__ __launch_bounds__(kThreads, 4) void k_small(
   __shared__ SmallShared sh;
   Column cd = one;
   if (desc) {
-    if (blockIdx.x >= desc->dims.ncols) return;
-    cd = desc_cols(desc)[blockIdx.x];
+    if (blockIdx.x >= desc->dims.shorts) return;
+    cd = desc_cols(desc)[desc->dims.ncols + blockIdx.x];
   }
   if (cd.n == 0) {
     if (threadIdx.x == 0) counts[cd.index] = wahgpu_counts_dev{};
@@ -286,7 +286,7 @@ __global__ __launch_bounds__(kThreads, 4) void k_small(
 }
 
 void launch_small(const BuildArgs& a, hipStream_t s) {
-  hipLaunchKernelGGL(k_small, dim3(a.inline_desc ? 1u : a.cols_cap), dim3(kThreads), 0, s,
+  hipLaunchKernelGGL(k_small, dim3(a.inline_desc ? 1u : a.shorts_cap), dim3(kThreads), 0, s,
                      a.inline_desc ? nullptr : a.desc, a.one, (int)a.atomic_rank, a.values,
                      a.out_keys, a.out_offsets, a.out_lengths, a.out_words, a.counts);
 }

@@ -192,15 +192,16 @@ struct Caps {
   uint64_t n;  // values of the concatenated input (its highest end)
   uint32_t cols, sort_tiles, tail_tiles, hist_chunks;
   uint32_t wide_slots = 0, wide_tiles = 0;  // columns that may take wide digits, their tiles
+  uint32_t desc_cols = 0;                   // columns of a descriptor, the short ones too
   bool operator==(const Caps& o) const {
     return n == o.n && cols == o.cols && sort_tiles == o.sort_tiles &&
            tail_tiles == o.tail_tiles && hist_chunks == o.hist_chunks &&
-           wide_slots == o.wide_slots && wide_tiles == o.wide_tiles;
+           wide_slots == o.wide_slots && wide_tiles == o.wide_tiles && desc_cols == o.desc_cols;
   }
   bool covers(const Caps& o) const {
     return n >= o.n && cols >= o.cols && sort_tiles >= o.sort_tiles &&
            tail_tiles >= o.tail_tiles && hist_chunks >= o.hist_chunks &&
-           wide_slots >= o.wide_slots && wide_tiles >= o.wide_tiles;
+           wide_slots >= o.wide_slots && wide_tiles >= o.wide_tiles && desc_cols >= o.desc_cols;
   }
 };
 // Column-length bucket of n: < 2^14, < 2^17, < 2^20, the rest.
@@ -251,6 +252,7 @@ uint32_t wide_tiles_of(uint64_t n) { return (uint32_t)((n + wah::kWideTile - 1) 
 Caps caps_one(uint64_t n, int shape, bool wide = false) {
   Caps k{n, 1u, wah::sort_tiles_of(n, wah::radix_tile(shape)), wah::tail_tiles_of(n),
          wah::hist_chunks_of(n)};
+  k.desc_cols = 1;
   if (wide) {
     k.wide_slots = 1;
     k.wide_tiles = wide_tiles_of(n);
@@ -263,12 +265,12 @@ Caps caps_for(const wahgpu_ctx* c, uint64_t n) {
 }
 
 // Bytes of scratch a fused build needs (besides outputs), with `ndesc`
-// descriptor regions of k.cols columns each.
+// descriptor regions of k.desc_cols columns each.
 uint64_t build_scratch_bytes(const Caps& k, uint32_t ndesc = 1) {
   const uint64_t nn = k.n ? k.n : 1;
   uint64_t b = 0;
   b += 6 * align_up(nn * 4);                       // keys, rids and lits of A and B
-  b += ndesc * align_up(sizeof(wah::DescHead) + (uint64_t)k.cols * sizeof(wah::Column));
+  b += ndesc * align_up(sizeof(wah::DescHead) + (uint64_t)k.desc_cols * sizeof(wah::Column));
   b += align_up(sizeof(wah::Header));
   b += align_up((uint64_t)k.cols * sizeof(wah::ColState));
   b += align_up(2ull * k.sort_tiles * 256 * 4);
@@ -291,7 +293,7 @@ void carve_build(wahgpu_ctx* c, BuildArgs* a, const Caps& k, int shape) {
   a->litsA = take<uint32_t>(c, nn);
   a->litsB = take<uint32_t>(c, nn);
   a->desc = reinterpret_cast<wah::DescHead*>(
-      take<char>(c, sizeof(wah::DescHead) + (uint64_t)k.cols * sizeof(wah::Column)));
+      take<char>(c, sizeof(wah::DescHead) + (uint64_t)k.desc_cols * sizeof(wah::Column)));
   a->hdr = take<wah::Header>(c, 1);
   a->cs = take<wah::ColState>(c, k.cols);
   a->sort_status_stride = (uint64_t)k.sort_tiles * 256;
@@ -878,15 +880,15 @@ namespace {
 
 // One launch set of a batch: the columns whose length bucket maps to one
 // radix tile shape, with their descriptor (dims + columns with tile and
-// chunk prefixes in that shape's tiles) in host memory.
+// chunk prefixes in that shape's tiles) in host memory.  The first set's
+// descriptor carries the batch's short columns too, which take a workgroup each.
 struct SubBatch {
-  int shape;  // kSmallShape: columns of one workgroup each
+  int shape;
+  uint32_t cols, shorts;
   std::vector<char> desc;
   Caps caps;
 };
 
-constexpr int kSmallShape = wah::kRadixShapes;
-constexpr int kSubShapes = wah::kRadixShapes + 1;  // launch sets a batch may need
 // Short columns join the launch set of a batch's longer ones where they are one
 // for two CUs at most and the long ones have this many rows for each: there a
 // few tiles more per pass cost less than the launch of one workgroup per column,
@@ -897,15 +899,16 @@ constexpr int kSubShapes = wah::kRadixShapes + 1;  // launch sets a batch may ne
 // 2^14.2) 143 / 129.
 constexpr uint64_t kJoinRows = 1u << 15;
 
-// Validates the columns and splits them into sub-batches: the short ones, which
-// take a workgroup each, and the others by tile shape (all that the context
-// may use when `all_shapes`, empty ones included, so that a captured graph fits
-// any batch of the reservation).  *shared = element-wise maximum of the
-// sub-batches' caps (the scratch they share, one after another).
+// Validates the columns and splits them into sub-batches by tile shape (all that
+// the context may use when `all_shapes`, empty ones included, so that a captured
+// graph fits any batch of the reservation), with the short ones, which take a
+// workgroup each, in the first (which has no others if the batch has none).
+// *shared = element-wise maximum of the sub-batches' caps (the scratch they share,
+// one after another).
 int plan_batch(wahgpu_ctx* c, const wahgpu_column* cols, uint32_t ncols, uint64_t values_len,
                bool all_shapes, std::vector<SubBatch>* subs, Caps* shared) {
   uint64_t end = 0;
-  std::vector<uint32_t> members[kSubShapes];
+  std::vector<uint32_t> members[wah::kRadixShapes], shorts;
   // a captured graph has to fit any batch of the reservation, so its shape
   // goes by the reservation
   const bool table = c->tuned || c->force_shape >= 0;
@@ -929,38 +932,42 @@ int plan_batch(wahgpu_ctx* c, const wahgpu_column* cols, uint32_t ncols, uint64_
       return fail(c, WAHGPU_EINVAL, "column " + std::to_string(i) +
                                         " overlaps the previous one or exceeds values_len");
     end = col.offset + col.n;
-    members[small_ok(c, col.n) ? kSmallShape : table ? shape_for(c, col.n) : rule].push_back(i);
+    if (small_ok(c, col.n)) shorts.push_back(i);
+    else members[table ? shape_for(c, col.n) : rule].push_back(i);
   }
   if (join) {
     std::vector<uint32_t> rest;
-    for (uint32_t i : members[kSmallShape]) {
+    for (uint32_t i : shorts) {
       auto& m = members[table ? shape_for(c, cols[i].n) : rule];
       if (m.empty() || !cols[i].n) rest.push_back(i);
       else m.push_back(i);
     }
-    members[kSmallShape].swap(rest);
-    for (int sh = 0; sh < kSmallShape; ++sh) std::sort(members[sh].begin(), members[sh].end());
+    shorts.swap(rest);
+    for (auto& m : members) std::sort(m.begin(), m.end());
   }
   subs->clear();
   *shared = Caps{values_len, 0, 0, 0, 0};
-  bool tuned[kSubShapes] = {};
+  bool tuned[wah::kRadixShapes] = {};
   for (uint32_t b = 0; b < WAHGPU_TUNE_BUCKETS; ++b)
     tuned[table ? (int)c->tune_shape[b] : rule] = true;
-  tuned[kSmallShape] = true;
-  for (int sh = 0; sh < kSubShapes; ++sh) {
-    if (members[sh].empty() && !(all_shapes && tuned[sh])) continue;
+  bool any = all_shapes;  // a set for some column of more rows
+  for (const auto& m : members) any |= !m.empty();
+  for (int sh = 0; sh < wah::kRadixShapes; ++sh) {
+    if (members[sh].empty() && !(all_shapes && tuned[sh]) && !(!any && sh == 0)) continue;
     SubBatch sb;
     sb.shape = sh;
     const uint32_t m = (uint32_t)members[sh].size();
-    sb.desc.assign(sizeof(wah::DescHead) + (uint64_t)m * sizeof(wah::Column), 0);
+    sb.cols = m;
+    sb.shorts = subs->empty() ? (uint32_t)shorts.size() : 0u;
+    sb.desc.assign(sizeof(wah::DescHead) + (uint64_t)(m + sb.shorts) * sizeof(wah::Column), 0);
     auto* head = reinterpret_cast<wah::DescHead*>(sb.desc.data());
     wah::Column* dc = wah::desc_cols(head);
     uint64_t st = 0, tt = 0, hc = 0, wt = 0;
     uint32_t ws = 0;  // columns that may take wide digits, each with a WideState
-    const uint32_t tile = wah::radix_tile(sh);  // (a short column's counts are bounds only)
+    const uint32_t tile = wah::radix_tile(sh);
     for (uint32_t j = 0; j < m; ++j) {
       const wahgpu_column& col = cols[members[sh][j]];
-      const bool wide = sh != kSmallShape && wide_ok(c, col.n);
+      const bool wide = wide_ok(c, col.n);
       dc[j] = wah::Column{col.offset, col.n, col.rid_base, (uint32_t)st, (uint32_t)tt,
                           (uint32_t)hc, members[sh][j], wide ? ws + 1u : 0u, (uint32_t)wt, 0u};
       st += wah::sort_tiles_of(col.n, tile);
@@ -971,18 +978,24 @@ int plan_batch(wahgpu_ctx* c, const wahgpu_column* cols, uint32_t ncols, uint64_
         wt += wide_tiles_of(col.n);
       }
     }
+    for (uint32_t j = 0; j < sb.shorts; ++j) {
+      const wahgpu_column& col = cols[shorts[j]];
+      dc[m + j] = wah::Column{col.offset, col.n, col.rid_base, 0u, 0u, 0u, shorts[j], 0u, 0u, 0u};
+    }
     if (st > 0xFFFFFFF0ull || hc > 0xFFFFFFF0ull)
       return fail(c, WAHGPU_ERANGE, "batch too large for 32-bit tile numbering");
-    head->dims = wah::Dims{m, (uint32_t)st, (uint32_t)tt, (uint32_t)hc, (uint32_t)wt, 0u};
+    head->dims = wah::Dims{m, (uint32_t)st, (uint32_t)tt, (uint32_t)hc, (uint32_t)wt, sb.shorts};
     sb.caps = Caps{values_len, m, (uint32_t)st, (uint32_t)tt, (uint32_t)hc};
     sb.caps.wide_slots = ws;
     sb.caps.wide_tiles = (uint32_t)wt;
+    sb.caps.desc_cols = m + sb.shorts;
     shared->cols = std::max(shared->cols, m);
     shared->sort_tiles = std::max(shared->sort_tiles, (uint32_t)st);
     shared->tail_tiles = std::max(shared->tail_tiles, (uint32_t)tt);
     shared->hist_chunks = std::max(shared->hist_chunks, (uint32_t)hc);
     shared->wide_slots = std::max(shared->wide_slots, ws);
     shared->wide_tiles = std::max(shared->wide_tiles, (uint32_t)wt);
+    shared->desc_cols = std::max(shared->desc_cols, sb.caps.desc_cols);
     subs->push_back(std::move(sb));
   }
   return WAHGPU_OK;
@@ -1015,6 +1028,7 @@ Caps reserved_caps(const wahgpu_ctx* c) {
   Caps k{v, c->res_cols, (uint32_t)(v / min_tile + c->res_cols),
          (uint32_t)(v / wah::kTailTile + c->res_cols),
          (uint32_t)(v / wah::kHistChunk + c->res_cols)};
+  k.desc_cols = c->res_cols;
   bool wide = false;  // some bucket allows wide digits
   for (uint32_t b = 1; b < WAHGPU_TUNE_BUCKETS; ++b) wide |= c->tune_digits[b] == 11u;
   if (wide) {
@@ -1081,7 +1095,8 @@ int batch_device_impl(wahgpu_ctx* c, const uint32_t* d_values, uint64_t values_l
   for (size_t i = 0; i < subs.size(); ++i) {
     BuildArgs a = base;
     a.shape = subs[i].shape;
-    if (i > 0) a.desc = carve_desc(c, k.cols);
+    if (i > 0) a.desc = carve_desc(c, k.desc_cols);
+    a.shorts_cap = graph && i == 0 ? k.desc_cols : subs[i].shorts;
     a.inline_desc = false;
     a.values = d_values;
     a.out_keys = d_keys;
@@ -1107,10 +1122,7 @@ int batch_device_impl(wahgpu_ctx* c, const uint32_t* d_values, uint64_t values_l
       }
       HIPCHK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
       for (const BuildArgs& a : args) {
-        if (a.shape == kSmallShape) {
-          wah::launch_small(a, c->stream);
-          continue;
-        }
+        if (a.shorts_cap) wah::launch_small(a, c->stream);
         wah::launch_sort(a, c->stream);
         wah::launch_tail(a, c->stream);
       }
@@ -1132,12 +1144,13 @@ int batch_device_impl(wahgpu_ctx* c, const uint32_t* d_values, uint64_t values_l
     return WAHGPU_OK;
   }
   ORDERED(c);
-  for (const BuildArgs& a : args) {
-    if (a.shape == kSmallShape) {
+  for (size_t i = 0; i < args.size(); ++i) {
+    const BuildArgs& a = args[i];
+    if (a.shorts_cap) {
       wah::launch_small(a, c->stream);
       LAUNCHCHK(c);
-      continue;
     }
+    if (!subs[i].cols) continue;
     EventHook hook;
     EventHook* hp = nullptr;
     if (c->timing && c->tcalls < c->tmax && args.size() == 1) {
@@ -1732,9 +1745,10 @@ void wah_batch_acc_add(wah_batch_acc* acc, uint64_t n) {
 
 uint64_t wah_batch_acc_scratch(const wah_batch_acc* acc) {
   // one descriptor region per compiled tile shape: the most sub-batches
-  const Caps k{acc->values, acc->cols, (uint32_t)acc->sort_tiles, (uint32_t)acc->tail_tiles,
-               (uint32_t)acc->hist_chunks};
-  return build_scratch_bytes(k, kSubShapes);
+  Caps k{acc->values, acc->cols, (uint32_t)acc->sort_tiles, (uint32_t)acc->tail_tiles,
+         (uint32_t)acc->hist_chunks};
+  k.desc_cols = acc->cols;
+  return build_scratch_bytes(k, wah::kRadixShapes);
 }
 
 int wah_build_batch_ws(wahgpu_ctx* c, const uint32_t* d_values, uint64_t values_len,

@@ -181,7 +181,7 @@ void launch_tail(const BuildArgs& a, hipStream_t s, LaunchHook* hook) {
 }
 void launch_sort_finalize(const BuildArgs&, hipStream_t) { note("finalize"); }
 void launch_small(const BuildArgs& a, hipStream_t) {
-  note("small cols=%u", a.inline_desc ? 1u : a.cols_cap);
+  note("small cols=%u", a.inline_desc ? 1u : a.shorts_cap);
   g_clock += 100;
 }
 void launch_rank_selftest(uint32_t*, hipStream_t) {}

@@ -292,3 +292,55 @@ def test_a_context_holds_status_words_for_what_it_scans(lib):
     assert lib.fake_device_bytes() - start == held + 15 * 2**20  # 2^21 words in all
     c.close()
     assert lib.fake_device_bytes() == start
+
+
+class Column(ctypes.Structure):
+    _fields_ = [("offset", U64), ("n", U64), ("rid_base", ctypes.c_uint32),
+                ("reserved", ctypes.c_uint32)]
+
+
+def batch(ctx, lens):
+    cols, at = (Column * len(lens))(), 0
+    for c, n in zip(cols, lens):
+        c.offset, c.n = at, n
+        at += n
+    return ctx.call("build_batch_device", None, at, cols, ctypes.c_uint32(len(lens)), None, None,
+                    None, None, None)
+
+
+def test_a_reservation_that_fits_a_fixed_arena_builds_in_it(lib):
+    """What wahgpu_batch_reserve lays out is enough for batches of short and long
+    columns; no build asks for more than the reservation did."""
+    values, cols = 2**24, 65536
+    c = Ctx(lib)
+    assert c.call("batch_reserve", values, ctypes.c_uint32(cols)) == OK
+    need = int(lib.wahgpu_arena_bytes(c.h))
+    for lens in ([20000, 5], [5, 1000], [20000] * 3, [20000, 0] * 4):
+        assert batch(c, lens) == OK
+        assert int(lib.wahgpu_arena_bytes(c.h)) == need
+    c.close()
+    f = Ctx(lib, need)
+    assert f.call("batch_reserve", values, ctypes.c_uint32(cols)) == OK
+    for lens in ([20000, 5], [5, 1000], [20000] * 3, [20000, 0] * 4):
+        assert batch(f, lens) == OK, f.error()
+    assert f.log().count("graph") == 4
+    f.close()
+
+
+def test_short_columns_add_no_scratch_to_a_batch(lib):
+    """A batch whose last columns are short, or empty, fits where it fits with
+    long columns in their place."""
+    sizes = []
+    for last in (20000, 5, 0):
+        c = Ctx(lib)
+        assert batch(c, [20000] * 65536 + [last] * 200) == OK
+        sizes.append(int(lib.wahgpu_arena_bytes(c.h)))
+        launches = [x.split()[0] for x in c.log()]
+        assert launches == (["small"] if last < 20000 else []) + ["sort", "tail"]
+        c.close()
+    assert sizes[1] <= sizes[0] and sizes[2] <= sizes[0]
+
+
+def test_a_batch_of_short_columns_alone_is_one_launch(ctx):
+    assert batch(ctx, [5, 0, 16384, 1000]) == OK
+    assert ctx.log() == ["small cols=4"]
