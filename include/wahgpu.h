@@ -150,13 +150,16 @@ int wahgpu_build_device_noalloc(wahgpu_ctx* ctx, const uint32_t* d_values, uint6
                                 uint32_t* d_lengths, uint32_t* d_words,
                                 wahgpu_counts* d_counts);
 
-/* Per-kernel timing of wahgpu_build_device calls, for measurement: between
- * wahgpu_timing_begin and wahgpu_timing_end every build_device call records
- * HIP events around its kernels on the context's stream (at most max_calls
- * calls).  timing_end waits for them and writes, per kernel group, the summed
+/* Per-kernel timing of device builds, for measurement: between
+ * wahgpu_timing_begin and wahgpu_timing_end every build_device call, and every
+ * build_batch_device call that neither replays a graph nor mixes tile shapes,
+ * records HIP events around its kernels on the context's stream (at most
+ * max_calls calls).  timing_end waits for them and writes, per kernel group, the summed
  * milliseconds over the recorded calls:
  *   ms[0] histogram + digit scan, ms[1..4] radix passes of digits 0..3
- *   (inactive passes are near zero), ms[5] tail, ms[6] lengths.
+ *   (inactive passes are near zero), ms[5] tail, ms[6] lengths.  The build of
+ *   columns that one workgroup each makes (at most 2^14 values) is one launch
+ *   and counts as ms[0].
  * *calls receives the number of recorded calls. */
 #define WAHGPU_TIMING_GROUPS 7
 int wahgpu_timing_begin(wahgpu_ctx* ctx, uint32_t max_calls);

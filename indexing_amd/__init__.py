@@ -126,7 +126,8 @@ class Context:
         self._check(self._lib.wahgpu_synchronize(self._h))
 
     def timing_begin(self, max_calls):
-        """Record per-kernel HIP events for the next build_device calls."""
+        """Record per-kernel HIP events for the next build_device and (outside a
+        reservation) build_batch_device calls."""
         self._check(self._lib.wahgpu_timing_begin(self._h, int(max_calls)))
 
     def timing_end(self):

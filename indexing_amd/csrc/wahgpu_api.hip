@@ -1146,11 +1146,7 @@ int batch_device_impl(wahgpu_ctx* c, const uint32_t* d_values, uint64_t values_l
   ORDERED(c);
   for (size_t i = 0; i < args.size(); ++i) {
     const BuildArgs& a = args[i];
-    if (a.shorts_cap) {
-      wah::launch_small(a, c->stream);
-      LAUNCHCHK(c);
-    }
-    if (!subs[i].cols) continue;
+    // timed: batches of one launch set, whose short columns count as the first group
     EventHook hook;
     EventHook* hp = nullptr;
     if (c->timing && c->tcalls < c->tmax && args.size() == 1) {
@@ -1158,6 +1154,14 @@ int batch_device_impl(wahgpu_ctx* c, const uint32_t* d_values, uint64_t values_l
       hp = &hook;
       ++c->tcalls;
       hook.mark(c->stream);
+    }
+    if (a.shorts_cap) {
+      wah::launch_small(a, c->stream);
+      LAUNCHCHK(c);
+    }
+    if (!subs[i].cols) {
+      if (hp) hook.rest(c->stream);
+      continue;
     }
     wah::launch_sort(a, c->stream, hp);
     LAUNCHCHK(c);

@@ -344,3 +344,15 @@ def test_short_columns_add_no_scratch_to_a_batch(lib):
 def test_a_batch_of_short_columns_alone_is_one_launch(ctx):
     assert batch(ctx, [5, 0, 16384, 1000]) == OK
     assert ctx.log() == ["small cols=4"]
+
+
+def test_timing_covers_batches_of_short_and_long_columns(ctx):
+    """Each batch of one launch set is a timed call, short columns beside it or
+    alone; the short ones' launch (100 ticks of the harness's clock) is ms[0]."""
+    ms, calls = (ctypes.c_double * 7)(), ctypes.c_uint32(0)
+    assert ctx.call("timing_begin", ctypes.c_uint32(8)) == OK
+    for lens in ([20000] * 3, [5] * 200 + [40000], [20000, 0], [5, 1000]):
+        assert batch(ctx, lens) == OK
+    assert ctx.call("timing_end", ms, ctypes.byref(calls)) == OK
+    assert calls.value == 4
+    assert 300 <= ms[0] < 400 and all(0 < x < 50 for x in ms[1:])

@@ -228,3 +228,19 @@ def test_autotune_reports_a_table():
         assert t["ms"][b][t["shape"][b]] == min(t["ms"][b])
         ms8, ms11 = t["digit_ms"][b]
         assert t["digit_bits"][b] == (8 if b == 0 or ms8 <= ms11 else 11)
+
+
+def test_timing_of_batches_with_short_columns():
+    """timing_begin / timing_end record a batch of short and long columns, and of
+    short ones alone, as they do one of long columns."""
+    import torch
+    v = torch.arange(200_000, dtype=torch.int32, device="cuda:0") % 1000
+    with ia.Context(0) as c:
+        for cols in ([(0, 100_000)], [(0, 100_000), (100_000, 0)], [(0, 900), (1000, 5000)],
+                     [(i * 20, 20) for i in range(200)] + [(4000, 150_000)]):
+            c.build_batch_device(v, cols)
+            c.timing_begin(4)
+            for _ in range(2):
+                c.build_batch_device(v, cols)
+            ms, calls = c.timing_end()
+            assert calls == 2 and ms[0] > 0 and sum(ms) < 50
