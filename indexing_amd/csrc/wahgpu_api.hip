@@ -334,10 +334,18 @@ void set_one(BuildArgs* a, uint64_t n, uint32_t rid_base, bool wide = false) {
 
 // Scans keep their state in the context and take nothing from the arena, but a
 // fixed arena still bounds what a call on its context may ask for: bytes a scan
-// of n elements counts as, and the check.
+// of n elements counts as, and the check.  A growing arena gets its first 2 MB by
+// any call that is not captured: a build that is captured after it finds what it
+// needs for up to some 80000 rows, whichever call warmed the context up.
 uint64_t scan_scratch_bytes(uint64_t n) { return align_up(2080 + (n + 2047) / 2048 * 8); }
 int arena_limit(wahgpu_ctx* c, uint64_t bytes) {
-  if (!c->fixed || bytes <= c->arena_cap) return WAHGPU_OK;
+  if (bytes <= c->arena_cap) return WAHGPU_OK;
+  if (!c->fixed) {
+    if (c->arena_cap) return WAHGPU_OK;
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    HIPCHK(c, hipStreamIsCapturing(c->stream, &cs));
+    return cs == hipStreamCaptureStatusNone ? arena_reserve(c, 1) : WAHGPU_OK;
+  }
   return fail(c, WAHGPU_ENOMEM, "arena of " + std::to_string(c->arena_cap) +
                                     " bytes is too small for " + std::to_string(bytes));
 }

@@ -218,6 +218,11 @@ def test_range_on_a_fixed_arena_is_refused_before_it_decodes(lib, arena):
     c.close()
 
 
+def device_bytes(ctx):
+    """Device memory in use beside the context's arena."""
+    return ctx.lib.fake_device_bytes() - int(ctx.lib.wahgpu_arena_bytes(ctx.h))
+
+
 def launched(ctx):
     """Table entries and `grow` of the range launches so far."""
     lines = [x for x in ctx.log() if x.startswith("range")]
@@ -227,25 +232,25 @@ def launched(ctx):
 def test_range_table_is_bounded_by_what_ranges_need(ctx):
     """An index of many keys and rows: a query brings 8 MB whatever its range
     could need, and keeps more only for a range that decodes by it."""
-    start = ctx.lib.fake_device_bytes()
+    start = device_bytes(ctx)
     for extra in ((3, 100), (10**6, 5 * 10**7), (0, 0)):  # few words, few per key and slice, none
         ctx.script("range", extra=extra)
         assert query(ctx, keycnt=10**8, nrows=2**32) == OK
     assert launched(ctx) == [(2**20, 1)] * 3
-    assert ctx.lib.fake_device_bytes() - start == 8 << 20
+    assert device_bytes(ctx) - start == 8 << 20
 
 
 def test_range_comes_back_for_a_larger_table(ctx):
     nrows, keys = 2**24, 5000
     slices = 256  # one per CU up to 10240 chunks each
     words = 13 * keys * slices
-    start = ctx.lib.fake_device_bytes()
+    start = device_bytes(ctx)
     for _ in range(2):  # the launch that finds it too small, then the one that decodes
         ctx.script("range", extra=(keys, words))
     assert query(ctx, keycnt=2 * keys, nrows=nrows) == OK
     (first, grow), (second, again) = launched(ctx)
     assert (first, grow, again) == (2**20, 1, 0) and second >= 0.99 * keys * slices
-    held = ctx.lib.fake_device_bytes() - start
+    held = device_bytes(ctx) - start
     assert held == 8 * second < words  # 8 bytes for 13 words
     ctx.script("range", extra=(keys, words))  # the table is kept
     assert query(ctx, keycnt=2 * keys, nrows=nrows) == OK
@@ -277,9 +282,9 @@ def test_a_context_holds_status_words_for_what_it_scans(lib):
     assert c.call("stream_compaction", None, None, 2**30 - 1, None, ctypes.byref(out)) == OK
     assert c.call("decode_device", None, 2**29, 2**32, None, ctypes.byref(out)) == OK
     assert c.call("encode_device", None, 2**32, None, 100, ctypes.byref(out)) == OK
-    assert lib.fake_device_bytes() - start == held and len(states()) == 1
+    assert device_bytes(c) - start == held and len(states()) == 1
     assert c.call("decode_device", None, 2**29 + 1, 2**32, None, ctypes.byref(out)) == OK
-    assert lib.fake_device_bytes() - start == held + 8
+    assert device_bytes(c) - start == held + 8
     assert any(x.startswith("fill") and int(x.split("=")[1]) > 2**18 for x in c.log())
     for words in (2**29 + 4097, 2**33 - 2):  # found, then decoded
         at = len(launched(c))
@@ -289,7 +294,7 @@ def test_a_context_holds_status_words_for_what_it_scans(lib):
         most = [int(x.split("most=")[1].split()[0]) for x in c.log() if x.startswith("range")]
         assert most[at] < words <= most[at + 1]
     assert c.call("decode_device", None, 2**32, 2**32, None, ctypes.byref(out)) == OK
-    assert lib.fake_device_bytes() - start == held + 15 * 2**20  # 2^21 words in all
+    assert device_bytes(c) - start == held + 15 * 2**20  # 2^21 words in all
     c.close()
     assert lib.fake_device_bytes() == start
 
@@ -356,3 +361,28 @@ def test_timing_covers_batches_of_short_and_long_columns(ctx):
     assert ctx.call("timing_end", ms, ctypes.byref(calls)) == OK
     assert calls.value == 4
     assert 300 <= ms[0] < 400 and all(0 < x < 50 for x in ms[1:])
+
+
+def build_device(ctx, n):
+    return ctx.call("build_device", None, n, ctypes.c_uint32(0), None, None, None, None, None)
+
+
+@pytest.mark.parametrize("warm_up", ["build", "scan", "query"])
+def test_any_call_warms_up_for_a_captured_build(ctx, warm_up):
+    """A context's first call lays out 2 MB of arena, also one that needs none, so
+    that a column of 50000 rows can be captured next; a captured short column
+    needs no call before it and lays out nothing."""
+    stream = VP(ctx.lib.wahgpu_stream(ctx.h))
+    ctx.lib.fake_capture(stream, 1)
+    assert build_device(ctx, 1000) == OK and ctx.lib.wahgpu_arena_bytes(ctx.h) == 0
+    assert build_device(ctx, 50000) == EHIP  # the arena cannot grow in a capture
+    ctx.lib.fake_capture(stream, 0)
+    if warm_up == "build":
+        assert build_device(ctx, 1000) == OK
+    elif warm_up == "scan":
+        assert ctx.call("exclusive_scan", None, 1000, None) == OK
+    else:
+        assert query(ctx) == OK
+    ctx.lib.fake_capture(stream, 1)
+    assert build_device(ctx, 50000) == OK
+    ctx.lib.fake_capture(stream, 0)

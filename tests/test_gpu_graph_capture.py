@@ -90,3 +90,29 @@ def test_scan_replayed_beside_the_contexts_own_work(ctx, segmented):
         torch.cuda.synchronize()
         for got in (out, eager):
             assert np.array_equal(got.cpu().numpy().view(np.uint32), want)
+
+
+def test_a_short_column_warms_up_for_a_captured_longer_one():
+    """The first call sizes the arena for some 80000 rows, also where it needs
+    none itself."""
+    import torch
+    n = 50_000
+    inputs = [ia.generate(n, "uniform", seed=i, lo=0, hi=5000) for i in range(3)]
+    s = torch.cuda.Stream()
+    with ia.Context(0) as c:
+        d_in = dev(inputs[0])
+        out = tuple(torch.zeros(m, dtype=torch.int32, device="cuda:0") for m in (n, n, n, 2 * n, 16))
+        with torch.cuda.stream(s):
+            c.build_device(d_in[:1000])
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=s):
+            c.build_device(d_in, out=out)
+        for rep, v in enumerate(inputs):
+            d_in.copy_(dev(v))
+            torch.cuda.synchronize()
+            g.replay()
+            torch.cuda.synchronize()
+            cnt = c.read_counts(out[4])
+            assert cnt.fault == 0
+            assert_same(per_column(out, [cnt], [(0, n)])[0], oracle.build(v), f"replay {rep}")
