@@ -323,3 +323,89 @@ def test_streams_of_more_words_than_a_context_starts_with():
                                          0, 10, nrows)
             want = rows(at[at < half], second)
             assert m == 2 and np.array_equal(bitmap_rows(u32(bm), nrows), want[want < nrows])
+
+
+def long_stream(n, seed, odd):
+    """n words whose fills are short, so that their chunks fit a bit array."""
+    rng = np.random.default_rng(seed)
+    w = (rng.integers(0, 1 << 31, n) | 0x80000000).astype(np.uint32)
+    kind = rng.random(n)
+    w[kind < 0.3] = rng.integers(1, 4, n)[kind < 0.3]
+    if odd:
+        w[kind < 0.04] = 0x40000000 | rng.integers(0, 4, n)[kind < 0.04]  # 1-fills, some of nothing
+        w[(kind >= 0.04) & (kind < 0.06)] = 0
+        w[(kind >= 0.06) & (kind < 0.08)] = 0x80000000
+    return w
+
+
+def stream_bits(words):
+    """Rows of a stream as an array of bits, 31 per chunk."""
+    lit = (words >> 31) == 1
+    chunks = np.where(lit, 1, words & 0x3FFFFFFF).astype(np.int64)
+    start = np.cumsum(chunks) - chunks
+    payload = np.zeros(int(chunks.sum()), np.uint32)
+    payload[start[lit]] = words[lit] & 0x7FFFFFFF
+    ones = (words >> 30) == 1
+    edge = np.zeros(payload.size + 1, np.int64)
+    np.add.at(edge, start[ones], 1)
+    np.add.at(edge, (start + chunks)[ones], -1)
+    payload[np.cumsum(edge)[:-1] > 0] = 0x7FFFFFFF
+    bits = np.unpackbits(payload.view(np.uint8).reshape(-1, 4), axis=1, bitorder="little")
+    return bits[:, :31].reshape(-1)
+
+
+def pack(bits):
+    out = np.zeros((bits.size + 31) // 32 * 4, np.uint8)
+    out[:(bits.size + 7) // 8] = np.packbits(bits, bitorder="little")
+    return out.view(np.uint32)
+
+
+def canonical_of(bits):
+    """The words of an array of bits: a fill where chunks were skipped, then the
+    literal, per chunk with a row."""
+    chunks = np.zeros((bits.size + 30) // 31 * 31, np.uint8)
+    chunks[:bits.size] = bits
+    payload = np.zeros((chunks.size // 31, 32), np.uint8)
+    payload[:, :31] = chunks.reshape(-1, 31)
+    payload = np.packbits(payload, axis=1, bitorder="little").view(np.uint32).reshape(-1)
+    at = np.flatnonzero(payload)
+    fill = np.diff(at, prepend=-1) - 1
+    words = np.stack([fill.astype(np.uint32), payload[at] | np.uint32(0x80000000)], 1).reshape(-1)
+    return words[words != 0]
+
+
+@pytest.mark.parametrize("odd", [False, True], ids=["canonical", "odd"])
+def test_decode_of_more_tiles_than_blocks(ctx, odd):
+    """More tiles than a launch has blocks (512), so blocks draw theirs and the
+    look-back goes over many windows; twice, on the state the first left."""
+    words = long_stream(600 * 4096 + 77, 3 + odd, odd)
+    bits = stream_bits(words)
+    for nrows in (bits.size, bits.size // 2 + 5):
+        want, last = pack(bits[:nrows]), int(np.flatnonzero(bits)[-1]) + 1
+        for rep in range(2):
+            print(f"[decode] odd={odd} nrows={nrows} {rep}", flush=True)
+            bm, got = ctx.decode_device(dev(words, rep), nrows)
+            assert np.array_equal(u32(bm), want) and got == last
+
+
+@pytest.mark.parametrize("density", [0.0005, 0.02, 0.6])
+def test_encode_of_more_tiles_than_blocks(ctx, density):
+    n = 31 * 4096 * 1100 + 1234  # 1100 tiles and a part, 1024 blocks
+    bits = (np.random.default_rng(9).random(n, dtype=np.float32) < density).astype(np.uint8)
+    bits[n // 4:n // 4 + 31 * 4096 * 70] = 0  # more than a window of tiles without a row
+    want, bitmap = canonical_of(bits), dev(pack(bits))
+    for rep in range(2):
+        print(f"[encode] density={density} {rep}", flush=True)
+        assert np.array_equal(u32(ctx.encode_device(bitmap, n)), want)
+
+
+@pytest.mark.parametrize("op", ["and", "xor"])
+def test_combine_of_long_streams(ctx, op):
+    """The second stream's tiles start past the first look-back window, and both
+    streams' together are more than the blocks."""
+    a, b = long_stream(300 * 4096 + 5, 21, True), long_stream(280 * 4096 + 900, 22, False)
+    x, y = stream_bits(a), stream_bits(b)
+    n = min(x.size, y.size) - 7
+    want = canonical_of(x[:n] & y[:n] if op == "and" else x[:n] ^ y[:n])
+    for rep in range(2):
+        assert np.array_equal(u32(ctx.combine_device(op, dev(a), dev(b), n)), want)
