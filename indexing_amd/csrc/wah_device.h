@@ -58,11 +58,6 @@ __device__ __forceinline__ uint64_t shfl_up64(uint64_t x, int d) {
   uint32_t hi = __shfl_up((uint32_t)(x >> 32), d, kWave);
   return ((uint64_t)hi << 32) | lo;
 }
-__device__ __forceinline__ uint64_t shfl64(uint64_t x, int src) {
-  uint32_t lo = __shfl((uint32_t)x, src, kWave);
-  uint32_t hi = __shfl((uint32_t)(x >> 32), src, kWave);
-  return ((uint64_t)hi << 32) | lo;
-}
 
 // Tile scheduling for the single-pass kernels (wah_tiles.h has the rules; the
 // scans' own is in wah_scan.h).  Tiles are handed out by
@@ -101,21 +96,6 @@ __device__ __forceinline__ uint32_t next_tile(uint32_t* counters, uint32_t lanes
   __syncthreads();
   return *s_tile;
 #endif
-}
-
-// Asynchronous copy of 16 bytes per lane from global memory straight into
-// LDS (gfx950 global_load_lds_dwordx4): lane l's bytes land at
-// lds_wave_base + 16 * l.  The base must be the same for the whole wave.
-// Completion is tracked by vmcnt; see wait_vm().
-__device__ __forceinline__ void load_lds16(const void* g, uint32_t* lds_wave_base) {
-  __builtin_amdgcn_global_load_lds(g, (__attribute__((address_space(3))) void*)lds_wave_base,
-                                   16, 0, 0);
-}
-// s_waitcnt vmcnt(N) with lgkmcnt/expcnt left alone (gfx9 encoding).
-template <int N>
-__device__ __forceinline__ void wait_vm() {
-  static_assert(N >= 0 && N < 64, "vmcnt range");
-  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
 }
 
 // Inclusive uint32 prefix sum across the wave with DPP row shifts and row

@@ -106,12 +106,11 @@ __host__ __device__ constexpr int tail_waves_per_eu(int items) {
 constexpr uint32_t kHistMaxBlocks = 2048;
 // Tile counters: radix launches 0-3 of pair-mode columns, then their tail;
 // radix launches 0-3 of run-mode columns, then their tail.
-constexpr int kCounters = 14;
+constexpr int kCounters = 13;
 constexpr int kCounterTail = 4;
 constexpr int kCounterRun = 5;
 constexpr int kCounterRunTail = 9;
-constexpr int kCounterCut = 10;
-constexpr int kCounterWide = 11;  // wide-digit launches 0-2
+constexpr int kCounterWide = 10;  // wide-digit launches 0-2
 
 // Wide digits.  A pair-mode column whose keys take fewer passes of up to 11
 // bits than of 8 (9-11, 17-22 or 25-32 significant bits, trivial 8-bit

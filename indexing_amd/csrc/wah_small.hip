@@ -29,7 +29,7 @@ static_assert(kSmallMax == 16u * kThreads && 2 * kSmallMax < 65536, "16 rows a t
 struct SmallShared {
   // sort: keys, 16-bit rows, the waves' digit counts; then the index's words
   alignas(16) uint32_t raw[2 * kSmallMax];
-  uint32_t excl[256], dsum[4];
+  uint32_t dsum[4];
   uint32_t vary[kWaves16], vmax[kWaves16], runs[kWaves16], tot[kWaves16], ent[kWaves16];
 };
 
