@@ -29,7 +29,9 @@ constexpr int kDecRows = 2;
 constexpr uint32_t kDecTile = kScanTileOf<kDecRows>;  // words per decode tile
 // Resident blocks per CU.
 constexpr int kDecBlocks = 2;
-constexpr int kEncBlocks = 4;  // 20.2 us for 2^27 rows; 2 and 3 blocks 24.5, 23.1 us
+// 20.2 us for 2^27 rows, with 2 and 3 blocks 24.5 and 23.1 (timed with blocks that
+// took their first tile by index; 21.3 with all tiles drawn)
+constexpr int kEncBlocks = 4;
 static_assert(kDecTile == kDecodeTileWords, "what the host counts status words by");
 constexpr int query_waves_per_eu(int blocks) { return blocks * kScanWaves / 4; }
 
@@ -141,7 +143,7 @@ static_assert(kEnterTile >= kDecTile, "a range has no more of these");
 // the first chunk of its four words only, and looks for a slice's start among
 // all of their chunks at once; a tile in which no key starts, which is most of
 // them, skips everything about keys.
-// (54 MB of words take 31 us.)
+// (54 MB of words take 31 us, 35 as profiled.)
 __device__ __forceinline__ void enter_slices(const uint32_t* __restrict__ words,
                                              const uint32_t* __restrict__ offsets, uint32_t span,
                                              uint32_t slices, uint64_t* __restrict__ table,

@@ -14,14 +14,15 @@ namespace wah {
 
 namespace {
 
-// Rows per tile and blocks per CU of each kernel.  A launch has no more blocks
-// than the registers and LDS of a block let the device hold at once.  What a
-// tile costs besides its bytes is one look-back (its wait is for the tiles just
-// before it), so the largest tiles that leave two blocks per CU are the fastest: 2^24 elements, 16384-element tiles at two blocks
-// per CU against 8192 at four and 4096 at four: scan 31.7 / 35.8 / 46.9 us,
-// compaction 40.2 / 42.6 / 51.4 us, fuse (half the elements) 20.6 / 22.7 /
-// 28.9 us on 2^22.  The segmented scan and the column lengths hold more
-// registers per row and gain nothing from a larger tile (39.4 and 16.6 us).
+// Rows per tile and blocks per CU of each kernel. A launch has no more blocks
+// than the registers and LDS of a block let the device hold at once. What a tile
+// costs besides its bytes is one look-back (its wait is for the tiles just
+// before it), so the largest tiles that leave two blocks per CU are the fastest:
+// 2^24 elements, 16384-element tiles at two blocks per CU against 8192 at four
+// and 4096 at four: scan 31.7 / 35.8 / 46.9 us, compaction 40.2 / 42.6 / 51.4
+// us, fuse (half the elements) 20.6 / 22.7 / 28.9 us on 2^22 (timed with blocks
+// that took their first tile by index). The segmented scan and the column
+// lengths hold more registers per row and gain nothing from a larger tile.
 constexpr int kScanRows = 8, kCompactRows = 8, kFuseRows = 4, kSegRows = 4, kMergeRows = 4,
               kColenRows = 4;
 constexpr int kScanBlocks = 2;
@@ -44,7 +45,7 @@ __device__ __forceinline__ uint32_t waves_before(const uint32_t* s_tot, int w, u
 }  // namespace
 
 // Exclusive uint32 sum scan (include/scan.cl), wrapping mod 2^32.  2^24
-// elements: 31.7 us (4.2 TB/s); 184 us as one look-back thread per tile of
+// elements: 34.5 us (3.9 TB/s); 184 us as one look-back thread per tile of
 // 2048 elements and lanes that load 8 consecutive ones.
 template <int ROWS>
 __global__ __launch_bounds__(kScanThreads, waves_per_eu(kScanBlocks)) void k_scan(
@@ -105,7 +106,7 @@ __global__ __launch_bounds__(kScanThreads, waves_per_eu(kScanBlocks)) void k_sca
 // of a scan whose every step selects.  Elements of a segment that began before
 // the wave are "open" and take the carry once it is known.  A tile with a head
 // publishes its last segment's sum as a prefix at once: later tiles need
-// nothing from before it.  2^24 elements: 39.4 us (5.1 TB/s; was 230 us).
+// nothing from before it.  2^24 elements: 41.6 us (4.8 TB/s; was 230 us).
 __global__ __launch_bounds__(kScanThreads, waves_per_eu(kScanBlocks)) void k_segscan(
     const uint32_t* in, const uint32_t* heads, uint64_t n, uint32_t* out, ScanState* st,
     uint64_t* status, uint32_t tiles, uint64_t* kept) {
@@ -215,7 +216,7 @@ __global__ __launch_bounds__(kScanThreads, waves_per_eu(kScanBlocks)) void k_seg
 // (a[i], b[i]) with zero words dropped (fuse_fill_literals); half the
 // elements per tile, since each may leave two words.  The kept words are
 // placed in LDS by a scan of the lanes' counts and stored contiguously.  2^24
-// elements, half kept: 40 us (4.2 TB/s; was 204 us); 2^22 entries fused: 21 us
+// elements, half kept: 42 us (4.0 TB/s; was 204 us); 2^22 entries fused: 21 us
 // (3.2 TB/s; was 85 us).
 template <int ROWS, bool FUSE>
 __global__ __launch_bounds__(kScanThreads, waves_per_eu(kScanBlocks)) void k_compact(
@@ -292,7 +293,7 @@ __global__ __launch_bounds__(kScanThreads, waves_per_eu(kScanBlocks)) void k_com
 // along the lane's four elements, then across lanes with DPP steps that stop
 // at the lane of the nearest head, then across waves and tiles by carries.
 // The three output arrays leave through one LDS buffer, one after another.
-// 2^22 pairs: 29 us (3.5 TB/s; was 124 us with a 64-bit scan operator over
+// 2^22 pairs: 32 us (3.2 TB/s; was 124 us with a 64-bit scan operator over
 // shuffles, three reads of the inputs and one look-back thread).
 __global__ __launch_bounds__(kScanThreads, waves_per_eu(kScanBlocks)) void k_merge(
     const uint32_t* __restrict__ vals, const uint32_t* __restrict__ chids,

@@ -44,7 +44,9 @@ constexpr uint32_t tile_group(uint32_t tiles, uint32_t grid, uint32_t lanes, uin
 // that saves the smallest calls two draws.  With more tiles than blocks every
 // tile, a block's first one too, is drawn: a block that stays for another tile
 // then never waits for a tile that belongs to a block without a place, which
-// work on another stream may withhold for as long as it runs.
+// work on another stream may withhold for as long as it runs.  (That draw costs
+// the encode of 2^27 rows, 1058 tiles, 18.7 -> 21.3 us and three primitives of
+// 2^24 elements 144 -> 148; the next tile drawn ahead of its use 24 and 154.)
 constexpr bool scan_draws(uint32_t tiles, uint32_t grid) { return tiles > grid; }
 
 // Polls of a look-back wait that see nothing new before it gives up.

@@ -404,7 +404,8 @@ int wait_stream(wahgpu_ctx* c) {
     *kept = 0;
     reset_scan_state(c);
     return fail(c, WAHGPU_EHIP, "an earlier exclusive or segmented scan reported fault " +
-                                    std::to_string(f) + " (look-back wait gave up); its sums are wrong");
+                                    std::to_string(f) +
+                                    " (look-back wait gave up); its sums are wrong");
   }
   return WAHGPU_OK;
 }
