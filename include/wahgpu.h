@@ -444,7 +444,9 @@ int wahgpu_decode_device(wahgpu_ctx* ctx, const uint32_t* d_words, uint64_t len,
 
 /* Range query on an equality index (keys ascending; offsets, lengths and
  * words as a build writes them): d_bitmap = OR of the row bitmaps of every
- * key in [lo, hi].  *keys_matched (may be NULL) = keys in the range. */
+ * key in [lo, hi].  *keys_matched (may be NULL) = keys in the range.  A range
+ * whose offsets descend (WAHGPU_EINVAL), or whose words are more than a fixed
+ * arena allows (WAHGPU_ENOMEM), leaves the bitmap empty. */
 int wahgpu_query_range_device(wahgpu_ctx* ctx, const uint32_t* d_keys,
                               const uint32_t* d_offsets, const uint32_t* d_lengths,
                               uint64_t keycnt, const uint32_t* d_words, uint32_t lo,
