@@ -123,7 +123,8 @@ class DeviceOrder {
     slot_->mu.lock();
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     st_ = hipStreamIsCapturing(c->stream, &cs);
-    if (st_ != hipSuccess || cs != hipStreamCaptureStatusNone) return;
+    captured_ = cs != hipStreamCaptureStatusNone;
+    if (st_ != hipSuccess || captured_) return;
     if (!slot_->last) st_ = hipEventCreateWithFlags(&slot_->last, hipEventDisableTiming);
     if (st_ == hipSuccess) st_ = hipStreamWaitEvent(c->stream, slot_->last, 0);
     record_ = st_ == hipSuccess;
@@ -141,12 +142,14 @@ class DeviceOrder {
   DeviceOrder(const DeviceOrder&) = delete;
   DeviceOrder& operator=(const DeviceOrder&) = delete;
   hipError_t status() const { return st_; }
+  bool captured() const { return captured_; }  // into a graph: not ordered
 
  private:
   wahgpu_ctx* c_;
   OrderSlot* slot_ = nullptr;
   hipError_t st_ = hipSuccess;
   bool record_ = false;
+  bool captured_ = false;
 };
 
 #define ORDERED(ctx)                  \
@@ -431,18 +434,16 @@ ScanRun scan_run(wahgpu_ctx* c, bool launched) {
   return ScanRun{c->scan_state, reinterpret_cast<uint64_t*>(c->scan_state + 1), c->scan_host,
                  c->scan_host + kKeptSlot, c->cus, false};
 }
-// The same for a scan that nobody waits for; one that its stream captures takes
-// the graphs' state.
-int scan_run_async(wahgpu_ctx* c, ScanRun* run) {
-  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-  HIPCHK(c, hipStreamIsCapturing(c->stream, &cs));
-  *run = scan_run(c, false);
-  if (cs != hipStreamCaptureStatusNone) {
-    run->state = c->graph_state;
-    run->status = reinterpret_cast<uint64_t*>(c->graph_state + 1);
-    run->captured = true;
+// The same for a scan that nobody waits for; a captured one takes the graphs'
+// state.
+ScanRun scan_run_async(wahgpu_ctx* c, bool captured) {
+  ScanRun run = scan_run(c, false);
+  if (captured) {
+    run.state = c->graph_state;
+    run.status = reinterpret_cast<uint64_t*>(c->graph_state + 1);
+    run.captured = true;
   }
-  return WAHGPU_OK;
+  return run;
 }
 // Waits for the stream and reads the result of the scan that wrote `slot`.
 int scan_result(wahgpu_ctx* c, uint64_t* out, int slot = 0) {
@@ -1718,10 +1719,8 @@ int wahgpu_exclusive_scan(wahgpu_ctx* c, const uint32_t* d_in, uint64_t n, uint3
   rc = arena_limit(c, scan_scratch_bytes(n));
   if (rc) return rc;
   ORDERED(c);
-  ScanRun run;
-  rc = scan_run_async(c, &run);
-  if (rc) return rc;
-  wah::launch_scan(run, d_in, nullptr, n, d_out, false, c->stream);
+  wah::launch_scan(scan_run_async(c, order_guard_.captured()), d_in, nullptr, n, d_out, false,
+                   c->stream);
   LAUNCHCHK(c);
   return WAHGPU_OK;
 }
@@ -1736,10 +1735,8 @@ int wahgpu_segmented_inclusive_scan(wahgpu_ctx* c, const uint32_t* d_in, const u
   rc = arena_limit(c, scan_scratch_bytes(n));
   if (rc) return rc;
   ORDERED(c);
-  ScanRun run;
-  rc = scan_run_async(c, &run);
-  if (rc) return rc;
-  wah::launch_scan(run, d_in, d_heads, n, d_out, true, c->stream);
+  wah::launch_scan(scan_run_async(c, order_guard_.captured()), d_in, d_heads, n, d_out, true,
+                   c->stream);
   LAUNCHCHK(c);
   return WAHGPU_OK;
 }
